@@ -73,6 +73,9 @@ SIGNATURES = {
     "pa_mlp_bias_grad": (i32, [i32, i32, vp, vp, vp]),
     "pa_mlp_head_loss": (i32, [i32, i32, vp, vp, vp, f32, f32, vp, vp, vp]),
     "pa_mlp_adam": (i32, [i32, vp, vp, vp, vp, f32, f32, f32, f32, i32, vp]),
+    "pa_mlp_loss_grads_scratch": (i64, [i32, vp, i32]),
+    "pa_mlp_loss_grads": (i32, [i32, vp, i32, vp, vp, vp, vp, f32, f32, vp, vp, vp, vp]),
+    "pa_mlp_adam_multi": (i32, [i32, vp, vp, vp, vp, vp, f32, f32, f32, f32, i32, vp]),
     "pa_mlp_to_bf16": (i32, [i64, vp, vp, vp]),
     "pa_mlp_layer_bf16": (i32, [i32, i32, i32, vp, vp, vp, vp, i32, vp]),
 }
@@ -118,6 +121,15 @@ def ptr(t) -> Optional[int]:
     if t is None:
         return None
     return t.data_ptr()
+
+
+def ptr_array(tensors) -> C.Array:
+    """Host array of the tensors' device pointers."""
+    return (vp * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def int_array(values) -> C.Array:
+    return (i32 * len(values))(*values)
 
 
 def stream_handle() -> Optional[int]:

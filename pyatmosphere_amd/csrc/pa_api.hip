@@ -4,6 +4,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <climits>
+
 #include "pa_internal.h"
 
 namespace pa {
@@ -71,6 +73,12 @@ int mlp_head_loss(int M, int NB, const float* out, const float* target, const fl
                   float* loss, float* dout, hipStream_t s);
 int mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, float b1, float b2, float eps,
              int t, hipStream_t s);
+long long mlp_loss_grads_scratch(int layers, const int* sizes, int M);
+int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
+                   const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
+                   float* scratch, hipStream_t s);
+int mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
+                   float* const* v, float lr, float b1, float b2, float eps, int t, hipStream_t s);
 int mlp_to_bf16(long long n, const float* x, unsigned short* y, hipStream_t s);
 int mlp_layer_bf16(int M, int N, int K, const float* X, const unsigned short* W, const float* bias, float* Y,
                    int act, hipStream_t s);
@@ -364,6 +372,32 @@ int pa_mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, f
                 int t, void* stream) {
   REQUIRE(n > 0 && w && g && m && v && t >= 1, "mlp_adam: bad argument");
   return mlp_adam(n, w, g, m, v, lr, b1, b2, eps, t, STREAM(stream));
+}
+static bool mlp_sizes_ok(int layers, const int* sizes, int M) {
+  if (!sizes || layers < 1 || layers > kMlpMaxLayers || M < 1) return false;
+  for (int i = 0; i <= layers; ++i)
+    if (sizes[i] < 1) return false;
+  return sizes[layers] >= 2 && sizes[layers] <= 65;
+}
+long long pa_mlp_loss_grads_scratch(int layers, const int* sizes, int M) {
+  REQUIRE(mlp_sizes_ok(layers, sizes, M), "mlp_loss_grads: bad layer sizes or batch");
+  return mlp_loss_grads_scratch(layers, sizes, M);
+}
+int pa_mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
+                      const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
+                      void* scratch, void* stream) {
+  REQUIRE(mlp_sizes_ok(layers, sizes, M), "mlp_loss_grads: bad layer sizes or batch");
+  REQUIRE(X && params && target && tvar && loss && grads && scratch, "mlp_loss_grads: null pointer");
+  for (int i = 0; i < 2 * layers; ++i) REQUIRE(params[i] && grads[i], "mlp_loss_grads: null pointer");
+  return mlp_loss_grads(layers, sizes, M, X, params, target, tvar, wv, wc, loss, grads,
+                        reinterpret_cast<float*>(scratch), STREAM(stream));
+}
+int pa_mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
+                      float* const* v, float lr, float b1, float b2, float eps, int t, void* stream) {
+  REQUIRE(count > 0 && n && w && g && m && v && t >= 1, "mlp_adam_multi: bad argument");
+  for (int i = 0; i < count; ++i)
+    REQUIRE(n[i] > 0 && n[i] <= INT_MAX - 1024 && w[i] && g[i] && m[i] && v[i], "mlp_adam_multi: bad tensor");
+  return mlp_adam_multi(count, n, w, g, m, v, lr, b1, b2, eps, t, STREAM(stream));
 }
 int pa_mlp_to_bf16(long long n, const float* x, void* y, void* stream) {
   REQUIRE(n > 0 && x && y, "mlp_to_bf16: bad argument");

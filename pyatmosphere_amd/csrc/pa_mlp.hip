@@ -1,7 +1,6 @@
 // Kernels of the transmittance-PDT surrogate: a small MLP trained and evaluated
-// on the device.  Training runs in float32 (LDS-tiled GEMMs on the vector
-// units, which are exact enough for gradient checks against a float64 host
-// MLP); inference GEMMs run on bf16 MFMA with float32 accumulation and fused
+// on the device.  Training runs in float32 (float32 MFMA products, exact enough
+// for gradient checks against a float64 host MLP); inference GEMMs run on bf16 MFMA with float32 accumulation and fused
 // bias + activation.  Activation: SiLU, z * sigmoid(z).  Output head: NB
 // logits (softmax PDT over NB transmittance bins) and one log-variance.
 #include "pa_internal.h"
@@ -13,56 +12,120 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 typedef unsigned short us8 __attribute__((ext_vector_type(8)));
 
 // ------------------------------------------------------------------ fp32 GEMM
-// C[M][N] = alpha * op(A) op(B) + beta * C, row-major, op = transpose when t* != 0:
-// op(A) is M x K (A is M x K, or K x M when ta), op(B) is K x N (B is K x N, or N x K when tb).
-constexpr int GT = 64, GK = 16;
+// C[M][N] = op(A) op(B), row-major, op = transpose when t* is set: op(A) is M x K
+// (A is M x K, or K x M when TA), op(B) is K x N (B is K x N, or N x K when TB).
+//
+// The training shapes (1024 x 384 x 384 and the like) are small: what bounds
+// them is latency, not the 2 GFLOP of a step (13 us at the float32 matrix
+// rate).  One block owns one 32 x 32 tile of C and its WK waves split K, so a
+// 384-deep product is 12 loads deep per wave and a 384 x 384 weight gradient
+// still gives 144 blocks of 16 waves; the waves' partial tiles are added in LDS
+// in wave order (deterministic).  Operands go from L2 straight to registers
+// on v_mfma_f32_32x32x2f32 (float32 products and sums): lane l supplies row
+// (column) l % 32 at k = k0 + 4 (l / 32) + i for i = 0..3, so an operand whose
+// K is contiguous is read as one float4 per lane and 8 k (VA / VB), and one
+// whose rows are contiguous as four coalesced dwords.  Rows past M and columns
+// past N repeat the last one (their results are not stored); k past the end
+// is zero in both operands.
+// Measured, a 1024-pair step of the 384-wide network (loss, gradients, Adam):
+// 1856 us with 64 x 64 LDS tiles on the vector units (94 us a product, 36 to 96
+// blocks), serial column sums for db (194 us) and a launch per pass and tensor;
+// 94 us with these kernels (10-12 us a product, 21 us for all weight gradients).
+typedef float f16v __attribute__((ext_vector_type(16)));
+constexpr int GT = 32;             // C tile
+constexpr int GU = 4;              // groups of 8 k in flight per wave
 
-__global__ void __launch_bounds__(256)
-k_gemm_f32(int M, int N, int K, const float* __restrict__ A, int lda, int ta, const float* __restrict__ B,
-           int ldb, int tb, float* __restrict__ C, int ldc, float alpha, float beta) {
-  __shared__ float sa[GK][GT + 4];
-  __shared__ float sb[GK][GT + 4];
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += GK) {
-    for (int i = threadIdx.x; i < GK * GT; i += 256) {
-      const int kk = i / GT, mm = i % GT;
-      const int m = m0 + mm, k = k0 + kk;
-      float va = 0.f;
-      if (m < M && k < K) va = ta ? A[(size_t)k * lda + m] : A[(size_t)m * lda + k];
-      sa[kk][mm] = va;
-      const int n = n0 + mm;
-      float vb = 0.f;
-      if (n < N && k < K) vb = tb ? B[(size_t)n * ldb + k] : B[(size_t)k * ldb + n];
-      sb[kk][mm] = vb;
+template <bool T, bool VEC>
+__device__ __forceinline__ void gemm_load(float (&x)[4], const float* __restrict__ P, int ld, int row, int k, int kend) {
+  // T: element (row, k) at P[k ld + row], else P[row ld + k]
+  if constexpr (!T && VEC) {
+    const int kk = min(k, kend - 4);
+    const f4v v = *reinterpret_cast<const f4v*>(P + (size_t)row * ld + kk);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = k < kend ? v[i] : 0.f;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int kk = min(k + i, kend - 1);
+      const float v = T ? P[(size_t)kk * ld + row] : P[(size_t)row * ld + kk];
+      x[i] = k + i < kend ? v : 0.f;
     }
-    __syncthreads();
+  }
+}
+
+// The sum of the tile at (m0, n0) over K into red[0 .. WK) (32 x 32 partial
+// tiles, row stride 33).  With SUMA, rs[wave][row] receives the wave's sums of
+// op(A)'s rows over K.  Ends with a barrier.
+template <int WK, bool TA, bool TB, bool VA, bool VB, bool SUMA>
+__device__ __forceinline__ void gemm_tile32(int M, int N, int K, int m0, int n0, const float* __restrict__ A, int lda,
+                                            const float* __restrict__ B, int ldb, float* red, float* rs) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
+  const int row = min(m0 + r, M - 1), col = min(n0 + r, N - 1);
+  const int per = ((K + 7) / 8 + WK - 1) / WK * 8;       // k per wave, a multiple of 8
+  const int kb = wave * per, ke = min(K, kb + per);
+  f16v acc;
 #pragma unroll
-    for (int kk = 0; kk < GK; ++kk) {
-      float a[4], b[4];
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  float sum = 0.f;
+  if (kb < ke) {
+    float a[GU][4], b[GU][4];
+    auto fetch = [&](int k0) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = sa[kk][ty * 4 + i];
+      for (int u = 0; u < GU; ++u) {
+        gemm_load<TA, VA>(a[u], A, lda, row, k0 + 8 * u + 4 * h, ke);
+        gemm_load<!TB, VB>(b[u], B, ldb, col, k0 + 8 * u + 4 * h, ke);
+      }
+    };
+    fetch(kb);
+    for (int k0 = kb; k0 < ke; k0 += 8 * GU) {
+      float ca[GU][4], cb[GU][4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = sb[kk][tx * 4 + j];
+      for (int u = 0; u < GU; ++u)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+          ca[u][i] = a[u][i];
+          cb[u][i] = b[u][i];
+        }
+      if (k0 + 8 * GU < ke) fetch(k0 + 8 * GU);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+      for (int u = 0; u < GU; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ca[u][i], cb[u][i], acc, 0, 0, 0);
+          if constexpr (SUMA) sum += ca[u][i];
+        }
     }
-    __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
+  for (int v = 0; v < 16; ++v) red[wave * (GT * 33) + (8 * (v / 4) + 4 * h + v % 4) * 33 + r] = acc[v];
+  if constexpr (SUMA) {
+    sum += __shfl_xor(sum, 32, 64);
+    if (h == 0) rs[wave * GT + r] = sum;
+  }
+  __syncthreads();
+}
+
+template <int WK>
+__device__ __forceinline__ float gemm_sum(const float* red, int r, int c) {
+  float s = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float* c = C + (size_t)m * ldc + n;
-      *c = alpha * acc[i][j] + (beta != 0.f ? beta * *c : 0.f);
-    }
+  for (int w = 0; w < WK; ++w) s += red[w * (GT * 33) + r * 33 + c];
+  return s;
+}
+
+constexpr int kGemmWaves = 4;
+template <bool TA, bool TB, bool VA, bool VB>
+__global__ void __launch_bounds__(64 * kGemmWaves)
+k_gemm_f32(int M, int N, int K, const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb,
+           float* __restrict__ C, int ldc, float alpha, float beta) {
+  __shared__ float red[kGemmWaves * GT * 33];
+  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
+  gemm_tile32<kGemmWaves, TA, TB, VA, VB, false>(M, N, K, m0, n0, A, lda, B, ldb, red, nullptr);
+  for (int e = threadIdx.x; e < GT * GT; e += 64 * kGemmWaves) {
+    const int r = e / GT, c = e % GT;
+    if (m0 + r >= M || n0 + c >= N) continue;
+    float* o = C + (size_t)(m0 + r) * ldc + n0 + c;
+    *o = alpha * gemm_sum<kGemmWaves>(red, r, c) + (beta != 0.f ? beta * *o : 0.f);
   }
 }
 
@@ -96,6 +159,76 @@ __global__ void k_bias_grad(int M, int N, const float* __restrict__ dZ, float* _
   for (int m = 0; m < M; ++m) s += dZ[(size_t)m * N + n];
   db[n] = s;
 }
+
+// Z = X W^T + bias and (Y non-null) Y = SiLU(Z) of one layer, X M x K, W N x K:
+// the bias and the activation ride on the product's epilogue instead of two
+// more passes over the M x N values.
+template <bool VEC>
+__global__ void __launch_bounds__(64 * kGemmWaves)
+k_layer_forward(int M, int N, int K, const float* __restrict__ X, const float* __restrict__ W,
+                const float* __restrict__ bias, float* __restrict__ Z, float* __restrict__ Y) {
+  __shared__ float red[kGemmWaves * GT * 33];
+  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
+  gemm_tile32<kGemmWaves, false, true, VEC, VEC, false>(M, N, K, m0, n0, X, K, W, K, red, nullptr);
+  for (int e = threadIdx.x; e < GT * GT; e += 64 * kGemmWaves) {
+    const int r = e / GT, c = e % GT;
+    if (m0 + r >= M || n0 + c >= N) continue;
+    const float z = gemm_sum<kGemmWaves>(red, r, c) + bias[n0 + c];
+    const size_t o = (size_t)(m0 + r) * N + n0 + c;
+    Z[o] = z;
+    if (Y) Y[o] = z * sigm(z);
+  }
+}
+
+// dZ = (D W) * SiLU'(Z) of the layer below: D M x K (this layer's dZ), W K x N,
+// Z the lower layer's M x N pre-activations.
+template <bool VEC>
+__global__ void __launch_bounds__(64 * kGemmWaves)
+k_layer_backward(int M, int N, int K, const float* __restrict__ D, const float* __restrict__ W,
+                 const float* __restrict__ Z, float* __restrict__ dZ) {
+  __shared__ float red[kGemmWaves * GT * 33];
+  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
+  gemm_tile32<kGemmWaves, false, false, VEC, false, false>(M, N, K, m0, n0, D, K, W, N, red, nullptr);
+  for (int e = threadIdx.x; e < GT * GT; e += 64 * kGemmWaves) {
+    const int r = e / GT, c = e % GT;
+    if (m0 + r >= M || n0 + c >= N) continue;
+    const size_t o = (size_t)(m0 + r) * N + n0 + c;
+    const float z = Z[o], s = sigm(z);
+    dZ[o] = gemm_sum<kGemmWaves>(red, r, c) * s * (1.f + z * (1.f - s));
+  }
+}
+
+// Every layer's dW = D^T H (fo x fi over K = M rows) and db = column sums of D
+// in one launch: the products do not depend on each other, and together they
+// fill the chip (336 tiles of 16 waves for the 16-384-384-384-65 network).
+constexpr int kGradLayers = 8;      // layers per launch
+constexpr int kGradWaves = 16;
+struct GradLayers {
+  const float* d[kGradLayers];
+  const float* h[kGradLayers];
+  float* dw[kGradLayers];
+  float* db[kGradLayers];
+  int fo[kGradLayers], fi[kGradLayers], first[kGradLayers + 1];   // first: tiles before this layer
+};
+__global__ void __launch_bounds__(64 * kGradWaves)
+k_weight_grads(int layers, int M, GradLayers g) {
+  __shared__ float red[kGradWaves * GT * 33];
+  __shared__ float rs[kGradWaves * GT];
+  int i = 0;
+  while (i + 1 < layers && (int)blockIdx.x >= g.first[i + 1]) ++i;
+  const int fo = g.fo[i], fi = g.fi[i], nx = (fi + GT - 1) / GT, tile = blockIdx.x - g.first[i];
+  const int m0 = tile / nx * GT, n0 = tile % nx * GT;
+  gemm_tile32<kGradWaves, true, false, false, false, true>(fo, fi, M, m0, n0, g.d[i], fo, g.h[i], fi, red, rs);
+  const int r = threadIdx.x / GT, c = threadIdx.x % GT;
+  if (m0 + r < fo && n0 + c < fi) g.dw[i][(size_t)(m0 + r) * fi + n0 + c] = gemm_sum<kGradWaves>(red, r, c);
+  if (n0 == 0 && threadIdx.x < GT && m0 + (int)threadIdx.x < fo) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kGradWaves; ++w) s += rs[w * GT + threadIdx.x];
+    g.db[i][m0 + threadIdx.x] = s;
+  }
+}
+static_assert(GT * GT == 64 * kGradWaves, "one thread per element of the tile");
 
 // Head: row m of out holds NB logits and one log-variance.  Loss per row:
 //   -sum_j t_j log p_j + wc sum_j (P_j - T_j)^2 + wv (lv - tv)^2
@@ -150,16 +283,44 @@ k_head_loss(int M, int NB, const float* __restrict__ out, const float* __restric
 }
 
 // Adam with bias correction; w, m, v float32.
-__global__ void k_adam(int n, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+__device__ __forceinline__ void adam_update(int i, float* __restrict__ w, const float* __restrict__ g,
+                                            float* __restrict__ m, float* __restrict__ v, float lr, float b1,
+                                            float b2, float eps, float c1, float c2) {
   const float gi = g[i];
   const float mi = b1 * m[i] + (1.f - b1) * gi;
   const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
   w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+}
+
+__global__ void k_adam(int n, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
+                       float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) adam_update(i, w, g, m, v, lr, b1, b2, eps, c1, c2);
+}
+
+// The same update of several tensors in one launch (kAdamPer values per block).
+constexpr int kAdamTensors = 16, kAdamPer = 1024;
+struct AdamTensors {
+  float* w[kAdamTensors];
+  const float* g[kAdamTensors];
+  float* m[kAdamTensors];
+  float* v[kAdamTensors];
+  int n[kAdamTensors], first[kAdamTensors];   // first: blocks before this tensor
+};
+__global__ void __launch_bounds__(256)
+k_adam_multi(int count, AdamTensors a, float lr, float b1, float b2, float eps, float c1, float c2) {
+  int t = 0;
+  while (t + 1 < count && (int)blockIdx.x >= a.first[t + 1]) ++t;
+  const int base = (blockIdx.x - a.first[t]) * kAdamPer + threadIdx.x;
+  float *w = a.w[t], *m = a.m[t], *v = a.v[t];
+  const float* g = a.g[t];
+#pragma unroll
+  for (int j = 0; j < kAdamPer / 256; ++j) {
+    const int i = base + 256 * j;
+    if (i < a.n[t]) adam_update(i, w, g, m, v, lr, b1, b2, eps, c1, c2);
+  }
 }
 
 __device__ __forceinline__ unsigned short f2bf(float f) {
@@ -183,7 +344,6 @@ k_layer_bf16(int M, int N, int K, const float* __restrict__ X, const unsigned sh
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 128 + wave * 32;
   if (n0 >= N) return;
-  typedef float f16v __attribute__((ext_vector_type(16)));
   f16v acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
@@ -210,11 +370,127 @@ k_layer_bf16(int M, int N, int K, const float* __restrict__ X, const unsigned sh
 }
 
 // ------------------------------------------------------------------ launchers
+// float4 reads of an operand whose K is contiguous need whole quads of k at 16-byte addresses
+static bool quads(const float* p, int ld, int K) {
+  return K % 4 == 0 && ld % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+}
+
 int mlp_gemm_f32(int M, int N, int K, const float* A, int lda, int ta, const float* B, int ldb, int tb, float* C,
                  int ldc, float alpha, float beta, hipStream_t s) {
-  dim3 g((N + GT - 1) / GT, (M + GT - 1) / GT);
-  hipLaunchKernelGGL(k_gemm_f32, g, dim3(256), 0, s, M, N, K, A, lda, ta, B, ldb, tb, C, ldc, alpha, beta);
+  const dim3 g((N + GT - 1) / GT, (M + GT - 1) / GT);
+  const bool va = !ta && quads(A, lda, K), vb = tb && quads(B, ldb, K);
+#define G_(TA, TB, VA, VB)                                                                                      \
+  hipLaunchKernelGGL((k_gemm_f32<TA, TB, VA, VB>), g, dim3(64 * kGemmWaves), 0, s, M, N, K, A, lda, B, ldb, C, \
+                     ldc, alpha, beta)
+  if (ta && tb) {
+    if (vb) G_(true, true, false, true);
+    else G_(true, true, false, false);
+  } else if (ta) {
+    G_(true, false, false, false);
+  } else if (tb) {
+    if (va && vb) G_(false, true, true, true);
+    else G_(false, true, false, false);
+  } else {
+    if (va) G_(false, false, true, false);
+    else G_(false, false, false, false);
+  }
+#undef G_
   return check_launch("mlp_gemm_f32");
+}
+
+// Floats of scratch for mlp_loss_grads: per layer Z and dZ (M x fo), and Y for
+// the hidden ones; each starts at a multiple of 4 floats.
+static size_t padded(size_t n) { return (n + 3) / 4 * 4; }
+long long mlp_loss_grads_scratch(int layers, const int* sizes, int M) {
+  size_t n = 0;
+  for (int i = 0; i < layers; ++i) n += (i < layers - 1 ? 3 : 2) * padded((size_t)M * sizes[i + 1]);
+  return (long long)(n * sizeof(float));
+}
+
+int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
+                   const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
+                   float* scratch, hipStream_t s) {
+  const int NB = sizes[layers] - 1;
+  // scratch: every layer's Z, then every layer's dZ, then the hidden layers' Y
+  size_t all = 0;
+  for (int i = 0; i < layers; ++i) all += padded((size_t)M * sizes[i + 1]);
+  const float* h = X;
+  float *z = scratch, *d = scratch + all, *y = scratch + 2 * all;
+  for (int i = 0; i < layers; ++i) {
+    const int fi = sizes[i], fo = sizes[i + 1];
+    const dim3 g((fo + GT - 1) / GT, (M + GT - 1) / GT);
+    const float* W = params[2 * i];
+    float* Y = i < layers - 1 ? y : nullptr;
+    if (quads(h, fi, fi) && quads(W, fi, fi))
+      hipLaunchKernelGGL(k_layer_forward<true>, g, dim3(64 * kGemmWaves), 0, s, M, fo, fi, h, W, params[2 * i + 1], z, Y);
+    else
+      hipLaunchKernelGGL(k_layer_forward<false>, g, dim3(64 * kGemmWaves), 0, s, M, fo, fi, h, W, params[2 * i + 1], z, Y);
+    if (i < layers - 1) {
+      h = y;
+      y += padded((size_t)M * fo);
+      z += padded((size_t)M * fo);
+      d += padded((size_t)M * fo);
+    }
+  }
+  // z, d: the last layer's
+  hipLaunchKernelGGL(k_head_loss, dim3(M), dim3(64), 0, s, M, NB, z, target, tvar, wv, wc, loss, d);
+  const float* dl[kMlpMaxLayers];
+  const float* hl[kMlpMaxLayers];
+  for (int i = layers - 1; i >= 0; --i) {
+    const int fi = sizes[i], fo = sizes[i + 1];
+    dl[i] = d;
+    if (i > 0) {
+      y -= padded((size_t)M * fi);
+      z -= padded((size_t)M * fi);
+      float* dn = d - padded((size_t)M * fi);
+      hl[i] = y;
+      const dim3 g((fi + GT - 1) / GT, (M + GT - 1) / GT);
+      if (quads(d, fo, fo))
+        hipLaunchKernelGGL(k_layer_backward<true>, g, dim3(64 * kGemmWaves), 0, s, M, fi, fo, d, params[2 * i], z, dn);
+      else
+        hipLaunchKernelGGL(k_layer_backward<false>, g, dim3(64 * kGemmWaves), 0, s, M, fi, fo, d, params[2 * i], z, dn);
+      d = dn;
+    } else {
+      hl[i] = X;
+    }
+  }
+  for (int i0 = 0; i0 < layers; i0 += kGradLayers) {
+    const int cnt = layers - i0 < kGradLayers ? layers - i0 : kGradLayers;
+    GradLayers g = {};
+    for (int j = 0; j < cnt; ++j) {
+      const int fi = sizes[i0 + j], fo = sizes[i0 + j + 1];
+      g.d[j] = dl[i0 + j];
+      g.h[j] = hl[i0 + j];
+      g.dw[j] = grads[2 * (i0 + j)];
+      g.db[j] = grads[2 * (i0 + j) + 1];
+      g.fo[j] = fo;
+      g.fi[j] = fi;
+      g.first[j + 1] = g.first[j] + ((fo + GT - 1) / GT) * ((fi + GT - 1) / GT);
+    }
+    hipLaunchKernelGGL(k_weight_grads, dim3(g.first[cnt]), dim3(64 * kGradWaves), 0, s, cnt, M, g);
+  }
+  return check_launch("mlp_loss_grads");
+}
+
+int mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
+                   float* const* v, float lr, float b1, float b2, float eps, int t, hipStream_t s) {
+  const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
+  for (int i0 = 0; i0 < count; i0 += kAdamTensors) {
+    const int cnt = count - i0 < kAdamTensors ? count - i0 : kAdamTensors;
+    AdamTensors a = {};
+    int blocks = 0;
+    for (int j = 0; j < cnt; ++j) {
+      a.w[j] = w[i0 + j];
+      a.g[j] = g[i0 + j];
+      a.m[j] = m[i0 + j];
+      a.v[j] = v[i0 + j];
+      a.n[j] = n[i0 + j];
+      a.first[j] = blocks;
+      blocks += (n[i0 + j] + kAdamPer - 1) / kAdamPer;
+    }
+    hipLaunchKernelGGL(k_adam_multi, dim3(blocks), dim3(256), 0, s, cnt, a, lr, b1, b2, eps, c1, c2);
+  }
+  return check_launch("mlp_adam_multi");
 }
 int mlp_bias_act(int M, int N, float* Z, const float* bias, float* Y, int act, hipStream_t s) {
   hipLaunchKernelGGL(k_bias_act, dim3((unsigned)(((size_t)M * N + 255) / 256)), dim3(256), 0, s, M, N, Z, bias,

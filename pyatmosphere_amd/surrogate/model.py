@@ -6,7 +6,7 @@ aperture radius a, wavelength.  Outputs: NB = 64 logits of the transmittance
 PDT over [0, 1] (softmax -> bin probabilities) and log of the beam-wander
 variance sigma_BW,x^2 = <x_c^2> (simulations/beam.py:35-38).
 
-Training: float32 master weights, float32 GEMMs on the vector units, softmax
+Training: float32 master weights, float32 MFMA GEMMs, softmax
 cross-entropy + a ranked-probability (squared CDF distance) term + weighted
 log-variance MSE, Adam.  Inference: bf16 MFMA GEMMs
 with float32 accumulation and fused bias + SiLU.
@@ -19,7 +19,7 @@ import numpy as np
 import torch
 
 from .. import _lib
-from .._lib import call, ptr
+from .._lib import call, ptr, ptr_array
 
 NB = 64
 IN_FEATURES = 5
@@ -48,6 +48,10 @@ def encode(log10_cn2, L, w0, a, wvl) -> np.ndarray:
 
 def in_domain(x: np.ndarray, tol: float = 1e-6) -> np.ndarray:
     return np.all(np.abs(x) <= 1 + tol, axis=-1)
+
+
+def _flat(pairs) -> List[torch.Tensor]:
+    return [t for pair in pairs for t in pair]
 
 
 class PDTSurrogate:
@@ -113,55 +117,24 @@ class PDTSurrogate:
         xp[:, :IN_FEATURES] = x
         return torch.from_numpy(xp).to(self.device)
 
-    def _forward(self, X: torch.Tensor):
-        s = _lib.stream_handle()
-        M = X.shape[0]
-        hs, zs = [X], []
-        for i, (W, b) in enumerate(self.params):
-            fo, fi = W.shape
-            Z = torch.empty(M, fo, dtype=torch.float32, device=self.device)
-            call("pa_mlp_gemm_f32", M, fo, fi, ptr(hs[-1]), fi, 0, ptr(W), fi, 1, ptr(Z), fo, 1.0, 0.0, s)
-            Y = torch.empty_like(Z)
-            call("pa_mlp_bias_act", M, fo, ptr(Z), ptr(b), ptr(Y), int(i < len(self.params) - 1), s)
-            zs.append(Z)
-            hs.append(Y)
-        return hs, zs
-
     def loss_and_grads(self, X: torch.Tensor, T: torch.Tensor, TV: torch.Tensor):
         """Mean loss (device scalar) and gradients [(dW, db)] for one batch."""
-        s = _lib.stream_handle()
-        M = X.shape[0]
-        hs, zs = self._forward(X)
-        out = hs[-1]
+        M, layers = X.shape[0], len(self.params)
+        sizes = _lib.int_array([self.params[0][0].shape[1]] + [W.shape[0] for W, _ in self.params])
         loss = torch.empty(M, dtype=torch.float32, device=self.device)
-        d = torch.empty_like(out)
-        call("pa_mlp_head_loss", M, NB, ptr(out), ptr(T), ptr(TV), float(self.wv), float(self.wc), ptr(loss),
-             ptr(d), s)
-        grads = [None] * len(self.params)
-        for i in reversed(range(len(self.params))):
-            W, b = self.params[i]
-            fo, fi = W.shape
-            if i < len(self.params) - 1:
-                dz = torch.empty_like(d)
-                call("pa_mlp_act_backward", M, fo, ptr(zs[i]), ptr(d), ptr(dz), s)
-                d = dz
-            dW = torch.empty_like(W)
-            db = torch.empty_like(b)
-            call("pa_mlp_gemm_f32", fo, fi, M, ptr(d), fo, 1, ptr(hs[i]), fi, 0, ptr(dW), fi, 1.0, 0.0, s)
-            call("pa_mlp_bias_grad", M, fo, ptr(d), ptr(db), s)
-            grads[i] = (dW, db)
-            if i > 0:
-                dh = torch.empty(M, fi, dtype=torch.float32, device=self.device)
-                call("pa_mlp_gemm_f32", M, fi, fo, ptr(d), fo, 0, ptr(W), fi, 0, ptr(dh), fi, 1.0, 0.0, s)
-                d = dh
+        scratch = torch.empty(call("pa_mlp_loss_grads_scratch", layers, sizes, M), dtype=torch.uint8,
+                              device=self.device)
+        grads = [(torch.empty_like(W), torch.empty_like(b)) for W, b in self.params]
+        call("pa_mlp_loss_grads", layers, sizes, M, ptr(X), ptr_array(_flat(self.params)), ptr(T), ptr(TV),
+             float(self.wv), float(self.wc), ptr(loss), ptr_array(_flat(grads)), ptr(scratch), _lib.stream_handle())
         return loss.mean(), grads
 
     def adam_step(self, grads, lr: float, b1=0.9, b2=0.999, eps=1e-8) -> None:
-        s = _lib.stream_handle()
         self.t += 1
-        for (W, b), (gW, gb), (mW, mb), (vW, vb) in zip(self.params, grads, self.m, self.v):
-            call("pa_mlp_adam", W.numel(), ptr(W), ptr(gW), ptr(mW), ptr(vW), lr, b1, b2, eps, self.t, s)
-            call("pa_mlp_adam", b.numel(), ptr(b), ptr(gb), ptr(mb), ptr(vb), lr, b1, b2, eps, self.t, s)
+        layers = list(zip(self.params, grads, self.m, self.v))
+        w, g, m, v = (_flat(pairs) for pairs in zip(*layers))
+        call("pa_mlp_adam_multi", len(w), _lib.int_array([p.numel() for p in w]), ptr_array(w), ptr_array(g),
+             ptr_array(m), ptr_array(v), lr, b1, b2, eps, self.t, _lib.stream_handle())
         self._bf16 = None
 
     def train(self, x: np.ndarray, target: np.ndarray, tvar: np.ndarray, steps: int, batch: int = 512,

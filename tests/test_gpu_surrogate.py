@@ -129,3 +129,44 @@ def test_fallback_runs_the_simulation(dev):
     assert np.isclose(pdt[0].sum(), 1.0) and np.isclose(pdt[1].sum(), 1.0)
     direct = simulated_pdt(outside, 0.1, 300, 5)
     assert np.array_equal(pdt[0], direct)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 33, 7), (32, 32, 8), (65, 17, 100), (100, 384, 16), (384, 65, 1001)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("pad", [0, 1, 4])
+def test_gemm_f32_edges(dev, M, N, K, ta, tb, pad):
+    """Tile remainders, every transposition, and leading dimensions that do and
+    do not allow quad reads, against float64.  Tolerance: the float32 sum of K
+    products is within K 2^-24 of sum |a b| (any order), plus the epilogue's
+    three roundings."""
+    from pyatmosphere_amd._lib import call, ptr
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.normal(size=(K, M) if ta else (M, K)), rng.normal(size=(N, K) if tb else (K, N))
+    C = rng.normal(size=(M, N)).astype(np.float32)
+    Ap, Bp = (np.pad(x, ((0, 0), (0, pad)), constant_values=np.nan).astype(np.float32) for x in (A, B))
+    a, b, c = (torch.from_numpy(x).to(dev) for x in (Ap, Bp, C.copy()))
+    call("pa_mlp_gemm_f32", M, N, K, ptr(a), a.shape[1], ta, ptr(b), b.shape[1], tb, ptr(c), N, 0.5, 2.0, None)
+    A, B = (x.astype(np.float32).astype(np.float64) for x in (A, B))
+    A, B = A.T if ta else A, B.T if tb else B
+    bound = (K + 4) * 2.0 ** -24 * (0.5 * np.abs(A) @ np.abs(B) + 2 * np.abs(C))
+    assert np.all(np.abs(c.cpu().numpy() - (0.5 * A @ B + 2.0 * C)) <= bound)
+
+
+@pytest.mark.parametrize("width,depth,M", [(32, 2, 1), (64, 3, 33), (96, 4, 1000), (40, 10, 65)])
+def test_loss_and_grads_edges(dev, width, depth, M):
+    """Batches and widths off the tile sizes, and more layers than one gradient
+    launch holds, against the float64 oracle.  Tolerance: M + width roundings
+    of 2^-24 per product chain, a few chains deep, of the largest gradient."""
+    rng = np.random.default_rng(width + M)
+    net = PDTSurrogate(width=width, depth=depth, seed=3, device=dev)
+    x, t, tv = _batch(rng, M)
+    loss, grads = net.loss_and_grads(net._pad(x), torch.from_numpy(t).to(dev), torch.from_numpy(tv).to(dev))
+    ref_loss, ref = omlp.loss_and_grad(net.numpy_params(), x.astype(np.float64), t.astype(np.float64),
+                                       tv.astype(np.float64), net.wv, net.wc)
+    tol = 2.0 ** -24 * (M + width) * depth + 2.0 ** -18
+    assert abs(loss.item() - ref_loss) <= tol * max(1, abs(ref_loss))
+    for i, (got, want) in enumerate(zip(grads, ref)):
+        for g, r in zip(got, want):
+            g = g.cpu().numpy().astype(np.float64)
+            g = g[:, :5] if i == 0 and g.ndim == 2 else g
+            assert np.abs(g - r).max() <= tol * np.abs(r).max() + 1e-7, i
