@@ -357,6 +357,21 @@ int pa_mlp_to_bf16(long long n, const float* x, void* y, void* stream);
  * K multiple of 16, N multiple of 32. */
 int pa_mlp_layer_bf16(int M, int N, int K, const float* X, const void* W, const float* bias, float* Y, int act,
                       void* stream);
+/* The whole network in one launch, bit-equal to pa_mlp_layer_bf16 layer by
+ * layer (SiLU between layers), for at most 16 layers whose inputs are at most
+ * 512 wide and multiples of 16 (pa_mlp_pack_bytes is 0 otherwise).
+ * pa_mlp_pack_bf16 lays out one member's weights and biases (params as for
+ * pa_mlp_loss_grads) in pa_mlp_pack_bytes bytes, 16-byte aligned; pa_mlp_infer
+ * takes x[M][inputs] (float32; inputs <= sizes[0], the rest zero) through each
+ * of `members` packed networks into out[members][M][sizes[layers]]. */
+long long pa_mlp_pack_bytes(int layers, const int* sizes);
+int pa_mlp_pack_bf16(int layers, const int* sizes, const float* const* params, void* packed, void* stream);
+int pa_mlp_infer(int layers, const int* sizes, int inputs, int members, const void* const* packed, int M,
+                 const float* x, float* out, void* stream);
+/* Ensemble PDTs of logits[members][M][65] (64 bins and a log-variance; at most
+ * 8 members), in float64: out = the members' mean softmax [M][64], their mean
+ * log-variance [M], and the largest CDF distance of a member from the mean [M]. */
+int pa_mlp_pdt(int members, int M, const float* logits, double* out, void* stream);
 
 #ifdef __cplusplus
 }

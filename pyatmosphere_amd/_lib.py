@@ -77,6 +77,10 @@ SIGNATURES = {
     "pa_mlp_loss_grads": (i32, [i32, vp, i32, vp, vp, vp, vp, f32, f32, vp, vp, vp, vp]),
     "pa_mlp_adam_multi": (i32, [i32, vp, vp, vp, vp, vp, f32, f32, f32, f32, i32, vp]),
     "pa_mlp_to_bf16": (i32, [i64, vp, vp, vp]),
+    "pa_mlp_pack_bytes": (i64, [i32, vp]),
+    "pa_mlp_pack_bf16": (i32, [i32, vp, vp, vp, vp]),
+    "pa_mlp_infer": (i32, [i32, vp, i32, i32, vp, i32, vp, vp, vp]),
+    "pa_mlp_pdt": (i32, [i32, i32, vp, vp, vp]),
     "pa_mlp_layer_bf16": (i32, [i32, i32, i32, vp, vp, vp, vp, i32, vp]),
 }
 

@@ -79,6 +79,12 @@ int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const fl
                    float* scratch, hipStream_t s);
 int mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
                    float* const* v, float lr, float b1, float b2, float eps, int t, hipStream_t s);
+bool mlp_infer_fits(int layers, const int* sizes);
+long long mlp_pack_bytes(int layers, const int* sizes);
+int mlp_pack_bf16(int layers, const int* sizes, const float* const* params, void* packed, hipStream_t s);
+int mlp_infer(int layers, const int* sizes, int inputs, int members, const void* const* packed, int M, const float* x,
+              float* out, hipStream_t s);
+int mlp_pdt(int members, int M, const float* logits, double* out, hipStream_t s);
 int mlp_to_bf16(long long n, const float* x, unsigned short* y, hipStream_t s);
 int mlp_layer_bf16(int M, int N, int K, const float* X, const unsigned short* W, const float* bias, float* Y,
                    int act, hipStream_t s);
@@ -408,6 +414,35 @@ int pa_mlp_layer_bf16(int M, int N, int K, const float* X, const void* W, const 
   REQUIRE(M > 0 && N > 0 && K > 0 && X && W && bias && Y, "mlp_layer_bf16: bad argument");
   REQUIRE(K % 16 == 0 && N % 32 == 0, "mlp_layer_bf16: K must be a multiple of 16 and N of 32");
   return mlp_layer_bf16(M, N, K, X, reinterpret_cast<const unsigned short*>(W), bias, Y, act, STREAM(stream));
+}
+
+static bool mlp_layers_ok(int layers, const int* sizes) {
+  if (!sizes || layers < 1 || layers > kMlpMaxLayers) return false;
+  for (int i = 0; i <= layers; ++i)
+    if (sizes[i] < 1) return false;
+  return true;
+}
+long long pa_mlp_pack_bytes(int layers, const int* sizes) {
+  REQUIRE(mlp_layers_ok(layers, sizes), "mlp_pack: bad layer sizes");
+  return mlp_infer_fits(layers, sizes) ? mlp_pack_bytes(layers, sizes) : 0;
+}
+int pa_mlp_pack_bf16(int layers, const int* sizes, const float* const* params, void* packed, void* stream) {
+  REQUIRE(mlp_layers_ok(layers, sizes) && mlp_infer_fits(layers, sizes), "mlp_pack: bad layer sizes");
+  REQUIRE(params && packed, "mlp_pack: null pointer");
+  for (int i = 0; i < 2 * layers; ++i) REQUIRE(params[i], "mlp_pack: null pointer");
+  return mlp_pack_bf16(layers, sizes, params, packed, STREAM(stream));
+}
+int pa_mlp_infer(int layers, const int* sizes, int inputs, int members, const void* const* packed, int M,
+                 const float* x, float* out, void* stream) {
+  REQUIRE(mlp_layers_ok(layers, sizes) && mlp_infer_fits(layers, sizes), "mlp_infer: bad layer sizes");
+  REQUIRE(inputs > 0 && inputs <= sizes[0] && members > 0 && M > 0, "mlp_infer: bad argument");
+  REQUIRE(packed && x && out, "mlp_infer: null pointer");
+  for (int i = 0; i < members; ++i) REQUIRE(packed[i], "mlp_infer: null pointer");
+  return mlp_infer(layers, sizes, inputs, members, packed, M, x, out, STREAM(stream));
+}
+int pa_mlp_pdt(int members, int M, const float* logits, double* out, void* stream) {
+  REQUIRE(members > 0 && M > 0 && logits && out, "mlp_pdt: bad argument");
+  return mlp_pdt(members, M, logits, out, STREAM(stream));
 }
 
 }  // extern "C"

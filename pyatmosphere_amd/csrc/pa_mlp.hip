@@ -369,6 +369,146 @@ k_layer_bf16(int M, int N, int K, const float* __restrict__ X, const unsigned sh
   }
 }
 
+// ------------------------------------------------------------------ fused bf16 inference
+// The whole network in one launch, for layers up to kInferWidth values wide.  A
+// block takes 32 rows of one member through every layer; the activations stay
+// in LDS as the bf16 values the next product reads, so nothing but the inputs,
+// the weights (L2) and the outputs moves.  Weights are packed once per set of
+// weights in the order the products read them (pack_bf16): the fragment of
+// (32-column tile, 16-wide K chunk) is 1 KB, 16 bytes per lane, where rows of
+// the plain matrix gave 32 scattered 32-byte pieces.  A wave owns a tile and
+// walks K with kInferAhead fragments in flight (the products are a serial
+// chain per tile, so the loads' latency bounds it); 12 waves cover a 384-wide
+// layer at once.  Chunk order, operand roles and roundings are k_layer_bf16's,
+// so the outputs are bit-equal to running the layers one by one.
+// Measured, 4096 rows x 3 members of width 384: 720 us of layer launches.
+constexpr int kInferRows = 32, kInferWaves = 12, kInferWidth = 512, kInferAhead = 8;
+constexpr int kInferLayers = 16, kInferMembers = 8;
+constexpr int kInferStride = kInferWidth + 8;   // bf16 per LDS row: 16-byte reads of 32 rows hit all banks
+
+struct InferNet {
+  const float* bias[kInferMembers];             // packed: every layer's biases, then the fragments
+  int sizes[kInferLayers + 1];
+};
+
+static __host__ __device__ inline int tiles32(int n) { return (n + 31) / 32; }
+
+__global__ void __launch_bounds__(64 * kInferWaves)
+k_mlp_infer(int layers, int inputs, int M, const float* __restrict__ x, InferNet net, float* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) unsigned short act[2][kInferRows * kInferStride];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
+  const int m0 = blockIdx.x * kInferRows, member = blockIdx.y;
+  const float* bias = net.bias[member];
+  int nb = 0;
+  for (int i = 0; i < layers; ++i) nb += 32 * tiles32(net.sizes[i + 1]);
+  const unsigned short* w = reinterpret_cast<const unsigned short*>(bias + nb);
+  for (int e = threadIdx.x; e < kInferRows * net.sizes[0]; e += 64 * kInferWaves) {
+    const int rr = e / net.sizes[0], k = e % net.sizes[0];
+    act[0][rr * kInferStride + k] = m0 + rr < M && k < inputs ? f2bf(x[(size_t)(m0 + rr) * inputs + k]) : 0;
+  }
+  for (int i = 0; i < layers; ++i) {
+    __syncthreads();
+    const unsigned short* cur = act[i & 1] + r * kInferStride + 8 * h;
+    unsigned short* nxt = act[(i + 1) & 1];
+    const int nc = net.sizes[i] / 16, fo = net.sizes[i + 1], nt = tiles32(fo);
+    for (int t = wave; t < nt; t += kInferWaves) {
+      const us8* f = reinterpret_cast<const us8*>(w) + (size_t)t * nc * 64 + lane;
+      f16v acc;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+      us8 q[kInferAhead];
+#pragma unroll
+      for (int u = 0; u < kInferAhead; ++u) q[u] = f[(size_t)min(u, nc - 1) * 64];
+      for (int c0 = 0; c0 < nc; c0 += kInferAhead) {
+#pragma unroll
+        for (int u = 0; u < kInferAhead; ++u) {
+          if (c0 + u >= nc) break;
+          const us8 b = q[u];
+          q[u] = f[(size_t)min(c0 + u + kInferAhead, nc - 1) * 64];
+          const us8 a = *reinterpret_cast<const us8*>(cur + 16 * (c0 + u));
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), acc, 0,
+                                                        0, 0);
+        }
+      }
+      const int col = 32 * t + r;
+      const float bc = bias[col];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int rr = 8 * (v / 4) + 4 * h + v % 4;
+        const float z = acc[v] + bc;
+        if (i < layers - 1) {
+          nxt[rr * kInferStride + col] = f2bf(z * sigm(z));
+        } else if (col < fo && m0 + rr < M) {
+          out[((size_t)member * M + m0 + rr) * fo + col] = z;
+        }
+      }
+    }
+    bias += 32 * nt;
+    w += (size_t)nt * nc * 512;
+  }
+}
+
+// One layer's weights W[fo][fi] and biases into the packed order.
+__global__ void k_pack_bf16(int fo, int fi, const float* __restrict__ W, const float* __restrict__ b,
+                            float* __restrict__ pb, unsigned short* __restrict__ pw) {
+  const int nc = fi / 16, nt = tiles32(fo), i = blockIdx.x * 256 + threadIdx.x;
+  if (i < 32 * nt) pb[i] = i < fo ? b[i] : 0.f;
+  if (i >= nt * nc * 512) return;
+  const int j = i & 7, l = (i >> 3) & 63, c = (i >> 9) % nc, t = (i >> 9) / nc;
+  const int col = 32 * t + (l & 31), k = 16 * c + 8 * (l >> 5) + j;
+  pw[i] = col < fo ? f2bf(W[(size_t)col * fi + k]) : 0;
+}
+
+// Softmax in float64 of every member's 64 logits, their mean, the mean of the
+// log-variances and the members' spread: the largest |CDF difference| of a
+// member and the mean (NaN where a logit is NaN, as numpy's max gives).  One
+// wave per row, lane = bin.  out: mean [M][64], log-variance [M], spread [M].
+__device__ __forceinline__ double nan_max(double a, double b) { return a != a ? a : b != b ? b : fmax(a, b); }
+template <class F>
+__device__ __forceinline__ double wave_fold(double v, F f) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = f(v, __shfl_xor(v, o, 64));
+  return v;
+}
+__device__ __forceinline__ double wave_cumsum(double v, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double a = __shfl_up(v, o, 64);
+    if (lane >= o) v += a;
+  }
+  return v;
+}
+__global__ void __launch_bounds__(256)
+k_mlp_pdt(int members, int M, const float* __restrict__ logits, double* __restrict__ out) {
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= M) return;
+  double p[kInferMembers], mean = 0.0, lv = 0.0;
+#pragma unroll
+  for (int i = 0; i < kInferMembers; ++i) {
+    p[i] = 0.0;
+    if (i < members) {
+      const float* l = logits + ((size_t)i * M + row) * 65;
+      const double x = l[lane];
+      const double e = exp(x - wave_fold(x, nan_max));
+      p[i] = e / wave_fold(e, [](double a, double b) { return a + b; });
+      mean += p[i];
+      lv += (double)l[64];
+    }
+  }
+  mean /= members;
+  const double cm = wave_cumsum(mean, lane);
+  double spread = 0.0;
+#pragma unroll
+  for (int i = 0; i < kInferMembers; ++i)
+    if (i < members) spread = nan_max(spread, fabs(wave_cumsum(p[i], lane) - cm));
+  spread = wave_fold(spread, nan_max);
+  out[(size_t)row * 64 + lane] = mean;
+  if (lane == 0) {
+    out[(size_t)M * 64 + row] = lv / members;
+    out[(size_t)M * 65 + row] = spread;
+  }
+}
+
 // ------------------------------------------------------------------ launchers
 // float4 reads of an operand whose K is contiguous need whole quads of k at 16-byte addresses
 static bool quads(const float* p, int ld, int K) {
@@ -526,6 +666,50 @@ int mlp_layer_bf16(int M, int N, int K, const float* X, const unsigned short* W,
   dim3 g((N + 127) / 128, (M + 31) / 32);
   hipLaunchKernelGGL(k_layer_bf16, g, dim3(256), 0, s, M, N, K, X, W, bias, Y, act);
   return check_launch("mlp_layer_bf16");
+}
+
+
+bool mlp_infer_fits(int layers, const int* sizes) {
+  if (layers > kInferLayers) return false;
+  for (int i = 0; i < layers; ++i)
+    if (sizes[i] % 16 || sizes[i] > kInferWidth) return false;
+  return true;
+}
+long long mlp_pack_bytes(int layers, const int* sizes) {
+  long long n = 0;
+  for (int i = 0; i < layers; ++i) n += tiles32(sizes[i + 1]) * (128ll + (long long)sizes[i] / 16 * 1024);
+  return n;
+}
+int mlp_pack_bf16(int layers, const int* sizes, const float* const* params, void* packed, hipStream_t s) {
+  float* pb = reinterpret_cast<float*>(packed);
+  int nb = 0;
+  for (int i = 0; i < layers; ++i) nb += 32 * tiles32(sizes[i + 1]);
+  unsigned short* pw = reinterpret_cast<unsigned short*>(pb + nb);
+  for (int i = 0; i < layers; ++i) {
+    const int fi = sizes[i], fo = sizes[i + 1], nt = tiles32(fo), n = nt * (fi / 16) * 512;
+    hipLaunchKernelGGL(k_pack_bf16, dim3((n + 255) / 256), dim3(256), 0, s, fo, fi, params[2 * i], params[2 * i + 1], pb,
+                       pw);
+    pb += 32 * nt;
+    pw += n;
+  }
+  return check_launch("mlp_pack_bf16");
+}
+int mlp_infer(int layers, const int* sizes, int inputs, int members, const void* const* packed, int M, const float* x,
+              float* out, hipStream_t s) {
+  for (int i0 = 0; i0 < members; i0 += kInferMembers) {
+    const int cnt = members - i0 < kInferMembers ? members - i0 : kInferMembers;
+    InferNet net = {};
+    for (int j = 0; j < cnt; ++j) net.bias[j] = reinterpret_cast<const float*>(packed[i0 + j]);
+    for (int i = 0; i <= layers; ++i) net.sizes[i] = sizes[i];
+    hipLaunchKernelGGL(k_mlp_infer, dim3((M + kInferRows - 1) / kInferRows, cnt), dim3(64 * kInferWaves), 0, s, layers,
+                       inputs, M, x, net, out + (size_t)i0 * M * sizes[layers]);
+  }
+  return check_launch("mlp_infer");
+}
+int mlp_pdt(int members, int M, const float* logits, double* out, hipStream_t s) {
+  if (members > kInferMembers) return set_error(PA_ERR_ARG, "mlp_pdt: at most 8 members");
+  hipLaunchKernelGGL(k_mlp_pdt, dim3((M + 3) / 4), dim3(256), 0, s, members, M, logits, out);
+  return check_launch("mlp_pdt");
 }
 
 }  // namespace pa

@@ -24,6 +24,7 @@ from .._lib import call, ptr, ptr_array
 NB = 64
 IN_FEATURES = 5
 IN_PAD = 16
+MAX_FUSED_MEMBERS = 8        # pa_mlp_pdt's limit
 DOMAIN = {
     "log10_cn2": (-16.0, -14.0),
     "L": (1e3, 50e3),
@@ -120,7 +121,7 @@ class PDTSurrogate:
     def loss_and_grads(self, X: torch.Tensor, T: torch.Tensor, TV: torch.Tensor):
         """Mean loss (device scalar) and gradients [(dW, db)] for one batch."""
         M, layers = X.shape[0], len(self.params)
-        sizes = _lib.int_array([self.params[0][0].shape[1]] + [W.shape[0] for W, _ in self.params])
+        sizes = self._layer_sizes()
         loss = torch.empty(M, dtype=torch.float32, device=self.device)
         scratch = torch.empty(call("pa_mlp_loss_grads_scratch", layers, sizes, M), dtype=torch.uint8,
                               device=self.device)
@@ -157,11 +158,28 @@ class PDTSurrogate:
         return hist
 
     # ------------------------------------------------------------ inference (bf16 MFMA)
-    def _bf16_weights(self):
+    def _layer_sizes(self):
+        return _lib.int_array([self.params[0][0].shape[1]] + [W.shape[0] for W, _ in self.params])
+
+    def _packed(self) -> Optional[torch.Tensor]:
+        """The weights in the fused network's order (pa_mlp_pack_bf16), laid out
+        once per set of weights; None for networks too wide or deep for it."""
         if self._bf16 is None:
-            s = _lib.stream_handle()
+            sizes, layers = self._layer_sizes(), len(self.params)
+            size = call("pa_mlp_pack_bytes", layers, sizes)
+            if not size:
+                return None
+            packed = torch.empty(size, dtype=torch.uint8, device=self.device)
+            call("pa_mlp_pack_bf16", layers, sizes, ptr_array(_flat(self.params)), ptr(packed), _lib.stream_handle())
+            self._bf16 = packed
+        return self._bf16 if torch.is_tensor(self._bf16) else None
+
+    def _bf16_layers(self):
+        """Per layer (weights, bias, width, padded width, inputs) for the networks
+        that the fused launch does not take."""
+        if self._bf16 is None:
             layers = []
-            for i, (W, b) in enumerate(self.params):
+            for W, b in self.params:
                 fo, fi = W.shape
                 fo_p = ((fo + 31) // 32) * 32
                 Wp = torch.zeros(fo_p, fi, dtype=torch.float32, device=self.device)
@@ -169,29 +187,64 @@ class PDTSurrogate:
                 bp = torch.zeros(fo_p, dtype=torch.float32, device=self.device)
                 bp[:fo] = b
                 Wb = torch.empty(fo_p, fi, dtype=torch.int16, device=self.device)
-                call("pa_mlp_to_bf16", Wp.numel(), ptr(Wp), ptr(Wb), s)
+                call("pa_mlp_to_bf16", Wp.numel(), ptr(Wp), ptr(Wb), _lib.stream_handle())
                 layers.append((Wb, bp, fo, fo_p, fi))
             self._bf16 = layers
         return self._bf16
 
-    def predict_raw(self, x: np.ndarray) -> np.ndarray:
-        """(M, NB + 1) outputs on bf16 MFMA."""
-        s = _lib.stream_handle()
+    def _layer_by_layer(self, x: np.ndarray) -> torch.Tensor:
+        """(M, outputs) device outputs, one launch per layer."""
         h = self._pad(x)
-        M = h.shape[0]
-        layers = self._bf16_weights()
+        M, layers = h.shape[0], self._bf16_layers()
         for i, (Wb, bp, fo, fo_p, fi) in enumerate(layers):
             y = torch.empty(M, fo_p, dtype=torch.float32, device=self.device)
-            call("pa_mlp_layer_bf16", M, fo_p, fi, ptr(h), ptr(Wb), ptr(bp), ptr(y), int(i < len(layers) - 1), s)
-            h = y
-        return h[:, :NB + 1].cpu().numpy().astype(np.float64)
+            call("pa_mlp_layer_bf16", M, fo_p, fi, ptr(h), ptr(Wb), ptr(bp), ptr(y), int(i < len(layers) - 1),
+                 _lib.stream_handle())
+            h = y if fo_p == fo else y[:, :fo].contiguous()
+        return h
+
+    def predict_raw(self, x: np.ndarray) -> np.ndarray:
+        """(M, NB + 1) outputs on bf16 MFMA."""
+        return _outputs([self], x)[0].cpu().numpy().astype(np.float64)
 
     def predict(self, x: np.ndarray) -> Tuple[np.ndarray, np.ndarray]:
         """Bin probabilities (M, NB) of the transmittance PDT and log sigma_BW,x^2."""
-        out = self.predict_raw(x)
-        lg = out[:, :NB]
-        p = np.exp(lg - lg.max(axis=1, keepdims=True))
-        return p / p.sum(axis=1, keepdims=True), out[:, NB]
+        return _distributions([self], x)[:2]
+
+
+def _outputs(members: Sequence[PDTSurrogate], x: np.ndarray) -> torch.Tensor:
+    """(members, M, NB + 1) float32 device outputs; the members share a device.
+    Networks of one shape run in one launch."""
+    dev, M = members[0].device, x.shape[0]
+    shapes = {tuple(p.shape for p in _flat(m.params)) for m in members}
+    packs = [m._packed() for m in members]
+    if len(shapes) > 1 or any(p is None for p in packs):
+        if len(members) > 1:
+            return torch.cat([_outputs([m], x) for m in members])
+        return members[0]._layer_by_layer(x)[None, :, :NB + 1].contiguous()
+    xs = np.empty((M, IN_FEATURES), np.float32)
+    xs[:] = x
+    xd = torch.empty(M, IN_FEATURES, dtype=torch.float32, device=dev)
+    xd.copy_(torch.from_numpy(xs).pin_memory(), non_blocking=True)
+    out = torch.empty(len(members), M, members[0].params[-1][0].shape[0], dtype=torch.float32, device=dev)
+    call("pa_mlp_infer", len(members[0].params), members[0]._layer_sizes(), IN_FEATURES, len(members),
+         ptr_array(packs), M, ptr(xd), ptr(out), _lib.stream_handle())
+    return out[:, :, :NB + 1].contiguous()
+
+
+def _distributions(members: Sequence[PDTSurrogate], x: np.ndarray):
+    """The members' mean PDT (M, NB), mean log variance (M,) and spread (M,)
+    (KS distance between a member and the mean), float64: softmax and ensemble
+    statistics on the device, one copy back."""
+    logits = _outputs(members, x)
+    M = logits.shape[1]
+    dist = torch.empty(M * (NB + 2), dtype=torch.float64, device=logits.device)
+    call("pa_mlp_pdt", len(members), M, ptr(logits), ptr(dist), _lib.stream_handle())
+    host = torch.empty(dist.shape, dtype=dist.dtype, pin_memory=True)
+    host.copy_(dist, non_blocking=True)
+    torch.cuda.current_stream(dist.device).synchronize()
+    flat = host.numpy()
+    return flat[:M * NB].reshape(M, NB), flat[M * NB:M * (NB + 1)], flat[M * (NB + 1):]
 
 
 def ks_binned(p: np.ndarray, q: np.ndarray) -> np.ndarray:
@@ -212,10 +265,14 @@ class SurrogateEnsemble:
         self.max_spread = max_spread
 
     def pdt(self, x: np.ndarray):
-        preds = [m.predict(x) for m in self.members]
-        ps = np.stack([p for p, _ in preds])
-        mean = ps.mean(axis=0)
-        spread = np.max([ks_binned(p, mean) for p in ps], axis=0)
-        lv = np.mean([v for _, v in preds], axis=0)
+        if 0 < len(self.members) <= MAX_FUSED_MEMBERS and all(type(m) is PDTSurrogate for m in self.members) \
+                and len({m.device for m in self.members}) == 1:
+            mean, lv, spread = _distributions(self.members, x)
+        else:
+            preds = [m.predict(x) for m in self.members]
+            ps = np.stack([p for p, _ in preds])
+            mean = ps.mean(axis=0)
+            spread = np.max([ks_binned(p, mean) for p in ps], axis=0)
+            lv = np.mean([v for _, v in preds], axis=0)
         fallback = (spread > self.max_spread) | ~in_domain(x)
         return mean, lv, spread, fallback

@@ -170,3 +170,39 @@ def test_loss_and_grads_edges(dev, width, depth, M):
             g = g.cpu().numpy().astype(np.float64)
             g = g[:, :5] if i == 0 and g.ndim == 2 else g
             assert np.abs(g - r).max() <= tol * np.abs(r).max() + 1e-7, i
+
+
+@pytest.mark.parametrize("width,depth", [(16, 2), (32, 4), (48, 3), (384, 4), (400, 4), (512, 4), (64, 16)])
+@pytest.mark.parametrize("M", [1, 31, 33, 200])
+def test_fused_inference_equals_the_layers(dev, width, depth, M):
+    """The fused network's outputs are bit-equal to one launch per layer: the
+    chunk order and every rounding are the same."""
+    rng = np.random.default_rng(width + M)
+    net = PDTSurrogate(width=width, depth=depth, seed=3, device=dev)
+    x = rng.uniform(-1, 1, size=(M, 5)).astype(np.float32)
+    assert net._packed() is not None
+    got = net.predict_raw(x)
+    net._bf16 = None
+    assert np.array_equal(got, net._layer_by_layer(x).cpu().numpy()[:, :NB + 1].astype(np.float64))
+
+
+@pytest.mark.parametrize("widths,M", [((32,), 1), ((64, 64), 5), ((64, 96, 544), 37), ((32,) * 8, 6), ((32,) * 9, 3)])
+def test_ensemble_statistics(dev, widths, M):
+    """Ensembles of one shape, of several, with a network too wide for the fused
+    launch, of 8 and more members, and with NaN requests, against numpy on the
+    members' own outputs: float64 on both sides, 64-term sums."""
+    from pyatmosphere_amd.surrogate import SurrogateEnsemble
+    rng = np.random.default_rng(M)
+    members = [PDTSurrogate(width=w, depth=3, seed=i, device=dev) for i, w in enumerate(widths)]
+    x = rng.uniform(-1.1, 1.1, size=(M, 5)).astype(np.float32)
+    x[M // 2, 1] = np.nan if M > 1 else 0.5
+    raw = np.stack([m.predict_raw(x) for m in members])
+    p = np.exp(raw[:, :, :NB] - raw[:, :, :NB].max(axis=2, keepdims=True))
+    p /= p.sum(axis=2, keepdims=True)
+    mean = p.mean(axis=0)
+    spread = np.max([ks_binned(q, mean) for q in p], axis=0)
+    got = SurrogateEnsemble(members).pdt(x)
+    for a, b in zip(got, (mean, raw[:, :, NB].mean(axis=0), spread)):
+        np.testing.assert_allclose(a, b, rtol=0, atol=1e-13 * max(1.0, np.nanmax(np.abs(b))), equal_nan=True)
+    inside = np.all(np.abs(x) <= 1 + 1e-6, axis=1)
+    assert np.array_equal(got[3], (spread > 0.04) | ~inside)
