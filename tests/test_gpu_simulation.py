@@ -178,6 +178,20 @@ def test_structure_function_kernel(dev, n):
     assert np.array_equal(got, want) if n <= 256 else np.allclose(got, want, rtol=1.5 * n / 4 * 2.0 ** -24, atol=0)
 
 
+@pytest.mark.parametrize("n", [64, 256, 1024])
+def test_structure_function_of_an_unaligned_screen(dev, n):
+    """A screen that starts off a 16-byte boundary gives the same bits as its
+    aligned copy, alone and as one of three."""
+    import torch
+    from pyatmosphere_amd import engine
+    g = torch.Generator(device=dev).manual_seed(n)
+    buf = torch.randn(3 * n * n + 1, device=dev, generator=g)
+    phi = buf[1:].view(3, n, n)
+    got = engine.structure_function(phi)
+    assert np.array_equal(got, engine.structure_function(phi.clone()))
+    assert np.array_equal(got[1], engine.structure_function(phi[1]))
+
+
 def test_structure_function_result_matches_oracle(dev):
     """StructureFunctionResult (simulations/structure_function.py): the first
     screen of each realization, device synthesis and device structure function,
