@@ -935,14 +935,17 @@ def field_moments(u: torch.Tensor, delta: float, pupils: Sequence[Tuple[float, f
     T = call("pa_tile_rows", n)
     dev = u.device
     stream = _lib.stream_handle()
-    chp = torch.tensor([[delta, 0.0, 0.0, 0.0]], dtype=torch.float64, device=dev)
-    pup_np = np.zeros((1, _lib.PA_MAX_PUPILS, 3))
+    # one channel's parameters and pupils, in one upload
+    host = np.zeros(_lib.PA_CH_PARAMS + 3 * _lib.PA_MAX_PUPILS)
+    host[0] = delta
     for j, p in enumerate(pupils):
-        pup_np[0, j] = p
-    pup = torch.from_numpy(pup_np).to(dev)
+        host[_lib.PA_CH_PARAMS:].reshape(-1, 3)[j] = p
+    chp = torch.empty(len(host), dtype=torch.float64, device=dev)
+    upload(chp, host, np.float64)
+    pup = chp[_lib.PA_CH_PARAMS:]
     part = torch.empty(B, n // T, _lib.PA_PART_SUMS, dtype=torch.float64, device=dev)
     out = torch.empty(B, _lib.PA_NUM_MOMENTS, dtype=torch.float64, device=dev)
-    chan = torch.zeros(B, dtype=torch.int32, device=dev)
+    chan = None
     if tracked:
         call("pa_field_partials", n, ptr(u), ptr(part), ptr(chp), ptr(pup), 0, None, ptr(chan), B, stream)
         call("pa_moments_finalize", n, ptr(part), ptr(chp), 0, ptr(chan), ptr(out), B, stream)

@@ -534,3 +534,35 @@ def test_ragged_batch_with_vacuum_element(dev):
         engine.run_batch(w1, t1, np.zeros(1), ns[b:b + 1], seed=3, rid=np.array([b]), field_out=o1, reduce=False,
                          separable=False)
         assert torch.equal(out[b], o1[0]), b
+
+
+@pytest.mark.parametrize("n", [64, 128, 256, 1024, 4096])
+@pytest.mark.parametrize("npup", [0, 1, 8])
+def test_field_moments_match_numpy(dev, n, npup):
+    """Moments and pupil sums of given fields on every tile geometry, with pupils
+    that hold the whole grid, a few columns, or nothing, at 16-byte aligned and
+    unaligned fields, fixed and centroid-tracked: float64 sums of the same
+    terms on both sides, so 1e-12 of the sum of their magnitudes; the pupils
+    hold exactly the same elements."""
+    g = torch.Generator(device=dev).manual_seed(n + npup)
+    buf = torch.randn(2 * n * n + 1, 2, device=dev, generator=g)
+    u = torch.view_as_complex(buf)[1:].view(2, n, n)
+    delta = 2.0 / n
+    pupils = [(0.3, 0.1, -0.2), (9.0, 0.0, 0.0), (0.4 * delta, 0.0, 0.0), (0.2, 5.0, 0.0), (0.5, -0.9, 0.9),
+              (1.0, 0.0, 0.0), (0.0, 0.0, 0.0), (1.2, 0.3, 0.3)][:npup]
+    x = (np.arange(n) - n // 2) * delta
+    for tracked in (False, True):
+        got = engine.field_moments(u, delta, pupils, tracked=tracked)
+        assert np.array_equal(got, engine.field_moments(u.clone(), delta, pupils, tracked=tracked))
+        for b in range(2):
+            f = u[b].cpu().numpy().astype(np.complex128)
+            i = (f.real ** 2 + f.imag ** 2) * delta ** 2
+            X, Y = x[None, :], x[:, None]
+            want = [i.sum(), (i * X).sum(), -(i * Y).sum(), (i * X * X).sum(), -(i * X * Y).sum(), (i * Y * Y).sum()]
+            assert np.abs(got[b, :6] - want).max() <= 1e-12 * i.sum()
+            for p, (r, sx, sy) in enumerate(pupils):
+                if tracked:
+                    sx, sy = got[b, 1], got[b, 2]
+                m = (X - sx) ** 2 + (Y + sy) ** 2 <= r ** 2
+                assert abs(got[b, 7 + p] - i[m].sum()) <= 1e-12 * i[m].sum()
+        assert np.all(got[:, 7 + npup:] == 0)
