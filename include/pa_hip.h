@@ -171,7 +171,7 @@ int pa_ensemble_accumulate(int batch, const double* moments, const int* slot_cha
 /* pa_field_partials followed by pa_moments_finalize without the caller's
  * partials buffer: no counterpart in pyAtmosphere.  For callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops): the
- * per-tile partials go to a fixed 8 MiB device array inside the library (one
+ * per-tile partials go to a fixed 16 MiB device array inside the library (one
  * per GPU, held until the process ends), so the call allocates nothing; u,
  * chparam, pup, pup_moments, chan and out[b][PA_NUM_MOMENTS] are as for
  * pa_field_partials / pa_moments_finalize, and the results are identical.

@@ -56,8 +56,7 @@ int apply_pupil(int n, float2* u, double delta, double radius, double sx, double
 int ensemble_accumulate(int batch, const double* mom, const int* slot_chan, int nchan, int npup, int beam_cap,
                         int pdt_cap, double* acc, long long* counts, unsigned long long* hist, hipStream_t s);
 int hbm_stream(int kind, const void* src, void* dst, long long bytes, int unroll, int nt, hipStream_t s);
-long long static_scratch_bytes();
-long long moments_scratch_bytes(int n, int batch);
+int static_max_fields(int n);
 int field_moments_static(int n, const float2* u, const double* chparam, const double* pup, int npup,
                          const double* pup_moments, const int* chan, double* out, int batch, hipStream_t s);
 int fill_twiddles(int n, float2* tw, hipStream_t s);
@@ -241,7 +240,7 @@ int pa_field_moments_static(int n, const void* u, const double* chparam, const d
                             const double* pup_moments, const int* chan, double* out, int batch, void* stream) {
   REQUIRE_N(n);
   REQUIRE(batch > 0, "field_moments_static: batch must be positive");
-  if (moments_scratch_bytes(n, batch) > static_scratch_bytes())
+  if (batch > static_max_fields(n))
     return set_error(PA_ERR_SIZE, "field_moments_static: batch * (n / tile rows) * PA_PART_SUMS * 8 bytes of "
                                   "partials exceed the library's static scratch (pa_field_moments_static_max)");
   REQUIRE(u && chparam && out, "field_moments_static: null argument");
@@ -272,7 +271,7 @@ int pa_fft_screen(int n, const void* coeff, void* work, const void* sub, int nsu
 
 int pa_field_moments_static_max(int n) {
   REQUIRE_N(n);
-  return (int)(static_scratch_bytes() / moments_scratch_bytes(n, 1));
+  return static_max_fields(n);
 }
 
 int pa_spectral_draw(int points, const float* base, const float* sqrt_psd, const int* chan,

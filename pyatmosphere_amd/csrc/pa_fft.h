@@ -145,12 +145,20 @@ __host__ __device__ __forceinline__ void dft(float2 (&u)[R]) {
 template <int N>
 struct Plan;
 // E: points per thread; R0..R2: radices (0 = unused); T: rows per tile of the
-// field layout and per row-pass block; C: columns per column-pass block.
+// field layout and per row-pass block; C: columns per column-pass block.  T
+// makes row-pass blocks of 128 (256^2) to 256 or 512 threads: the fewer waves
+// meet at a block's barriers the better its loads overlap its transforms, down
+// to the T C 8-byte runs of the column pass (128 bytes and more where T is not
+// 2).  Measured, T against twice that: k_row_mid 8.4 against 10.8 us (one
+// 1024^2 field), 100 against 108 (27), 5.0 against 6.5 (one 512^2), 230 against
+// 242 (256); k_row_last 242 against 276 (128 of 1024^2).  At 2048 half the T
+// slows the column pass (967 against 867 us, 64 fields), at 4096 twice the T
+// the row passes (167 against 135 us, two fields).
 template <> struct Plan<64>   { static constexpr int E = 8,  NP = 2, R0 = 8,  R1 = 8,  R2 = 0,  T = 8,  C = 16; };
 template <> struct Plan<128>  { static constexpr int E = 16, NP = 2, R0 = 16, R1 = 8,  R2 = 0,  T = 8,  C = 16; };
-template <> struct Plan<256>  { static constexpr int E = 16, NP = 2, R0 = 16, R1 = 16, R2 = 0,  T = 16, C = 16; };
-template <> struct Plan<512>  { static constexpr int E = 8,  NP = 3, R0 = 8,  R1 = 8,  R2 = 8,  T = 8,  C = 8; };
-template <> struct Plan<1024> { static constexpr int E = 16, NP = 3, R0 = 16, R1 = 8,  R2 = 8,  T = 8,  C = 8; };
+template <> struct Plan<256>  { static constexpr int E = 16, NP = 2, R0 = 16, R1 = 16, R2 = 0,  T = 8,  C = 16; };
+template <> struct Plan<512>  { static constexpr int E = 8,  NP = 3, R0 = 8,  R1 = 8,  R2 = 8,  T = 4,  C = 8; };
+template <> struct Plan<1024> { static constexpr int E = 16, NP = 3, R0 = 16, R1 = 8,  R2 = 8,  T = 4,  C = 8; };
 template <> struct Plan<2048> { static constexpr int E = 16, NP = 3, R0 = 16, R1 = 16, R2 = 8,  T = 4,  C = 4; };
 template <> struct Plan<4096> { static constexpr int E = 16, NP = 3, R0 = 16, R1 = 16, R2 = 16, T = 2,  C = 2; };
 

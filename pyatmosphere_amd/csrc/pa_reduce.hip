@@ -284,15 +284,18 @@ int moments_finalize(int n, const double* part, const double* chparam, int npup,
 // (different streams, or threads) race; calls in one stream do not.  Nothing
 // needs clearing: k_field_partials writes every partial k_moments_finalize
 // reads.
-constexpr long long kStaticScratchBytes = 8ll << 20;
+constexpr long long kStaticScratchBytes = 16ll << 20;
 static __device__ __align__(256) double scratch[kStaticScratchBytes / sizeof(double)];
 
-long long static_scratch_bytes() { return kStaticScratchBytes; }
-
-long long moments_scratch_bytes(int n, int batch) {
+// Fields per call.  The limit is that of 8 MiB of partials for tiles of at least
+// these heights; the tiles of 256^2 to 1024^2 grids are half as high, for which
+// the array has its other half.
+int static_max_fields(int n) {
   const int T = tile_rows(n);
   if (T <= 0) return T;
-  return (long long)batch * (n / T) * kMaxSums * (long long)sizeof(double);
+  const int rows = n == 256 ? 16 : n == 512 || n == 1024 ? 8 : T;
+  static_assert(Geo<256>::T >= 8 && Geo<512>::T >= 4 && Geo<1024>::T >= 4, "partials fit the array");
+  return (int)(kStaticScratchBytes / 2 / ((long long)(n / rows) * kMaxSums * (long long)sizeof(double)));
 }
 
 static std::mutex g_scratch_mutex;

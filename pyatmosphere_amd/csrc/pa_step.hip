@@ -161,12 +161,18 @@ k_row_mid_source(float2* __restrict__ work, const float2* __restrict__ sep, cons
 // ------------------------------------------------------------------ col_step
 // Column FFT, transfer function, inverse column FFT, in place on work[b].
 // htab layout: [channel][step][2][N] (row factor, then column factor holding s).
-// One block per item (element b, group of C columns), items element-major, so
-// the blocks the device holds at once cover one element's field; the point
-// (l + L e, c) of the tiled field is at the lane offset of e = 0 plus e L N
-// points (L is a multiple of T), one buffer load per point with the stride in
-// the instruction's SGPR offset.  (Measured: a persistent form that prefetches
-// the next item, and non-temporal hints, are both slower for this pass.)
+// One block per item (element b, group of C columns).  Consecutive blocks go
+// round-robin over the 8 XCDs, each with an L2 of its own, so each XCD takes a
+// contiguous eighth of every element's groups: neighbouring groups share cache
+// lines (a run of C columns is 32 bytes of a tile at 4096^2) and DRAM pages, and
+// elements that have no such step leave no XCD idle.  Measured against
+// element-major blocks: 72 against 134 us for a 4096^2 field, 867 against 908
+// for 64 of 2048^2, 205 against 215 for 256 of 512^2, the same at 1024^2.  The
+// point (l + L e, c) of the tiled field is at the lane offset of e = 0 plus
+// e L N points (L is a multiple of T), one buffer load per point with the
+// stride in the instruction's SGPR offset.  (Measured: a persistent form that
+// prefetches the next item, and non-temporal hints, are both slower for this
+// pass.)
 template <int N, int C>
 __global__ void __launch_bounds__(C * Geo<N>::L)
 k_col_step(float2* __restrict__ work, const float2* __restrict__ htab,
@@ -176,12 +182,19 @@ k_col_step(float2* __restrict__ work, const float2* __restrict__ htab,
   static_assert((C * L) % 64 == 0 && C * L <= 1024 && N % C == 0, "column group");
   __shared__ float2 lds[C * Geo<N>::LINE_COL];
   __shared__ float2 s_tw[TwTable<N>::SIZE];
-  const int item = blockIdx.x;
-  const int b = item / G;
+  int b, g;
+  if constexpr (G % 8 == 0) {
+    const int j = blockIdx.x / 8;
+    b = j / (G / 8);
+    g = (blockIdx.x % 8) * (G / 8) + j % (G / 8);
+  } else {
+    b = blockIdx.x / G;
+    g = blockIdx.x % G;
+  }
   if (nsteps && step >= nsteps[b] + 1) return;  // this element has no step `step`
   int cc, l;
   col_map<N, C>(threadIdx.x, cc, l);
-  const int c = (item - b * G) * C + cc;
+  const int c = g * C + cc;
   const rsrc_t rf = make_rsrc(work + (size_t)b * N * N, N * N * 8);
   const int fo = (((l / T) * N + c) * T + l % T) * 8;
   float2 v[E];
@@ -544,11 +557,29 @@ static int launch_col_group(float2* work, const float2* htab, const int* chan, c
   }
 }
 
+// With no choice given: half the layout's columns where that is faster.  Smaller
+// blocks overlap their loads and transforms better; longer runs use HBM better.
+// Half wins where the default's blocks would be fewer than four per CU (5.0
+// against 6.1 us for one 512^2 field, 5.0 against 5.8 of 256^2), at 1024^2 (8.4
+// against 10.4 us for one field, 81 against 95 for 32, 398 against 400 for 128),
+// and at 2048^2 while the batch's fields stay in the 256 MB Infinity Cache (52
+// against 61 us for 4; past it 900 against 867 for 64).  At 4096^2 half is one
+// column, and slower throughout.
+template <int N>
+static int col_group_default(int batch) {
+  constexpr int C = Geo<N>::C;
+  if (N > 2048 || !col_group_ok(N, Geo<N>::L, C / 2)) return C;
+  const bool few = (long long)(N / C) * batch <= 1024;
+  const bool cached = N == 2048 && (long long)batch * N * N * 8 <= (256ll << 20);
+  return few || cached || N == 1024 ? C / 2 : C;
+}
+
 template <int N>
 static int launch_col_step(float2* work, const float2* htab, const int* chan, const int* nsteps,
                            int step, int max_steps, const float2* tw, int cols, int batch, hipStream_t s) {
   constexpr int C = Geo<N>::C;
-  if (cols == 0 || cols == C) return launch_col_group<N, C>(work, htab, chan, nsteps, step, max_steps, tw, batch, s);
+  if (cols == 0) cols = col_group_default<N>(batch);
+  if (cols == C) return launch_col_group<N, C>(work, htab, chan, nsteps, step, max_steps, tw, batch, s);
   if (C / 2 >= 1 && cols == C / 2)
     return launch_col_group<N, (C / 2 >= 1 ? C / 2 : 1)>(work, htab, chan, nsteps, step, max_steps, tw, batch, s);
   if (cols == 2 * C) return launch_col_group<N, 2 * C>(work, htab, chan, nsteps, step, max_steps, tw, batch, s);

@@ -566,3 +566,30 @@ def test_field_moments_match_numpy(dev, n, npup):
                 m = (X - sx) ** 2 + (Y + sy) ** 2 <= r ** 2
                 assert abs(got[b, 7 + p] - i[m].sum()) <= 1e-12 * i[m].sum()
         assert np.all(got[:, 7 + npup:] == 0)
+
+
+@pytest.mark.parametrize("n,batch", [(64, 3), (128, 5), (256, 64), (256, 65), (512, 16), (512, 17), (1024, 3),
+                                     (2048, 2), (2048, 9), (4096, 1)])
+def test_default_column_groups(dev, n, batch):
+    """The default column group on either side of each of its lines gives the
+    bits of every explicit choice, elements without the step stay as they were,
+    and the last element's field is as the FP32 transform pair gives it."""
+    from pyatmosphere_amd import autotune
+    g = torch.Generator(device=dev).manual_seed(n)
+    field = torch.view_as_complex(torch.randn(batch, n, n, 2, device=dev, generator=g))
+    h = torch.polar(torch.ones(1, 3, 2, n, device=dev), 6.0 * torch.rand(1, 3, 2, n, device=dev, generator=g)) / n
+    ns = torch.full((batch,), 5, dtype=torch.int32, device=dev)
+    ns[0] = 0 if batch > 1 else 5           # element 0 has no step 1
+    out = []
+    for cols in (0,) + tuple(autotune.col_groups(n)):
+        w = field.clone()
+        engine.call("pa_col_step", n, engine.ptr(w), engine.ptr(h), None, engine.ptr(ns), 1, 3,
+                    engine.ptr(engine.twiddles(n, dev)), cols, batch, engine._lib.stream_handle())
+        out.append(w)
+    assert all(torch.equal(out[0], w) for w in out[1:])
+    assert batch == 1 or torch.equal(out[0][0], field[0])
+    T = engine.call("pa_tile_rows", n)
+    rows = lambda w: w.reshape(n // T, n, T).transpose(1, 2).reshape(n, n).to(torch.complex128)  # noqa: E731
+    spec = torch.fft.fft(rows(field[-1]), dim=0) * (h[0, 1, 0][:, None] * h[0, 1, 1][None, :])
+    want = torch.fft.ifft(spec, dim=0) * n
+    assert (rows(out[0][-1]) - want).norm() <= 2e-6 * want.norm()
