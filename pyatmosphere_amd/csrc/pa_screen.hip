@@ -287,11 +287,11 @@ constexpr int kLRCoefH = 8 + kLR * kLR, kLRCoefG = kLRCoefH + kLR;   // sparam o
 constexpr int kLRThreads = 512;                                       // waves 0-3: G, 4-7: h and g
 static_assert(PA_LOWRANK_TERMS == 32, "the block is 32 K columns (kbeg = 2 d0 - 32)");
 static_assert(2 * kLRChunk <= kLRThreads && kLRThreads == 512 && kLRChunk == 64, "polynomial block split");
-constexpr int kLRMaxPoints = 1024;   // cap on d0
-constexpr int kLRMaxChunks = kLRMaxPoints / kLRChunk;
+constexpr int kLRMaxPoints = 4096;   // cap on d0
+constexpr int kLRAhead = 16;         // chunks' partials in flight in the sum
 static inline int lowrank_chunks(int P) { return (std::min(P, kLRMaxPoints) + kLRChunk - 1) / kLRChunk; }
 constexpr int kColLowMax = 64;       // column-smooth points per element (LDS rows of the A tables)
-constexpr int kClassThreads = 1024;   // points that may move: the first 1024 (the low radii)
+constexpr int kClassThreads = 1024;   // points that may move: the first 4096 (the low radii), up to 4 per thread
 // sparam slots of the grouping: [4] kbeg, [5] d0, [7] n2
 constexpr int kSpKbeg = 4, kSpD0 = 5, kSpN2 = 7;
 
@@ -317,6 +317,12 @@ __device__ __forceinline__ int block_rank(bool flag, int& total, int* s_w) {
   return pre + below;
 }
 
+// CH points per thread (k = thread + 1024 c): every point that may move is in
+// registers before the first one is written.  With one point per thread the
+// block would hold at most 1024 points, which at 4096 points and 4096^2 left
+// over 1500 smooth points to the GEMM (K 6176 instead of about 3100; 10.1 ms for
+// 20 screens instead of 5.1).
+template <int CH>
 __global__ void __launch_bounds__(kClassThreads)
 k_screen_classify(int n, int P, double2* __restrict__ fxy, const double* __restrict__ chparam,
                   const int* __restrict__ chan, double* __restrict__ sparam, int nc_max,
@@ -326,19 +332,28 @@ k_screen_classify(int n, int P, double2* __restrict__ fxy, const double* __restr
   const int ch = chan ? chan[b] : 0;
   const double X = 0.5 * n * chparam[ch * kChParams + 0];
   double* sp = sparam + (size_t)b * PA_SCREEN_PARAMS;
-  const int G = min(P, kClassThreads), k = threadIdx.x;
+  const int G = min(P, CH * kClassThreads);
   __shared__ int s_w[kClassThreads / 64];
-  double2 f = make_double2(0.0, 0.0), a = make_double2(0.0, 0.0);
-  int cls = 3;
-  if (k < G) {
-    f = fxy[((size_t)b * P + k) * 2];
-    a = fxy[((size_t)b * P + k) * 2 + 1];
-    const bool col = fabs(kTwoPi * f.x) * X <= kLowRankZ, row = fabs(kTwoPi * f.y) * X <= kLowRankZ;
-    cls = col && row ? 0 : col ? 1 : 2;
+  double2 f[CH], a[CH];
+  int cls[CH], e0[CH], e1[CH], n2 = 0, n1 = 0;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int k = threadIdx.x + c * kClassThreads;
+    f[c] = a[c] = make_double2(0.0, 0.0);
+    cls[c] = 3;
+    if (k < G) {
+      f[c] = fxy[((size_t)b * P + k) * 2];
+      a[c] = fxy[((size_t)b * P + k) * 2 + 1];
+      const bool col = fabs(kTwoPi * f[c].x) * X <= kLowRankZ, row = fabs(kTwoPi * f[c].y) * X <= kLowRankZ;
+      cls[c] = col && row ? 0 : col ? 1 : 2;
+    }
+    // ranks among all points of the class, in point order
+    int t0, t1;
+    e0[c] = n2 + block_rank(cls[c] == 0, t0, s_w);
+    e1[c] = n1 + block_rank(cls[c] == 1, t1, s_w);
+    n2 += t0;
+    n1 += t1;
   }
-  int n2, n1;
-  const int e0 = block_rank(cls == 0, n2, s_w);
-  const int e1 = block_rank(cls == 1, n1, s_w);
   const int nc = min(n1, nc_max);
   int d0 = min((n2 + nc) / 16 * 16, kLRMaxPoints);
   if (d0 < 32) d0 = 0;
@@ -347,11 +362,16 @@ k_screen_classify(int n, int P, double2* __restrict__ fxy, const double* __restr
     sp[kSpD0] = d0;
     sp[kSpN2] = min(n2, d0);
   }
-  if (!d0 || k >= G) return;   // no block: the points stay as drawn
+  if (!d0) return;   // no block: the points stay as drawn
   // every point was loaded (into registers) before the barriers above
-  const int slot = cls == 0 ? e0 : (cls == 1 && e1 < nc) ? n2 + e1 : n2 + nc + (k - e0 - min(e1, nc));
-  fxy[((size_t)b * P + slot) * 2] = f;
-  fxy[((size_t)b * P + slot) * 2 + 1] = a;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int k = threadIdx.x + c * kClassThreads;
+    if (k >= G) continue;
+    const int slot = cls[c] == 0 ? e0[c] : (cls[c] == 1 && e1[c] < nc) ? n2 + e1[c] : n2 + nc + (k - e0[c] - min(e1[c], nc));
+    fxy[((size_t)b * P + slot) * 2] = f[c];
+    fxy[((size_t)b * P + slot) * 2 + 1] = a[c];
+  }
 }
 
 __global__ void __launch_bounds__(kLRThreads)
@@ -454,16 +474,18 @@ k_screen_lowrank_sum(int P, const double2* __restrict__ fxy, double* __restrict_
   double* sp = sparam + (size_t)b * PA_SCREEN_PARAMS;
   const int d0 = (int)sp[kSpD0], n2 = (int)sp[kSpN2];
   if (!d0) return;   // prep's scales stand
-  const int used = (d0 + kLRChunk - 1) / kLRChunk;   // <= chunks <= kLRMaxChunks
+  const int used = (d0 + kLRChunk - 1) / kLRChunk;   // <= chunks
   __shared__ double s_g[kLR * kLR];
   for (int e = threadIdx.x; e < kLRSums; e += 1024) {
     const double* pb = part + (size_t)b * chunks * kLRSums + e;
-    double v[kLRMaxChunks];
-#pragma unroll
-    for (int c = 0; c < kLRMaxChunks; ++c) v[c] = c < used ? pb[(size_t)c * kLRSums] : 0.0;
     double sum = 0.0;
+    for (int c0 = 0; c0 < used; c0 += kLRAhead) {
+      double v[kLRAhead];
 #pragma unroll
-    for (int c = 0; c < kLRMaxChunks; ++c) sum += v[c];
+      for (int c = 0; c < kLRAhead; ++c) v[c] = c0 + c < used ? pb[(size_t)(c0 + c) * kLRSums] : 0.0;
+#pragma unroll
+      for (int c = 0; c < kLRAhead; ++c) sum += v[c];
+    }
     sp[8 + e] = sum;
     if (e < kLR * kLR) s_g[e] = sum;
   }
@@ -1328,8 +1350,13 @@ static void tables_launch(int n, int P, double* fxy, double* sparam,
   double* part = reinterpret_cast<double*>(opb);
   double2* pcoef = reinterpret_cast<double2*>(part + (size_t)batch * chunks * kLRSums);
   double2* f2 = reinterpret_cast<double2*>(fxy);
-  hipLaunchKernelGGL(k_screen_classify, dim3(batch), dim3(kClassThreads), 0, s, n, P, f2, chparam, chan, sparam,
-                     nc_max, nsteps, step);
+#define CL_(CH)                                                                                                       \
+  hipLaunchKernelGGL(k_screen_classify<CH>, dim3(batch), dim3(kClassThreads), 0, s, n, P, f2, chparam, chan, sparam, \
+                     nc_max, nsteps, step)
+  if (P <= kClassThreads) CL_(1);
+  else if (P <= 2 * kClassThreads) CL_(2);
+  else CL_(4);
+#undef CL_
   hipLaunchKernelGGL(k_screen_lowrank_part, dim3(batch, chunks), dim3(kLRThreads), 0, s, n, P, f2, chparam, chan,
                      sparam, part, pcoef, nc_max, nsteps, step);
   hipLaunchKernelGGL(k_screen_lowrank_sum, dim3(batch), dim3(1024), 0, s, P, f2, sparam, part, pcoef, nc_max,

@@ -593,3 +593,54 @@ def test_default_column_groups(dev, n, batch):
     spec = torch.fft.fft(rows(field[-1]), dim=0) * (h[0, 1, 0][:, None] * h[0, 1, 1][None, :])
     want = torch.fft.ifft(spec, dim=0) * n
     assert (rows(out[0][-1]) - want).norm() <= 2e-6 * want.norm()
+
+
+@pytest.mark.parametrize("P", [1024, 1025, 2048, 2500, 4096, 4200])
+def test_polynomial_block_past_1024_points(dev, P):
+    """Points grouped several per thread: the grouping is the stable one of the
+    first 4096 points (both axes smooth, then at most 64 smooth along the columns
+    as far as multiples of 16 reach, then the rest; points past 4096 stay), the
+    polynomial block's sums are numpy's over those slots, and the screen is
+    within the split GEMM's 2e-5 rad of the plane-wave sum."""
+    from scipy.special import jv
+    n, T = 256, 32
+    spec = channel_spec(n, 0.002, 808e-9, 0.05, 5e3, 3, P, 1e-15)
+    spectra, per_real = host_spectra(spec, 1, seed=P)
+    tables = engine.DeviceTables([spec], dev)
+    ws = engine.Workspace(n, P, 1, "f16x3", dev)
+    engine.upload_spectra(ws, *spectra[0], batch=1)
+    ws.chan[:1].zero_()
+    engine.prep_screen(ws, tables, 0, 1, None, None)
+    drawn = ws.fxy[0].cpu().numpy().copy()
+    engine.synth_screen(ws, tables, 0, 1, None, None, phi2=ws.phi2_buffer(), prepped=True)
+    X = n / 2 * spec.delta
+    low = np.abs(2 * np.pi * drawn[:4096, :2]) * X <= 14
+    both = np.nonzero(low[:, 0] & low[:, 1])[0]
+    cols = np.nonzero(low[:, 0] & ~low[:, 1])[0][:64]
+    d0 = (len(both) + len(cols)) // 16 * 16
+    rest = np.setdiff1d(np.arange(P), np.concatenate([both, cols]))
+    order = np.concatenate([both, cols, rest])
+    assert np.all(rest[rest >= 4096] == np.arange(4096, P)) and d0 > min(P, 1024) // 2
+    f, sp = ws.fxy[0].cpu().numpy(), ws.sparam[0].cpu().numpy()
+    n2 = min(len(both), d0)
+    assert (sp[4], sp[5], sp[7]) == (2 * d0 - 32, d0, n2)
+    assert np.array_equal(f, drawn[order])
+    m = np.arange(T)
+
+    def coef(w):
+        c = 2 * (1j) ** m[None, :] * jv(m[None, :], (2 * np.pi * w * X)[:, None])
+        c[:, 0] = c[:, 0] / 2 - 1
+        return c
+    a = f[:, 2] + 1j * f[:, 3]
+    Q, Pm = coef(f[:d0, 1]), coef(f[:d0, 0])
+    scale = 4 * np.abs(a[:d0]).sum()
+    G = ((a[:n2, None] * Q[:n2]).T @ Pm[:n2]).real
+    assert np.abs(sp[8:8 + T * T].reshape(T, T) - G).max() < 1e-13 * scale
+    assert np.abs(sp[8 + T * T:8 + T * T + T] - (a[:n2] @ Q[:n2]).real).max() < 1e-13 * scale
+    assert np.abs(sp[8 + T * T + T:8 + T * T + 2 * T] - (a[:d0] @ Pm).real).max() < 1e-13 * scale
+    phi = torch.empty(1, n, n, dtype=torch.float32, device=dev)
+    engine.call("pa_screen_compose", n, engine.ptr(ws.sparam), engine.ptr(ws.hg), engine.ptr(ws.phi2),
+                engine.ptr(phi), 1, None)
+    ref = o.screen_phase(n, spec.delta, per_real[0][0])
+    excess = np.abs(phi[0].cpu().numpy().astype(np.float64) - ref) - np.abs(ref) * 2 ** -24
+    assert excess.max() < 2e-5
