@@ -109,8 +109,8 @@ def timed_region(engine, torch, ws, tables, B, steps, warmup, seed):
         sep = engine.SEPARABLE_SOURCE
         angs = None
         if engine.SYNTH_WHOLE_BATCH and run.whole_batch_synthesis():
-            # all screens' synthesis first: the draw per screen, the tables and
-            # the GEMM once over the S x B (screen, realization) pairs
+            # all screens' synthesis first: the draws, the tables and the GEMM once
+            # each over the S x B (screen, realization) pairs
             angs = run.synthesize_all(seed, timed=lambda name, fn: timed(name, fn, record))
         timed("source_fresnel" if sep else "row_first", lambda: run.begin(None, sep), record)
         for k in range(S + 1):
@@ -435,7 +435,7 @@ def main():
     issued = 1.0 if args.mode == "f32" else 3.0
     peak = 157.3 if args.mode == "f32" else F16_PEAK_TFLOPS
     # the chain's time per B screens
-    t_chain = ((kt["screen_gemm"] + kt["screen_tables"]) * B / G + kt["screen_draw_prep"]) * 1e-3
+    t_chain = (kt["screen_gemm"] + kt["screen_tables"] + kt["screen_draw_prep"]) * B / G * 1e-3
     # HBM-bound FFT passes: algorithmic bytes per element (read + write the
     # field; the row pass also reads the float32 screen angle)
     # (bytes per element, the streaming ceiling of the same direction)

@@ -232,12 +232,24 @@ int pa_screen_prep(int points, const float* rho, const float* theta, const void*
 int pa_screen_draw_prep(int points, const float* base, const float* sqrt_psd, const int* chan,
                         const uint64_t* rid, uint64_t seed, int screen, double* fxy, double* sparam, int mode,
                         const double* chparam, const int* nsteps, int step, int batch, void* stream);
+/* pa_screen_draw_prep of screens 0 .. screens - 1 of every element in one launch:
+ * element v = screen * batch + b of fxy and sparam holds screen `screen` of
+ * element b (chan, rid and nsteps are per element b, as for one screen). */
+int pa_screens_draw_prep(int points, const float* base, const float* sqrt_psd, const int* chan, const uint64_t* rid,
+                         uint64_t seed, int screens, double* fxy, double* sparam, int mode, const double* chparam,
+                         const int* nsteps, int batch, void* stream);
 int pa_screen_tables(int n, int points, double* fxy, double* sparam, const double* chparam,
                      const int* chan, void* opa, void* opb, double* hg, void* esc, int mode, int rows,
                      const int* nsteps, int step, int batch, void* stream);
 int pa_screen_gemm(int n, int points, const void* opa, const void* opb, const double* sparam,
                    const void* esc, float* phi2, float* ang, void* fac, int mode, int tile,
                    const int* nsteps, int step, int batch, void* stream);
+/* pa_screen_gemm followed by pa_screen_compose: the full screen phi (row-major
+ * float32, the same bits) from the GEMM itself, and the screen angle ang
+ * (nullable, as pa_screen_gemm writes it). */
+int pa_screen_gemm_compose(int n, int points, const void* opa, const void* opb, const double* sparam, const void* esc,
+                           const double* hg, float* phi, float* ang, int mode, int tile, const int* nsteps, int step,
+                           int batch, void* stream);
 /* Full screen phi = phi0 + h(r) + g(c) + phi2 as a row-major float32 array
  * (the value PhaseScreen.generate returns, phase_screens.py:25-28). */
 int pa_screen_compose(int n, const double* sparam, const double* hg, const float* phi2,
@@ -270,6 +282,10 @@ int pa_structure_function(int n, const float* phi, double* scratch, double* out,
 /* u[b] *= mask(pupil) for row-major fields (pupils.py:8-13). */
 int pa_apply_pupil(int n, void* u, double delta, double radius, double shift_x, double shift_y,
                    int batch, void* stream);
+
+/* out[b] = u[b] * mask(pupil) as a new row-major field (out must not overlap u). */
+int pa_pupil_output(int n, const void* u, void* out, double delta, double radius, double shift_x, double shift_y,
+                    int batch, void* stream);
 
 /* out[b][r][c] = gy[b][r] * gx[b][c]: the separable Gaussian source field
  * (theory/sources.py:16-18 on RectGrid.get_rho2, grids.py:74-76). */

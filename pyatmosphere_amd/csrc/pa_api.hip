@@ -38,13 +38,13 @@ int screen_prep(int P, const float* rho, const float* theta, const float2* value
                 int batch, hipStream_t s);
 int screen_draw_prep(int P, const float* base, const float* sqrt_psd, const int* chan, const uint64_t* rid,
                      uint64_t seed, int screen, double* fxy, double* sparam, int mode, const double* chparam,
-                     const int* nsteps, int step, int batch, hipStream_t s);
+                     const int* nsteps, int step, int screens, int batch, hipStream_t s);
 int screen_tables(int n, int P, double* fxy, double* sparam,
                   const double* chparam, const int* chan, void* opa, void* opb, double* hg,
                   float2* esc, int mode, int rows, const int* nsteps, int step, int batch, hipStream_t s);
 int screen_gemm(int n, int P, const void* opa, const void* opb, const double* sparam, const float2* esc,
-                float* phi2, float* ang, float2* fac, int mode, int tile, const int* nsteps, int step, int batch,
-                hipStream_t s);
+                float* phi2, float* ang, float2* fac, const double* hg, float* phi, int mode, int tile,
+                const int* nsteps, int step, int batch, hipStream_t s);
 int screen_compose(int n, const double* sparam, const double* hg, const float* phi2, float* phi,
                    int batch, hipStream_t s);
 int field_partials(int n, const float2* u, double* part, const double* chparam, const double* pup,
@@ -53,6 +53,8 @@ int moments_finalize(int n, const double* part, const double* chparam, int npup,
                      double* out, int batch, hipStream_t s);
 int apply_pupil(int n, float2* u, double delta, double radius, double sx, double sy, int batch,
                 hipStream_t s);
+int pupil_output(int n, const float2* u, float2* out, double delta, double radius, double sx, double sy, int batch,
+                 hipStream_t s);
 int ensemble_accumulate(int batch, const double* mom, const int* slot_chan, int nchan, int npup, int beam_cap,
                         int pdt_cap, double* acc, long long* counts, unsigned long long* hist, hipStream_t s);
 int hbm_stream(int kind, const void* src, void* dst, long long bytes, int unroll, int nt, hipStream_t s);
@@ -300,6 +302,17 @@ int pa_screen_draw_prep(int points, const float* base, const float* sqrt_psd, co
   REQUIRE(base && sqrt_psd && rid && fxy && sparam && chparam, "screen_draw_prep: null argument");
   REQUIRE(mode >= 0 && mode <= 2, "screen_draw_prep: unknown GEMM mode");
   return screen_draw_prep(points, base, sqrt_psd, chan, rid, seed, screen, fxy, sparam, mode, chparam, nsteps, step,
+                          1, batch, STREAM(stream));
+}
+
+int pa_screens_draw_prep(int points, const float* base, const float* sqrt_psd, const int* chan, const uint64_t* rid,
+                         uint64_t seed, int screens, double* fxy, double* sparam, int mode, const double* chparam,
+                         const int* nsteps, int batch, void* stream) {
+  REQUIRE(points > 0 && batch > 0, "screens_draw_prep: points and batch must be positive");
+  REQUIRE(screens > 0 && screens <= 65535, "screens_draw_prep: screens must be in 1..65535");
+  REQUIRE(base && sqrt_psd && rid && fxy && sparam && chparam, "screens_draw_prep: null argument");
+  REQUIRE(mode >= 0 && mode <= 2, "screens_draw_prep: unknown GEMM mode");
+  return screen_draw_prep(points, base, sqrt_psd, chan, rid, seed, 0, fxy, sparam, mode, chparam, nsteps, 0, screens,
                           batch, STREAM(stream));
 }
 
@@ -321,7 +334,18 @@ int pa_screen_gemm(int n, int points, const void* opa, const void* opb, const do
   REQUIRE(opa && opb && sparam && esc && (phi2 || ang || fac), "screen_gemm: null argument");
   REQUIRE(mode >= 0 && mode <= 2, "screen_gemm: unknown GEMM mode");
   return screen_gemm(n, points, opa, opb, sparam, reinterpret_cast<const float2*>(esc), phi2, ang,
-                     reinterpret_cast<float2*>(fac), mode, tile, nsteps, step, batch, STREAM(stream));
+                     reinterpret_cast<float2*>(fac), nullptr, nullptr, mode, tile, nsteps, step, batch, STREAM(stream));
+}
+
+int pa_screen_gemm_compose(int n, int points, const void* opa, const void* opb, const double* sparam, const void* esc,
+                           const double* hg, float* phi, float* ang, int mode, int tile, const int* nsteps, int step,
+                           int batch, void* stream) {
+  REQUIRE_N(n);
+  REQUIRE(points > 0 && batch > 0, "screen_gemm_compose: points and batch must be positive");
+  REQUIRE(mode >= 0 && mode <= 2, "screen_gemm_compose: unknown GEMM mode");
+  REQUIRE(opa && opb && sparam && esc && hg && phi, "screen_gemm_compose: null argument");
+  return screen_gemm(n, points, opa, opb, sparam, reinterpret_cast<const float2*>(esc), nullptr, ang, nullptr, hg, phi,
+                     mode, tile, nsteps, step, batch, STREAM(stream));
 }
 
 int pa_screen_compose(int n, const double* sparam, const double* hg, const float* phi2, float* phi,
@@ -337,6 +361,14 @@ int pa_apply_pupil(int n, void* u, double delta, double radius, double shift_x, 
   REQUIRE(u && batch > 0, "apply_pupil: null field or batch <= 0");
   return apply_pupil(n, reinterpret_cast<float2*>(u), delta, radius, shift_x, shift_y, batch,
                      STREAM(stream));
+}
+
+int pa_pupil_output(int n, const void* u, void* out, double delta, double radius, double shift_x, double shift_y,
+                    int batch, void* stream) {
+  REQUIRE_N(n);
+  REQUIRE(u && out && batch > 0, "pupil_output: null field or batch <= 0");
+  return pupil_output(n, reinterpret_cast<const float2*>(u), reinterpret_cast<float2*>(out), delta, radius, shift_x,
+                      shift_y, batch, STREAM(stream));
 }
 
 int pa_outer(int n, void* out, const void* gy, const void* gx, int batch, void* stream) {

@@ -24,13 +24,13 @@ int screen_prep(int P, const float* rho, const float* theta, const float2* value
                 hipStream_t s);
 int screen_draw_prep(int P, const float* base, const float* sqrt_psd, const int* chan, const uint64_t* rid,
                      uint64_t seed, int screen, double* fxy, double* sparam, int mode, const double* chparam,
-                     const int* nsteps, int step, int batch, hipStream_t s);
+                     const int* nsteps, int step, int screens, int batch, hipStream_t s);
 int screen_tables(int n, int P, double* fxy, double* sparam, const double* chparam, const int* chan,
                   void* opa, void* opb, double* hg, float2* esc, int mode, int rows, const int* nsteps, int step,
                   int batch, hipStream_t s);
 int screen_gemm(int n, int P, const void* opa, const void* opb, const double* sparam, const float2* esc,
-                float* phi2, float* ang, float2* fac, int mode, int tile, const int* nsteps, int step, int batch,
-                hipStream_t s);
+                float* phi2, float* ang, float2* fac, const double* hg, float* phi, int mode, int tile,
+                const int* nsteps, int step, int batch, hipStream_t s);
 int moments_finalize(int n, const double* part, const double* chparam, int npup, const int* chan, double* out,
                      int batch, hipStream_t s);
 int fill_twiddles(int n, float2* tw, hipStream_t s);
@@ -224,11 +224,11 @@ int pa_channel_run(pa_channel* c, int batch, const float* rho, const float* thet
                         c->mode, c->chparam, c->chan, nullptr, i, batch, s));
     } else {
       CHECK(screen_draw_prep(P, c->base, c->sqrt_psd, c->chan, rid, seed, i, c->fxy, c->sparam, c->mode,
-                             c->chparam, nullptr, i, batch, s));
+                             c->chparam, nullptr, i, 1, batch, s));
     }
     CHECK(screen_tables(n, P, c->fxy, c->sparam, c->chparam, c->chan, c->opa, c->opb, c->hg, c->esc, c->mode, 0,
                         nullptr, i, batch, s));
-    CHECK(screen_gemm(n, P, c->opa, c->opb, c->sparam, c->esc, nullptr, c->ang, nullptr, c->mode, 0, nullptr, i,
+    CHECK(screen_gemm(n, P, c->opa, c->opb, c->sparam, c->esc, nullptr, c->ang, nullptr, nullptr, nullptr, c->mode, 0, nullptr, i,
                       batch, s));
     if (sep && i == 0) {
       CHECK(row_mid_source(n, c->work, c->sep, c->ang, c->tw, batch, s));

@@ -201,6 +201,36 @@ __global__ void k_apply_pupil(int n, float2* __restrict__ u, double delta, doubl
     u[(size_t)b * n * n + idx] = make_float2(0.f, 0.f);
 }
 
+// out = u inside the pupil, 0 outside, as a new field: a row's columns inside are
+// one interval (circle_cols, the exact predicate), found by one thread per row
+// of the block, so the field is read inside the pupil only and nothing is
+// tested in float64 per element.  The 8 bytes written per element bound it: a
+// 1024^2 field, where a copy and a pass over it took 16).
+constexpr int kPupilRows = 8;
+__global__ void __launch_bounds__(256)
+k_pupil_output(int n, const float2* __restrict__ u, float2* __restrict__ out, double delta, double rad2, double sx,
+               double sy) {
+  __shared__ int2 s_pc[kPupilRows];
+  const size_t o = (size_t)blockIdx.y * n * n + (size_t)blockIdx.x * kPupilRows * n;
+  if (threadIdx.x < kPupilRows) {
+    int lo, hi;
+    circle_cols(n, delta, grid_offset(blockIdx.x * kPupilRows + threadIdx.x, n, delta, -sy), sx, rad2, lo, hi);
+    s_pc[threadIdx.x] = make_int2(lo, hi);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kPupilRows * n / 2; i += 256) {
+    const int r = 2 * i / n, c = 2 * i % n;
+    const int2 q = s_pc[r];
+    pa_f4c v = {0.f, 0.f, 0.f, 0.f};
+    if (q.x <= c + 1 && q.y >= c) {
+      const pa_f4c w = reinterpret_cast<const pa_f4c*>(u + o)[i];
+      if (q.x <= c && c <= q.y) v.x = w.x, v.y = w.y;
+      if (q.x <= c + 1 && c + 1 <= q.y) v.z = w.z, v.w = w.w;
+    }
+    reinterpret_cast<pa_f4c*>(out + o)[i] = v;
+  }
+}
+
 __global__ void k_expmi(int count, const float* __restrict__ x, float2* __restrict__ out) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < count) out[i] = expmi_fast(x[i]);
@@ -397,6 +427,13 @@ int apply_pupil(int n, float2* u, double delta, double radius, double sx, double
   hipLaunchKernelGGL(k_apply_pupil, dim3((n * n + 255) / 256, batch), dim3(256), 0, s, n, u, delta,
                      radius * radius, sx, sy);
   return check_launch("apply_pupil");
+}
+
+int pupil_output(int n, const float2* u, float2* out, double delta, double radius, double sx, double sy, int batch,
+                 hipStream_t s) {
+  hipLaunchKernelGGL(k_pupil_output, dim3(n / kPupilRows, batch), dim3(256), 0, s, n, u, out, delta, radius * radius, sx,
+                     sy);
+  return check_launch("pupil_output");
 }
 
 // ------------------------------------------------------------------ structure function

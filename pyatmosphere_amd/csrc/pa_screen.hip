@@ -197,10 +197,14 @@ k_screen_prep(int P, const float* __restrict__ rho, const float* __restrict__ th
 }
 
 // The spectral draw and the prep in one launch (one block of 1024 threads per
-// element): the same per-point arithmetic and the same summation order as
+// element b and screen `screen` + y, whose results go to element y batch + b of
+// fxy and sparam): the same per-point arithmetic and the same summation order as
 // k_spectral_draw followed by k_screen_prep (thread t < 256 adds points t,
 // t + 256, t + 512, ... in turn), so fxy and sparam are identical; the
-// draw's rho, theta, value are not stored.
+// draw's rho, theta, value are not stored.  A block's chain of float64 log, sine
+// and cosine bounds it (8 to 20 us whatever the batch), so all screens of a
+// batch go in one launch: 20 us instead of 196 for ten screens of 4096 points,
+// 13 instead of 130 for a mixed batch's ten.
 constexpr int kDrawPrepThreads = 1024;
 __global__ void __launch_bounds__(kDrawPrepThreads)
 k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restrict__ sqrt_psd,
@@ -208,7 +212,9 @@ k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restric
                    double* __restrict__ sparam, int mode, const double* __restrict__ chparam,
                    const int* __restrict__ chan, const int* __restrict__ nsteps, int step) {
   const int b = blockIdx.x;
-  if (nsteps && step >= nsteps[b]) return;
+  const size_t o = (size_t)blockIdx.y * gridDim.x + b;
+  screen += blockIdx.y;
+  if (nsteps && step + (int)blockIdx.y >= nsteps[b]) return;
   const int ch = chan ? chan[b] : 0;
   const uint64_t id = rid[b];
   const double x0 = chparam[ch * kChParams + 1], y0 = chparam[ch * kChParams + 2];
@@ -224,8 +230,8 @@ k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restric
       draw_point(P, base, sqrt_psd, ch, id, seed, screen, k, U, r, t, v);
       double2 f, a;
       am = prep_point(r, t, v, x0, y0, f, a);
-      fxy[((size_t)b * P + k) * 2] = f;
-      fxy[((size_t)b * P + k) * 2 + 1] = a;
+      fxy[(o * P + k) * 2] = f;
+      fxy[(o * P + k) * 2 + 1] = a;
       re = a.x;
     }
     s_re[threadIdx.x] = re;
@@ -247,7 +253,7 @@ k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restric
     s_am[threadIdx.x] = amax;
   }
   __syncthreads();
-  prep_finish(s_re, s_am, sparam + (size_t)b * PA_SCREEN_PARAMS, mode);
+  prep_finish(s_re, s_am, sparam + o * PA_SCREEN_PARAMS, mode);
 }
 
 // ------------------------------------------------------------------ polynomial block
@@ -895,11 +901,18 @@ __device__ __forceinline__ void st_nt(float* p, float a, float b) {
   __builtin_nontemporal_store(v, reinterpret_cast<pa_f2v*>(p));
 }
 
-template <int N, int MI, int NI>
+//
+// COMPOSE: also the full screen phi0 + h(r) + g(c) + phi2 (float64 sum, rounded
+// to float32) into the row-major `po`.  A template of its own, so that the batches' GEMM
+// keeps its registers; it saves the compose pass and its 8 bytes per element
+// (2048^2, one screen: 15 us of pass and 4 us of stores).
+template <int N, int MI, int NI, bool COMPOSE>
 __device__ __forceinline__ void gemm_epilogue(const f16v (&acc)[MI][NI], int m0, int n0, int r0, int c0, int lane,
                                               float inv, float* __restrict__ out, float* __restrict__ ao,
                                               float2* __restrict__ fo, const float2* seh, const float2* seg,
-                                              const float* sah, const float* sag) {
+                                              const float* sah, const float* sag, double phi0,
+                                              const double* __restrict__ h, const double* __restrict__ g,
+                                              float* __restrict__ po) {
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -913,6 +926,12 @@ __device__ __forceinline__ void gemm_epilogue(const f16v (&acc)[MI][NI], int m0,
         float v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) v[u] = acc[i][j][4 * q + u] * inv;
+        if constexpr (COMPOSE) {
+          const double gd = g[col];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            po[(size_t)(row + u) * N + col] = (float)(phi0 + h[row + u] + gd + (double)v[u]);
+        }
         if (out) {
           if constexpr (Geo<N>::T >= 4) {
             st_nt(out + tiled<N>(row, col), v[0], v[1], v[2], v[3]);
@@ -1076,12 +1095,12 @@ __device__ __forceinline__ void split_mma(f16v (&acc)[G::MI][G::NI], const Split
     }
 }
 
-template <int N, int MODE, int CFG>
+template <int N, int MODE, int CFG, bool COMPOSE>
 __global__ void __launch_bounds__((SplitGeo<N, CFG>::NT))
 k_screen_gemm_split(const void* __restrict__ opa, const void* __restrict__ opb,
                     const double* __restrict__ sparam, const float2* __restrict__ esc, float* __restrict__ phi2,
                     float* __restrict__ ang, float2* __restrict__ fac, int Kp, const int* __restrict__ nsteps,
-                    int step, int batch) {
+                    int step, int batch, const double* __restrict__ hg, float* __restrict__ phi) {
   using G = SplitGeo<N, CFG>;
   constexpr int BM = G::BM, MI = G::MI, NI = G::NI, DEPTH = G::DEPTH;
 
@@ -1176,9 +1195,12 @@ k_screen_gemm_split(const void* __restrict__ opa, const void* __restrict__ opb,
       sa[tid + u * G::NT] = -atan2f(fct[u].y, fct[u].x);
     }
   __syncthreads();
-  gemm_epilogue<N, MI, NI>(acc, m0, n0, wm * G::WM, wn * G::WN, lane, (float)sparam[(size_t)b * PA_SCREEN_PARAMS + 3],
-                           phi2 ? phi2 + (size_t)b * N * N : nullptr, ang ? ang + (size_t)b * N * N : nullptr,
-                           fac ? fac + (size_t)b * N * N : nullptr, sf, sf + BM, sa, sa + BM);
+  const double* hb = hg + (size_t)b * 2 * N;
+  gemm_epilogue<N, MI, NI, COMPOSE>(acc, m0, n0, wm * G::WM, wn * G::WN, lane,
+                                    (float)sparam[(size_t)b * PA_SCREEN_PARAMS + 3],
+                                    phi2 ? phi2 + (size_t)b * N * N : nullptr, ang ? ang + (size_t)b * N * N : nullptr,
+                                    fac ? fac + (size_t)b * N * N : nullptr, sf, sf + BM, sa, sa + BM,
+                                    sparam[(size_t)b * PA_SCREEN_PARAMS], hb, hb + N, phi + (size_t)b * N * N);
 }
 
 // ---- float32 GEMM (v_mfma_f32_32x32x2f32): the full-precision reference mode
@@ -1188,12 +1210,12 @@ struct F32Geo {
   static constexpr int NTM = N / BM, NTN = N / BN;
 };
 
-template <int N>
+template <int N, bool COMPOSE>
 __global__ void __launch_bounds__(256)
 k_screen_gemm_f32(const void* __restrict__ opa, const void* __restrict__ opb,
                   const double* __restrict__ sparam, const float2* __restrict__ esc, float* __restrict__ phi2,
                   float* __restrict__ ang, float2* __restrict__ fac, int Kp, const int* __restrict__ nsteps,
-                  int step, int batch) {
+                  int step, int batch, const double* __restrict__ hg, float* __restrict__ phi) {
   constexpr int BM = F32Geo<N>::BM, BN = F32Geo<N>::BN;
   constexpr int WM = BM / 2, WN = BN / 2, MI = WM / 32, NI = WN / 32;
   constexpr int BK = 32;
@@ -1285,9 +1307,12 @@ k_screen_gemm_f32(const void* __restrict__ opa, const void* __restrict__ opb,
     sa[tid] = -atan2f(e.y, e.x);
   }
   __syncthreads();
-  gemm_epilogue<N, MI, NI>(acc, m0, n0, wm * WM, wn * WN, lane, (float)sparam[(size_t)b * PA_SCREEN_PARAMS + 3],
-                           phi2 ? phi2 + (size_t)b * N * N : nullptr, ang ? ang + (size_t)b * N * N : nullptr,
-                           fac ? fac + (size_t)b * N * N : nullptr, sf, sf + BM, sa, sa + BM);
+  const double* hb = hg + (size_t)b * 2 * N;
+  gemm_epilogue<N, MI, NI, COMPOSE>(acc, m0, n0, wm * WM, wn * WN, lane,
+                                    (float)sparam[(size_t)b * PA_SCREEN_PARAMS + 3],
+                                    phi2 ? phi2 + (size_t)b * N * N : nullptr, ang ? ang + (size_t)b * N * N : nullptr,
+                                    fac ? fac + (size_t)b * N * N : nullptr, sf, sf + BM, sa, sa + BM,
+                                    sparam[(size_t)b * PA_SCREEN_PARAMS], hb, hb + N, phi + (size_t)b * N * N);
 }
 
 // ------------------------------------------------------------------ compose
@@ -1323,8 +1348,8 @@ int spectral_draw(int P, const float* base, const float* sqrt_psd, const int* ch
 
 int screen_draw_prep(int P, const float* base, const float* sqrt_psd, const int* chan, const uint64_t* rid,
                      uint64_t seed, int screen, double* fxy, double* sparam, int mode, const double* chparam,
-                     const int* nsteps, int step, int batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_screen_draw_prep, dim3(batch), dim3(kDrawPrepThreads), 0, s, P, base, sqrt_psd, rid, seed,
+                     const int* nsteps, int step, int screens, int batch, hipStream_t s) {
+  hipLaunchKernelGGL(k_screen_draw_prep, dim3(batch, screens), dim3(kDrawPrepThreads), 0, s, P, base, sqrt_psd, rid, seed,
                      screen, reinterpret_cast<double2*>(fxy), sparam, mode, chparam, chan, nsteps, step);
   return check_launch("screen_draw_prep");
 }
@@ -1422,10 +1447,16 @@ int screen_tables(int n, int P, double* fxy, double* sparam,
 
 template <int N, int MODE, int CFG>
 static void gemm_split_launch(int Kp, const void* opa, const void* opb, const double* sparam, const float2* esc,
-                              float* phi2, float* ang, float2* fac, const int* nsteps, int step, int batch, hipStream_t s) {
+                              float* phi2, float* ang, float2* fac, const double* hg, float* phi, const int* nsteps,
+                              int step, int batch, hipStream_t s) {
   using G = SplitGeo<N, CFG>;
-  hipLaunchKernelGGL((k_screen_gemm_split<N, MODE, CFG>), dim3(G::NTM * G::NTN * batch), dim3(G::NT), 0, s, opa,
-                     opb, sparam, esc, phi2, ang, fac, Kp, nsteps, step, batch);
+  const dim3 g(G::NTM * G::NTN * batch);
+  if (phi)
+    hipLaunchKernelGGL((k_screen_gemm_split<N, MODE, CFG, true>), g, dim3(G::NT), 0, s, opa, opb, sparam, esc, phi2,
+                       ang, fac, Kp, nsteps, step, batch, hg, phi);
+  else
+    hipLaunchKernelGGL((k_screen_gemm_split<N, MODE, CFG, false>), g, dim3(G::NT), 0, s, opa, opb, sparam, esc, phi2,
+                       ang, fac, Kp, nsteps, step, batch, hg, phi);
 }
 
 // GEMM tile: the 256 x 256 tiles when they give at least two blocks per CU
@@ -1435,29 +1466,37 @@ static int gemm_tile_default(int n, int batch) {
 
 template <int N>
 static int gemm_n(int P, const void* opa, const void* opb, const double* sparam, const float2* esc, float* phi2,
-                  float* ang, float2* fac, int mode, int tile, const int* nsteps, int step, int batch, hipStream_t s) {
+                  float* ang, float2* fac, const double* hg, float* phi, int mode, int tile, const int* nsteps, int step,
+                  int batch, hipStream_t s) {
   const int Kp = kpad(P);
   if (tile == 0) tile = gemm_tile_default(N, batch);
   if (tile != 1 && tile != 2) return set_error(PA_ERR_ARG, "screen_gemm: tile must be 0, 1 or 2");
   if (N < 512) tile = 2;   // one geometry below 512
+#define G_(MODE, CFG) \
+  gemm_split_launch<N, MODE, CFG>(Kp, opa, opb, sparam, esc, phi2, ang, fac, hg, phi, nsteps, step, batch, s)
   switch (mode) {
     case PA_GEMM_F16X3:
-      if (tile == 1) gemm_split_launch<N, PA_GEMM_F16X3, 1>(Kp, opa, opb, sparam, esc, phi2, ang, fac, nsteps, step, batch, s);
-      else gemm_split_launch<N, PA_GEMM_F16X3, 2>(Kp, opa, opb, sparam, esc, phi2, ang, fac, nsteps, step, batch, s);
+      if (tile == 1) G_(PA_GEMM_F16X3, 1);
+      else G_(PA_GEMM_F16X3, 2);
       break;
     case PA_GEMM_BF16X3:
-      if (tile == 1) gemm_split_launch<N, PA_GEMM_BF16X3, 1>(Kp, opa, opb, sparam, esc, phi2, ang, fac, nsteps, step, batch, s);
-      else gemm_split_launch<N, PA_GEMM_BF16X3, 2>(Kp, opa, opb, sparam, esc, phi2, ang, fac, nsteps, step, batch, s);
+      if (tile == 1) G_(PA_GEMM_BF16X3, 1);
+      else G_(PA_GEMM_BF16X3, 2);
       break;
     case PA_GEMM_F32: {
       const dim3 gf(F32Geo<N>::NTM * F32Geo<N>::NTN * batch);
-      hipLaunchKernelGGL((k_screen_gemm_f32<N>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang, fac, Kp, nsteps,
-                         step, batch);
+      if (phi)
+        hipLaunchKernelGGL((k_screen_gemm_f32<N, true>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang, fac, Kp,
+                           nsteps, step, batch, hg, phi);
+      else
+        hipLaunchKernelGGL((k_screen_gemm_f32<N, false>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang, fac,
+                           Kp, nsteps, step, batch, hg, phi);
       break;
     }
     default:
       return set_error(PA_ERR_ARG, "unknown GEMM mode");
   }
+#undef G_
   return check_launch("screen_gemm");
 }
 
@@ -1482,9 +1521,9 @@ static int compose_n(const double* sparam, const double* hg, const float* phi2, 
   }
 
 int screen_gemm(int n, int P, const void* opa, const void* opb, const double* sparam, const float2* esc,
-                float* phi2, float* ang, float2* fac, int mode, int tile, const int* nsteps, int step, int batch,
-                hipStream_t s) {
-#define C_(NN) gemm_n<NN>(P, opa, opb, sparam, esc, phi2, ang, fac, mode, tile, nsteps, step, batch, s)
+                float* phi2, float* ang, float2* fac, const double* hg, float* phi, int mode, int tile,
+                const int* nsteps, int step, int batch, hipStream_t s) {
+#define C_(NN) gemm_n<NN>(P, opa, opb, sparam, esc, phi2, ang, fac, hg, phi, mode, tile, nsteps, step, batch, s)
   PA_DISPATCH_N(n, C_)
 #undef C_
 }

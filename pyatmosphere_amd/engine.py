@@ -273,14 +273,14 @@ SYNTH_BATCH_MAX_BYTES = 16 << 30
 def synth_bytes_per_element(n: int, points: int, mode: int) -> int:
     """Device bytes of one (screen, realization) pair in SynthBuffers."""
     opb = call("pa_operand_bytes", n, points, mode)
-    return 2 * opb + points * 32 + _lib.PA_SCREEN_PARAMS * 8 + 2 * n * (8 + 8) + n * n * 4 + 12
+    return 2 * opb + points * (32 + 16) + _lib.PA_SCREEN_PARAMS * 8 + 2 * n * (8 + 8) + n * n * 4 + 12
 
 
 class SynthBuffers:
     """Screen synthesis of every screen of a batch as one virtual batch:
     element v = i * B + b is screen i of realization b (B the run's batch).
-    The device draw runs per screen into its slice (it takes the screen index);
-    the plane-wave tables and the GEMM then run once over all S * B pairs.
+    The draws, the plane-wave tables and the GEMM each run once over all S * B
+    pairs (host draws are uploaded in one copy).
     Every pair is computed exactly as in the screen-by-screen schedule, so the
     angles are bit-identical; what changes is five times fewer launches of the
     small latency-bound kernels, each with a five times larger grid.  Launch
@@ -303,17 +303,24 @@ class SynthBuffers:
         self.chan = e(V, dt=torch.int32)
         self.active = e(V, dt=torch.int32)
 
-    def draw_view(self, ws: "Workspace", screen: int, batch: int):
-        """The workspace as the device draw of screen `screen` sees it: the
-        batch's channels and realization ids, this screen's fxy and sparam slice."""
-        lo, hi = screen * batch, (screen + 1) * batch
-        return _View(points=self.points, mode=self.mode, chan=ws.chan, rid=ws.rid,
-                     fxy=self.fxy[lo:hi], sparam=self.sparam[lo:hi])
+        self.spectra: Optional[torch.Tensor] = None    # host draws (upload), allocated on first use
 
-
-class _View:
-    def __init__(self, **kw):
-        self.__dict__.update(kw)
+    def upload(self, host_spectra, batch: int):
+        """The host draws of every screen, (rho, theta, value) arrays (B, P) each, in
+        one copy; returns the device addresses of rho, theta, value in pair order."""
+        P, V = self.points, len(host_spectra) * batch
+        stage = torch.empty(4 * V * P, dtype=torch.float32, pin_memory=True)
+        flat = stage.numpy()
+        rho, theta = flat[:V * P].reshape(V, P), flat[V * P:2 * V * P].reshape(V, P)
+        value = flat[2 * V * P:].view(np.complex64).reshape(V, P)
+        for i, (r, t, v) in enumerate(host_spectra):
+            rho[i * batch:(i + 1) * batch], theta[i * batch:(i + 1) * batch] = r, t
+            value[i * batch:(i + 1) * batch] = v
+        if self.spectra is None:
+            self.spectra = torch.empty(4 * self.capacity * P, dtype=torch.float32, device=self.ang.device)
+        self.spectra[:4 * V * P].copy_(stage, non_blocking=True)
+        at = self.spectra.data_ptr()
+        return at, at + 4 * V * P, at + 8 * V * P
 
 
 # ---------------------------------------------------------------- pipeline pieces
@@ -336,9 +343,15 @@ def plane_wave_tables(ws: Workspace, tables: DeviceTables, step: int, batch: int
 def screen_gemm(ws: Workspace, step: int, batch: int, nsteps: Optional[torch.Tensor], stream,
                 fac: Optional[torch.Tensor] = None, esc: Optional[torch.Tensor] = None,
                 phi2: Optional[torch.Tensor] = None, ang: Optional[torch.Tensor] = None,
-                tile: Optional[int] = None) -> None:
+                tile: Optional[int] = None, phi: Optional[torch.Tensor] = None) -> None:
     """phi2 = A B^T of screen `step`, into any of: the screen angle `ang` (what
-    the row pass applies), the real phi2 `phi2`, the complex factor `fac`."""
+    the row pass applies), the real phi2 `phi2`, the complex factor `fac`; or
+    into the full row-major screen `phi` (and `ang`)."""
+    if phi is not None:
+        call("pa_screen_gemm_compose", ws.n, ws.points, ptr(ws.opa), ptr(ws.opb), ptr(ws.sparam),
+             ptr(ws.esc if esc is None else esc), ptr(ws.hg), ptr(phi), ptr(ang), ws.mode,
+             ws.gemm_tile if tile is None else tile, ptr(nsteps), step, batch, stream)
+        return
     call("pa_screen_gemm", ws.n, ws.points, ptr(ws.opa), ptr(ws.opb), ptr(ws.sparam),
          ptr(ws.esc if esc is None else esc), ptr(phi2), ptr(ang), ptr(fac), ws.mode,
          ws.gemm_tile if tile is None else tile, ptr(nsteps), step, batch, stream)
@@ -347,16 +360,18 @@ def screen_gemm(ws: Workspace, step: int, batch: int, nsteps: Optional[torch.Ten
 def synth_screen(ws: Workspace, tables: DeviceTables, step: int, batch: int,
                  nsteps: Optional[torch.Tensor], stream, fac: Optional[torch.Tensor] = None,
                  esc: Optional[torch.Tensor] = None, phi2: Optional[torch.Tensor] = None,
-                 ang: Optional[torch.Tensor] = None, prepped: bool = False) -> None:
+                 ang: Optional[torch.Tensor] = None, prepped: bool = False,
+                 phi: Optional[torch.Tensor] = None) -> None:
     """Screen `step` of every active element from ws.rho/theta/value
     (phase_screens.py:108-136): prep, plane-wave tables, GEMM.  The GEMM writes
     the screen angle into `ang` (default ws.ang), and the real phi2 and the
-    complex factor eh eg e^{-i phi2} into `phi2` / `fac` when given."""
-    ang = ws.ang if ang is None else ang
+    complex factor eh eg e^{-i phi2} into `phi2` / `fac` when given; or the full
+    row-major screen into `phi` (and the angle into `ang` when given)."""
+    ang = ws.ang if ang is None and phi is None else ang
     if not prepped:   # (else draw_prep_device has done it)
         prep_screen(ws, tables, step, batch, nsteps, stream)
     plane_wave_tables(ws, tables, step, batch, nsteps, stream, esc=esc)
-    screen_gemm(ws, step, batch, nsteps, stream, fac=fac, esc=esc, phi2=phi2, ang=ang)
+    screen_gemm(ws, step, batch, nsteps, stream, fac=fac, esc=esc, phi2=phi2, ang=ang, phi=phi)
 
 
 def draw_prep_device(ws: Workspace, tables: DeviceTables, seed: int, screen: int, batch: int,
@@ -420,14 +435,15 @@ class StepRunner:
         need = self.smax * self.B * synth_bytes_per_element(ws.n, ws.points, ws.mode)
         return self.smax > 0 and need <= SYNTH_BATCH_MAX_BYTES
 
-    def synthesize_all(self, seed: int, stream=None, timed=None, upload_ids: bool = True) -> List[torch.Tensor]:
+    def synthesize_all(self, seed: Optional[int], stream=None, timed=None, upload_ids: bool = True,
+                       host: Optional[Sequence] = None) -> List[torch.Tensor]:
         """Every screen's synthesis for the batch as one virtual batch
-        (SynthBuffers): the device draw per screen, then the tables and the GEMM
-        once over all (screen, realization) pairs.  Returns the screen angles
-        of screen i as a (B, n, n) view.  `timed(name, fn)`, when given, runs
-        each launch (a timing hook).  Without `upload_ids` the pairs' channels
-        and activity flags are taken as an earlier call left them (graph
-        capture records no host uploads)."""
+        (SynthBuffers): the draws (on the device, or `host` as run_batch takes
+        them), the tables and the GEMM once each over all (screen, realization)
+        pairs.  Returns the screen angles of screen i as a (B, n, n) view.
+        `timed(name, fn)`, when given, runs each launch (a timing hook).
+        Without `upload_ids` the pairs' channels and activity flags are taken
+        as an earlier call left them (graph capture records no host uploads)."""
         ws, B, S = self.ws, self.B, self.smax
         sb = ws.synth_buffers(S)
         st = self.stream if stream is None else stream
@@ -438,10 +454,16 @@ class StepRunner:
                 act = (np.arange(S)[:, None] < np.asarray(self.nscreens_np)[None, :]).astype(np.int32).reshape(-1)
                 upload(sb.active[:S * B], act, np.int32)
         nv = None if self.ns is None else sb.active
-        for i in range(S):
-            run("screen_draw_prep",
-                lambda i=i: draw_prep_device(sb.draw_view(ws, i, B), self.tables, seed, i, B, self.ns, st))
-        run("screen_tables", lambda: plane_wave_tables(sb, self.tables, 0, S * B, nv, st))
+        t = self.tables
+        if host is not None:
+            rho, theta, value = sb.upload(host[:S], B)
+            call("pa_screen_prep", sb.points, rho, theta, value, ptr(sb.fxy), ptr(sb.sparam), sb.mode,
+                 ptr(t.chparam), ptr(sb.chan), ptr(nv), 0, S * B, st)
+        else:
+            run("screen_draw_prep", lambda: call(
+                "pa_screens_draw_prep", sb.points, ptr(t.base), ptr(t.sqrt_psd), ptr(ws.chan), ptr(ws.rid),
+                int(seed) & (2 ** 64 - 1), S, ptr(sb.fxy), ptr(sb.sparam), sb.mode, ptr(t.chparam), ptr(self.ns), B, st))
+        run("screen_tables", lambda: plane_wave_tables(sb, t, 0, S * B, nv, st))
         run("screen_gemm", lambda: screen_gemm(sb, 0, S * B, nv, st, ang=sb.ang))
         return [sb.ang[i * B:(i + 1) * B] for i in range(S)]
 
@@ -487,12 +509,9 @@ class StepRunner:
             upload_spectra(ws, *host, batch=self.B)
         else:
             draw_prep_device(ws, self.tables, seed, step, self.B, self.ns, st)
-        p2 = ws.phi2_buffer() if compose else None
-        synth_screen(ws, self.tables, step, self.B, self.ns, st, esc=esc, phi2=p2, ang=ang, prepped=host is None)
-        phi = None
-        if compose:
-            phi = torch.empty(self.B, ws.n, ws.n, dtype=torch.float32, device=ws.device)
-            call("pa_screen_compose", ws.n, ptr(ws.sparam), ptr(ws.hg), ptr(p2), ptr(phi), self.B, st)
+        phi = torch.empty(self.B, ws.n, ws.n, dtype=torch.float32, device=ws.device) if compose else None
+        synth_screen(ws, self.tables, step, self.B, self.ns, st, esc=esc, ang=ws.ang if ang is None else ang,
+                     prepped=host is None, phi=phi)
         return phi
 
     def apply(self, step: int, ang: Optional[torch.Tensor] = None) -> None:
@@ -561,11 +580,11 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
     if overlap is None:
         overlap = use_overlap(ws, len(chan), int(np.max(nscreens)) if len(nscreens) else 0)
     device_draws = host_spectra is None and screens_out is None and run.smax > 0
-    whole = device_draws and SYNTH_WHOLE_BATCH and run.whole_batch_synthesis()
+    whole = screens_out is None and run.smax > 0 and SYNTH_WHOLE_BATCH and run.whole_batch_synthesis()
     if device_draws and overlap:
         overlapped_body(run, seed, field_in, sep, whole)
     elif whole:
-        angs = run.synthesize_all(seed)
+        angs = run.synthesize_all(seed, host=host_spectra)
         run.begin(field_in, sep)
         for i in range(run.smax + 1):
             run.fresnel(i)
@@ -587,8 +606,8 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
 
 
 OVERLAP_DEFAULT = True
-# device-drawn batches synthesize all their screens at once (SynthBuffers)
-# when the buffers fit SYNTH_BATCH_MAX_BYTES
+# batches synthesize all their screens at once (SynthBuffers) when the buffers
+# fit SYNTH_BATCH_MAX_BYTES
 SYNTH_WHOLE_BATCH = True
 # the Gaussian source's first Fresnel step as two 1-D propagations (exact:
 # source and transfer function are separable; StepRunner.begin)

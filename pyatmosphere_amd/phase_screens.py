@@ -70,11 +70,8 @@ def _synthesize(screen, spectrum: PolarDiscreteFunction, shift=(0.0, 0.0), imagi
     engine.upload_spectra(ws, np.asarray(spectrum.rho)[None], np.asarray(spectrum.theta)[None], value[None], batch=1)
     ws.chan[:1].zero_()
     stream = engine._lib.stream_handle()
-    p2 = ws.phi2_buffer()
-    engine.synth_screen(ws, tables, 0, 1, None, stream, phi2=p2)
     phi = torch.empty(1, n, n, dtype=torch.float32, device=dev)
-    engine.call("pa_screen_compose", n, engine.ptr(ws.sparam), engine.ptr(ws.hg), engine.ptr(p2),
-                engine.ptr(phi), 1, stream)
+    engine.synth_screen(ws, tables, 0, 1, None, stream, phi=phi)
     return phi[0]
 
 

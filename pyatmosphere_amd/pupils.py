@@ -19,9 +19,10 @@ class CirclePupil:
     def output(self, input, shift=(0, 0), **kwargs):
         """input * mask as a new device array."""
         grid = self.channel.grid
-        u = input.to(torch.complex64).clone().contiguous()
+        u = input.to(torch.complex64).contiguous()
+        out = torch.empty_like(u)
         n = u.shape[-1]
         batch = u.numel() // (n * n)
-        call("pa_apply_pupil", n, ptr(u), float(grid.delta), float(self.radius), float(shift[0]),
+        call("pa_pupil_output", n, ptr(u), ptr(out), float(grid.delta), float(self.radius), float(shift[0]),
              float(shift[1]), batch, _lib.stream_handle())
-        return u
+        return out

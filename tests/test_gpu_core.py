@@ -644,3 +644,90 @@ def test_polynomial_block_past_1024_points(dev, P):
     ref = o.screen_phase(n, spec.delta, per_real[0][0])
     excess = np.abs(phi[0].cpu().numpy().astype(np.float64) - ref) - np.abs(ref) * 2 ** -24
     assert excess.max() < 2e-5
+
+
+@pytest.mark.parametrize("P", [16, 1000, 2048])
+def test_draws_of_all_screens_equal_one_by_one(dev, P):
+    """pa_screens_draw_prep's element screen * batch + b holds the bits of
+    pa_screen_draw_prep for that screen, and elements without the screen are
+    left alone."""
+    S, B = 3, 4
+    spec = channel_spec(256, 0.002, 808e-9, 0.05, 5e3, S, P, 1e-15)
+    tables = engine.DeviceTables([spec], dev)
+    ws = engine.Workspace(256, P, B, "f16x3", dev)
+    ws.chan.zero_()
+    ws.rid.copy_(torch.tensor([5, 2 ** 33, 7, 1]))
+    ns = torch.tensor([3, 1, 0, 2], dtype=torch.int32, device=dev)
+    fxy = torch.full((S * B, P, 4), 7.0, dtype=torch.float64, device=dev)
+    sp = torch.full((S * B, engine._lib.PA_SCREEN_PARAMS), 7.0, dtype=torch.float64, device=dev)
+    p = engine.ptr
+    engine.call("pa_screens_draw_prep", P, p(tables.base), p(tables.sqrt_psd), None, p(ws.rid), 99, S, p(fxy), p(sp), 0,
+                p(tables.chparam), p(ns), B, None)
+    for i in range(S):
+        ws.fxy.fill_(7.0)
+        ws.sparam.fill_(7.0)
+        engine.draw_prep_device(ws, tables, 99, i, B, ns, None)
+        assert torch.equal(ws.fxy, fxy[i * B:(i + 1) * B]) and torch.equal(ws.sparam, sp[i * B:(i + 1) * B])
+
+
+@pytest.mark.parametrize("mode", ["f16x3", "bf16x3", "f32"])
+@pytest.mark.parametrize("n,tile", [(64, 0), (256, 0), (512, 1), (512, 2), (4096, 1)])
+def test_composed_screen_from_the_gemm(dev, mode, n, tile):
+    """pa_screen_gemm_compose's screen and angle are the bits of pa_screen_gemm
+    followed by pa_screen_compose, for an element that is active and not."""
+    P, B = 200, 2 if n < 4096 else 1
+    spec = channel_spec(n, 0.002, 808e-9, 0.05, 5e3, 3, P, 1e-15)
+    spectra, _ = host_spectra(spec, B, seed=n)
+    tables = engine.DeviceTables([spec], dev)
+    ws = engine.Workspace(n, P, B, mode, dev)
+    engine.upload_spectra(ws, *spectra[0], batch=B)
+    ws.chan.zero_()
+    ns = torch.tensor([1, 0][:B], dtype=torch.int32, device=dev)
+    engine.synth_screen(ws, tables, 0, B, None, None, phi2=ws.phi2_buffer())
+    want, got = (torch.full((B, n, n), 3.0, dtype=torch.float32, device=dev) for _ in range(2))
+    engine.call("pa_screen_compose", n, engine.ptr(ws.sparam), engine.ptr(ws.hg), engine.ptr(ws.phi2),
+                engine.ptr(want), B, None)
+    ang = torch.full_like(got, 3.0)
+    engine.screen_gemm(ws, 0, B, ns, None, tile=tile, phi=got, ang=ang)
+    assert torch.equal(got[0], want[0]) and torch.equal(ang[0], ws.ang[0])
+    assert B == 1 or bool((got[1] == 3.0).all() and (ang[1] == 3.0).all())
+
+
+@pytest.mark.parametrize("n", [64, 256, 2048])
+def test_pupil_output_is_the_masked_copy(dev, n):
+    """pa_pupil_output against the in-place pupil on a copy, bits and all (NaN
+    and negative zero inside kept, outside replaced by zero), at aligned and
+    unaligned fields, for pupils that hold nothing, part, and everything."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    buf = torch.randn(2 * n * n + 1, 2, device=dev, generator=g)
+    buf[::7] = float("nan")
+    buf[1::5] = -0.0
+    delta = 2.0 / n
+    p = engine.ptr
+    for u in (torch.view_as_complex(buf)[:2 * n * n].view(2, n, n), torch.view_as_complex(buf)[1:].view(2, n, n)):
+        for r, sx, sy in [(0.3, 0.1, -0.2), (9.0, 0.0, 0.0), (0.4 * delta, 0.0, 0.0), (0.2, 5.0, 0.0), (0.5, -0.9, 0.9),
+                          (0.5 * delta, 0.5 * delta, 0.0), (float("nan"), 0.0, 0.0)]:
+            want, out = u.clone(), torch.full_like(u, 7.0)
+            engine.call("pa_apply_pupil", n, p(want), delta, r, sx, sy, 2, None)
+            engine.call("pa_pupil_output", n, p(u), p(out), delta, r, sx, sy, 2, None)
+            assert torch.equal(torch.view_as_real(out).view(torch.int32), torch.view_as_real(want).view(torch.int32))
+
+
+@pytest.mark.parametrize("screens", [[3, 3, 3], [3, 0, 2]])
+def test_host_draws_synthesize_whole(dev, monkeypatch, screens):
+    """Host-drawn batches synthesized as one virtual batch give the bits of the
+    screen-by-screen schedule, with uniform and mixed screen counts."""
+    n, P, B, S = 256, 100, len(screens), 3
+    spec = channel_spec(n, 0.002, 808e-9, 0.05, 5e3, S, P, 1e-15, pupils=[(0.1, 0.0, 0.0)])
+    spectra, _ = host_spectra(spec, B, seed=4)
+    specs = [dataclasses.replace(spec, positions=spec.positions[:k]) for k in sorted(set(screens))]
+    tables = engine.DeviceTables(specs, dev)
+    chan = np.array([sorted(set(screens)).index(k) for k in screens])
+    got = []
+    for whole in (True, False):
+        monkeypatch.setattr(engine, "SYNTH_WHOLE_BATCH", whole)
+        ws = engine.Workspace(n, P, B, "f16x3", dev)
+        out = torch.empty(B, n, n, dtype=torch.complex64, device=dev)
+        mom = engine.run_batch(ws, tables, chan, np.array(screens), host_spectra=spectra, field_out=out)
+        got.append((out, mom.clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
