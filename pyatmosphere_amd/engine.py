@@ -17,6 +17,7 @@ random stream.
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -39,6 +40,18 @@ def axis_coords(n: int, delta: float) -> np.ndarray:
 def log_polar_base(points: int, f_min: float, f_max: float) -> np.ndarray:
     """RandLogPolarGrid.base (grids.py:94-96), float32."""
     return np.exp(np.linspace(np.log(f_min), np.log(f_max), points, dtype=np.float32))
+
+
+@functools.lru_cache(maxsize=64, typed=True)
+def log_polar_annuli(points: int, f_min: float, f_max: float) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
+    """(base, inner radii squared, differences of squared radii) of the log-polar
+    annuli, float32, read-only (grids.py:94-102)."""
+    f = log_polar_base(points, f_min, f_max)
+    prev = np.insert(f, 0, 0)[:-1]
+    out = (f, prev ** 2, f ** 2 - prev ** 2)
+    for a in out:
+        a.flags.writeable = False
+    return out
 
 
 def mvk_psd_n(kappa, Cn2, l0, L0):
@@ -160,6 +173,16 @@ def twiddles(n: int, device: torch.device) -> torch.Tensor:
     return t
 
 
+def to_device(arrays: Sequence[np.ndarray], device: torch.device) -> List[torch.Tensor]:
+    """Host arrays as device tensors that share one allocation and one copy."""
+    at = np.cumsum([0] + [-(-a.nbytes // 256) * 256 for a in arrays])
+    host = np.zeros(int(at[-1]), np.uint8)
+    for a, o in zip(arrays, at):
+        host[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
+    dev = torch.from_numpy(host).to(device)
+    return [dev[o:o + a.nbytes].view(torch.from_numpy(a).dtype).view(a.shape) for a, o in zip(arrays, at)]
+
+
 class DeviceTables:
     """Per-channel tables stacked for the channels of one batch (same N, P)."""
 
@@ -191,9 +214,32 @@ class DeviceTables:
             base[i] = s.base
             sq[i] = np.sqrt(s.psd.astype(np.float32))
         self.npup = max(len(s.pupils) for s in specs)
-        to = lambda a: torch.from_numpy(a).to(device)
-        self.src, self.htab, self.chparam, self.pup = to(src), to(htab), to(chp), to(pup)
-        self.base, self.sqrt_psd = to(base), to(sq)
+        self.src, self.htab, self.chparam, self.pup, self.base, self.sqrt_psd = \
+            to_device([src, htab, chp, pup, base, sq], device)
+
+
+class KeptTables:
+    """The device tables of the channels that one path ran last, at most KEEP of
+    them: rebuilt unless every value they are made from is what it was, on the
+    same device and stream."""
+    KEEP = 4
+
+    def __init__(self):
+        self._kept: tuple = ()
+
+    def get(self, spec: ChannelSpec, device: torch.device) -> DeviceTables:
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("a channel with host draws cannot be captured into a graph")
+        key = (spec.n, spec.delta, spec.wvl, spec.w0, spec.F0, spec.length, np.asarray(spec.positions).tobytes(),
+               spec.points, tuple(spec.pupils), spec.shift, None if spec.gains is None else tuple(spec.gains), device,
+               _lib.stream_handle())
+        for k, base, psd, tables in self._kept:
+            if k == key and np.array_equal(base, spec.base) and np.array_equal(psd, spec.psd):
+                return tables
+        tables = DeviceTables([spec], device)
+        entry = (key, np.array(spec.base), np.array(spec.psd), tables)
+        self._kept = ((entry,) + self._kept)[:self.KEEP]
+        return tables
 
 
 class Workspace:
@@ -236,9 +282,12 @@ class Workspace:
         self.value = e(B, points, dt=torch.complex64)
         self.part = e(B, self.tiles, _lib.PA_PART_SUMS, dt=torch.float64)
         self.moments = e(B, _lib.PA_NUM_MOMENTS, dt=torch.float64)
-        self.rid = e(B, dt=torch.int64)
-        self.chan = e(B, dt=torch.int32)
-        self.nsteps = e(B, dt=torch.int32)
+        # realization ids, channels and screen counts: one buffer, one upload
+        ids = e(16 * B, dt=torch.uint8)
+        self.rid = ids[:8 * B].view(torch.int64)
+        self.chan = ids[8 * B:12 * B].view(torch.int32)
+        self.nsteps = ids[12 * B:].view(torch.int32)
+        self._ids = (ids,)
 
     def phi2_buffer(self) -> torch.Tensor:
         if self.phi2 is None:
@@ -251,6 +300,19 @@ class Workspace:
             self.esc_s.append(torch.empty(self.batch, 2, self.n, dtype=torch.complex64, device=self.device))
         if self.side is None:
             self.side = torch.cuda.Stream(device=self.device)   # default priority
+
+    def upload_ids(self, chan, nsteps, rid=None) -> None:
+        """Channels, screen counts and (when given) realization ids of a batch."""
+        B, n = self.batch, len(chan)
+        stage = torch.zeros(16 * B, dtype=torch.uint8, pin_memory=True)
+        h = stage.numpy()
+        h[8 * B:12 * B].view(np.int32)[:n] = chan
+        h[12 * B:].view(np.int32)[:n] = nsteps
+        lo = 8 * B
+        if rid is not None:
+            h[:lo].view(np.int64)[:n] = rid
+            lo = 0
+        self._ids[0][lo:].copy_(stage[lo:], non_blocking=True)
 
     def synth_buffers(self, screens: int) -> "SynthBuffers":
         """Buffers for synthesizing `screens` screens of a whole batch at once
@@ -333,10 +395,12 @@ def prep_screen(ws: Workspace, tables: DeviceTables, step: int, batch: int, nste
 
 
 def plane_wave_tables(ws: Workspace, tables: DeviceTables, step: int, batch: int, nsteps: Optional[torch.Tensor],
-                      stream, esc: Optional[torch.Tensor] = None, rows: Optional[int] = None) -> None:
-    """GEMM operands, float64 1-D parts h, g and the row/column factors of screen `step`."""
+                      stream, esc: Optional[torch.Tensor] = None, rows: Optional[int] = None,
+                      single: bool = False) -> None:
+    """GEMM operands, float64 1-D parts h, g and the row/column factors of screen
+    `step`; `single`: every element is channel 0."""
     call("pa_screen_tables", ws.n, ws.points, ptr(ws.fxy), ptr(ws.sparam), ptr(tables.chparam),
-         ptr(ws.chan), ptr(ws.opa), ptr(ws.opb), ptr(ws.hg), ptr(ws.esc if esc is None else esc), ws.mode,
+         None if single else ptr(ws.chan), ptr(ws.opa), ptr(ws.opb), ptr(ws.hg), ptr(ws.esc if esc is None else esc), ws.mode,
          ws.table_rows if rows is None else rows, ptr(nsteps), step, batch, stream)
 
 
@@ -411,19 +475,20 @@ class StepRunner:
     the field after every screen, and by run_batch)."""
 
     def __init__(self, ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: np.ndarray,
-                 rid: Optional[np.ndarray] = None):
+                 rid: Optional[np.ndarray] = None, single: bool = False):
+        """`single`: every element is channel 0 with all its screens, and the
+        screens are synthesized whole or not at all; no ids are uploaded."""
         self.ws, self.tables = ws, tables
         self.B = B = len(chan)
         if B > ws.batch:
             raise ValueError("batch larger than the workspace")
         self.stream = _lib.stream_handle()
         self.tw = twiddles(ws.n, ws.device)
-        upload(ws.chan[:B], chan, np.int32)
-        upload(ws.nsteps[:B], nscreens, np.int32)
         uniform = bool(np.all(np.asarray(nscreens) == tables.max_screens))
         self.ns = None if uniform else ws.nsteps
-        if rid is not None:
-            upload(ws.rid[:B], rid, np.int64)
+        self.chan = None if single else ws.chan
+        if not single:
+            ws.upload_ids(chan, nscreens, rid)
         self.smax = int(np.max(nscreens)) if len(nscreens) else 0
         self.smin = int(np.min(nscreens)) if len(nscreens) else 0
         self.sep0 = False
@@ -448,8 +513,10 @@ class StepRunner:
         sb = ws.synth_buffers(S)
         st = self.stream if stream is None else stream
         run = timed if timed is not None else (lambda name, fn: fn())
+        single = not np.any(self.chan_np)     # every pair is channel 0
         if upload_ids:
-            upload(sb.chan[:S * B], np.tile(np.asarray(self.chan_np, np.int32), S), np.int32)
+            if not single:
+                upload(sb.chan[:S * B], np.tile(np.asarray(self.chan_np, np.int32), S), np.int32)
             if self.ns is not None:
                 act = (np.arange(S)[:, None] < np.asarray(self.nscreens_np)[None, :]).astype(np.int32).reshape(-1)
                 upload(sb.active[:S * B], act, np.int32)
@@ -458,12 +525,12 @@ class StepRunner:
         if host is not None:
             rho, theta, value = sb.upload(host[:S], B)
             call("pa_screen_prep", sb.points, rho, theta, value, ptr(sb.fxy), ptr(sb.sparam), sb.mode,
-                 ptr(t.chparam), ptr(sb.chan), ptr(nv), 0, S * B, st)
+                 ptr(t.chparam), None if single else ptr(sb.chan), ptr(nv), 0, S * B, st)
         else:
             run("screen_draw_prep", lambda: call(
-                "pa_screens_draw_prep", sb.points, ptr(t.base), ptr(t.sqrt_psd), ptr(ws.chan), ptr(ws.rid),
+                "pa_screens_draw_prep", sb.points, ptr(t.base), ptr(t.sqrt_psd), ptr(self.chan), ptr(ws.rid),
                 int(seed) & (2 ** 64 - 1), S, ptr(sb.fxy), ptr(sb.sparam), sb.mode, ptr(t.chparam), ptr(self.ns), B, st))
-        run("screen_tables", lambda: plane_wave_tables(sb, t, 0, S * B, nv, st))
+        run("screen_tables", lambda: plane_wave_tables(sb, t, 0, S * B, nv, st, single=single))
         run("screen_gemm", lambda: screen_gemm(sb, 0, S * B, nv, st, ang=sb.ang))
         return [sb.ang[i * B:(i + 1) * B] for i in range(S)]
 
@@ -476,17 +543,17 @@ class StepRunner:
         ws, t = self.ws, self.tables
         self.sep0 = bool(separable and field_in is None and self.smin >= 1)
         if self.sep0:
-            call("pa_source_fresnel", ws.n, ptr(ws.sep), ptr(t.src), ptr(t.htab), ptr(ws.chan), t.max_steps,
+            call("pa_source_fresnel", ws.n, ptr(ws.sep), ptr(t.src), ptr(t.htab), ptr(self.chan), t.max_steps,
                  ptr(self.tw), self.B, self.stream)
             return
         call("pa_row_first", ws.n, ptr(ws.work), ptr(field_in), None if field_in is not None else ptr(t.src),
-             ptr(ws.chan), ptr(self.tw), self.B, self.stream)
+             ptr(self.chan), ptr(self.tw), self.B, self.stream)
 
     def fresnel(self, step: int) -> None:
         ws, t = self.ws, self.tables
         if step == 0 and self.sep0:
             return          # taken by begin(separable=True)
-        call("pa_col_step", ws.n, ptr(ws.work), ptr(t.htab), ptr(ws.chan), ptr(self.ns), step, t.max_steps,
+        call("pa_col_step", ws.n, ptr(ws.work), ptr(t.htab), ptr(self.chan), ptr(self.ns), step, t.max_steps,
              ptr(self.tw), ws.col_group, self.B, self.stream)
 
     def screen(self, step: int, *, seed: Optional[int] = None,
@@ -527,9 +594,9 @@ class StepRunner:
         ws, t = self.ws, self.tables
         part = ws.part if reduce else None
         call("pa_row_last", ws.n, ptr(ws.work), ptr(field_out), ptr(part), ptr(t.chparam), ptr(t.pup), t.npup,
-             None, ptr(ws.chan), ptr(self.tw), self.B, self.stream)
+             None, ptr(self.chan), ptr(self.tw), self.B, self.stream)
         if reduce:
-            call("pa_moments_finalize", ws.n, ptr(ws.part), ptr(t.chparam), t.npup, ptr(ws.chan),
+            call("pa_moments_finalize", ws.n, ptr(ws.part), ptr(t.chparam), t.npup, ptr(self.chan),
                  ptr(ws.moments), self.B, self.stream)
             return ws.moments[:self.B]
         return None
@@ -549,8 +616,8 @@ class StepRunner:
         centroid = ws.moments[:self.B].clone()
         out = torch.empty_like(centroid)
         call("pa_row_last", ws.n, ptr(ws.work), None, ptr(ws.part), ptr(t.chparam), ptr(pup_t), len(radii),
-             ptr(centroid), ptr(ws.chan), ptr(self.tw), self.B, self.stream)
-        call("pa_moments_finalize", ws.n, ptr(ws.part), ptr(t.chparam), len(radii), ptr(ws.chan), ptr(out),
+             ptr(centroid), ptr(self.chan), ptr(self.tw), self.B, self.stream)
+        call("pa_moments_finalize", ws.n, ptr(ws.part), ptr(t.chparam), len(radii), ptr(self.chan), ptr(out),
              self.B, self.stream)
         return out
 
@@ -561,7 +628,7 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
               field_in: Optional[torch.Tensor] = None, field_out: Optional[torch.Tensor] = None,
               reduce: bool = True, screens_out: Optional[List[torch.Tensor]] = None,
               overlap: Optional[bool] = None, tracked: Optional[Sequence[float]] = None,
-              separable: Optional[bool] = None):
+              separable: Optional[bool] = None, single: bool = False):
     """Propagate `len(chan)` realizations through their channels.
 
     Spectra come from the device Philox stream (`seed`, `rid`) or from
@@ -573,9 +640,13 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
     each element's centroid (StepRunner.tracked).  `separable` (default
     SEPARABLE_SOURCE) takes the source's first Fresnel step as two 1-D
     propagations when there is no input field and every element has a screen
-    (StepRunner.begin).
+    (StepRunner.begin).  `single` says that every element is channel 0 with all
+    its screens: host-drawn batches then upload no ids (ws.chan and ws.nsteps
+    stay as they are).
     """
-    run = StepRunner(ws, tables, chan, nscreens, rid)
+    single = single and host_spectra is not None and screens_out is None and SYNTH_WHOLE_BATCH and \
+        tables.max_screens * len(chan) * synth_bytes_per_element(ws.n, ws.points, ws.mode) <= SYNTH_BATCH_MAX_BYTES
+    run = StepRunner(ws, tables, chan, nscreens, rid, single=single)
     sep = SEPARABLE_SOURCE if separable is None else bool(separable)
     if overlap is None:
         overlap = use_overlap(ws, len(chan), int(np.max(nscreens)) if len(nscreens) else 0)
@@ -721,6 +792,7 @@ class GraphedBatch:
         run.tw = twiddles(ws.n, ws.device)
         uniform = bool(np.all(self.nscreens == t.max_screens))
         run.ns = None if uniform else ws.nsteps
+        run.chan = ws.chan
         run.smax = int(np.max(self.nscreens))
         run.smin = int(np.min(self.nscreens))
         run.sep0 = False

@@ -107,13 +107,18 @@ class RandLogPolarGrid(Grid):
 
     @property
     def base(self):
-        return engine.log_polar_base(self.points, self.f_min, self.f_max)
+        return self._annuli()[0].copy()
+
+    def _annuli(self):
+        try:
+            return engine.log_polar_annuli(self.points, self.f_min, self.f_max)
+        except TypeError:       # limits that cannot be hashed (arrays)
+            return engine.log_polar_annuli.__wrapped__(self.points, self.f_min, self.f_max)
 
     def draw_rho(self):
         rand = np.random.random(size=(1,)).astype(np.float32)
-        f = self.base
-        f_prev = np.insert(f, 0, 0)[:-1]
-        return np.sqrt(f_prev ** 2 + rand * (f ** 2 - f_prev ** 2)).astype(np.float32)
+        _, prev2, d2 = self._annuli()
+        return np.sqrt(prev2 + rand * d2).astype(np.float32)
 
     def draw_theta(self):
         return (2 * np.pi * np.random.random(size=(self.points,)).astype(np.float32)).astype(np.float32)

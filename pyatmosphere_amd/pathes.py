@@ -85,11 +85,21 @@ class PhaseScreensPath(AbstractPath):
         self.phase_screens = phase_screens
         super().__init__(length, losses_db)
 
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_kept_tables"}
+
     def init_phase_screens(self):
         for phase_screen in self.phase_screens:
             phase_screen.channel = self.channel
 
     # -- device plumbing
+    def _tables(self, spec, dev):
+        """The device tables of `spec`, kept while its values stay the same."""
+        kept = self.__dict__.get("_kept_tables")
+        if kept is None:
+            kept = self._kept_tables = engine.KeptTables()
+        return kept.get(spec, dev)
+
     def _segment_gains(self, with_total):
         ds = engine.ChannelSpec.step_lengths(self)  # uses self.positions / self.length
         gains = []
@@ -146,12 +156,12 @@ class PhaseScreensPath(AbstractPath):
     def _run(self, input, shift=(0, 0), wind=False, with_total=False):
         spec = self._spec(shift, with_total)
         dev = device()
-        tables = engine.DeviceTables([spec], dev)
+        tables = self._tables(spec, dev)
         ws = engine.get_workspace(spec.n, spec.points, 1, config.get("gemm_mode", "f16x3"), dev)
         out = torch.empty(1, spec.n, spec.n, dtype=torch.complex64, device=dev)
         if all(isinstance(ps, _PLANE_WAVE) for ps in self.phase_screens):
             engine.run_batch(ws, tables, np.zeros(1), np.array([spec.nscreens]), host_spectra=self._draw(wind),
-                             field_in=_as_field(input, spec.n, dev), field_out=out, reduce=False)
+                             field_in=_as_field(input, spec.n, dev), field_out=out, reduce=False, single=True)
             return out[0]
         run = engine.StepRunner(ws, tables, np.zeros(1), np.array([spec.nscreens]))
         run.begin(_as_field(input, spec.n, dev))
@@ -173,7 +183,7 @@ class PhaseScreensPath(AbstractPath):
         (pathes.py:61-75)."""
         spec = self._spec(shift, with_total=False)
         dev = device()
-        tables = engine.DeviceTables([spec], dev)
+        tables = self._tables(spec, dev)
         ws = engine.get_workspace(spec.n, spec.points, 1, config.get("gemm_mode", "f16x3"), dev)
         run = engine.StepRunner(ws, tables, np.zeros(1), np.array([spec.nscreens]))
         run.begin(_as_field(input, spec.n, dev))

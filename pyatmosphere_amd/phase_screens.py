@@ -60,18 +60,28 @@ def _synthesize(screen, spectrum: PolarDiscreteFunction, shift=(0.0, 0.0), imagi
     P = len(spectrum.rho)
     dev = device()
     ws = engine.get_workspace(n, P, 1, config.get("gemm_mode", "f16x3"), dev)
-    spec = engine.ChannelSpec(n=n, delta=screen.grid.delta, wvl=screen.wvl, w0=1.0, F0=np.inf, length=0.0,
-                              positions=np.zeros(1), points=P, base=np.asarray(spectrum.rho, np.float32),
-                              psd=np.zeros(P, np.float32), shift=tuple(float(v) for v in shift))
-    tables = engine.DeviceTables([spec], dev)
     value = np.asarray(spectrum.value, np.complex64)
     if imaginary:
         value = (value * np.complex64(-1j)).astype(np.complex64)
-    engine.upload_spectra(ws, np.asarray(spectrum.rho)[None], np.asarray(spectrum.theta)[None], value[None], batch=1)
-    ws.chan[:1].zero_()
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a host-drawn screen cannot be captured into a graph")
+    # the grid's parameters and the draw in one upload
+    stage = torch.empty(32 + 16 * P, dtype=torch.uint8, pin_memory=True)
+    h = stage.numpy()
+    h[:32].view(np.float64)[:] = (screen.grid.delta, float(shift[0]), float(shift[1]), 0.0)
+    h[32:32 + 4 * P].view(np.float32)[:] = spectrum.rho
+    h[32 + 4 * P:32 + 8 * P].view(np.float32)[:] = spectrum.theta
+    h[32 + 8 * P:].view(np.complex64)[:] = value
+    d = torch.empty(stage.shape, dtype=torch.uint8, device=dev)
+    d.copy_(stage, non_blocking=True)
     stream = engine._lib.stream_handle()
+    at = d.data_ptr()
+    engine.call("pa_screen_prep", P, at + 32, at + 32 + 4 * P, at + 32 + 8 * P, engine.ptr(ws.fxy),
+                engine.ptr(ws.sparam), ws.mode, at, None, None, 0, 1, stream)
+    engine.call("pa_screen_tables", n, P, engine.ptr(ws.fxy), engine.ptr(ws.sparam), at, None, engine.ptr(ws.opa),
+                engine.ptr(ws.opb), engine.ptr(ws.hg), engine.ptr(ws.esc), ws.mode, ws.table_rows, None, 0, 1, stream)
     phi = torch.empty(1, n, n, dtype=torch.float32, device=dev)
-    engine.synth_screen(ws, tables, 0, 1, None, stream, phi=phi)
+    engine.screen_gemm(ws, 0, 1, None, stream, phi=phi)
     return phi[0]
 
 
@@ -107,7 +117,9 @@ class SSPhaseScreen(PhaseScreen):
         rho = self.f_grid.draw_rho()
         theta = self.f_grid.draw_theta()
         nrm = np.random.normal(size=(2, self.f_grid.points))
-        value = ((nrm[0] + 1j * nrm[1]).astype(np.complex64) * np.sqrt(self._get_psd())).astype(np.complex64)
+        value = np.empty(self.f_grid.points, np.complex64)
+        value.real, value.imag = nrm
+        value = (value * np.sqrt(self._get_psd())).astype(np.complex64, copy=False)
         spectrum = PolarDiscreteFunction(rho=rho, theta=theta, value=value)
         if use_cached_spectrum:
             self._cached_spectrum = spectrum

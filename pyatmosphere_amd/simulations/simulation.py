@@ -234,8 +234,11 @@ class Simulation:
             path.init_phase_screens()
             spec = path._spec((0.0, 0.0), with_total=False)  # Channel.generator output
             spec.pupils = [(r, sx, sy) for (r, sx, sy) in p["pupils"]]
-            tables = engine.DeviceTables([spec], dev)
-            prepared.append((p, spec, tables))
+            prepared.append((p, spec, path._tables(spec, dev)))
+        # with nothing to do between realizations a batch's values go in at once
+        measures = list(self.flattened_measures())
+        at_once = not (plot_step or save_step) and type(self).process_output is Simulation.process_output \
+            and all(type(m) is Measure for m in measures) and len({id(m) for m in measures}) == len(measures)
         iteration = 0
         while not self.is_measures_done():
             remaining = self._remaining()
@@ -273,16 +276,14 @@ class Simulation:
                 # work buffer (no field is stored)
                 mom, tr = (out[0].cpu().numpy(), out[1].cpu().numpy()) if p["tracked"] else (out.cpu().numpy(), None)
                 results[id(p)] = (mom, tr)
+            if at_once:
+                self._take(prepared, results, B)
+                continue
             for b in range(B):
                 for p, spec, _ in prepared:
                     mom, tr = results[id(p)]
                     for m, c in p["items"]:
-                        if c[0] == "moment":
-                            m.iteration_data = float(mom[b, c[1]])
-                        elif c[0] == "pupil":
-                            m.iteration_data = float(mom[b, 7 + c[1]])
-                        else:
-                            m.iteration_data = float(tr[b, 7 + c[1]])
+                        m.iteration_data = float(self._column(c, mom, tr)[b])
                     for m, c in p["items"]:
                         if c[0] == "tracked":
                             res = m.operations[0].__self__
@@ -294,3 +295,24 @@ class Simulation:
                 self.process_output(iteration, plot_step=plot_step, save_step=save_step)
                 if self.is_measures_done():
                     break
+
+    @staticmethod
+    def _column(c, mom, tr):
+        """One measure's values of a batch: a moment, a pupil's transmittance, or a
+        centroid-tracked pupil's."""
+        return mom[:, c[1]] if c[0] == "moment" else (mom if c[0] == "pupil" else tr)[:, 7 + c[1]]
+
+    def _take(self, prepared, results, B):
+        """A batch's values into the measures, as realization by realization would
+        put them there: each measure up to its size, and no realization after
+        the one that completes the last of them."""
+        items = [(m, c, results[id(p)]) for p, _, _ in prepared for m, c in p["items"]]
+        left = [B if m.max_size is None else max(0, min(B, m.max_size - len(m))) for m, _, _ in items]
+        if all(m.max_size is not None for m, _, _ in items):
+            B = max(left)
+        for (m, c, (mom, tr)), take in zip(items, left):
+            values = self._column(c, mom, tr)[:B].tolist()
+            m.data.extend(values[:take])
+            m.iteration_data = values[-1]
+            if c[0] == "tracked":
+                m.operations[0].__self__.pupil_shift = (float(mom[B - 1, 1]), float(mom[B - 1, 2]))

@@ -6,6 +6,7 @@ import torch
 
 from . import _lib
 from ._lib import call, ptr
+from .engine import gaussian_factors, to_device
 from .gpu import device
 from .theory.sources import GaussianBeam
 
@@ -30,18 +31,20 @@ class GaussianSource(GaussianBeam, Source):
     float64 factors."""
 
     def factors(self, n, delta):
-        from .engine import gaussian_factors
         return gaussian_factors(n, delta, self.wvl, self.w0, self.F0)
 
     def output(self):
         grid = self.channel.grid
         n = grid.resolution[0]
-        gy, gx = self.factors(n, grid.delta)
         dev = device()
+        # the two factors last used stay on the device, by the values they are made from
+        key = (n, grid.delta, self.wvl, self.w0, self.F0, dev, _lib.stream_handle())
+        kept = self.__dict__.get("_factors")
+        if kept is None or kept[0] != key:
+            kept = self._factors = (key, to_device(self.factors(n, grid.delta), dev))
         out = torch.empty(n, n, dtype=torch.complex64, device=dev)
-        # keep the factor tensors referenced until the launch is enqueued: a freed
-        # temporary's block can be handed to the next allocation before the kernel runs
-        gy_d = torch.from_numpy(gy).to(dev)
-        gx_d = torch.from_numpy(gx).to(dev)
-        call("pa_outer", n, ptr(out), ptr(gy_d), ptr(gx_d), 1, _lib.stream_handle())
+        call("pa_outer", n, ptr(out), ptr(kept[1][0]), ptr(kept[1][1]), 1, _lib.stream_handle())
         return out
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_factors"}

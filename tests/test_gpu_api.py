@@ -180,3 +180,56 @@ def test_channel_plan_matches_engine_and_oracle(dev):
         assert np.allclose(mom[:, :9].cpu().numpy(), ref_mom[:, :9].cpu().numpy(), rtol=1e-6, atol=1e-12)
     finally:
         lib.pa_channel_destroy(plan)
+
+
+def test_kept_tables_follow_the_channel(dev):
+    """A channel whose parts were changed after a run gives what a new channel
+    with those parts gives, on the same stream and on another, and a copy or a
+    pickle of a channel that has run carries no device tables."""
+    import copy
+    import pickle
+    import torch
+
+    def build(w0=0.04, delta=0.002, length=5e3, losses=0.0, Cn2=2e-15):
+        return pa.Channel(grid=pa.RectGrid(resolution=128, delta=delta),
+                          source=pa.GaussianSource(wvl=808e-9, w0=w0, F0=np.inf),
+                          path=pa.IdenticalPhaseScreensPath(
+                              phase_screen=pa.SSPhaseScreen(
+                                  model=pa.MVKModel(Cn2=Cn2, l0=6e-3, L0=1e3),
+                                  f_grid=pa.RandLogPolarGrid(points=100, f_min=1 / 15000, f_max=2 / 6e-3)),
+                              length=length, count=3, losses_db=losses),
+                          pupil=pa.CirclePupil(radius=0.05))
+
+    def run(ch):
+        np.random.seed(3)
+        return ch.run()
+
+    ch = build()
+    first = run(ch)
+    assert torch.equal(run(ch), first)
+    ch.source.w0 = 0.05
+    assert torch.equal(run(ch), run(build(w0=0.05)))
+    ch.grid.delta = 0.003
+    assert torch.equal(run(ch), run(build(w0=0.05, delta=0.003)))
+    ch.path.losses_db = 3.0
+    assert torch.equal(run(ch), run(build(w0=0.05, delta=0.003, losses=3.0)))
+    for ps in ch.path.phase_screens:
+        ps._psd *= 4.0            # in place: the values count, not the array
+    want = build(w0=0.05, delta=0.003, losses=3.0)
+    want.path.init_phase_screens()
+    for ps in want.path.phase_screens:
+        ps._psd = ps._get_psd() * np.float32(4.0)
+    assert torch.equal(run(ch), run(want))
+    ch.source.w0, ch.grid.delta, ch.path.losses_db = 0.04, 0.002, 0.0
+    for ps in ch.path.phase_screens:
+        ps._psd /= 4.0
+    assert torch.equal(run(ch), first)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        other = run(ch)
+    torch.cuda.synchronize()
+    assert torch.equal(other, first)
+    assert "_kept_tables" not in copy.copy(ch.path).__dict__ and "_factors" not in copy.deepcopy(ch.source).__dict__
+    again = pickle.loads(pickle.dumps(ch.source))
+    assert again == ch.source and "_factors" not in again.__dict__

@@ -176,3 +176,44 @@ def test_si_result_formula():
     r.measures[0].data = data.tolist()
     assert np.allclose(r.positions, [1.0, 2.0, 3.0])
     assert np.allclose(r.si, data.var(axis=0) / data.mean(axis=0) ** 2, rtol=1e-12)
+
+
+@pytest.mark.parametrize("sizes", [(5, 5), (3, 8), (None, 4), (2, 2, 7), (0, 3)])
+@pytest.mark.parametrize("batch", [1, 4, 9])
+def test_batch_values_taken_at_once(sizes, batch):
+    """Simulation._take leaves the measures as one realization after another
+    would: data, iteration_data, and the tracked pupil's last centroid."""
+    rng = np.random.default_rng(batch)
+    mom, tr = rng.normal(size=(batch, 15)), rng.normal(size=(batch, 15))
+
+    class Owner:
+        pupil_shift = None
+
+        def set(self, channel, output):
+            return output
+
+    def build():
+        owner = Owner()
+        ms = [Measure(None, "atmosphere", owner.set, max_size=n) for n in sizes]
+        for m in ms:
+            m.data = [0.5]
+        kinds = [("moment", 2), ("pupil", 1), ("tracked", 0)]
+        return owner, [(m, kinds[i % 3]) for i, m in enumerate(ms)]
+
+    owner, items = build()
+    for b in range(batch):
+        for m, c in items:
+            m.iteration_data = float(mom[b, c[1]] if c[0] == "moment" else (mom if c[0] == "pupil" else tr)[b, 7 + c[1]])
+            if c[0] == "tracked":
+                owner.pupil_shift = (float(mom[b, 1]), float(mom[b, 2]))
+        for m, _ in items:
+            if not m.is_done:
+                m.data.append(m.iteration_data)
+        if all(m.is_done for m, _ in items):
+            break
+    owner2, items2 = build()
+    plan = dict(items=items2)
+    if any(not m.is_done for m, _ in items2):
+        Simulation([])._take([(plan, None, None)], {id(plan): (mom, tr)}, batch)
+        assert [(m.data, m.iteration_data) for m, _ in items2] == [(m.data, m.iteration_data) for m, _ in items]
+        assert owner2.pupil_shift == owner.pupil_shift
