@@ -290,9 +290,10 @@ k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restric
 constexpr int kLRChunk = 64;                                          // points per chunk
 constexpr int kLRSums = kLR * kLR + 2 * kLR;                          // G, h and g sums
 constexpr int kLRCoefH = 8 + kLR * kLR, kLRCoefG = kLRCoefH + kLR;   // sparam offsets
-constexpr int kLRThreads = 512;                                       // waves 0-3: G, 4-7: h and g
+constexpr int kLRThreads = 256;
+constexpr int kLRRow = kLR + 1;                                       // doubles per LDS row of coefficients
 static_assert(PA_LOWRANK_TERMS == 32, "the block is 32 K columns (kbeg = 2 d0 - 32)");
-static_assert(2 * kLRChunk <= kLRThreads && kLRThreads == 512 && kLRChunk == 64, "polynomial block split");
+static_assert(kLRThreads == 256 && kLRChunk == 64, "polynomial block split");
 constexpr int kLRMaxPoints = 4096;   // cap on d0
 constexpr int kLRAhead = 16;         // chunks' partials in flight in the sum
 static inline int lowrank_chunks(int P) { return (std::min(P, kLRMaxPoints) + kLRChunk - 1) / kLRChunk; }
@@ -380,10 +381,19 @@ k_screen_classify(int n, int P, double2* __restrict__ fxy, const double* __restr
   }
 }
 
-__global__ void __launch_bounds__(kLRThreads)
+// Of P_km = 2 i^m J_m (J_0 - 1 for m = 0) and Q_kn only the real number beside
+// i^(m mod 2) is kept: u_jm = +-2 J_m, v_jn likewise, so with a' = x + i y
+//   Re(a' Q_n P_m) = x v u, -y v u, -y v u, -x v u  for (n, m) both even, odd and
+// even, even and odd, both odd, and G falls into four 16 x 16 products over the
+// chunk's points, one per wave (v_mfma_f64_16x16x4f64, K = one value per point).
+// The Bessel recurrences (two waves) and the barrier bound a block, so what
+// counts is blocks in flight: 35 KB of LDS and 4 waves let a CU hold four,
+// where complex coefficients and 8 waves allowed two (168 us for 1280 screens
+// of 1024 points instead of 268).
+__global__ void __launch_bounds__(kLRThreads, 4)
 k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const double* __restrict__ chparam,
                       const int* __restrict__ chan, const double* __restrict__ sparam, double* __restrict__ part,
-                      double2* __restrict__ pcoef, int nc_max, const int* __restrict__ nsteps, int step) {
+                      double* __restrict__ pcoef, int nc_max, const int* __restrict__ nsteps, int step) {
   const int b = blockIdx.x, k0 = blockIdx.y * kLRChunk;
   if (nsteps && step >= nsteps[b]) return;
   const int ch = chan ? chan[b] : 0;
@@ -392,13 +402,13 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
   const double* sp = sparam + (size_t)b * PA_SCREEN_PARAMS;
   const int d0 = (int)sp[kSpD0], n2 = (int)sp[kSpN2];
   if (k0 >= d0) return;   // the whole block: no chunk points in the polynomial block
-  __shared__ double2 s_p[kLRChunk][kLR];   // P_km
-  __shared__ double2 s_q[kLRChunk][kLR];   // a'_k Q_kn (zero for column-smooth slots)
-  __shared__ double2 s_a[kLRChunk];        // a'_k
+  __shared__ double s_u[kLRChunk][kLRRow];   // P_km
+  __shared__ double s_v[kLRChunk][kLRRow];   // Q_kn (zero for column-smooth slots)
+  __shared__ double2 s_a[kLRChunk];          // a'_k
   const int cnt = min(kLRChunk, d0 - k0);   // a multiple of 16
-  // (point j, side): Bessel values; side 1 (alpha, columns) gives P_km =
-  // 2 i^m J_m (m >= 1) or J_0 - 1, side 0 (beta, rows) a'_k Q_kn; points
-  // j >= cnt of a partial chunk, and side 0 of the column-smooth slots, are zero
+  // (point j, side): Bessel values; side 1 (alpha, columns) gives P_km, side 0
+  // (beta, rows) Q_kn; points j >= cnt of a partial chunk, and side 0 of the
+  // column-smooth slots, are zero
   if (threadIdx.x < 2 * kLRChunk) {
     const int j = threadIdx.x % kLRChunk, side = threadIdx.x / kLRChunk, slot = k0 + j;
     double J[kLR];
@@ -412,18 +422,15 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
       for (int m = 0; m < kLR; ++m) J[m] = m == 0 ? 1.0 : 0.0;
     }
     // a column-smooth slot's P_km is kept for the tables
-    double2* pc = (side == 1 && j < cnt && slot >= n2) ? pcoef + ((size_t)b * nc_max + (slot - n2)) * kLR : nullptr;
+    double* pc = (side == 1 && j < cnt && slot >= n2) ? pcoef + ((size_t)b * nc_max + (slot - n2)) * kLR : nullptr;
 #pragma unroll
     for (int m = 0; m < kLR; ++m) {
-      const double v = m == 0 ? J[0] - 1.0 : 2.0 * J[m];
-      // times i^m
-      const double cr = (m & 3) == 0 ? v : (m & 3) == 2 ? -v : 0.0;
-      const double ci = (m & 3) == 1 ? v : (m & 3) == 3 ? -v : 0.0;
+      const double v = m == 0 ? J[0] - 1.0 : (m & 2) ? -2.0 * J[m] : 2.0 * J[m];   // times i^(m mod 2)
       if (side == 1) {
-        s_p[j][m] = make_double2(cr, ci);
-        if (pc) pc[m] = make_double2(cr, ci);
+        s_u[j][m] = v;
+        if (pc) pc[m] = v;
       } else {
-        s_q[j][m] = make_double2(a.x * cr - a.y * ci, a.x * ci + a.y * cr);
+        s_v[j][m] = v;
       }
     }
     if (side == 1) s_a[j] = a;
@@ -431,39 +438,30 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
   __syncthreads();
   double* out = part + ((size_t)b * gridDim.y + blockIdx.y) * kLRSums;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (wave < 4) {
-    // G[n][m] = sum_k A[n][k] B[k][m] over K = 2 cnt on v_mfma_f64_16x16x4f64,
-    // A[n][2j] = Re(a'Q)_jn, A[n][2j+1] = -Im(a'Q)_jn, B[2j][m] = Re P_jm,
-    // B[2j+1][m] = Im P_jm; wave w: the 16 x 16 tile (rows 16 (w / 2),
-    // columns 16 (w % 2)).  Lane l supplies A[l % 16][l / 16] and
-    // B[l / 16][l % 16] of each K step of 4 and holds D[4 i + l / 16][l % 16].
-    const int n0 = 16 * (wave >> 1), m0 = 16 * (wave & 1);
-    const int r = lane & 15, kk = lane >> 4, jo = kk >> 1;
-    const bool im = kk & 1;
+  {
+    // Lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] of each K step of 4
+    // and holds D[4 i + l / 16][l % 16]
+    const int pn = wave >> 1, pm = wave & 1, r = lane & 15, kk = lane >> 4;
     d4v acc = {0.0, 0.0, 0.0, 0.0};
-    for (int j = 0; j < cnt; j += 2) {
-      const double2 q = s_q[j + jo][n0 + r], p = s_p[j + jo][m0 + r];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(im ? -q.y : q.x, im ? p.y : p.x, acc, 0, 0, 0);
+    for (int j = kk; j < cnt; j += 4) {
+      const double2 a = s_a[j];
+      const double c = pn != pm ? -a.y : pn ? -a.x : a.x;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(c * s_v[j][2 * r + pn], s_u[j][2 * r + pm], acc, 0, 0, 0);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[(n0 + 4 * i + kk) * kLR + m0 + r] = acc[i];
-  } else {
-    // h (t < 32) and g sums: 4 lanes per sum, 16 points each, then the 4
-    // lanes' values added by xor shuffles
-    const int t = threadIdx.x - 256, o = t >> 2, sub = t & 3;
-    double v = 0.0;
-    for (int j = sub; j < cnt; j += 4) {
-      if (o < kLR) {
-        v += s_q[j][o].x;                                        // h: Re sum a' Q_kn
-      } else {
-        const double2 aa = s_a[j], pp = s_p[j][o - kLR];
-        v += aa.x * pp.x - aa.y * pp.y;                          // g: Re sum a' P_km
-      }
-    }
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
-    if (sub == 0) out[kLR * kLR + o] = v;
+    for (int i = 0; i < 4; ++i) out[(2 * (4 * i + kk) + pn) * kLR + 2 * r + pm] = acc[i];
   }
+  // h (o < 32) and g sums: 4 lanes per sum, 16 points each, then the 4 lanes'
+  // values added by xor shuffles
+  const int o = threadIdx.x >> 2, sub = threadIdx.x & 3, m = o % kLR;
+  double v = 0.0;
+  for (int j = sub; j < cnt; j += 4) {
+    const double2 a = s_a[j];
+    v += ((m & 1) ? -a.y : a.x) * (o < kLR ? s_v[j][m] : s_u[j][m]);   // Re a' Q_kn, Re a' P_km
+  }
+  v += __shfl_xor(v, 1, 64);
+  v += __shfl_xor(v, 2, 64);
+  if (sub == 0) out[kLR * kLR + o] = v;
 }
 
 // One thread per sum: the chunks' partials in chunk order.  Then the A scale:
@@ -473,7 +471,7 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
 // in sp[3] for the GEMM.
 __global__ void __launch_bounds__(1024)
 k_screen_lowrank_sum(int P, const double2* __restrict__ fxy, double* __restrict__ sparam,
-                     const double* __restrict__ part, const double2* __restrict__ pcoef, int nc_max, int chunks,
+                     const double* __restrict__ part, const double* __restrict__ pcoef, int nc_max, int chunks,
                      int mode, const int* __restrict__ nsteps, int step) {
   const int b = blockIdx.x;
   if (nsteps && step >= nsteps[b]) return;
@@ -506,8 +504,7 @@ k_screen_lowrank_sum(int P, const double2* __restrict__ fxy, double* __restrict_
     double v = 0.0;
     for (int tt = t; tt < d0 - n2; tt += 1024 / kLR) {
       const double2 a = fxy[((size_t)b * P + n2 + tt) * 2 + 1];
-      const double2 pm = pcoef[((size_t)b * nc_max + tt) * kLR + m];
-      v += 2.0 * sqrt(a.x * a.x + a.y * a.y) * sqrt(pm.x * pm.x + pm.y * pm.y);
+      v += 2.0 * sqrt(a.x * a.x + a.y * a.y) * fabs(pcoef[((size_t)b * nc_max + tt) * kLR + m]);
     }
     s_v[t][m] = v;
   }
@@ -567,6 +564,24 @@ __device__ __forceinline__ uint32_t split_pack(double v0, double v1, uint32_t& l
 }
 
 // ------------------------------------------------------------------ tables
+// In lanes whose bit OFF is clear, a + (a of the lane OFF above); in the others
+// b + (b of the lane OFF below): gfx950's lane swaps exchange the upper part of
+// `a` with the lower part of `b` without the LDS pipe.
+template <int OFF>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 x = __builtin_bit_cast(u2, a), y = __builtin_bit_cast(u2, b);
+  u2 p, q;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false)
+                             : __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+    p[i] = r[0];
+    q[i] = r[1];
+  }
+  return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
+}
+
 // One block per RT = TC * RG consecutive rows (AXIS = 0: A operand, h, eh) or
 // columns (AXIS = 1: B operand, g, eg) of element b; threads stride over k.
 // Along the block's rows the plane wave advances by a fixed angle, so each
@@ -578,12 +593,22 @@ __device__ __forceinline__ uint32_t split_pack(double v0, double v1, uint32_t& l
 // the 1-D sums are accumulated times `scale` (a power of two, divided out
 // exactly at the end).  RT (4, 8, 16 or 32) trades sincos work and per-block
 // set-up against the number of blocks.
+//
+// The polynomial block's 32 columns come from the Chebyshev values T_q(u) of
+// the block's rows, formed once (one thread per row, the forward recurrence)
+// and kept in LDS: they are the B operand's columns, and the A operand's are
+// the products T G + Re V on v_mfma_f64_16x16x4f64: 16 rows by the 16 even and
+// the 16 odd columns (P_km is real or imaginary by the parity of m, so a
+// column-smooth slot is one K of either), K split over the waves that share a
+// row tile.  Measured, 1280 screens of 512^2 (320 of 2048^2): the two axes take
+// 452 + 281 us (559 + 372); with each entry's own Clenshaw recurrence and dot
+// product over the slots on LDS operands 538 + 365 (644 + 478).
 template <int MODE, int AXIS, int TC, int RG>
 __global__ void __launch_bounds__(256, 4)
 k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
                 double* __restrict__ sparam, const double* __restrict__ chparam,
                 const int* __restrict__ chan, void* __restrict__ op, double* __restrict__ hg,
-                float2* __restrict__ esc, const double2* __restrict__ pcoef, int nc_max,
+                float2* __restrict__ esc, const double* __restrict__ pcoef, int nc_max,
                 const int* __restrict__ nsteps, int step) {
   constexpr int RT = TC * RG;
   static_assert(RT == 4 || RT == 8 || RT == 16 || RT == 32, "rows per block");
@@ -599,13 +624,8 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
   const int kbeg = (int)sp[kSpKbeg], klow = (int)sp[kSpD0], n2 = (int)sp[kSpN2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // operand scales (k_screen_prep, the A scale lowered by k_screen_lowrank_sum
-  // for the polynomial block); AXIS 0 stages G in LDS for the block's columns
+  // for the polynomial block)
   const double scale = sp[AXIS == 0 ? 1 : 2];
-  __shared__ double s_g[AXIS == 0 ? kLR * kLR : 1];
-  if constexpr (AXIS == 0) {
-    if (klow)
-      for (int e = threadIdx.x; e < kLR * kLR; e += 256) s_g[e] = sp[8 + e];
-  }
   constexpr bool SPLIT = MODE != PA_GEMM_F32;
   const size_t plane_bytes = (size_t)n * Kp * (SPLIT ? 2 : 4);
   char* opb = reinterpret_cast<char*>(op) + (size_t)b * plane_bytes * (SPLIT ? 2 : 1);
@@ -615,87 +635,126 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
   // 32 TC bytes.  Rows are padded so that 8 consecutive pieces read from 8
   // distinct 16-byte bank groups.
   constexpr int SROW = 256 + 8;
-  // (before the direct points the same LDS stages the column-smooth slots'
-  // plane waves)
-  __shared__ __attribute__((aligned(16))) uint32_t s_stage[2 * TC * SROW];
-  uint32_t* s_hi = s_stage;
-  uint32_t* s_lo = s_stage + TC * SROW;
-  // AXIS 0, first: the column-smooth slots, CS at a time.  Their P_km go to
-  // LDS (s_pc) while their plane waves (a' q)(r) for the block's rows are
-  // formed by the same recurrence as the direct points, thread (slot t, row
-  // group g) from two float64 sincos at the group's first row, and staged
-  // unscaled (s_aq, in the operand staging LDS); then each thread adds their
-  // share of V_m(r) to its entries of the polynomial columns (vacc, entry e =
-  // tid + 256 i, column m = tid % 32) and thread j < RT their share of h(r)
-  // (hsh), in slot order.
-  constexpr int NV = (RT * kLR + 255) / 256;
-  constexpr int CS = 16, RGS = RT >= 16 ? 16 : RT, RPG = RT / RGS;   // slots, row groups, rows per group
-  static_assert(RT * CS * 16 <= 2 * TC * SROW * 4, "column-smooth staging fits the operand staging");
-  __shared__ double2 s_pc[AXIS == 0 ? CS * kLR : 1];
-  double vacc[NV];
+  // (before the direct points the same LDS holds the column-smooth slots' plane
+  // waves, CS slots at a time, and the partial tiles)
+  constexpr int CS = 48, CROW = CS + 1, RPG = RT / 4, MR = RT < 16 ? 16 : RT;
+  constexpr int STAGE_BYTES = 2 * TC * SROW * 4, WAVE_BYTES = AXIS == 0 ? MR * CROW * 16 : 0;
+  constexpr int TILE_BYTES = AXIS == 0 ? 4 * 64 * 8 * 8 : 0;
+  constexpr int BUF1 = STAGE_BYTES > WAVE_BYTES ? STAGE_BYTES : WAVE_BYTES;
+  constexpr int BUF = BUF1 > TILE_BYTES ? BUF1 : TILE_BYTES;
+  __shared__ __attribute__((aligned(16))) char s_buf[BUF];
+  uint32_t* s_hi = reinterpret_cast<uint32_t*>(s_buf);
+  uint32_t* s_lo = s_hi + TC * SROW;
+  constexpr int TROW = kLR + 1;
+  __shared__ double s_t[MR * TROW];              // T_q(u) of the block's rows
+  __shared__ double s_h[AXIS == 0 ? 4 * 16 : 1];  // the column-smooth slots' share of h, per wave and tile row
+  // (v0, v1) into the polynomial block's columns kbeg + 2 pr, + 1 of row i0 + j
+  auto put_block = [&](int j, int pr, double v0, double v1) {
+    if constexpr (SPLIT) {
+      uint32_t lo;
+      const uint32_t hi = split_pack<MODE>(v0, v1, lo);
+      const size_t go = ((size_t)(kbeg / 16 + pr / 8) * n + i0 + j) * 32 + (2 * pr % 16) * 2;
+      *reinterpret_cast<uint32_t*>(opb + go) = hi;
+      *reinterpret_cast<uint32_t*>(opb + plane_bytes + go) = lo;
+    } else {
+      put_pair_f32(opb, Kp, i0 + j, kbeg / 2 + pr, v0, v1);
+    }
+  };
+  if (klow) {
+    if (threadIdx.x < RT) {
+      const double u = (double)(i0 + (int)threadIdx.x - n / 2) / (double)(n / 2);
+      double* t = s_t + threadIdx.x * TROW;
+      double t0 = 1.0, t1 = u;
+      t[0] = t0;
+      t[1] = t1;
 #pragma unroll
-  for (int i = 0; i < NV; ++i) vacc[i] = 0.0;
-  double hsh = 0.0;
-  if constexpr (AXIS == 0) {
-    double2* s_aq = reinterpret_cast<double2*>(s_stage);
-    const double2* pc = pcoef + (size_t)b * nc_max * kLR;
-    const int ncs = klow - n2, t = threadIdx.x % CS, g = threadIdx.x / CS;
-    // the next sub-chunk's P_km entries (e = tid, tid + 256) and this thread's
-    // slot are fetched one sub-chunk ahead, so their latency overlaps the work
-    static_assert(CS * kLR == 2 * 256, "two P_km entries per thread and sub-chunk");
-    double2 pn[2], fn = make_double2(0.0, 0.0), an = make_double2(0.0, 0.0);
-    auto fetch = [&](int t0) {
-      const int cnt = min(CS, ncs - t0);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int e = threadIdx.x + 256 * u;
-        pn[u] = e < cnt * kLR ? pc[(size_t)t0 * kLR + e] : make_double2(0.0, 0.0);
+      for (int q = 2; q < kLR; ++q) {
+        const double t2 = 2.0 * u * t1 - t0;
+        t0 = t1;
+        t1 = t2;
+        t[q] = t2;
       }
-      if (t < cnt) {
-        fn = fxy[((size_t)b * P + n2 + t0 + t) * 2];
-        an = fxy[((size_t)b * P + n2 + t0 + t) * 2 + 1];
-      }
-    };
-    if (ncs > 0) fetch(0);
-    for (int t0 = 0; t0 < ncs; t0 += CS) {
-      const int cnt = min(CS, ncs - t0);
-      const double2 f = fn, a = an;
-      __syncthreads();   // the staging LDS is free
-      s_pc[threadIdx.x] = pn[0];
-      s_pc[threadIdx.x + 256] = pn[1];
-      if (t0 + CS < ncs) fetch(t0 + CS);
-      if (t < cnt && g < RGS) {
-        double s0, c0, sd, cd;
-        sincos(kTwoPi * f.y * (coord0 + (double)(g * RPG) * delta), &s0, &c0);
-        sincos(kTwoPi * f.y * delta, &sd, &cd);
-        double wr = a.x * c0 - a.y * s0, wi = a.x * s0 + a.y * c0;
+    }
+    if constexpr (AXIS == 0) {
+      // wave w: row tile w % NT, every KS-th K step; lane l: A row l % 16, K l / 16
+      constexpr int NT = MR / 16, KS = 4 / NT;
+      const int tile = wave % NT, ks = wave / NT, r = lane & 15, kk = lane >> 4, tr = 16 * tile + r;
+      d4v ev = {0.0, 0.0, 0.0, 0.0}, od = ev;
+      double hs = 0.0;
+      double2* s_aq = reinterpret_cast<double2*>(s_buf);
+      const double* pc = pcoef + (size_t)b * nc_max * kLR;
+      const int ncs = klow - n2;
+      for (int t0 = 0; t0 < ncs; t0 += CS) {
+        const int cnt = min(CS, ncs - t0);
+        if (t0) __syncthreads();     // the previous slots' waves have been read
+        // slot t, rows g RPG ..: (a' q)(r) by the recurrence from the first row
+        const int t = threadIdx.x % CS, g = threadIdx.x / CS;
+        if (g < 4) {
+          double2 f = make_double2(0.0, 0.0), a = f;
+          if (t < cnt) {
+            f = fxy[((size_t)b * P + n2 + t0 + t) * 2];
+            a = fxy[((size_t)b * P + n2 + t0 + t) * 2 + 1];
+          }
+          double s0, c0, sd, cd;
+          sincos(kTwoPi * f.y * (coord0 + (double)(g * RPG) * delta), &s0, &c0);
+          sincos(kTwoPi * f.y * delta, &sd, &cd);
+          double wr = a.x * c0 - a.y * s0, wi = a.x * s0 + a.y * c0;
 #pragma unroll
-        for (int j = 0; j < RPG; ++j) {
-          s_aq[(g * RPG + j) * CS + t] = make_double2(wr - a.x, wi - a.y);
-          const double nr = wr * cd - wi * sd;
-          wi = wr * sd + wi * cd;
-          wr = nr;
-        }
-      }
-      __syncthreads();
-      const int m = threadIdx.x % kLR;
-#pragma unroll 4
-      for (int tt = 0; tt < cnt; ++tt) {
-        const double2 pm = s_pc[tt * kLR + m];
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-          const int e = threadIdx.x + 256 * i;
-          if (e < RT * kLR) {
-            const double2 q = s_aq[(e / kLR) * CS + tt];
-            vacc[i] += q.x * pm.x - q.y * pm.y;
+          for (int j = 0; j < RPG; ++j) {
+            s_aq[(g * RPG + j) * CROW + t] = make_double2(wr - a.x, wi - a.y);
+            const double nr = wr * cd - wi * sd;
+            wi = wr * sd + wi * cd;
+            wr = nr;
           }
         }
+        __syncthreads();
+        for (int k = 4 * ks; k < cnt; k += 4 * KS) {
+          const int slot = k + kk;     // slots past cnt have zero waves (cnt <= CS, a multiple of 4)
+          const double2 q = s_aq[tr * CROW + slot];
+          const double2 pm = slot < cnt ? *reinterpret_cast<const double2*>(pc + (size_t)(t0 + slot) * kLR + 2 * r)
+                                        : make_double2(0.0, 0.0);
+          ev = __builtin_amdgcn_mfma_f64_16x16x4f64(q.x, pm.x, ev, 0, 0, 0);
+          od = __builtin_amdgcn_mfma_f64_16x16x4f64(-q.y, pm.y, od, 0, 0, 0);
+          hs += q.x;
+        }
       }
-      if ((int)threadIdx.x < RT)
-#pragma nounroll
-        for (int tt = 0; tt < cnt; ++tt) hsh += s_aq[threadIdx.x * CS + tt].x;
+      __syncthreads();                 // T; and the waves have been read
+      for (int k = 4 * ks; k < kLR; k += 4 * KS) {
+        const double t = s_t[tr * TROW + k + kk];
+        const double2 gm = *reinterpret_cast<const double2*>(sp + 8 + (k + kk) * kLR + 2 * r);
+        ev = __builtin_amdgcn_mfma_f64_16x16x4f64(t, gm.x, ev, 0, 0, 0);
+        od = __builtin_amdgcn_mfma_f64_16x16x4f64(t, gm.y, od, 0, 0, 0);
+      }
+      hs += __shfl_xor(hs, 16, 64);
+      hs += __shfl_xor(hs, 32, 64);
+      if (kk == 0) s_h[wave * 16 + r] = hs;
+      // the K parts of a tile meet in LDS; entry i of lane l: row 4 i + l / 16,
+      // columns 2 (l % 16) and + 1, finished by wave i % KS of the tile
+      double2* s_d = reinterpret_cast<double2*>(s_buf);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_d[(wave * 4 + i) * 64 + lane] = make_double2(ev[i], od[i]);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = 16 * tile + 4 * i + kk;
+        if (i % KS != ks || j >= RT) continue;
+        double v0 = 0.0, v1 = 0.0;
+#pragma unroll
+        for (int w = 0; w < KS; ++w) {
+          const double2 d = s_d[((w * NT + tile) * 4 + i) * 64 + lane];
+          v0 += d.x;
+          v1 += d.y;
+        }
+        put_block(j, r, v0 * scale, v1 * scale);
+      }
+    } else {
+      __syncthreads();
+      for (int e = threadIdx.x; e < RT * kLR / 2; e += 256) {
+        const int j = e / (kLR / 2), pr = e % (kLR / 2);
+        put_block(j, pr, s_t[j * TROW + 2 * pr] * scale, s_t[j * TROW + 2 * pr + 1] * scale);
+      }
     }
-    __syncthreads();   // before the direct points reuse the staging LDS
+    __syncthreads();   // before the direct points use the staging LDS
   }
   double acc[RT];   // this thread's share of the 1-D sums, times scale
 #pragma unroll
@@ -760,54 +819,6 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
       }
     }
   }
-  // the polynomial block's kLR = 32 columns [kbeg, kbeg + 32) of these rows
-  // (AXIS 0: sum_n T_n(s) Re G[n][m] by Clenshaw + Re V_m(r)) or columns (AXIS
-  // 1: T_m(t)); thread e: row e / 32, column e % 32, the even lane of each
-  // pair stores both values (RT * 32 is a multiple of 64, so the loop is
-  // uniform over each wave)
-  if (klow) {
-    if constexpr (AXIS == 0) __syncthreads();   // s_g
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int e = threadIdx.x + 256 * i;
-      if (e >= RT * kLR) break;
-      const int j = e / kLR, m = e % kLR;
-      const double u = (double)(i0 + j - n / 2) / (double)(n / 2);
-      double val;
-      if constexpr (AXIS == 0) {
-        double b1 = 0.0, b2 = 0.0;
-#pragma unroll
-        for (int q = kLR - 1; q >= 1; --q) {
-          const double b0 = s_g[q * kLR + m] + 2.0 * u * b1 - b2;
-          b2 = b1;
-          b1 = b0;
-        }
-        val = s_g[m] + u * b1 - b2 + vacc[i];
-      } else {
-        double t0 = 1.0, t1 = u;
-        for (int q = 1; q < m; ++q) {
-          const double t2 = 2.0 * u * t1 - t0;
-          t0 = t1;
-          t1 = t2;
-        }
-        val = m == 0 ? 1.0 : t1;
-      }
-      const double v0 = val * scale;
-      const double v1 = __shfl_down(v0, 1, 64);
-      if (!(m & 1)) {
-        const int pr = m / 2;
-        if constexpr (SPLIT) {
-          uint32_t lo;
-          const uint32_t hi = split_pack<MODE>(v0, v1, lo);
-          const size_t go = ((size_t)(kbeg / 16 + pr / 8) * n + i0 + j) * 32 + (2 * pr % 16) * 2;
-          *reinterpret_cast<uint32_t*>(opb + go) = hi;
-          *reinterpret_cast<uint32_t*>(opb + plane_bytes + go) = lo;
-        } else {
-          put_pair_f32(opb, Kp, i0 + j, kbeg / 2 + pr, v0, v1);
-        }
-      }
-    }
-  }
   // reduce the RT sums over the block.  Within a wave, halving exchanges:
   // at offset 32 a lane keeps the half of its sums selected by bit 5 of its
   // index and adds the partner's copy of that half, and so on down to one sum
@@ -820,9 +831,15 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
     const bool up = lane & off;
 #pragma unroll
     for (int t = 0; t < half; ++t) {
-      const double keep = up ? acc[t + half] : acc[t];
-      const double send = up ? acc[t] : acc[t + half];
-      acc[t] = keep + __shfl_xor(send, off, 64);
+      if (s < 2) {
+        // lanes of the lower half keep sum t, of the upper half sum t + half:
+        // the swap puts a lane's own and its partner's copy side by side
+        acc[t] = s == 0 ? swap_add<32>(acc[t], acc[t + half]) : swap_add<16>(acc[t], acc[t + half]);
+      } else {
+        const double keep = up ? acc[t + half] : acc[t];
+        const double send = up ? acc[t] : acc[t + half];
+        acc[t] = keep + __shfl_xor(send, off, 64);
+      }
     }
   }
   double tot = acc[0];
@@ -836,29 +853,32 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
   __shared__ double red[4][RT];
   if ((lane & ((32 >> (LG - 1)) - 1)) == 0) red[wave][jr] = tot;
   __syncthreads();
-  if (threadIdx.x < RT) {
-    const int j = threadIdx.x, i = i0 + j;
-    double v = (red[0][j] + red[1][j] + red[2][j] + red[3][j]) * (1.0 / scale);
-    if constexpr (AXIS == 0) v += hsh;   // the column-smooth slots' share
-    // the polynomial points' share of h(r) (AXIS 0) or g(c): sum_n T_n(u) c[n]
-    // by Clenshaw
+  // 8 lanes per row: the polynomial points' share of h(r) (AXIS 0) or g(c),
+  // sum_q T_q(u) c[q], four terms each; the first lane finishes the row
+  if (threadIdx.x < 8 * RT) {
+    const int j = threadIdx.x / 8, sub = threadIdx.x % 8, i = i0 + j;
+    double v = 0.0;
     if (klow) {
       const double* cc = sp + (AXIS == 0 ? kLRCoefH : kLRCoefG);
-      const double u = (double)(i - n / 2) / (double)(n / 2);
-      double b1 = 0.0, b2 = 0.0;
 #pragma unroll
-      for (int q = kLR - 1; q >= 1; --q) {
-        const double b0 = cc[q] + 2.0 * u * b1 - b2;
-        b2 = b1;
-        b1 = b0;
+      for (int q = 0; q < kLR / 8; ++q) v += s_t[j * TROW + sub + 8 * q] * cc[sub + 8 * q];
+      v += __shfl_xor(v, 1, 64);
+      v += __shfl_xor(v, 2, 64);
+      v += __shfl_xor(v, 4, 64);
+      if constexpr (AXIS == 0) {
+        constexpr int NT = MR / 16, KS = 4 / NT;
+#pragma unroll
+        for (int w = 0; w < KS; ++w) v += s_h[(w * NT + j / 16) * 16 + j % 16];   // the column-smooth slots' share
       }
-      v += cc[0] + u * b1 - b2;
     }
-    hg[((size_t)b * 2 + AXIS) * n + i] = v;
-    const double ph = AXIS == 0 ? v + sp[0] : v;  // fold the piston into the row factor
-    double sn, cs;
-    sincos(ph, &sn, &cs);
-    esc[((size_t)b * 2 + AXIS) * n + i] = make_float2((float)cs, (float)-sn);
+    if (sub == 0) {
+      v += (red[0][j] + red[1][j] + red[2][j] + red[3][j]) * (1.0 / scale);
+      hg[((size_t)b * 2 + AXIS) * n + i] = v;
+      const double ph = AXIS == 0 ? v + sp[0] : v;  // fold the piston into the row factor
+      double sn, cs;
+      sincos(ph, &sn, &cs);
+      esc[((size_t)b * 2 + AXIS) * n + i] = make_float2((float)cs, (float)-sn);
+    }
   }
 }
 
@@ -1373,7 +1393,7 @@ static void tables_launch(int n, int P, double* fxy, double* sparam,
   // k_screen_tables<.., 0, ..> have read them
   const int chunks = lowrank_chunks(P);
   double* part = reinterpret_cast<double*>(opb);
-  double2* pcoef = reinterpret_cast<double2*>(part + (size_t)batch * chunks * kLRSums);
+  double* pcoef = part + (size_t)batch * chunks * kLRSums;
   double2* f2 = reinterpret_cast<double2*>(fxy);
 #define CL_(CH)                                                                                                       \
   hipLaunchKernelGGL(k_screen_classify<CH>, dim3(batch), dim3(kClassThreads), 0, s, n, P, f2, chparam, chan, sparam, \
