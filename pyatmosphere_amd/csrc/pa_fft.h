@@ -417,6 +417,50 @@ __device__ __forceinline__ void buf_st2(float2 v, rsrc_t r, int voff, int soff) 
   __builtin_amdgcn_raw_buffer_store_b64(x, r, voff, soff, AUX);
 }
 
+// In lanes whose bit OFF is clear, a + (a of the lane OFF above); in the others
+// b + (b of the lane OFF below): gfx950's lane swaps exchange the upper part of
+// `a` with the lower part of `b` without the LDS pipe.
+template <int OFF>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 x = __builtin_bit_cast(u2, a), y = __builtin_bit_cast(u2, b);
+  u2 p, q;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false)
+                             : __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+    p[i] = r[0];
+    q[i] = r[1];
+  }
+  return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
+}
+
+// v + (v of the lane OFF further round the 16-lane row), OFF 2, 4 or 8 (DPP
+// rotation, no LDS pipe): after the step of 2 OFF the lane OFF above and the
+// lane OFF below hold the same value, so it is the xor exchange of a reduction.
+template <int OFF>
+__device__ __forceinline__ double row_add(double v) {
+  static_assert(OFF == 2 || OFF == 4 || OFF == 8, "within a row of lanes");
+  typedef int i2 __attribute__((ext_vector_type(2)));
+  const i2 x = __builtin_bit_cast(i2, v);
+  i2 y;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) y[i] = __builtin_amdgcn_mov_dpp(x[i], 0x120 + OFF, 0xf, 0xf, true);
+  return v + __builtin_bit_cast(double, y);
+}
+
+// The sum over the wave's lanes with the same index mod T (T = 2, 4, 8), in every lane.
+template <int T>
+__device__ __forceinline__ double wave_sum_mod(double v) {
+  static_assert(T == 2 || T == 4 || T == 8, "rows interleaved over the lanes");
+  v = swap_add<32>(v, v);
+  v = swap_add<16>(v, v);
+  v = row_add<8>(v);
+  if constexpr (T <= 4) v = row_add<4>(v);
+  if constexpr (T <= 2) v = row_add<2>(v);
+  return v;
+}
+
 // Field layout in HBM between passes ("row-tiled"): T consecutive rows form a
 // tile stored column-interleaved, element (r, c) at ((r/T)*N + c)*T + r%T.
 // A row pass block owns one tile (one contiguous T*N run); a column pass block

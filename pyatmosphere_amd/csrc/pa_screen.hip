@@ -564,24 +564,6 @@ __device__ __forceinline__ uint32_t split_pack(double v0, double v1, uint32_t& l
 }
 
 // ------------------------------------------------------------------ tables
-// In lanes whose bit OFF is clear, a + (a of the lane OFF above); in the others
-// b + (b of the lane OFF below): gfx950's lane swaps exchange the upper part of
-// `a` with the lower part of `b` without the LDS pipe.
-template <int OFF>
-__device__ __forceinline__ double swap_add(double a, double b) {
-  typedef unsigned u2 __attribute__((ext_vector_type(2)));
-  const u2 x = __builtin_bit_cast(u2, a), y = __builtin_bit_cast(u2, b);
-  u2 p, q;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false)
-                             : __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
-    p[i] = r[0];
-    q[i] = r[1];
-  }
-  return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
-}
-
 // One block per RT = TC * RG consecutive rows (AXIS = 0: A operand, h, eh) or
 // columns (AXIS = 1: B operand, g, eg) of element b; threads stride over k.
 // Along the block's rows the plane wave advances by a fixed angle, so each
