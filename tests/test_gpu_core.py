@@ -731,3 +731,35 @@ def test_host_draws_synthesize_whole(dev, monkeypatch, screens):
         mom = engine.run_batch(ws, tables, chan, np.array(screens), host_spectra=spectra, field_out=out)
         got.append((out, mom.clone()))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n", [64, 256, 512, 1024])
+@pytest.mark.parametrize("batch", [1, 7, 8, 11, 16])
+def test_gemm_tiles_cover_every_element(dev, n, batch):
+    """Every element's screen is formed whatever the batch's remainder of 8, by
+    both tile shapes and the float32 GEMM: equal to the element on its own, and
+    untouched where it has no screen."""
+    P = 64
+    spec = channel_spec(n, 0.002, 808e-9, 0.05, 5e3, 3, P, 1e-15)
+    spectra, _ = host_spectra(spec, batch, seed=batch)
+    tables = engine.DeviceTables([spec], dev)
+    ns = torch.ones(batch, dtype=torch.int32, device=dev)
+    ns[batch // 2] = 0 if batch > 1 else 1
+    for mode, tile in (("f16x3", 1), ("f16x3", 2), ("f32", 0)):
+        ws, one = engine.Workspace(n, P, batch, mode, dev), engine.Workspace(n, P, 1, mode, dev)
+        for w in (ws, one):
+            w.chan.zero_()
+        engine.upload_spectra(ws, *spectra[0], batch=batch)
+        ws.ang.fill_(7.0)
+        engine.prep_screen(ws, tables, 0, batch, None, None)
+        engine.plane_wave_tables(ws, tables, 0, batch, None, None, rows=8)
+        engine.screen_gemm(ws, 0, batch, ns, None, ang=ws.ang, tile=tile)
+        for b in range(batch):
+            if not int(ns[b]):
+                assert bool((ws.ang[b] == 7.0).all())
+                continue
+            engine.upload_spectra(one, *(a[b:b + 1] for a in spectra[0]), batch=1)
+            engine.prep_screen(one, tables, 0, 1, None, None)
+            engine.plane_wave_tables(one, tables, 0, 1, None, None, rows=8)
+            engine.screen_gemm(one, 0, 1, None, None, ang=one.ang, tile=tile)
+            assert torch.equal(one.ang[0], ws.ang[b])
