@@ -356,14 +356,14 @@ int pa_mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, f
 /* Loss and gradients of one minibatch of an MLP whose layer i maps sizes[i] to
  * sizes[i + 1] values (SiLU between layers, the head of pa_mlp_head_loss with
  * sizes[layers] - 1 <= 64 bins at the end): X[M][sizes[0]], params = (W0, b0,
- * W1, b1, ...) with W_i [sizes[i + 1]][sizes[i]], loss[M], grads laid out as
- * params (host arrays of device pointers).  The launches of a step in one call.
+ * W1, b1, ...) with W_i [sizes[i + 1]][sizes[i]], loss[M], mean (nullable) the
+ * mean of loss, grads laid out as params (host arrays of device pointers).  The launches of a step in one call.
  * scratch: pa_mlp_loss_grads_scratch(layers, sizes, M) bytes, 16-byte aligned.
  * layers <= 256. */
 long long pa_mlp_loss_grads_scratch(int layers, const int* sizes, int M);
 int pa_mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
-                      const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
-                      void* scratch, void* stream);
+                      const float* target, const float* tvar, float wv, float wc, float* loss, float* mean,
+                      float* const* grads, void* scratch, void* stream);
 /* pa_mlp_adam of `count` tensors (host arrays of sizes and device pointers). */
 int pa_mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
                       float* const* v, float lr, float b1, float b2, float eps, int t, void* stream);

@@ -77,7 +77,7 @@ SIGNATURES = {
     "pa_mlp_head_loss": (i32, [i32, i32, vp, vp, vp, f32, f32, vp, vp, vp]),
     "pa_mlp_adam": (i32, [i32, vp, vp, vp, vp, f32, f32, f32, f32, i32, vp]),
     "pa_mlp_loss_grads_scratch": (i64, [i32, vp, i32]),
-    "pa_mlp_loss_grads": (i32, [i32, vp, i32, vp, vp, vp, vp, f32, f32, vp, vp, vp, vp]),
+    "pa_mlp_loss_grads": (i32, [i32, vp, i32, vp, vp, vp, vp, f32, f32, vp, vp, vp, vp, vp]),
     "pa_mlp_adam_multi": (i32, [i32, vp, vp, vp, vp, vp, f32, f32, f32, f32, i32, vp]),
     "pa_mlp_to_bf16": (i32, [i64, vp, vp, vp]),
     "pa_mlp_pack_bytes": (i64, [i32, vp]),

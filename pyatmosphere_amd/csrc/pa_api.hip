@@ -76,8 +76,8 @@ int mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, floa
              int t, hipStream_t s);
 long long mlp_loss_grads_scratch(int layers, const int* sizes, int M);
 int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
-                   const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
-                   float* scratch, hipStream_t s);
+                   const float* target, const float* tvar, float wv, float wc, float* loss, float* mean,
+                   float* const* grads, float* scratch, hipStream_t s);
 int mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
                    float* const* v, float lr, float b1, float b2, float eps, int t, hipStream_t s);
 bool mlp_infer_fits(int layers, const int* sizes);
@@ -421,12 +421,12 @@ long long pa_mlp_loss_grads_scratch(int layers, const int* sizes, int M) {
   return mlp_loss_grads_scratch(layers, sizes, M);
 }
 int pa_mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
-                      const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
-                      void* scratch, void* stream) {
+                      const float* target, const float* tvar, float wv, float wc, float* loss, float* mean,
+                      float* const* grads, void* scratch, void* stream) {
   REQUIRE(mlp_sizes_ok(layers, sizes, M), "mlp_loss_grads: bad layer sizes or batch");
   REQUIRE(X && params && target && tvar && loss && grads && scratch, "mlp_loss_grads: null pointer");
   for (int i = 0; i < 2 * layers; ++i) REQUIRE(params[i] && grads[i], "mlp_loss_grads: null pointer");
-  return mlp_loss_grads(layers, sizes, M, X, params, target, tvar, wv, wc, loss, grads,
+  return mlp_loss_grads(layers, sizes, M, X, params, target, tvar, wv, wc, loss, mean, grads,
                         reinterpret_cast<float*>(scratch), STREAM(stream));
 }
 int pa_mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,

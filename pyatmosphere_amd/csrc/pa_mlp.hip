@@ -30,7 +30,8 @@ typedef unsigned short us8 __attribute__((ext_vector_type(8)));
 // Measured, a 1024-pair step of the 384-wide network (loss, gradients, Adam):
 // 1856 us with 64 x 64 LDS tiles on the vector units (94 us a product, 36 to 96
 // blocks), serial column sums for db (194 us) and a launch per pass and tensor;
-// 94 us with these kernels (10-12 us a product, 21 us for all weight gradients).
+// 91 us with these kernels (10-12 us a product, 20 us for all weight gradients;
+// 8 waves a tile or other depths of loads in flight are 8 to 25% slower).
 typedef float f16v __attribute__((ext_vector_type(16)));
 constexpr int GT = 32;             // C tile
 constexpr int GU = 4;              // groups of 8 k in flight per wave
@@ -199,7 +200,8 @@ k_layer_backward(int M, int N, int K, const float* __restrict__ D, const float* 
 }
 
 // Every layer's dW = D^T H (fo x fi over K = M rows) and db = column sums of D
-// in one launch: the products do not depend on each other, and together they
+// in one launch, and the mean of the rows' losses in a block of its own (the
+// last, mean non-null): the products do not depend on each other, and together they
 // fill the chip (336 tiles of 16 waves for the 16-384-384-384-65 network).
 constexpr int kGradLayers = 8;      // layers per launch
 constexpr int kGradWaves = 16;
@@ -211,9 +213,20 @@ struct GradLayers {
   int fo[kGradLayers], fi[kGradLayers], first[kGradLayers + 1];   // first: tiles before this layer
 };
 __global__ void __launch_bounds__(64 * kGradWaves)
-k_weight_grads(int layers, int M, GradLayers g) {
+k_weight_grads(int layers, int M, GradLayers g, const float* __restrict__ loss, float* __restrict__ mean) {
   __shared__ float red[kGradWaves * GT * 33];
   __shared__ float rs[kGradWaves * GT];
+  if ((int)blockIdx.x == g.first[layers]) {
+    float s = 0.f;
+    for (int i = threadIdx.x; i < M; i += 64 * kGradWaves) s += loss[i];
+    red[threadIdx.x] = s;
+    for (int o = 32 * kGradWaves; o > 0; o >>= 1) {
+      __syncthreads();
+      if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    }
+    if (threadIdx.x == 0) *mean = red[0] / M;
+    return;
+  }
   int i = 0;
   while (i + 1 < layers && (int)blockIdx.x >= g.first[i + 1]) ++i;
   const int fo = g.fo[i], fi = g.fi[i], nx = (fi + GT - 1) / GT, tile = blockIdx.x - g.first[i];
@@ -377,13 +390,15 @@ k_layer_bf16(int M, int N, int K, const float* __restrict__ X, const unsigned sh
 // weights in the order the products read them (pack_bf16): the fragment of
 // (32-column tile, 16-wide K chunk) is 1 KB, 16 bytes per lane, where rows of
 // the plain matrix gave 32 scattered 32-byte pieces.  A wave owns a tile and
-// walks K with kInferAhead fragments in flight (the products are a serial
-// chain per tile, so the loads' latency bounds it); 12 waves cover a 384-wide
-// layer at once.  Chunk order, operand roles and roundings are k_layer_bf16's,
+// walks K in groups of kInferAhead chunks, the next group's fragments loaded
+// before the current one's products (a serial chain per tile, so the loads'
+// latency bounds it); 12 waves cover a 384-wide layer at once, and two blocks
+// share a CU.  Chunk order, operand roles and roundings are k_layer_bf16's,
 // so the outputs are bit-equal to running the layers one by one.
 // Measured, 4096 rows x 3 members of width 384: 720 us of layer launches before,
-// 55 us now, the 0.7 MB of weights each block reads from L2.
-constexpr int kInferRows = 32, kInferWaves = 12, kInferWidth = 512, kInferAhead = 8;
+// 34 us now (55 with one guarded chunk at a time, which took 168 registers, one
+// block per CU, and waited for every load).
+constexpr int kInferRows = 32, kInferWaves = 12, kInferWidth = 512, kInferAhead = 4;
 constexpr int kInferLayers = 16, kInferMembers = 8;
 constexpr int kInferStride = kInferWidth + 8;   // bf16 per LDS row: 16-byte reads of 32 rows hit all banks
 
@@ -394,7 +409,7 @@ struct InferNet {
 
 static __host__ __device__ inline int tiles32(int n) { return (n + 31) / 32; }
 
-__global__ void __launch_bounds__(64 * kInferWaves)
+__global__ void __launch_bounds__(64 * kInferWaves, 2 * kInferWaves / 4)
 k_mlp_infer(int layers, int inputs, int M, const float* __restrict__ x, InferNet net, float* __restrict__ out) {
   __shared__ __attribute__((aligned(16))) unsigned short act[2][kInferRows * kInferStride];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
@@ -417,30 +432,46 @@ k_mlp_infer(int layers, int inputs, int M, const float* __restrict__ x, InferNet
       f16v acc;
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+      auto mma = [&](int c, us8 bf) {
+        const us8 a = *reinterpret_cast<const us8*>(cur + 16 * c);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, bf), acc, 0, 0, 0);
+      };
       us8 q[kInferAhead];
 #pragma unroll
       for (int u = 0; u < kInferAhead; ++u) q[u] = f[(size_t)min(u, nc - 1) * 64];
-      for (int c0 = 0; c0 < nc; c0 += kInferAhead) {
+      int c0 = 0;
+      for (; c0 + kInferAhead <= nc; c0 += kInferAhead) {
+        us8 nq[kInferAhead];
 #pragma unroll
-        for (int u = 0; u < kInferAhead; ++u) {
-          if (c0 + u >= nc) break;
-          const us8 b = q[u];
-          q[u] = f[(size_t)min(c0 + u + kInferAhead, nc - 1) * 64];
-          const us8 a = *reinterpret_cast<const us8*>(cur + 16 * (c0 + u));
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), acc, 0,
-                                                        0, 0);
-        }
+        for (int u = 0; u < kInferAhead; ++u) nq[u] = f[(size_t)min(c0 + kInferAhead + u, nc - 1) * 64];
+#pragma unroll
+        for (int u = 0; u < kInferAhead; ++u) mma(c0 + u, q[u]);
+#pragma unroll
+        for (int u = 0; u < kInferAhead; ++u) q[u] = nq[u];
       }
-      const int col = 32 * t + r;
-      const float bc = bias[col];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int rr = 8 * (v / 4) + 4 * h + v % 4;
-        const float z = acc[v] + bc;
-        if (i < layers - 1) {
-          nxt[rr * kInferStride + col] = f2bf(z * sigm(z));
-        } else if (col < fo && m0 + rr < M) {
-          out[((size_t)member * M + m0 + rr) * fo + col] = z;
+      for (int u = 0; u < kInferAhead - 1; ++u)
+        if (c0 + u < nc) mma(c0 + u, q[u]);
+      // an opaque copy of the lane index: the epilogue's addresses are formed
+      // here, not carried through the layers in registers
+      int el = lane;
+      asm volatile("" : "+v"(el));
+      const int col = 32 * t + (el & 31), row = 4 * (el >> 5);
+      const float bc = bias[col];
+      if (i < layers - 1) {
+        unsigned short* o = nxt + row * kInferStride + col;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const float z = acc[v] + bc;
+          o[(8 * (v / 4) + v % 4) * kInferStride] = f2bf(z * sigm(z));
+        }
+      } else if (col < fo) {
+        float* o = out + ((size_t)member * M + m0 + row) * fo + col;
+        const int left = M - m0 - row;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int rr = 8 * (v / 4) + v % 4;
+          if (rr < left) o[rr * fo] = acc[v] + bc;
         }
       }
     }
@@ -549,8 +580,8 @@ long long mlp_loss_grads_scratch(int layers, const int* sizes, int M) {
 }
 
 int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
-                   const float* target, const float* tvar, float wv, float wc, float* loss, float* const* grads,
-                   float* scratch, hipStream_t s) {
+                   const float* target, const float* tvar, float wv, float wc, float* loss, float* mean,
+                   float* const* grads, float* scratch, hipStream_t s) {
   const int NB = sizes[layers] - 1;
   // scratch: every layer's Z, then every layer's dZ, then the hidden layers' Y
   size_t all = 0;
@@ -608,7 +639,9 @@ int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const fl
       g.fi[j] = fi;
       g.first[j + 1] = g.first[j] + ((fo + GT - 1) / GT) * ((fi + GT - 1) / GT);
     }
-    hipLaunchKernelGGL(k_weight_grads, dim3(g.first[cnt]), dim3(64 * kGradWaves), 0, s, cnt, M, g);
+    const bool last = i0 + cnt == layers;
+    hipLaunchKernelGGL(k_weight_grads, dim3(g.first[cnt] + (last && mean ? 1 : 0)), dim3(64 * kGradWaves), 0, s, cnt, M,
+                       g, loss, mean);
   }
   return check_launch("mlp_loss_grads");
 }

@@ -122,13 +122,14 @@ class PDTSurrogate:
         """Mean loss (device scalar) and gradients [(dW, db)] for one batch."""
         M, layers = X.shape[0], len(self.params)
         sizes = self._layer_sizes()
-        loss = torch.empty(M, dtype=torch.float32, device=self.device)
+        loss = torch.empty(M + 1, dtype=torch.float32, device=self.device)    # the rows' losses, their mean
         scratch = torch.empty(call("pa_mlp_loss_grads_scratch", layers, sizes, M), dtype=torch.uint8,
                               device=self.device)
         grads = [(torch.empty_like(W), torch.empty_like(b)) for W, b in self.params]
         call("pa_mlp_loss_grads", layers, sizes, M, ptr(X), ptr_array(_flat(self.params)), ptr(T), ptr(TV),
-             float(self.wv), float(self.wc), ptr(loss), ptr_array(_flat(grads)), ptr(scratch), _lib.stream_handle())
-        return loss.mean(), grads
+             float(self.wv), float(self.wc), ptr(loss), ptr(loss) + 4 * M, ptr_array(_flat(grads)), ptr(scratch),
+             _lib.stream_handle())
+        return loss[M], grads
 
     def adam_step(self, grads, lr: float, b1=0.9, b2=0.999, eps=1e-8) -> None:
         self.t += 1
