@@ -393,7 +393,7 @@ k_screen_classify(int n, int P, double2* __restrict__ fxy, const double* __restr
 __global__ void __launch_bounds__(kLRThreads, 4)
 k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const double* __restrict__ chparam,
                       const int* __restrict__ chan, const double* __restrict__ sparam, double* __restrict__ part,
-                      double* __restrict__ pcoef, int nc_max, const int* __restrict__ nsteps, int step) {
+                      double* __restrict__ pcoef, size_t pstride, const int* __restrict__ nsteps, int step) {
   const int b = blockIdx.x, k0 = blockIdx.y * kLRChunk;
   if (nsteps && step >= nsteps[b]) return;
   const int ch = chan ? chan[b] : 0;
@@ -422,7 +422,7 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
       for (int m = 0; m < kLR; ++m) J[m] = m == 0 ? 1.0 : 0.0;
     }
     // a column-smooth slot's P_km is kept for the tables
-    double* pc = (side == 1 && j < cnt && slot >= n2) ? pcoef + ((size_t)b * nc_max + (slot - n2)) * kLR : nullptr;
+    double* pc = (side == 1 && j < cnt && slot >= n2) ? pcoef + (size_t)b * pstride + (slot - n2) * kLR : nullptr;
 #pragma unroll
     for (int m = 0; m < kLR; ++m) {
       const double v = m == 0 ? J[0] - 1.0 : (m & 2) ? -2.0 * J[m] : 2.0 * J[m];   // times i^(m mod 2)
@@ -436,7 +436,7 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
     if (side == 1) s_a[j] = a;
   }
   __syncthreads();
-  double* out = part + ((size_t)b * gridDim.y + blockIdx.y) * kLRSums;
+  double* out = part + (size_t)b * pstride + blockIdx.y * kLRSums;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   {
     // Lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] of each K step of 4
@@ -471,17 +471,17 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
 // in sp[3] for the GEMM.
 __global__ void __launch_bounds__(1024)
 k_screen_lowrank_sum(int P, const double2* __restrict__ fxy, double* __restrict__ sparam,
-                     const double* __restrict__ part, const double* __restrict__ pcoef, int nc_max, int chunks,
-                     int mode, const int* __restrict__ nsteps, int step) {
+                     const double* __restrict__ part, const double* __restrict__ pcoef, size_t pstride, int mode,
+                     const int* __restrict__ nsteps, int step) {
   const int b = blockIdx.x;
   if (nsteps && step >= nsteps[b]) return;
   double* sp = sparam + (size_t)b * PA_SCREEN_PARAMS;
   const int d0 = (int)sp[kSpD0], n2 = (int)sp[kSpN2];
   if (!d0) return;   // prep's scales stand
-  const int used = (d0 + kLRChunk - 1) / kLRChunk;   // <= chunks
+  const int used = (d0 + kLRChunk - 1) / kLRChunk;
   __shared__ double s_g[kLR * kLR];
   for (int e = threadIdx.x; e < kLRSums; e += 1024) {
-    const double* pb = part + (size_t)b * chunks * kLRSums + e;
+    const double* pb = part + (size_t)b * pstride + e;
     double sum = 0.0;
     for (int c0 = 0; c0 < used; c0 += kLRAhead) {
       double v[kLRAhead];
@@ -504,7 +504,7 @@ k_screen_lowrank_sum(int P, const double2* __restrict__ fxy, double* __restrict_
     double v = 0.0;
     for (int tt = t; tt < d0 - n2; tt += 1024 / kLR) {
       const double2 a = fxy[((size_t)b * P + n2 + tt) * 2 + 1];
-      v += 2.0 * sqrt(a.x * a.x + a.y * a.y) * fabs(pcoef[((size_t)b * nc_max + tt) * kLR + m]);
+      v += 2.0 * sqrt(a.x * a.x + a.y * a.y) * fabs(pcoef[(size_t)b * pstride + tt * kLR + m]);
     }
     s_v[t][m] = v;
   }
@@ -585,17 +585,40 @@ __device__ __forceinline__ uint32_t split_pack(double v0, double v1, uint32_t& l
 // row tile.  Measured, 1280 screens of 512^2 (320 of 2048^2): the two axes take
 // 452 + 281 us (559 + 372); with each entry's own Clenshaw recurrence and dot
 // product over the slots on LDS operands 538 + 365 (644 + 478).
+//
+// AXIS 0 and 1 fill one operand each; AXIS 2 fills both, axis blockIdx.z: the
+// polynomial part of A's blocks is a chain of latencies (sincos, barriers, MFMA)
+// and B's blocks are stores, so they overlap.  Measured, the whole of
+// pa_screen_tables with one launch against two: 16.3 against 22.4 us of kernels
+// for one 2048^2 screen, 50 against 62 us (ten of 2048^2), 57 against 67 (60 of
+// 512^2), 260 against 280 (189 of 1024^2), 944 against 975 (320 of 2048^2), 884
+// against 903 (1280 of 512^2).
+template <int AXIS, int TC, int RG>
+struct TablesLds {
+  static constexpr int RT = TC * RG, MR = RT < 16 ? 16 : RT;
+  // split modes stage TC rows x 256 points; before the direct points the same
+  // LDS holds the column-smooth slots' plane waves, CS slots at a time, and the
+  // partial tiles
+  static constexpr int SROW = 256 + 8, CS = 48, CROW = CS + 1, TROW = kLR + 1;
+  static constexpr int STAGE_BYTES = 2 * TC * SROW * 4, WAVE_BYTES = AXIS == 0 ? MR * CROW * 16 : 0;
+  static constexpr int TILE_BYTES = AXIS == 0 ? 4 * 64 * 8 * 8 : 0;
+  static constexpr int BUF1 = STAGE_BYTES > WAVE_BYTES ? STAGE_BYTES : WAVE_BYTES;
+  static constexpr int BUF = BUF1 > TILE_BYTES ? BUF1 : TILE_BYTES;
+  __attribute__((aligned(16))) char buf[BUF];
+  double t[MR * TROW];              // T_q(u) of the block's rows
+  double h[AXIS == 0 ? 4 * 16 : 1];  // the column-smooth slots' share of h, per wave and tile row
+  double red[4][RT];
+};
+
 template <int MODE, int AXIS, int TC, int RG>
-__global__ void __launch_bounds__(256, 4)
-k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
-                double* __restrict__ sparam, const double* __restrict__ chparam,
-                const int* __restrict__ chan, void* __restrict__ op, double* __restrict__ hg,
-                float2* __restrict__ esc, const double* __restrict__ pcoef, int nc_max,
-                const int* __restrict__ nsteps, int step) {
+__device__ __forceinline__ void
+tables_axis(TablesLds<AXIS, TC, RG>& lds, int n, int P, int Kp, const double2* __restrict__ fxy,
+            double* __restrict__ sparam, const double* __restrict__ chparam,
+            const int* __restrict__ chan, void* __restrict__ op, double* __restrict__ hg,
+            float2* __restrict__ esc, const double* __restrict__ pcoef, size_t pstride) {
   constexpr int RT = TC * RG;
   static_assert(RT == 4 || RT == 8 || RT == 16 || RT == 32, "rows per block");
   const int b = blockIdx.y;
-  if (nsteps && step >= nsteps[b]) return;
   const int i0 = blockIdx.x * RT;  // first row (AXIS 0) or column (AXIS 1)
   const int ch = chan ? chan[b] : 0;
   const double delta = chparam[ch * kChParams + 0];
@@ -616,20 +639,13 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
   // operand: the TC rows of one 16-element chunk are one contiguous run of
   // 32 TC bytes.  Rows are padded so that 8 consecutive pieces read from 8
   // distinct 16-byte bank groups.
-  constexpr int SROW = 256 + 8;
-  // (before the direct points the same LDS holds the column-smooth slots' plane
-  // waves, CS slots at a time, and the partial tiles)
-  constexpr int CS = 48, CROW = CS + 1, RPG = RT / 4, MR = RT < 16 ? 16 : RT;
-  constexpr int STAGE_BYTES = 2 * TC * SROW * 4, WAVE_BYTES = AXIS == 0 ? MR * CROW * 16 : 0;
-  constexpr int TILE_BYTES = AXIS == 0 ? 4 * 64 * 8 * 8 : 0;
-  constexpr int BUF1 = STAGE_BYTES > WAVE_BYTES ? STAGE_BYTES : WAVE_BYTES;
-  constexpr int BUF = BUF1 > TILE_BYTES ? BUF1 : TILE_BYTES;
-  __shared__ __attribute__((aligned(16))) char s_buf[BUF];
+  using Lds = TablesLds<AXIS, TC, RG>;
+  constexpr int SROW = Lds::SROW, CS = Lds::CS, CROW = Lds::CROW, TROW = Lds::TROW, RPG = RT / 4, MR = Lds::MR;
+  char* s_buf = lds.buf;
+  double* s_t = lds.t;
+  double* s_h = lds.h;
   uint32_t* s_hi = reinterpret_cast<uint32_t*>(s_buf);
   uint32_t* s_lo = s_hi + TC * SROW;
-  constexpr int TROW = kLR + 1;
-  __shared__ double s_t[MR * TROW];              // T_q(u) of the block's rows
-  __shared__ double s_h[AXIS == 0 ? 4 * 16 : 1];  // the column-smooth slots' share of h, per wave and tile row
   // (v0, v1) into the polynomial block's columns kbeg + 2 pr, + 1 of row i0 + j
   auto put_block = [&](int j, int pr, double v0, double v1) {
     if constexpr (SPLIT) {
@@ -664,7 +680,7 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
       d4v ev = {0.0, 0.0, 0.0, 0.0}, od = ev;
       double hs = 0.0;
       double2* s_aq = reinterpret_cast<double2*>(s_buf);
-      const double* pc = pcoef + (size_t)b * nc_max * kLR;
+      const double* pc = pcoef + (size_t)b * pstride;
       const int ncs = klow - n2;
       for (int t0 = 0; t0 < ncs; t0 += CS) {
         const int cnt = min(CS, ncs - t0);
@@ -832,7 +848,7 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
   int jr = 0;
 #pragma unroll
   for (int s = 0; s < LG; ++s) jr |= ((lane >> (5 - s)) & 1) << (LG - 1 - s);
-  __shared__ double red[4][RT];
+  auto& red = lds.red;
   if ((lane & ((32 >> (LG - 1)) - 1)) == 0) red[wave][jr] = tot;
   __syncthreads();
   // 8 lanes per row: the polynomial points' share of h(r) (AXIS 0) or g(c),
@@ -861,6 +877,30 @@ k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
       sincos(ph, &sn, &cs);
       esc[((size_t)b * 2 + AXIS) * n + i] = make_float2((float)cs, (float)-sn);
     }
+  }
+}
+
+template <int MODE, int AXIS, int TC, int RG>
+__global__ void __launch_bounds__(256, 4)
+k_screen_tables(int n, int P, int Kp, const double2* __restrict__ fxy,
+                double* __restrict__ sparam, const double* __restrict__ chparam,
+                const int* __restrict__ chan, void* __restrict__ opa, void* __restrict__ opb, double* __restrict__ hg,
+                float2* __restrict__ esc, const double* __restrict__ pcoef, size_t pstride,
+                const int* __restrict__ nsteps, int step) {
+  if (nsteps && step >= nsteps[blockIdx.y]) return;
+  if constexpr (AXIS == 2) {
+    __shared__ union {
+      TablesLds<0, TC, RG> a;
+      TablesLds<1, TC, RG> b;
+    } lds;
+    if (blockIdx.z == 0)
+      tables_axis<MODE, 0, TC, RG>(lds.a, n, P, Kp, fxy, sparam, chparam, chan, opa, hg, esc, pcoef, pstride);
+    else
+      tables_axis<MODE, 1, TC, RG>(lds.b, n, P, Kp, fxy, sparam, chparam, chan, opb, hg, esc, pcoef, pstride);
+  } else {
+    __shared__ TablesLds<AXIS, TC, RG> lds;
+    tables_axis<MODE, AXIS, TC, RG>(lds, n, P, Kp, fxy, sparam, chparam, chan, AXIS == 0 ? opa : opb, hg, esc, pcoef,
+                                    pstride);
   }
 }
 
@@ -1377,18 +1417,32 @@ int screen_prep(int P, const float* rho, const float* theta, const float2* value
   return check_launch("screen_prep");
 }
 
+static bool tables_at_once(int n, int mode) { return mode != PA_GEMM_F32 && n >= 128; }
+
+// Rows per table block.  With both axes in one launch, 32 from 6144 rows up
+// (screens times n; measured, 32 against 8 rows: 36.9 against 38.5 us at 7680,
+// 39.8 against 43.1 at 10240, 260 against 365 at 194000; 33.7 against 31.2 at
+// 5120), 4 up to 2560 (25.0 against 25.3 at 768, the same at 2048 and 2560; 36.2
+// against 31.2 at 5120), else 8.  With a launch per axis: 32 where that gives
+// four blocks per CU, else 8 or 4 by the same count.
+static int tables_rows_default(int n, int batch, int mode) {
+  const long long rows = (long long)n * batch;
+  if (tables_at_once(n, mode)) return rows >= 6144 ? 32 : rows > 2560 ? 8 : 4;
+  return rows / 32 >= 1024 ? 32 : (rows / 8 >= 1024 ? 8 : 4);
+}
+
 template <int MODE, int TC, int RG>
 static void tables_launch(int n, int P, double* fxy, double* sparam,
                           const double* chparam, const int* chan, void* opa, void* opb, double* hg, float2* esc,
                           int nc_max, const int* nsteps, int step, int batch, hipStream_t s) {
   const int Kp = kpad(P);
-  // the polynomial block's partial sums, then the column-smooth points' P_km
-  // (nc_max per element), go to the B operand buffer, which
-  // k_screen_tables<.., 1, ..> overwrites after k_screen_lowrank_sum and
-  // k_screen_tables<.., 0, ..> have read them
+  // the column-smooth points' P_km (at most nc_max) and the polynomial block's
+  // partial sums go to the start of each element's own B operand, which the B
+  // tables overwrite: the partial sums have been read by then
   const int chunks = lowrank_chunks(P);
-  double* part = reinterpret_cast<double*>(opb);
-  double* pcoef = part + (size_t)batch * chunks * kLRSums;
+  const size_t pstride = (size_t)n * Kp * 4 / sizeof(double);
+  double* pcoef = reinterpret_cast<double*>(opb);
+  double* part = pcoef + (size_t)nc_max * kLR;
   double2* f2 = reinterpret_cast<double2*>(fxy);
 #define CL_(CH)                                                                                                       \
   hipLaunchKernelGGL(k_screen_classify<CH>, dim3(batch), dim3(kClassThreads), 0, s, n, P, f2, chparam, chan, sparam, \
@@ -1398,28 +1452,32 @@ static void tables_launch(int n, int P, double* fxy, double* sparam,
   else CL_(4);
 #undef CL_
   hipLaunchKernelGGL(k_screen_lowrank_part, dim3(batch, chunks), dim3(kLRThreads), 0, s, n, P, f2, chparam, chan,
-                     sparam, part, pcoef, nc_max, nsteps, step);
-  hipLaunchKernelGGL(k_screen_lowrank_sum, dim3(batch), dim3(1024), 0, s, P, f2, sparam, part, pcoef, nc_max,
-                     chunks, MODE, nsteps, step);
-  dim3 g(n / (TC * RG), batch);
-  hipLaunchKernelGGL((k_screen_tables<MODE, 0, TC, RG>), g, dim3(256), 0, s, n, P, Kp, f2, sparam, chparam, chan,
-                     opa, hg, esc, pcoef, nc_max, nsteps, step);
-  hipLaunchKernelGGL((k_screen_tables<MODE, 1, TC, RG>), g, dim3(256), 0, s, n, P, Kp, f2, sparam, chparam, chan,
-                     opb, hg, esc, pcoef, nc_max, nsteps, step);
-}
-
-// rows per table block: 32 when that still gives >= 4 blocks per CU, else 8
-// or 4 (measured at 2048^2: 32 rows 0.14 ms per 32 screens, 8 rows 0.16)
-static int tables_rows_default(int n, int batch) {
-  const long long blocks32 = (long long)(n / 32) * batch, blocks8 = (long long)(n / 8) * batch;
-  return blocks32 >= 1024 ? 32 : (blocks8 >= 1024 ? 8 : 4);
+                     sparam, part, pcoef, pstride, nsteps, step);
+  hipLaunchKernelGGL(k_screen_lowrank_sum, dim3(batch), dim3(1024), 0, s, P, f2, sparam, part, pcoef, pstride,
+                     MODE, nsteps, step);
+#define TK_(AXIS, Z)                                                                                                 \
+  hipLaunchKernelGGL((k_screen_tables<MODE, AXIS, TC, RG>), dim3(n / (TC * RG), batch, Z), dim3(256), 0, s, n, P, Kp, \
+                     f2, sparam, chparam, chan, opa, opb, hg, esc, pcoef, pstride, nsteps, step)
+  // Both axes in one launch where the P_km, read by axis 0, lie where axis 1 does
+  // not write: in the split operands' first kbeg columns, 2 n kbeg contiguous
+  // bytes with kbeg = 2 d0 - 32, d0 >= 32 and d0 >= the points that have P_km
+  // (256 bytes each), which is room for them from n = 128 up.
+  if constexpr (MODE != PA_GEMM_F32) {
+    if (tables_at_once(n, MODE)) {
+      TK_(2, 2);
+      return;
+    }
+  }
+  TK_(0, 1);
+  TK_(1, 1);
+#undef TK_
 }
 
 template <int MODE>
 static int tables_mode(int n, int P, double* fxy, double* sparam,
                        const double* chparam, const int* chan, void* opa, void* opb, double* hg,
                        float2* esc, int rows, int nc_max, const int* nsteps, int step, int batch, hipStream_t s) {
-  if (rows == 0) rows = tables_rows_default(n, batch);
+  if (rows == 0) rows = tables_rows_default(n, batch, MODE);
 #define TL_(TC, RG) tables_launch<MODE, TC, RG>(n, P, fxy, sparam, chparam, chan, opa, opb, hg, esc, nc_max, \
                                                 nsteps, step, batch, s)
   switch (rows) {

@@ -763,3 +763,61 @@ def test_gemm_tiles_cover_every_element(dev, n, batch):
             engine.plane_wave_tables(one, tables, 0, 1, None, None, rows=8)
             engine.screen_gemm(one, 0, 1, None, None, ang=one.ang, tile=tile)
             assert torch.equal(one.ang[0], ws.ang[b])
+
+
+@pytest.mark.parametrize("mode", ["f16x3", "bf16x3", "f32"])
+@pytest.mark.parametrize("n", [64, 128, 512])
+@pytest.mark.parametrize("both,cols,direct", [(0, 32, 0), (0, 40, 3), (0, 64, 32), (16, 64, 8), (64, 0, 1), (0, 0, 40)])
+def test_tables_of_both_axes_at_once(dev, n, mode, both, cols, direct):
+    """Both axes in one launch (n >= 128 with split operands) or one each: the 1-D
+    parts against their expansion in float64 and the composed screen against the
+    plane-wave sum, from points smooth along both axes, along the columns only, and
+    along neither, two screens with different counts.  Bounds: a split operand is within 2^-22 (2^-16) of its
+    value and the lo lo product is left out; a point's or the block's terms sum to
+    at most 28 |a|; the composed float32 rounds at 2^-24."""
+    from scipy.special import jv
+    rng = np.random.default_rng(n + both + 10 * cols + 100 * direct)
+    P, B, delta = both + cols + direct, 2, 0.002
+    X = n / 2 * delta
+    low, high = 13.0 / (2 * np.pi * X), 0.2 / delta
+    fx = np.concatenate([rng.uniform(-low, low, both + cols), rng.uniform(0.1, 1, direct) * high])
+    fy = np.concatenate([rng.uniform(-low, low, both), rng.uniform(0.6, 1, cols + direct) * high])
+    if n == 64:
+        fy[both:] = 0.4 / delta
+        fx[both + cols:] = 0.45 / delta
+    a = rng.normal(size=(B, P)) + 1j * rng.normal(size=(B, P))
+    a *= 4 / np.abs(a).sum(axis=1, keepdims=True)
+    rho = np.repeat(np.hypot(fx, fy)[None], B, axis=0).astype(np.float32)
+    theta = np.repeat(np.arctan2(fy, fx)[None], B, axis=0).astype(np.float32)
+    if cols > 32:      # one point of the second screen is smooth along neither axis
+        theta[1, both] = np.float32(np.pi / 4)
+        rho[1, both] = np.float32(0.45 / delta)
+    spec = channel_spec(n, delta, 808e-9, 0.05, 5e3, 3, P, 1e-15)
+    tables = engine.DeviceTables([spec], dev)
+    ws = engine.Workspace(n, P, B, mode, dev)
+    engine.upload_spectra(ws, rho, theta, a.astype(np.complex64), batch=B)
+    ws.chan[:B].zero_()
+    ws.table_rows = {32: 4, 40: 8, 64: 16, 0: 32}[cols]
+    phi = torch.empty(B, n, n, dtype=torch.float32, device=dev)
+    engine.synth_screen(ws, tables, 0, B, None, None, phi=phi)
+    eps = 2.0 ** -16 if mode == "bf16x3" else 2.0 ** -22
+    x = (np.arange(n) - n // 2) * delta
+    for b in range(B):
+        f, d0 = ws.fxy[b].cpu().numpy().reshape(P, 4), int(ws.sparam[b, 5])
+        room = (4 * n * (-(-2 * P // 32) * 32) - 8 * (32 * 32 + 64) * -(-P // 64)) // 512   # of the B operand
+        low_x, low_y = np.abs(2 * np.pi * f[:, :2]).T * X <= 14
+        low_points = (low_x & low_y).sum() + min((low_x & ~low_y).sum(), room, 64)
+        assert d0 == (low_points // 16 * 16 if low_points >= 32 else 0)
+        amp = f[:, 2] + 1j * f[:, 3]
+        p, q = np.exp(2j * np.pi * np.outer(f[:, 0], x)), np.exp(2j * np.pi * np.outer(f[:, 1], x))
+        hg = ws.hg[b].cpu().numpy()
+        n2 = int(ws.sparam[b, 7])
+        for axis, w, waves, block in ((0, f[:, 1], q, n2), (1, f[:, 0], p, d0)):
+            one = waves - 1      # of the block's points, their 32 Chebyshev terms
+            cheb = np.cos(np.outer(np.arange(32), np.arccos(x / X)))
+            c = 2 * 1j ** np.arange(32) * jv(np.arange(32), (2 * np.pi * w[:block] * X)[:, None])
+            c[:, 0] = c[:, 0] / 2 - 1
+            one[:block] = c @ cheb
+            assert np.abs(hg[axis] - (amp @ one).real).max() < 1e-11
+        ref = ((amp[:, None] * q).T @ p).real
+        assert np.abs(phi[b].cpu().numpy() - ref).max() < 3 * 28 * 4 * eps + 8 * 2.0 ** -24
