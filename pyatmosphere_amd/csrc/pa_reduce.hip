@@ -204,9 +204,11 @@ __global__ void k_apply_pupil(int n, float2* __restrict__ u, double delta, doubl
 // out = u inside the pupil, 0 outside, as a new field: a row's columns inside are
 // one interval (circle_cols, the exact predicate), found by one thread per row
 // of the block, so the field is read inside the pupil only and nothing is
-// tested in float64 per element.  The 8 bytes written per element bound it
-// (9 us for a 1024^2 field, where a copy and a pass over it took 16).
-constexpr int kPupilRows = 8;
+// tested in float64 per element.  The 8 bytes written per element bound a large
+// batch; one field is bound by a block's chain (interval, read, write), so a
+// block takes two rows (5.3 us for a 1024^2 field, 10.2 with eight; a copy
+// and a pass over it took 16).
+constexpr int kPupilRows = 2;
 __global__ void __launch_bounds__(256)
 k_pupil_output(int n, const float2* __restrict__ u, float2* __restrict__ out, double delta, double rad2, double sx,
                double sy) {
@@ -219,7 +221,7 @@ k_pupil_output(int n, const float2* __restrict__ u, float2* __restrict__ out, do
   }
   __syncthreads();
   for (int i = threadIdx.x; i < kPupilRows * n / 2; i += 256) {
-    const int r = 2 * i / n, c = 2 * i % n;
+    const int r = 2 * i >= n, c = 2 * i - r * n;
     const int2 q = s_pc[r];
     pa_f4c v = {0.f, 0.f, 0.f, 0.f};
     if (q.x <= c + 1 && q.y >= c) {

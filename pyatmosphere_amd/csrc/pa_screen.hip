@@ -140,15 +140,23 @@ __device__ __forceinline__ double prep_point(double rr, double th, float2 a, dou
 }
 
 // Block reduction of the 256 per-thread (sum, max) pairs in s_sum / s_max
-// (tree, fixed order) and the element's sparam entries.
+// (tree, fixed order; its last six levels within the first wave) and the
+// element's sparam entries.
 __device__ __forceinline__ void prep_finish(double* __restrict__ s_sum, double* __restrict__ s_max, double* sp,
                                             int mode) {
-  for (int o = 128; o > 0; o >>= 1) {
+  for (int o = 128; o >= 64; o >>= 1) {
     if (threadIdx.x < o) {
       s_sum[threadIdx.x] += s_sum[threadIdx.x + o];
       s_max[threadIdx.x] = fmax(s_max[threadIdx.x], s_max[threadIdx.x + o]);
     }
     __syncthreads();
+  }
+  if (threadIdx.x >= 64) return;
+  double sum = s_sum[threadIdx.x], amax = s_max[threadIdx.x];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sum += __shfl_down(sum, o, 64);
+    amax = fmax(amax, __shfl_down(amax, o, 64));
   }
   if (threadIdx.x == 0) {
     double sa = 1.0, sb = 1.0;
@@ -156,11 +164,11 @@ __device__ __forceinline__ void prep_finish(double* __restrict__ s_sum, double* 
       // A entries: |a q| <= 2 max|a| scaled to <= 2^14 (lowered by
       // k_screen_lowrank_sum if the polynomial block needs it); B entries:
       // |p| <= 2 and |T_m| <= 1, scaled to <= 2^14
-      const double m = 2.0 * s_max[0];
+      const double m = 2.0 * amax;
       sa = m > 0 ? ldexp(1.0, 14 - (int)ceil(log2(m))) : 1.0;
       sb = ldexp(1.0, 13);
     }
-    sp[0] = s_sum[0];
+    sp[0] = sum;
     sp[1] = sa;
     sp[2] = sb;
     sp[3] = 1.0 / (sa * sb);
@@ -170,64 +178,26 @@ __device__ __forceinline__ void prep_finish(double* __restrict__ s_sum, double* 
   }
 }
 
-__global__ void __launch_bounds__(256)
-k_screen_prep(int P, const float* __restrict__ rho, const float* __restrict__ theta,
-              const float2* __restrict__ value, double2* __restrict__ fxy,
-              double* __restrict__ sparam, int mode, const double* __restrict__ chparam,
-              const int* __restrict__ chan, const int* __restrict__ nsteps, int step) {
-  const int b = blockIdx.x;
-  if (nsteps && step >= nsteps[b]) return;
-  const int ch = chan ? chan[b] : 0;
-  const double x0 = chparam[ch * kChParams + 1], y0 = chparam[ch * kChParams + 2];
-  __shared__ double s_sum[256], s_max[256];
+// One element's prep by a block of 1024 threads: point(k, r, t, v) gives the
+// spectrum's point k.  Thread t < 256 adds the points t, t + 256, t + 512, ... in
+// turn, so the sums do not depend on how many points are formed at once.  A
+// point's chain of float64 functions bounds a block (with the draw 8 to 20 us
+// whatever the batch), so every thread forms one; with 256 threads and four
+// points each, k_screen_prep took 6.7 us for a screen of 1024 points
+// instead of 4.9.
+constexpr int kPrepThreads = 1024;
+template <class Point>
+__device__ __forceinline__ void prep_block(int P, size_t o, double2* __restrict__ fxy, double* __restrict__ sparam,
+                                           int mode, double x0, double y0, Point point) {
+  __shared__ double s_re[kPrepThreads], s_am[kPrepThreads];
   double sum = 0, amax = 0;
-  for (int k = threadIdx.x; k < P; k += 256) {
-    double2 f, a;
-    const double am = prep_point(rho[(size_t)b * P + k], theta[(size_t)b * P + k], value[(size_t)b * P + k], x0,
-                                 y0, f, a);
-    fxy[((size_t)b * P + k) * 2] = f;
-    fxy[((size_t)b * P + k) * 2 + 1] = a;
-    sum += a.x;
-    amax = fmax(amax, am);
-  }
-  s_sum[threadIdx.x] = sum;
-  s_max[threadIdx.x] = amax;
-  __syncthreads();
-  prep_finish(s_sum, s_max, sparam + (size_t)b * PA_SCREEN_PARAMS, mode);
-}
-
-// The spectral draw and the prep in one launch (one block of 1024 threads per
-// element b and screen `screen` + y, whose results go to element y batch + b of
-// fxy and sparam): the same per-point arithmetic and the same summation order as
-// k_spectral_draw followed by k_screen_prep (thread t < 256 adds points t,
-// t + 256, t + 512, ... in turn), so fxy and sparam are identical; the
-// draw's rho, theta, value are not stored.  A block's chain of float64 log, sine
-// and cosine bounds it (8 to 20 us whatever the batch), so all screens of a
-// batch go in one launch: 20 us instead of 196 for ten screens of 4096 points,
-// 13 instead of 130 for a mixed batch's ten.
-constexpr int kDrawPrepThreads = 1024;
-__global__ void __launch_bounds__(kDrawPrepThreads)
-k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restrict__ sqrt_psd,
-                   const uint64_t* __restrict__ rid, uint64_t seed, int screen, double2* __restrict__ fxy,
-                   double* __restrict__ sparam, int mode, const double* __restrict__ chparam,
-                   const int* __restrict__ chan, const int* __restrict__ nsteps, int step) {
-  const int b = blockIdx.x;
-  const size_t o = (size_t)blockIdx.y * gridDim.x + b;
-  screen += blockIdx.y;
-  if (nsteps && step + (int)blockIdx.y >= nsteps[b]) return;
-  const int ch = chan ? chan[b] : 0;
-  const uint64_t id = rid[b];
-  const double x0 = chparam[ch * kChParams + 1], y0 = chparam[ch * kChParams + 2];
-  const float U = (float)u01(stream_word(id, screen, 0, seed));
-  __shared__ double s_re[kDrawPrepThreads], s_am[kDrawPrepThreads];
-  double sum = 0, amax = 0;
-  for (int k0 = 0; k0 < P; k0 += kDrawPrepThreads) {
+  for (int k0 = 0; k0 < P; k0 += kPrepThreads) {
     const int k = k0 + threadIdx.x;
     double re = 0.0, am = 0.0;
     if (k < P) {
       float r, t;
       float2 v;
-      draw_point(P, base, sqrt_psd, ch, id, seed, screen, k, U, r, t, v);
+      point(k, r, t, v);
       double2 f, a;
       am = prep_point(r, t, v, x0, y0, f, a);
       fxy[(o * P + k) * 2] = f;
@@ -239,7 +209,7 @@ k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restric
     __syncthreads();
     if (threadIdx.x < 256) {
 #pragma unroll
-      for (int i = 0; i < kDrawPrepThreads / 256; ++i) {
+      for (int i = 0; i < kPrepThreads / 256; ++i) {
         if (k0 + threadIdx.x + 256 * i < P) {
           sum += s_re[threadIdx.x + 256 * i];
           amax = fmax(amax, s_am[threadIdx.x + 256 * i]);
@@ -254,6 +224,46 @@ k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restric
   }
   __syncthreads();
   prep_finish(s_re, s_am, sparam + o * PA_SCREEN_PARAMS, mode);
+}
+
+__global__ void __launch_bounds__(kPrepThreads)
+k_screen_prep(int P, const float* __restrict__ rho, const float* __restrict__ theta,
+              const float2* __restrict__ value, double2* __restrict__ fxy,
+              double* __restrict__ sparam, int mode, const double* __restrict__ chparam,
+              const int* __restrict__ chan, const int* __restrict__ nsteps, int step) {
+  const int b = blockIdx.x;
+  if (nsteps && step >= nsteps[b]) return;
+  const int ch = chan ? chan[b] : 0;
+  prep_block(P, b, fxy, sparam, mode, chparam[ch * kChParams + 1], chparam[ch * kChParams + 2],
+             [&](int k, float& r, float& t, float2& v) {
+               r = rho[(size_t)b * P + k];
+               t = theta[(size_t)b * P + k];
+               v = value[(size_t)b * P + k];
+             });
+}
+
+// The spectral draw and the prep in one launch (one block per element b and
+// screen `screen` + y, whose results go to element y batch + b of fxy and
+// sparam): the same per-point arithmetic and the same summation order as
+// k_spectral_draw followed by k_screen_prep, so fxy and sparam are identical; the
+// draw's rho, theta, value are not stored.  All screens of a batch go in one
+// launch: 20 us instead of 196 for ten screens of 4096 points, 13 instead of 130
+// for a mixed batch's ten.
+__global__ void __launch_bounds__(kPrepThreads)
+k_screen_draw_prep(int P, const float* __restrict__ base, const float* __restrict__ sqrt_psd,
+                   const uint64_t* __restrict__ rid, uint64_t seed, int screen, double2* __restrict__ fxy,
+                   double* __restrict__ sparam, int mode, const double* __restrict__ chparam,
+                   const int* __restrict__ chan, const int* __restrict__ nsteps, int step) {
+  const int b = blockIdx.x;
+  screen += blockIdx.y;
+  if (nsteps && step + (int)blockIdx.y >= nsteps[b]) return;
+  const int ch = chan ? chan[b] : 0;
+  const uint64_t id = rid[b];
+  const float U = (float)u01(stream_word(id, screen, 0, seed));
+  prep_block(P, (size_t)blockIdx.y * gridDim.x + b, fxy, sparam, mode, chparam[ch * kChParams + 1],
+             chparam[ch * kChParams + 2], [&](int k, float& r, float& t, float2& v) {
+               draw_point(P, base, sqrt_psd, ch, id, seed, screen, k, U, r, t, v);
+             });
 }
 
 // ------------------------------------------------------------------ polynomial block
@@ -1404,7 +1414,7 @@ int spectral_draw(int P, const float* base, const float* sqrt_psd, const int* ch
 int screen_draw_prep(int P, const float* base, const float* sqrt_psd, const int* chan, const uint64_t* rid,
                      uint64_t seed, int screen, double* fxy, double* sparam, int mode, const double* chparam,
                      const int* nsteps, int step, int screens, int batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_screen_draw_prep, dim3(batch, screens), dim3(kDrawPrepThreads), 0, s, P, base, sqrt_psd, rid, seed,
+  hipLaunchKernelGGL(k_screen_draw_prep, dim3(batch, screens), dim3(kPrepThreads), 0, s, P, base, sqrt_psd, rid, seed,
                      screen, reinterpret_cast<double2*>(fxy), sparam, mode, chparam, chan, nsteps, step);
   return check_launch("screen_draw_prep");
 }
@@ -1412,7 +1422,7 @@ int screen_draw_prep(int P, const float* base, const float* sqrt_psd, const int*
 int screen_prep(int P, const float* rho, const float* theta, const float2* value, double* fxy,
                 double* sparam, int mode, const double* chparam, const int* chan, const int* nsteps, int step,
                 int batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_screen_prep, dim3(batch), dim3(256), 0, s, P, rho, theta, value,
+  hipLaunchKernelGGL(k_screen_prep, dim3(batch), dim3(kPrepThreads), 0, s, P, rho, theta, value,
                      reinterpret_cast<double2*>(fxy), sparam, mode, chparam, chan, nsteps, step);
   return check_launch("screen_prep");
 }
