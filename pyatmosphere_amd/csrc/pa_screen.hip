@@ -1269,19 +1269,24 @@ k_screen_gemm_split(const void* __restrict__ opa, const void* __restrict__ opb,
 }
 
 // ---- float32 GEMM (v_mfma_f32_32x32x2f32): the full-precision reference mode
-template <int N>
+// BT x BT tiles of four waves, a wave's K chain being what bounds a small launch:
+// with 128 a wave runs 2 K MFMAs one after the other, with 64 K / 2.  64 where the
+// 128 x 128 tiles would leave CUs idle (one screen, 64 against 128: 16 against 38
+// us at 256^2, 20 against 45 at 1024^2; 192 tiles 41 against 48 us; the same at 256
+// tiles, 10% slower at 4096, where 128 reach 112 TFLOP/s).  Reading the K of four
+// MFMAs by one 16-byte LDS load (a chunk's K stored in that order) is no faster.
+template <int N, int BT>
 struct F32Geo {
-  static constexpr int BM = N < 128 ? N : 128, BN = BM;
-  static constexpr int NTM = N / BM, NTN = N / BN;
+  static constexpr int NTM = N / BT, NTN = NTM;
 };
 
-template <int N, bool COMPOSE>
+template <int N, int BT, bool COMPOSE>
 __global__ void __launch_bounds__(256)
 k_screen_gemm_f32(const void* __restrict__ opa, const void* __restrict__ opb,
                   const double* __restrict__ sparam, const float2* __restrict__ esc, float* __restrict__ phi2,
                   float* __restrict__ ang, float2* __restrict__ fac, int Kp, const int* __restrict__ nsteps,
                   int step, int batch, const double* __restrict__ hg, float* __restrict__ phi) {
-  constexpr int BM = F32Geo<N>::BM, BN = F32Geo<N>::BN;
+  constexpr int BM = BT, BN = BT;
   constexpr int WM = BM / 2, WN = BN / 2, MI = WM / 32, NI = WN / 32;
   constexpr int BK = 32;
   constexpr int LDSROW = BK * 4 + 16;          // padded LDS row (bytes)
@@ -1291,7 +1296,7 @@ k_screen_gemm_f32(const void* __restrict__ opa, const void* __restrict__ opb,
   constexpr int STA = BM * LDSROW, STB = BN * LDSROW;
 
   int b, ty, tx;
-  gemm_tile<F32Geo<N>::NTM, F32Geo<N>::NTN>(blockIdx.x, batch, b, ty, tx);
+  gemm_tile<F32Geo<N, BT>::NTM, F32Geo<N, BT>::NTN>(blockIdx.x, batch, b, ty, tx);
   if (nsteps && step >= nsteps[b]) return;
   __shared__ __attribute__((aligned(16))) char sA[2 * STA];
   __shared__ __attribute__((aligned(16))) char sB[2 * STB];
@@ -1567,14 +1572,25 @@ static int gemm_n(int P, const void* opa, const void* opb, const double* sparam,
       else G_(PA_GEMM_BF16X3, 2);
       break;
     case PA_GEMM_F32: {
-      const dim3 gf(F32Geo<N>::NTM * F32Geo<N>::NTN * batch);
-      if (phi)
-        hipLaunchKernelGGL((k_screen_gemm_f32<N, true>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang, fac, Kp,
-                           nsteps, step, batch, hg, phi);
-      else
-        hipLaunchKernelGGL((k_screen_gemm_f32<N, false>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang, fac,
-                           Kp, nsteps, step, batch, hg, phi);
+#define F_(BT)                                                                                                        \
+  do {                                                                                                                \
+    const dim3 gf(F32Geo<N, BT>::NTM * F32Geo<N, BT>::NTN * batch);                                                   \
+    if (phi)                                                                                                          \
+      hipLaunchKernelGGL((k_screen_gemm_f32<N, BT, true>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang,     \
+                         fac, Kp, nsteps, step, batch, hg, phi);                                                      \
+    else                                                                                                              \
+      hipLaunchKernelGGL((k_screen_gemm_f32<N, BT, false>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang,    \
+                         fac, Kp, nsteps, step, batch, hg, phi);                                                      \
+  } while (0)
+      if constexpr (N >= 128) {
+        if ((long long)(N / 128) * (N / 128) * batch >= 256) {
+          F_(128);
+          break;
+        }
+      }
+      F_(64);
       break;
+#undef F_
     }
     default:
       return set_error(PA_ERR_ARG, "unknown GEMM mode");

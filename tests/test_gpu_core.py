@@ -821,3 +821,27 @@ def test_tables_of_both_axes_at_once(dev, n, mode, both, cols, direct):
             assert np.abs(hg[axis] - (amp @ one).real).max() < 1e-11
         ref = ((amp[:, None] * q).T @ p).real
         assert np.abs(phi[b].cpu().numpy() - ref).max() < 3 * 28 * 4 * eps + 8 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n,batch", [(64, 3), (128, 1), (256, 1), (1024, 3), (1024, 4), (2048, 1)])
+def test_float32_gemm_tiles(dev, n, batch):
+    """The float32 GEMM on both sides of its tile rule (64 x 64 below 256 tiles of
+    128 x 128): phi2 against the float64 product of the operands.  A term has one
+    rounding and each of K additions one of a partial sum that a row's and a
+    column's |a| |b| bound."""
+    P = 96
+    spec = channel_spec(n, 0.002, 808e-9, 0.05, 5e3, 3, P, 1e-15)
+    spectra, _ = host_spectra(spec, batch, seed=n)
+    tables = engine.DeviceTables([spec], dev)
+    ws = engine.Workspace(n, P, batch, "f32", dev)
+    engine.upload_spectra(ws, *spectra[0], batch=batch)
+    ws.chan[:batch].zero_()
+    phi2 = ws.phi2_buffer()
+    engine.synth_screen(ws, tables, 0, batch, None, None, phi2=phi2)
+    T = n // ws.tiles
+    for b in range(batch):
+        kbeg = int(ws.sparam[b, 4])
+        A, B = (op[b].view(torch.float32).reshape(n, -1)[:, kbeg:].double() for op in (ws.opa, ws.opb))
+        got = phi2[b].reshape(ws.tiles, n, T).transpose(1, 2).reshape(n, n).double()
+        bound = (A.shape[1] + 1) * 2.0 ** -24 * (A.abs() @ B.abs().T) + 1e-30
+        assert bool(((got - A @ B.T).abs() <= bound).all())
