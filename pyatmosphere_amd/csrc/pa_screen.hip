@@ -1043,11 +1043,14 @@ __device__ __forceinline__ void gemm_epilogue(const f16v (&acc)[MI][NI], int m0,
 // 256 x 256 block tiles (8 waves of 128 x 64); smaller grids 128 x 128 (or
 // N x N) with 4 waves.
 // CFG 1: 256 x 256 block tiles (8 waves of 128 x 64) for grids of 512 and up;
-// CFG 2: 128 x 128 (or N x N) tiles with 4 waves of 64 x 64, 4x the blocks.
+// CFG 2: 128 x 128 (or N x N) tiles with 4 waves of 64 x 64, 4x the blocks;
+// CFG 3: 64 x 64 tiles with 4 waves of 32 x 32 and six stages, for launches whose
+// 128 x 128 tiles would leave half the CUs idle: a block's time is then its chain of chunks,
+// a quarter of the MFMAs each, and more of them in flight.
 template <int N, int CFG>
 struct SplitGeo {
   static constexpr bool BIG = N >= 512 && CFG == 1;
-  static constexpr int BM = BIG ? 256 : (N < 128 ? N : 128);
+  static constexpr int BM = BIG ? 256 : (N < 128 || CFG == 3 ? 64 : 128);
   static constexpr int BN = BM;
   static constexpr int WGM = 2, WGN = BIG ? 4 : 2;
   static constexpr int NT = 64 * WGM * WGN;
@@ -1058,7 +1061,7 @@ struct SplitGeo {
   static constexpr int STAGE = 64 * (BM + BN);
   static constexpr int SEGS = 2 * (BM + BN) / 32;
   static constexpr int SEG_PER_WAVE = SEGS / (NT / 64);
-  static constexpr int DEPTH = 4;                 // LDS stages: 2 chunks in flight, 1 in registers
+  static constexpr int DEPTH = CFG == 3 ? 6 : 4;  // LDS stages: 2 (4) chunks in flight, 1 in registers
   static_assert(MI >= 1 && NI >= 1, "wave tile");
   static_assert(SEGS % (NT / 64) == 0, "segments per wave");
   static_assert(DEPTH * STAGE <= 160 * 1024 && DEPTH >= 3, "LDS stages");
@@ -1547,9 +1550,17 @@ static void gemm_split_launch(int Kp, const void* opa, const void* opb, const do
                        ang, fac, Kp, nsteps, step, batch, hg, phi);
 }
 
-// GEMM tile: the 256 x 256 tiles when they give at least two blocks per CU
+// GEMM tile: the 256 x 256 tiles when they give at least two blocks per CU; 64 x 64
+// where the 128 x 128 ones would be at most one for every other CU.  Measured, 64
+// against 128: one screen of 512^2 9.7 against 15.2 us, of 1024^2 10.8 against 17.2,
+// thirty of 256^2 (120 tiles) 12.7 against 17.5, a whole 512^2 realization as a
+// graph (80 tiles) 134 against 140; 192 tiles 18.0 against 19.2 but, beside the field
+// passes, three 512^2 realizations (240 tiles) 169 against 166; 256 tiles (one
+// 2048^2) 26.7 against 22.5.  (With five or eight stages 128 x 128 is no faster;
+// with four or eight 64 x 64 is up to 1.4 us slower.)
 static int gemm_tile_default(int n, int batch) {
-  return (n >= 512 && (long long)(n / 256) * (n / 256) * batch >= 512) ? 1 : 2;
+  if (n >= 512 && (long long)(n / 256) * (n / 256) * batch >= 512) return 1;
+  return (long long)(n / 128) * (n / 128) * batch <= 128 ? 3 : 2;
 }
 
 template <int N>
@@ -1557,19 +1568,21 @@ static int gemm_n(int P, const void* opa, const void* opb, const double* sparam,
                   float* ang, float2* fac, const double* hg, float* phi, int mode, int tile, const int* nsteps, int step,
                   int batch, hipStream_t s) {
   const int Kp = kpad(P);
+  if (tile != 0 && tile != 1 && tile != 2) return set_error(PA_ERR_ARG, "screen_gemm: tile must be 0, 1 or 2");
+  if (N < 512 && tile == 1) tile = 2;   // no 256 x 256 tiles below 512
   if (tile == 0) tile = gemm_tile_default(N, batch);
-  if (tile != 1 && tile != 2) return set_error(PA_ERR_ARG, "screen_gemm: tile must be 0, 1 or 2");
-  if (N < 512) tile = 2;   // one geometry below 512
 #define G_(MODE, CFG) \
   gemm_split_launch<N, MODE, CFG>(Kp, opa, opb, sparam, esc, phi2, ang, fac, hg, phi, nsteps, step, batch, s)
   switch (mode) {
     case PA_GEMM_F16X3:
       if (tile == 1) G_(PA_GEMM_F16X3, 1);
-      else G_(PA_GEMM_F16X3, 2);
+      else if (tile == 2) G_(PA_GEMM_F16X3, 2);
+      else G_(PA_GEMM_F16X3, 3);
       break;
     case PA_GEMM_BF16X3:
       if (tile == 1) G_(PA_GEMM_BF16X3, 1);
-      else G_(PA_GEMM_BF16X3, 2);
+      else if (tile == 2) G_(PA_GEMM_BF16X3, 2);
+      else G_(PA_GEMM_BF16X3, 3);
       break;
     case PA_GEMM_F32: {
 #define F_(BT)                                                                                                        \

@@ -845,3 +845,27 @@ def test_float32_gemm_tiles(dev, n, batch):
         got = phi2[b].reshape(ws.tiles, n, T).transpose(1, 2).reshape(n, n).double()
         bound = (A.shape[1] + 1) * 2.0 ** -24 * (A.abs() @ B.abs().T) + 1e-30
         assert bool(((got - A @ B.T).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("mode", ["f16x3", "bf16x3"])
+@pytest.mark.parametrize("n,batch,points", [(64, 3, 40), (128, 1, 8), (256, 30, 100), (512, 1, 1024), (512, 8, 50),
+                                            (512, 9, 50), (1024, 2, 33), (1024, 3, 33)])
+def test_small_launches_take_the_same_products(dev, n, batch, points, mode):
+    """The library's own tile choice (64 x 64 up to 128 tiles of 128 x 128, with
+    more K chunks in flight than some of these have) gives the bits of the 128 x
+    128 tiles, angle, phi2 and composed screen."""
+    spec = channel_spec(n, 0.002, 808e-9, 0.05, 5e3, 3, points, 1e-15)
+    spectra, _ = host_spectra(spec, batch, seed=n + points)
+    tables = engine.DeviceTables([spec], dev)
+    ws = engine.Workspace(n, points, batch, mode, dev)
+    engine.upload_spectra(ws, *spectra[0], batch=batch)
+    ws.chan[:batch].zero_()
+    engine.prep_screen(ws, tables, 0, batch, None, None)
+    engine.plane_wave_tables(ws, tables, 0, batch, None, None)
+    got = []
+    for tile in (0, 2):
+        ang, phi2, phi = (torch.full((batch, n, n), 7.0, dtype=torch.float32, device=dev) for _ in range(3))
+        engine.screen_gemm(ws, 0, batch, None, None, ang=ang, phi2=phi2, tile=tile)
+        engine.screen_gemm(ws, 0, batch, None, None, phi=phi, tile=tile)
+        got.append((ang, phi2, phi))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
