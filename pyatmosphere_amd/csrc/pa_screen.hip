@@ -314,6 +314,12 @@ constexpr int kSpKbeg = 4, kSpD0 = 5, kSpN2 = 7;
 
 typedef double d4v __attribute__((ext_vector_type(4)));
 
+// The rounded product: not fused into a following addition.
+__device__ __forceinline__ double mul_rn(double a, double b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
 // Exclusive count of the block's threads below this one with flag set, and
 // the total into `total`.
 __device__ __forceinline__ int block_rank(bool flag, int& total, int* s_w) {
@@ -396,10 +402,11 @@ k_screen_classify(int n, int P, double2* __restrict__ fxy, const double* __restr
 //   Re(a' Q_n P_m) = x v u, -y v u, -y v u, -x v u  for (n, m) both even, odd and
 // even, even and odd, both odd, and G falls into four 16 x 16 products over the
 // chunk's points, one per wave (v_mfma_f64_16x16x4f64, K = one value per point).
-// The Bessel recurrences (two waves) and the barrier bound a block, so what
-// counts is blocks in flight: 35 KB of LDS and 4 waves let a CU hold four,
-// where complex coefficients and 8 waves allowed two (168 us for 1280 screens
-// of 1024 points instead of 268).
+// A product's terms are added one after the other in point order, as in a complex
+// sum (whose other terms are zero), so G keeps its bits.  The Bessel recurrences
+// (two waves) and the barrier bound a block, so what counts is blocks in flight: 35
+// KB of LDS and 4 waves let a CU hold four, where complex coefficients and 8 waves
+// allowed two (168 us for 1280 screens of 1024 points instead of 268).
 __global__ void __launch_bounds__(kLRThreads, 4)
 k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const double* __restrict__ chparam,
                       const int* __restrict__ chan, const double* __restrict__ sparam, double* __restrict__ part,
@@ -467,7 +474,7 @@ k_screen_lowrank_part(int n, int P, const double2* __restrict__ fxy, const doubl
   double v = 0.0;
   for (int j = sub; j < cnt; j += 4) {
     const double2 a = s_a[j];
-    v += ((m & 1) ? -a.y : a.x) * (o < kLR ? s_v[j][m] : s_u[j][m]);   // Re a' Q_kn, Re a' P_km
+    v += mul_rn((m & 1) ? -a.y : a.x, o < kLR ? s_v[j][m] : s_u[j][m]);   // Re a' Q_kn, Re a' P_km
   }
   v += __shfl_xor(v, 1, 64);
   v += __shfl_xor(v, 2, 64);
@@ -586,37 +593,36 @@ __device__ __forceinline__ uint32_t split_pack(double v0, double v1, uint32_t& l
 // exactly at the end).  RT (4, 8, 16 or 32) trades sincos work and per-block
 // set-up against the number of blocks.
 //
-// The polynomial block's 32 columns come from the Chebyshev values T_q(u) of
-// the block's rows, formed once (one thread per row, the forward recurrence)
-// and kept in LDS: they are the B operand's columns, and the A operand's are
-// the products T G + Re V on v_mfma_f64_16x16x4f64: 16 rows by the 16 even and
-// the 16 odd columns (P_km is real or imaginary by the parity of m, so a
-// column-smooth slot is one K of either), K split over the waves that share a
-// row tile.  Measured, 1280 screens of 512^2 (320 of 2048^2): the two axes take
-// 452 + 281 us (559 + 372); with each entry's own Clenshaw recurrence and dot
-// product over the slots on LDS operands 538 + 365 (644 + 478).
+// The polynomial block's 32 columns: B's are the Chebyshev values T_q(u) of the
+// block's columns, formed once (one thread per column, the forward recurrence) and
+// kept in LDS; A's are sum_n T_n(s) Re G[n][m] by Clenshaw on G in LDS plus
+// Re V_m(r), added over the column-smooth slots in order (P_km is real or imaginary
+// by the parity of m, so a term is one product).  The order of these float64 sums
+// and of the 1-D ones below stays: as the products T G + Re V on float64 MFMA the
+// tables took 884 us instead of 990 for 1280 screens of 512^2 (945, 1053 for 320 of
+// 2048^2), but another last bit in the sums now and then turns an operand's or a
+// row factor's rounding, and with it a realization's moments by up to 2e-8.  (With
+// B's columns recomputed per entry, complex P_km and a launch per axis: 1208.)
 //
 // AXIS 0 and 1 fill one operand each; AXIS 2 fills both, axis blockIdx.z: the
-// polynomial part of A's blocks is a chain of latencies (sincos, barriers, MFMA)
-// and B's blocks are stores, so they overlap.  Measured, the whole of
-// pa_screen_tables with one launch against two: 16.3 against 22.4 us of kernels
-// for one 2048^2 screen, 50 against 62 us (ten of 2048^2), 57 against 67 (60 of
-// 512^2), 260 against 280 (189 of 1024^2), 944 against 975 (320 of 2048^2), 884
-// against 903 (1280 of 512^2).
+// polynomial part of A's blocks is a chain of latencies (sincos, barriers,
+// recurrences) and B's blocks are stores, so they overlap.  Measured with A's
+// columns on MFMA, all of pa_screen_tables with one launch against two: 16.3 against
+// 22.4 us of kernels for one 2048^2 screen, 50 against 62 us (ten of 2048^2), 57
+// against 67 (60 of 512^2), 260 against 280 (189 of 1024^2), 944 against 975 (320 of
+// 2048^2).
 template <int AXIS, int TC, int RG>
 struct TablesLds {
-  static constexpr int RT = TC * RG, MR = RT < 16 ? 16 : RT;
+  static constexpr int RT = TC * RG;
   // split modes stage TC rows x 256 points; before the direct points the same
-  // LDS holds the column-smooth slots' plane waves, CS slots at a time, and the
-  // partial tiles
-  static constexpr int SROW = 256 + 8, CS = 48, CROW = CS + 1, TROW = kLR + 1;
-  static constexpr int STAGE_BYTES = 2 * TC * SROW * 4, WAVE_BYTES = AXIS == 0 ? MR * CROW * 16 : 0;
-  static constexpr int TILE_BYTES = AXIS == 0 ? 4 * 64 * 8 * 8 : 0;
-  static constexpr int BUF1 = STAGE_BYTES > WAVE_BYTES ? STAGE_BYTES : WAVE_BYTES;
-  static constexpr int BUF = BUF1 > TILE_BYTES ? BUF1 : TILE_BYTES;
+  // LDS holds the column-smooth slots' plane waves, CS slots at a time
+  static constexpr int SROW = 256 + 8, CS = 32, CROW = CS + 1, TROW = kLR + 1;
+  static constexpr int STAGE_BYTES = 2 * TC * SROW * 4, WAVE_BYTES = AXIS == 0 ? RT * CROW * 16 : 0;
+  static constexpr int BUF = STAGE_BYTES > WAVE_BYTES ? STAGE_BYTES : WAVE_BYTES;
   __attribute__((aligned(16))) char buf[BUF];
-  double t[MR * TROW];              // T_q(u) of the block's rows
-  double h[AXIS == 0 ? 4 * 16 : 1];  // the column-smooth slots' share of h, per wave and tile row
+  double p[AXIS == 0 ? CS * kLR : 1];      // the slots' P_km
+  double g[AXIS == 0 ? kLR * kLR : 1];     // G
+  double t[AXIS == 1 ? RT * TROW : 1];     // T_q(u) of the block's columns
   double red[4][RT];
 };
 
@@ -650,10 +656,8 @@ tables_axis(TablesLds<AXIS, TC, RG>& lds, int n, int P, int Kp, const double2* _
   // 32 TC bytes.  Rows are padded so that 8 consecutive pieces read from 8
   // distinct 16-byte bank groups.
   using Lds = TablesLds<AXIS, TC, RG>;
-  constexpr int SROW = Lds::SROW, CS = Lds::CS, CROW = Lds::CROW, TROW = Lds::TROW, RPG = RT / 4, MR = Lds::MR;
+  constexpr int SROW = Lds::SROW, CS = Lds::CS, CROW = Lds::CROW, TROW = Lds::TROW;
   char* s_buf = lds.buf;
-  double* s_t = lds.t;
-  double* s_h = lds.h;
   uint32_t* s_hi = reinterpret_cast<uint32_t*>(s_buf);
   uint32_t* s_lo = s_hi + TC * SROW;
   // (v0, v1) into the polynomial block's columns kbeg + 2 pr, + 1 of row i0 + j
@@ -668,41 +672,29 @@ tables_axis(TablesLds<AXIS, TC, RG>& lds, int n, int P, int Kp, const double2* _
       put_pair_f32(opb, Kp, i0 + j, kbeg / 2 + pr, v0, v1);
     }
   };
+  double hsh = 0.0;   // thread j < RT: the column-smooth slots' share of h
   if (klow) {
-    if (threadIdx.x < RT) {
-      const double u = (double)(i0 + (int)threadIdx.x - n / 2) / (double)(n / 2);
-      double* t = s_t + threadIdx.x * TROW;
-      double t0 = 1.0, t1 = u;
-      t[0] = t0;
-      t[1] = t1;
-#pragma unroll
-      for (int q = 2; q < kLR; ++q) {
-        const double t2 = 2.0 * u * t1 - t0;
-        t0 = t1;
-        t1 = t2;
-        t[q] = t2;
-      }
-    }
     if constexpr (AXIS == 0) {
-      // wave w: row tile w % NT, every KS-th K step; lane l: A row l % 16, K l / 16
-      constexpr int NT = MR / 16, KS = 4 / NT;
-      const int tile = wave % NT, ks = wave / NT, r = lane & 15, kk = lane >> 4, tr = 16 * tile + r;
-      d4v ev = {0.0, 0.0, 0.0, 0.0}, od = ev;
-      double hs = 0.0;
+      constexpr int NV = (RT * kLR + 255) / 256;               // entries per thread: e = tid + 256 i, column tid % 32
+      constexpr int RGS = RT >= 16 ? 16 : RT, RPG = RT / RGS;  // row groups, rows per group
       double2* s_aq = reinterpret_cast<double2*>(s_buf);
       const double* pc = pcoef + (size_t)b * pstride;
-      const int ncs = klow - n2;
+      const int ncs = klow - n2, m = threadIdx.x % kLR;
+      double vacc[NV];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) vacc[i] = 0.0;
+      for (int e = threadIdx.x; e < kLR * kLR; e += 256) lds.g[e] = sp[8 + e];
       for (int t0 = 0; t0 < ncs; t0 += CS) {
         const int cnt = min(CS, ncs - t0);
         if (t0) __syncthreads();     // the previous slots' waves have been read
-        // slot t, rows g RPG ..: (a' q)(r) by the recurrence from the first row
-        const int t = threadIdx.x % CS, g = threadIdx.x / CS;
-        if (g < 4) {
-          double2 f = make_double2(0.0, 0.0), a = f;
-          if (t < cnt) {
-            f = fxy[((size_t)b * P + n2 + t0 + t) * 2];
-            a = fxy[((size_t)b * P + n2 + t0 + t) * 2 + 1];
-          }
+        for (int e = threadIdx.x; e < cnt * kLR; e += 256) {
+          const double v = pc[(size_t)t0 * kLR + e];
+          lds.p[e] = (e & 1) ? -v : v;   // Re q P = q.x v for even m, -q.y v for odd
+        }
+        // slot t, rows g RPG ..: (a' q)(r) by the recurrence from the group's first row
+        const int g = threadIdx.x % RGS;
+        for (int t = threadIdx.x / RGS; t < cnt; t += 256 / RGS) {
+          const double2 f = fxy[((size_t)b * P + n2 + t0 + t) * 2], a = fxy[((size_t)b * P + n2 + t0 + t) * 2 + 1];
           double s0, c0, sd, cd;
           sincos(kTwoPi * f.y * (coord0 + (double)(g * RPG) * delta), &s0, &c0);
           sincos(kTwoPi * f.y * delta, &sd, &cd);
@@ -716,53 +708,62 @@ tables_axis(TablesLds<AXIS, TC, RG>& lds, int n, int P, int Kp, const double2* _
           }
         }
         __syncthreads();
-        for (int k = 4 * ks; k < cnt; k += 4 * KS) {
-          const int slot = k + kk;     // slots past cnt have zero waves (cnt <= CS, a multiple of 4)
-          const double2 q = s_aq[tr * CROW + slot];
-          const double2 pm = slot < cnt ? *reinterpret_cast<const double2*>(pc + (size_t)(t0 + slot) * kLR + 2 * r)
-                                        : make_double2(0.0, 0.0);
-          ev = __builtin_amdgcn_mfma_f64_16x16x4f64(q.x, pm.x, ev, 0, 0, 0);
-          od = __builtin_amdgcn_mfma_f64_16x16x4f64(-q.y, pm.y, od, 0, 0, 0);
-          hs += q.x;
+        const double* q = reinterpret_cast<const double*>(s_aq) + (m & 1);
+#pragma unroll 4
+        for (int t = 0; t < cnt; ++t) {
+          const double pm = lds.p[t * kLR + m];
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            const int e = threadIdx.x + 256 * i;
+            if (e < RT * kLR) vacc[i] += mul_rn(q[2 * ((e / kLR) * CROW + t)], pm);
+          }
         }
+        if ((int)threadIdx.x < RT)
+#pragma unroll 4
+          for (int t = 0; t < cnt; ++t) hsh += s_aq[threadIdx.x * CROW + t].x;
       }
-      __syncthreads();                 // T; and the waves have been read
-      for (int k = 4 * ks; k < kLR; k += 4 * KS) {
-        const double t = s_t[tr * TROW + k + kk];
-        const double2 gm = *reinterpret_cast<const double2*>(sp + 8 + (k + kk) * kLR + 2 * r);
-        ev = __builtin_amdgcn_mfma_f64_16x16x4f64(t, gm.x, ev, 0, 0, 0);
-        od = __builtin_amdgcn_mfma_f64_16x16x4f64(t, gm.y, od, 0, 0, 0);
-      }
-      hs += __shfl_xor(hs, 16, 64);
-      hs += __shfl_xor(hs, 32, 64);
-      if (kk == 0) s_h[wave * 16 + r] = hs;
-      // the K parts of a tile meet in LDS; entry i of lane l: row 4 i + l / 16,
-      // columns 2 (l % 16) and + 1, finished by wave i % KS of the tile
-      double2* s_d = reinterpret_cast<double2*>(s_buf);
+      __syncthreads();   // G; and the waves have been read
+      // sum_n T_n(s) Re G[n][m] by Clenshaw + Re V_m(r); the even lane of each pair
+      // stores both values (RT * 32 is a multiple of 64: uniform over each wave)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s_d[(wave * 4 + i) * 64 + lane] = make_double2(ev[i], od[i]);
-      __syncthreads();
+      for (int i = 0; i < NV; ++i) {
+        const int e = threadIdx.x + 256 * i;
+        if (e >= RT * kLR) break;
+        const int j = e / kLR;
+        const double u = (double)(i0 + j - n / 2) / (double)(n / 2);
+        double b1 = 0.0, b2 = 0.0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = 16 * tile + 4 * i + kk;
-        if (i % KS != ks || j >= RT) continue;
-        double v0 = 0.0, v1 = 0.0;
-#pragma unroll
-        for (int w = 0; w < KS; ++w) {
-          const double2 d = s_d[((w * NT + tile) * 4 + i) * 64 + lane];
-          v0 += d.x;
-          v1 += d.y;
+        for (int q = kLR - 1; q >= 1; --q) {
+          const double b0 = lds.g[q * kLR + m] + 2.0 * u * b1 - b2;
+          b2 = b1;
+          b1 = b0;
         }
-        put_block(j, r, v0 * scale, v1 * scale);
+        const double val = lds.g[m] + u * b1 - b2 + vacc[i];
+        const double v0 = val * scale;
+        const double v1 = __shfl_down(v0, 1, 64);
+        if (!(m & 1)) put_block(j, m / 2, v0, v1);
       }
     } else {
+      if (threadIdx.x < RT) {
+        const double u = (double)(i0 + (int)threadIdx.x - n / 2) / (double)(n / 2);
+        double* t = lds.t + threadIdx.x * TROW;
+        double t0 = 1.0, t1 = u;
+        t[0] = t0;
+        t[1] = t1;
+#pragma unroll
+        for (int q = 2; q < kLR; ++q) {
+          const double t2 = 2.0 * u * t1 - t0;
+          t0 = t1;
+          t1 = t2;
+          t[q] = t2;
+        }
+      }
       __syncthreads();
       for (int e = threadIdx.x; e < RT * kLR / 2; e += 256) {
         const int j = e / (kLR / 2), pr = e % (kLR / 2);
-        put_block(j, pr, s_t[j * TROW + 2 * pr] * scale, s_t[j * TROW + 2 * pr + 1] * scale);
+        put_block(j, pr, lds.t[j * TROW + 2 * pr] * scale, lds.t[j * TROW + 2 * pr + 1] * scale);
       }
     }
-    __syncthreads();   // before the direct points use the staging LDS
   }
   double acc[RT];   // this thread's share of the 1-D sums, times scale
 #pragma unroll
@@ -861,32 +862,29 @@ tables_axis(TablesLds<AXIS, TC, RG>& lds, int n, int P, int Kp, const double2* _
   auto& red = lds.red;
   if ((lane & ((32 >> (LG - 1)) - 1)) == 0) red[wave][jr] = tot;
   __syncthreads();
-  // 8 lanes per row: the polynomial points' share of h(r) (AXIS 0) or g(c),
-  // sum_q T_q(u) c[q], four terms each; the first lane finishes the row
-  if (threadIdx.x < 8 * RT) {
-    const int j = threadIdx.x / 8, sub = threadIdx.x % 8, i = i0 + j;
-    double v = 0.0;
+  if (threadIdx.x < RT) {
+    const int j = threadIdx.x, i = i0 + j;
+    double v = (red[0][j] + red[1][j] + red[2][j] + red[3][j]) * (1.0 / scale);
+    if constexpr (AXIS == 0) v += hsh;
+    // the polynomial points' share of h(r) (AXIS 0) or g(c): sum_n T_n(u) c[n]
+    // by Clenshaw
     if (klow) {
       const double* cc = sp + (AXIS == 0 ? kLRCoefH : kLRCoefG);
+      const double u = (double)(i - n / 2) / (double)(n / 2);
+      double b1 = 0.0, b2 = 0.0;
 #pragma unroll
-      for (int q = 0; q < kLR / 8; ++q) v += s_t[j * TROW + sub + 8 * q] * cc[sub + 8 * q];
-      v += __shfl_xor(v, 1, 64);
-      v += __shfl_xor(v, 2, 64);
-      v += __shfl_xor(v, 4, 64);
-      if constexpr (AXIS == 0) {
-        constexpr int NT = MR / 16, KS = 4 / NT;
-#pragma unroll
-        for (int w = 0; w < KS; ++w) v += s_h[(w * NT + j / 16) * 16 + j % 16];   // the column-smooth slots' share
+      for (int q = kLR - 1; q >= 1; --q) {
+        const double b0 = cc[q] + 2.0 * u * b1 - b2;
+        b2 = b1;
+        b1 = b0;
       }
+      v += cc[0] + u * b1 - b2;
     }
-    if (sub == 0) {
-      v += (red[0][j] + red[1][j] + red[2][j] + red[3][j]) * (1.0 / scale);
-      hg[((size_t)b * 2 + AXIS) * n + i] = v;
-      const double ph = AXIS == 0 ? v + sp[0] : v;  // fold the piston into the row factor
-      double sn, cs;
-      sincos(ph, &sn, &cs);
-      esc[((size_t)b * 2 + AXIS) * n + i] = make_float2((float)cs, (float)-sn);
-    }
+    hg[((size_t)b * 2 + AXIS) * n + i] = v;
+    const double ph = AXIS == 0 ? v + sp[0] : v;  // fold the piston into the row factor
+    double sn, cs;
+    sincos(ph, &sn, &cs);
+    esc[((size_t)b * 2 + AXIS) * n + i] = make_float2((float)cs, (float)-sn);
   }
 }
 
@@ -1437,15 +1435,15 @@ int screen_prep(int P, const float* rho, const float* theta, const float2* value
 
 static bool tables_at_once(int n, int mode) { return mode != PA_GEMM_F32 && n >= 128; }
 
-// Rows per table block.  With both axes in one launch, 32 from 6144 rows up
-// (screens times n; measured, 32 against 8 rows: 36.9 against 38.5 us at 7680,
-// 39.8 against 43.1 at 10240, 260 against 365 at 194000; 33.7 against 31.2 at
-// 5120), 4 up to 2560 (25.0 against 25.3 at 768, the same at 2048 and 2560; 36.2
-// against 31.2 at 5120), else 8.  With a launch per axis: 32 where that gives
-// four blocks per CU, else 8 or 4 by the same count.
+// Rows per table block.  With both axes in one launch, 32 from 8192 rows up (screens
+// times n; measured, 32 against 8 rows: 44.5 against 47.2 us at 10240, 50 against 68
+// at 20480, 297 against 520 at 194000; 45.4 against 43.5 at 7680), 4 up to 2560
+// (26.2 against 27.1 at 768, 32.4 against 33.0 at 2048, the same at 2560; 38.4
+// against 34.9 at 5120), else 8.  With a launch per axis: 32 where that gives four
+// blocks per CU, else 8 or 4 by the same count.
 static int tables_rows_default(int n, int batch, int mode) {
   const long long rows = (long long)n * batch;
-  if (tables_at_once(n, mode)) return rows >= 6144 ? 32 : rows > 2560 ? 8 : 4;
+  if (tables_at_once(n, mode)) return rows >= 8192 ? 32 : rows > 2560 ? 8 : 4;
   return rows / 32 >= 1024 ? 32 : (rows / 8 >= 1024 ? 8 : 4);
 }
 
