@@ -523,7 +523,7 @@ class StepRunner:
         nv = None if self.ns is None else sb.active
         t = self.tables
         if host is not None:
-            rho, theta, value = sb.upload(host[:S], B)
+            rho, theta, value = sb.upload([host[i] for i in range(S)], B)
             call("pa_screen_prep", sb.points, rho, theta, value, ptr(sb.fxy), ptr(sb.sparam), sb.mode,
                  ptr(t.chparam), None if single else ptr(sb.chan), ptr(nv), 0, S * B, st)
         else:
@@ -644,6 +644,9 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
     its screens: host-drawn batches then upload no ids (ws.chan and ws.nsteps
     stay as they are).
     """
+    if host_spectra is not None:
+        # a screen without a draw is an IndexError here, before anything is launched
+        host_spectra = [host_spectra[i] for i in range(int(np.max(nscreens)) if len(nscreens) else 0)]
     single = single and host_spectra is not None and screens_out is None and SYNTH_WHOLE_BATCH and \
         tables.max_screens * len(chan) * synth_bytes_per_element(ws.n, ws.points, ws.mode) <= SYNTH_BATCH_MAX_BYTES
     run = StepRunner(ws, tables, chan, nscreens, rid, single=single)

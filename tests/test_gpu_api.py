@@ -233,3 +233,24 @@ def test_kept_tables_follow_the_channel(dev):
     assert "_kept_tables" not in copy.copy(ch.path).__dict__ and "_factors" not in copy.deepcopy(ch.source).__dict__
     again = pickle.loads(pickle.dumps(ch.source))
     assert again == ch.source and "_factors" not in again.__dict__
+
+
+def test_path_with_too_few_screens_raises(dev):
+    """Two screens at three positions: IndexError, through run_batch's whole-batch
+    synthesis and screen by screen; a third screen past two positions is drawn
+    and left out, as the loop over positions does."""
+    from pyatmosphere_amd import engine
+    ch = _quick()
+    ch.path.phase_screens = ch.path.phase_screens[:2]
+    for whole in (True, False):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setattr(engine, "SYNTH_WHOLE_BATCH", whole)
+            with pytest.raises(IndexError):
+                ch.run()
+    ch = _quick()
+    ch.path.positions = ch.path.positions[:2]
+    np.random.seed(7)
+    got = ch.run()
+    ch.path.phase_screens = ch.path.phase_screens[:2]
+    np.random.seed(7)
+    assert torch.equal(got, ch.run())

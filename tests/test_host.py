@@ -335,3 +335,12 @@ def test_padded_exchange_offsets(n):
         ns *= r
     loads = [[lpad(l) + lpad(L * e) for e in range(e_pt)] for l in range(L)]
     assert loads == [[lpad(l + L * e) for e in range(e_pt)] for l in range(L)]
+
+
+@pytest.mark.parametrize("given, screens", [(0, 1), (2, 3)])
+def test_missing_host_draw_is_refused_before_a_launch(given, screens):
+    """run_batch with fewer draws than screens raises IndexError before it
+    looks at the workspace or the tables."""
+    draw = (np.ones((1, 4), np.float32), np.zeros((1, 4), np.float32), np.ones((1, 4), np.complex64))
+    with pytest.raises(IndexError):
+        engine.run_batch(None, None, np.zeros(1), np.array([screens]), host_spectra=[draw] * given)
