@@ -19,7 +19,7 @@ class CirclePupil:
     def output(self, input, shift=(0, 0), **kwargs):
         """input * mask as a new device array."""
         grid = self.channel.grid
-        u = input.to(torch.complex64).contiguous()
+        u = input.to(torch.complex64).resolve_conj().resolve_neg().contiguous()
         out = torch.empty_like(u)
         n = u.shape[-1]
         batch = u.numel() // (n * n)

@@ -254,3 +254,22 @@ def test_path_with_too_few_screens_raises(dev):
     ch.path.phase_screens = ch.path.phase_screens[:2]
     np.random.seed(7)
     assert torch.equal(got, ch.run())
+
+
+@pytest.mark.parametrize("view", ["conj", "neg", "conj_transposed", "expanded", "strided"])
+def test_pupil_of_lazy_and_strided_views(dev, view):
+    """The pupil of a lazily conjugated or negated field, or of a strided view, is
+    the mask times its values, and the input stays as it was: exact."""
+    ch = _quick()
+    ch.pupil.channel = ch
+    g = torch.Generator(device=dev).manual_seed(3)
+    a = torch.randn(256, 512, dtype=torch.complex64, device=dev, generator=g)
+    u = {"conj": lambda: a[:, :256].contiguous().conj(), "neg": lambda: torch._neg_view(a[:, :256].contiguous()),
+         "conj_transposed": lambda: a[:, :256].mH, "expanded": lambda: a[:1, :256].expand(256, 256),
+         "strided": lambda: a[:, ::2]}[view]()
+    want = u.clone().cpu().numpy()
+    got = ch.pupil.output(u, shift=(0.01, -0.02))
+    x = (np.arange(256) - 128) * ch.grid.delta
+    mask = (x[None, :] - 0.01) ** 2 + (x[:, None] - 0.02) ** 2 <= ch.pupil.radius ** 2
+    assert np.array_equal(got.cpu().numpy(), np.where(mask, want, 0))
+    assert np.array_equal(u.cpu().numpy(), want)
