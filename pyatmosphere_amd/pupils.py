@@ -25,4 +25,6 @@ class CirclePupil:
         batch = u.numel() // (n * n)
         call("pa_pupil_output", n, ptr(u), ptr(out), float(grid.delta), float(self.radius), float(shift[0]),
              float(shift[1]), batch, _lib.stream_handle())
+        if batch * n * n < u.numel():       # past the last whole field: as it is
+            out.view(-1)[batch * n * n:] = u.view(-1)[batch * n * n:]
         return out

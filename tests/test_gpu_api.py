@@ -273,3 +273,14 @@ def test_pupil_of_lazy_and_strided_views(dev, view):
     mask = (x[None, :] - 0.01) ** 2 + (x[:, None] - 0.02) ** 2 <= ch.pupil.radius ** 2
     assert np.array_equal(got.cpu().numpy(), np.where(mask, want, 0))
     assert np.array_equal(u.cpu().numpy(), want)
+
+
+def test_pupil_keeps_what_lies_past_the_last_whole_field(dev):
+    """Rows past the last whole n x n field stay as they are in the output."""
+    ch = _quick()
+    ch.pupil.channel = ch
+    u = torch.randn(256 + 3, 256, dtype=torch.complex64, device=dev, generator=torch.Generator(device=dev).manual_seed(4))
+    torch.full((256 + 3, 256), float("nan"), dtype=torch.complex64, device=dev)     # what a new allocation may hold
+    got = ch.pupil.output(u)
+    assert torch.equal(got[:256], ch.pupil.output(u[:256]))
+    assert torch.equal(got[256:], u[256:])
