@@ -42,13 +42,17 @@ def log_polar_base(points: int, f_min: float, f_max: float) -> np.ndarray:
     return np.exp(np.linspace(np.log(f_min), np.log(f_max), points, dtype=np.float32))
 
 
+def annuli(f: np.ndarray) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
+    """(f, inner radii squared, differences of squared radii) of the annuli
+    with outer radii f (grids.py:98-102)."""
+    prev = np.insert(f, 0, 0)[:-1]
+    return f, prev ** 2, f ** 2 - prev ** 2
+
+
 @functools.lru_cache(maxsize=64, typed=True)
 def log_polar_annuli(points: int, f_min: float, f_max: float) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
-    """(base, inner radii squared, differences of squared radii) of the log-polar
-    annuli, float32, read-only (grids.py:94-102)."""
-    f = log_polar_base(points, f_min, f_max)
-    prev = np.insert(f, 0, 0)[:-1]
-    out = (f, prev ** 2, f ** 2 - prev ** 2)
+    """`annuli` of the log-polar base (grids.py:94-102), float32, read-only."""
+    out = annuli(log_polar_base(points, f_min, f_max))
     for a in out:
         a.flags.writeable = False
     return out

@@ -110,6 +110,8 @@ class RandLogPolarGrid(Grid):
         return self._annuli()[0].copy()
 
     def _annuli(self):
+        if type(self).base is not RandLogPolarGrid.base:    # a subclass with its own annuli
+            return engine.annuli(self.base)
         try:
             return engine.log_polar_annuli(self.points, self.f_min, self.f_max)
         except TypeError:       # limits that cannot be hashed (arrays)

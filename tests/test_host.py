@@ -344,3 +344,24 @@ def test_missing_host_draw_is_refused_before_a_launch(given, screens):
     draw = (np.ones((1, 4), np.float32), np.zeros((1, 4), np.float32), np.ones((1, 4), np.complex64))
     with pytest.raises(IndexError):
         engine.run_batch(None, None, np.zeros(1), np.array([screens]), host_spectra=[draw] * given)
+
+
+def _drawn_rho(base, seed):
+    """RandLogPolarGrid.draw_rho's formula (grids.py:98-102) for annuli `base`."""
+    rand = np.random.RandomState(seed).random_sample(size=(1,)).astype(np.float32)
+    prev = np.insert(base, 0, 0)[:-1]
+    return np.sqrt(prev ** 2 + rand * (base ** 2 - prev ** 2)).astype(np.float32)
+
+
+def test_radii_are_drawn_from_the_grids_own_annuli():
+    """draw_rho follows `base` where a subclass has its own: exact."""
+    from pyatmosphere_amd import RandLogPolarGrid
+
+    class Linear(RandLogPolarGrid):
+        @property
+        def base(self):
+            return np.linspace(self.f_min, self.f_max, self.points, dtype=np.float32)
+
+    for g in (Linear(points=16, f_min=0.1, f_max=300.0), RandLogPolarGrid(points=16, f_min=0.1, f_max=300.0)):
+        np.random.seed(5)
+        assert np.array_equal(g.draw_rho(), _drawn_rho(g.base, 5))
