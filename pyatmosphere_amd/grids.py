@@ -107,15 +107,19 @@ class RandLogPolarGrid(Grid):
 
     @property
     def base(self):
-        return self._annuli()[0].copy()
+        if not self._plain_limits():
+            return engine.log_polar_base(self.points, self.f_min, self.f_max)
+        return engine.log_polar_annuli(self.points, self.f_min, self.f_max)[0].copy()
+
+    def _plain_limits(self):
+        """Whether the annuli can be kept by value: numbers, not arrays or
+        tensors, which hash by identity (or not at all) and may change in place."""
+        return all(isinstance(v, (int, float, np.number)) for v in (self.points, self.f_min, self.f_max))
 
     def _annuli(self):
-        if type(self).base is not RandLogPolarGrid.base:    # a subclass with its own annuli
-            return engine.annuli(self.base)
-        try:
-            return engine.log_polar_annuli(self.points, self.f_min, self.f_max)
-        except TypeError:       # limits that cannot be hashed (arrays)
-            return engine.log_polar_annuli.__wrapped__(self.points, self.f_min, self.f_max)
+        if type(self).base is not RandLogPolarGrid.base or not self._plain_limits():
+            return engine.annuli(self.base)     # a subclass's own, or not kept
+        return engine.log_polar_annuli(self.points, self.f_min, self.f_max)
 
     def draw_rho(self):
         rand = np.random.random(size=(1,)).astype(np.float32)

@@ -365,3 +365,20 @@ def test_radii_are_drawn_from_the_grids_own_annuli():
     for g in (Linear(points=16, f_min=0.1, f_max=300.0), RandLogPolarGrid(points=16, f_min=0.1, f_max=300.0)):
         np.random.seed(5)
         assert np.array_equal(g.draw_rho(), _drawn_rho(g.base, 5))
+
+
+@pytest.mark.parametrize("kind", ["array", "tensor"])
+def test_annuli_follow_limits_changed_in_place(kind):
+    """Limits that can change in place (0-d arrays, and tensors, of which only
+    `base` can be formed) give the annuli of the values they hold: exact."""
+    import torch
+    from pyatmosphere_amd import RandLogPolarGrid
+    limit = np.array(0.1) if kind == "array" else torch.tensor(0.1, dtype=torch.float64)
+    g = RandLogPolarGrid(points=16, f_min=limit, f_max=300.0)
+    for _ in range(2):
+        want = o.log_polar_base(16, float(limit), 300.0)
+        assert np.array_equal(np.asarray(g.base), want)
+        if kind == "array":
+            np.random.seed(5)
+            assert np.array_equal(g.draw_rho(), _drawn_rho(want, 5))
+        limit *= 2
