@@ -37,11 +37,15 @@ class GaussianSource(GaussianBeam, Source):
         grid = self.channel.grid
         n = grid.resolution[0]
         dev = device()
-        # the two factors last used stay on the device, by the values they are made from
-        key = (n, grid.delta, self.wvl, self.w0, self.F0, dev, _lib.stream_handle())
-        kept = self.__dict__.get("_factors")
-        if kept is None or kept[0] != key:
-            kept = self._factors = (key, to_device(self.factors(n, grid.delta), dev))
+        if getattr(self.factors, "__func__", None) is not GaussianSource.factors:
+            # a subclass's or instance's own factors may depend on anything
+            kept = (None, to_device(self.factors(n, grid.delta), dev))
+        else:
+            # the two factors last used stay on the device, by the values they are made from
+            key = (n, grid.delta, self.wvl, self.w0, self.F0, dev, _lib.stream_handle())
+            kept = self.__dict__.get("_factors")
+            if kept is None or kept[0] != key:
+                kept = self._factors = (key, to_device(self.factors(n, grid.delta), dev))
         out = torch.empty(n, n, dtype=torch.complex64, device=dev)
         call("pa_outer", n, ptr(out), ptr(kept[1][0]), ptr(kept[1][1]), 1, _lib.stream_handle())
         return out

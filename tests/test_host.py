@@ -382,3 +382,47 @@ def test_annuli_follow_limits_changed_in_place(kind):
             np.random.seed(5)
             assert np.array_equal(g.draw_rho(), _drawn_rho(want, 5))
         limit *= 2
+
+
+@pytest.fixture
+def outer(monkeypatch):
+    """GaussianSource.output on the CPU: pa_outer formed from the addresses it is given."""
+    import ctypes
+    import torch
+    from pyatmosphere_amd import _lib, sources
+
+    def call(name, n, out, gy, gx, batch, stream):
+        assert name == "pa_outer" and batch == 1
+        view = lambda at, size: np.ctypeslib.as_array((ctypes.c_float * (2 * size)).from_address(at)).view(np.complex64)
+        view(out, n * n).reshape(n, n)[:] = view(gy, n)[:, None] * view(gx, n)[None, :]
+
+    monkeypatch.setattr(sources, "device", lambda: torch.device("cpu"))
+    monkeypatch.setattr(sources, "call", call)
+    monkeypatch.setattr(_lib, "stream_handle", lambda: 0)
+
+
+def test_source_follows_a_subclass_or_instance_factors(outer):
+    """GaussianSource.output takes the factors that `factors` gives at the call: exact."""
+    import pyatmosphere_amd as pa
+
+    class Tilted(pa.GaussianSource):
+        tilt = 0.0
+
+        def factors(self, n, delta):
+            gy, gx = super().factors(n, delta)
+            return gy, (gx * np.exp(1j * self.tilt * np.arange(n))).astype(np.complex64)
+
+    def check(s):
+        gy, gx = s.factors(16, 0.01)
+        assert np.array_equal(s.output().numpy(), gy[:, None] * gx[None, :])
+
+    s = Tilted(wvl=808e-9, w0=0.05, F0=np.inf)
+    s.channel = pa.Channel(grid=pa.RectGrid(resolution=16, delta=0.01), source=s, path=pa.VacuumPath(length=1e3))
+    for tilt in (0.0, 0.3):
+        s.tilt = tilt
+        check(s)
+    s = pa.GaussianSource(wvl=808e-9, w0=0.05, F0=np.inf)
+    s.channel = pa.Channel(grid=pa.RectGrid(resolution=16, delta=0.01), source=s, path=pa.VacuumPath(length=1e3))
+    check(s)
+    s.factors = lambda n, delta: (np.ones(n, np.complex64), np.full(n, 2j, np.complex64))
+    check(s)
