@@ -222,6 +222,19 @@ class DeviceTables:
             to_device([src, htab, chp, pup, base, sq], device)
 
 
+def value_key(*values) -> tuple:
+    """The values themselves, to compare with others by: numbers as they are, arrays
+    (and whatever numpy takes as one) by their bytes, as they may change in place;
+    the types too, which numpy's promotion depends on."""
+    out = []
+    for v in values:
+        if not isinstance(v, (int, float, np.number, type(None))):
+            a = np.asarray(v)
+            v = (type(v), a.dtype.str, a.shape, a.tobytes())
+        out.append((type(v), v))
+    return tuple(out)
+
+
 class KeptTables:
     """The device tables of the channels that one path ran last, at most KEEP of
     them: rebuilt unless every value they are made from is what it was, on the
@@ -234,9 +247,8 @@ class KeptTables:
     def get(self, spec: ChannelSpec, device: torch.device) -> DeviceTables:
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("a channel with host draws cannot be captured into a graph")
-        key = (spec.n, spec.delta, spec.wvl, spec.w0, spec.F0, spec.length, np.asarray(spec.positions).tobytes(),
-               spec.points, tuple(spec.pupils), spec.shift, None if spec.gains is None else tuple(spec.gains), device,
-               _lib.stream_handle())
+        key = value_key(spec.n, spec.delta, spec.wvl, spec.w0, spec.F0, spec.length, spec.positions, spec.points,
+                        *spec.shift, *(() if spec.gains is None else spec.gains), *spec.pupils), len(spec.pupils), device, _lib.stream_handle()
         for k, base, psd, tables in self._kept:
             if k == key and np.array_equal(base, spec.base) and np.array_equal(psd, spec.psd):
                 return tables

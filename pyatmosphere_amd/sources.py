@@ -6,7 +6,7 @@ import torch
 
 from . import _lib
 from ._lib import call, ptr
-from .engine import gaussian_factors, to_device
+from .engine import gaussian_factors, to_device, value_key
 from .gpu import device
 from .theory.sources import GaussianBeam
 
@@ -42,7 +42,7 @@ class GaussianSource(GaussianBeam, Source):
             kept = (None, to_device(self.factors(n, grid.delta), dev))
         else:
             # the two factors last used stay on the device, by the values they are made from
-            key = (n, grid.delta, self.wvl, self.w0, self.F0, dev, _lib.stream_handle())
+            key = value_key(n, grid.delta, self.wvl, self.w0, self.F0), dev, _lib.stream_handle()
             kept = self.__dict__.get("_factors")
             if kept is None or kept[0] != key:
                 kept = self._factors = (key, to_device(self.factors(n, grid.delta), dev))

@@ -426,3 +426,66 @@ def test_source_follows_a_subclass_or_instance_factors(outer):
     check(s)
     s.factors = lambda n, delta: (np.ones(n, np.complex64), np.full(n, 2j, np.complex64))
     check(s)
+
+
+@pytest.fixture
+def no_stream(monkeypatch):
+    """Stands in for the current stream, which is not being captured."""
+    import torch
+    from pyatmosphere_amd import _lib
+    monkeypatch.setattr(_lib, "stream_handle", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+
+@pytest.mark.parametrize("field", ["delta", "wvl", "w0", "F0", "length", "gains", "pupils", "positions", "base", "psd"])
+def test_kept_tables_follow_values_changed_in_place(no_stream, field):
+    """KeptTables gives the tables of the values that a spec holds at the call, also
+    where an array among them was changed in place, and keeps them while nothing
+    has changed: exact."""
+    import torch
+    cpu = torch.device("cpu")
+    spec = _spec(S=2)
+    spec.F0 = 3e3
+    spec.gains, spec.pupils, spec.positions = [1.0, 0.5, 0.25], [(0.05, 0.0, 0.0)], np.array([2e3, 6e3])
+    box = {"gains": lambda: spec.gains, "pupils": lambda: spec.pupils}.get(field)
+    if box is None and not isinstance(getattr(spec, field), np.ndarray):
+        setattr(spec, field, np.array(getattr(spec, field)))
+    elif field == "gains":
+        spec.gains[1] = np.array(0.5)
+    elif field == "pupils":
+        spec.pupils[0] = np.array([0.05, 0.0, 0.0])
+    value = box()[1 if field == "gains" else 0] if box else getattr(spec, field)
+    kept = engine.KeptTables()
+    first = kept.get(spec, cpu)
+    assert kept.get(spec, cpu) is first
+    value *= 0.9
+    got, want = kept.get(spec, cpu), engine.DeviceTables([spec], cpu)
+    assert all(torch.equal(getattr(got, k), getattr(want, k)) for k in
+               ("src", "htab", "chparam", "pup", "base", "sqrt_psd"))
+    assert not all(torch.equal(getattr(got, k), getattr(first, k)) for k in
+                   ("src", "htab", "chparam", "pup", "base", "sqrt_psd"))
+
+
+def test_kept_tables_tell_types_apart(no_stream):
+    """A float32 beam radius and the float of the same value give tables that differ
+    in the last bits: each gets its own."""
+    import torch
+    kept, spec = engine.KeptTables(), _spec(S=2)
+    for w0 in (np.float32(0.0437), float(np.float32(0.0437))):
+        spec.w0 = w0
+        assert torch.equal(kept.get(spec, torch.device("cpu")).src,
+                           engine.DeviceTables([spec], torch.device("cpu")).src)
+
+
+def test_source_factors_follow_values_changed_in_place(outer):
+    """The kept factors are those of the values at the call: exact."""
+    import pyatmosphere_amd as pa
+    for name in ("wvl", "w0", "F0"):
+        s = pa.GaussianSource(wvl=808e-9, w0=0.05, F0=2e3)
+        setattr(s, name, np.array(getattr(s, name)))
+        s.channel = pa.Channel(grid=pa.RectGrid(resolution=16, delta=0.01), source=s, path=pa.VacuumPath(length=1e3))
+        for _ in range(2):
+            gy, gx = s.factors(16, 0.01)
+            assert np.array_equal(s.output().numpy(), gy[:, None] * gx[None, :]), name
+            value = getattr(s, name)
+            value *= 1.5
