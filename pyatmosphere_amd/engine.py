@@ -246,9 +246,11 @@ class KeptTables:
 
     def get(self, spec: ChannelSpec, device: torch.device) -> DeviceTables:
         if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("a channel with host draws cannot be captured into a graph")
+            raise RuntimeError("the tables of a channel cannot be uploaded or shared under graph capture: "
+                               "capture engine.run_batch on DeviceTables of its own")
         key = value_key(spec.n, spec.delta, spec.wvl, spec.w0, spec.F0, spec.length, spec.positions, spec.points,
-                        *spec.shift, *(() if spec.gains is None else spec.gains), *spec.pupils), len(spec.pupils), device, _lib.stream_handle()
+                        *spec.shift, *(() if spec.gains is None else spec.gains), *spec.pupils), \
+            len(spec.pupils), device, _lib.stream_handle()
         for k, base, psd, tables in self._kept:
             if k == key and np.array_equal(base, spec.base) and np.array_equal(psd, spec.psd):
                 return tables

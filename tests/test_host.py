@@ -489,3 +489,12 @@ def test_source_factors_follow_values_changed_in_place(outer):
             assert np.array_equal(s.output().numpy(), gy[:, None] * gx[None, :]), name
             value = getattr(s, name)
             value *= 1.5
+
+
+def test_channel_tables_under_capture_say_what_is_refused(no_stream, monkeypatch):
+    """Host- and device-drawn runs both ask for the tables: the refusal names these."""
+    import torch
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="tables of a channel") as e:
+        engine.KeptTables().get(_spec(S=2), torch.device("cpu"))
+    assert "host draws" not in str(e.value)
