@@ -37,6 +37,8 @@ class GaussianSource(GaussianBeam, Source):
         grid = self.channel.grid
         n = grid.resolution[0]
         dev = device()
+        if torch.cuda.is_current_stream_capturing():    # a graph would keep the factors' addresses
+            raise RuntimeError("a source's factors cannot be uploaded or shared under graph capture")
         if getattr(self.factors, "__func__", None) is not GaussianSource.factors:
             # a subclass's or instance's own factors may depend on anything
             kept = (None, to_device(self.factors(n, grid.delta), dev))

@@ -396,6 +396,7 @@ def outer(monkeypatch):
         view = lambda at, size: np.ctypeslib.as_array((ctypes.c_float * (2 * size)).from_address(at)).view(np.complex64)
         view(out, n * n).reshape(n, n)[:] = view(gy, n)[:, None] * view(gx, n)[None, :]
 
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(sources, "device", lambda: torch.device("cpu"))
     monkeypatch.setattr(sources, "call", call)
     monkeypatch.setattr(_lib, "stream_handle", lambda: 0)
@@ -498,3 +499,16 @@ def test_channel_tables_under_capture_say_what_is_refused(no_stream, monkeypatch
     with pytest.raises(RuntimeError, match="tables of a channel") as e:
         engine.KeptTables().get(_spec(S=2), torch.device("cpu"))
     assert "host draws" not in str(e.value)
+
+
+def test_source_output_under_capture_is_refused_with_kept_factors(outer, monkeypatch):
+    """A graph would hold the address of factors that the source may replace: refused
+    whether or not factors are kept, as the copy to the device was."""
+    import torch
+    import pyatmosphere_amd as pa
+    s = pa.GaussianSource(wvl=808e-9, w0=0.05, F0=np.inf)
+    s.channel = pa.Channel(grid=pa.RectGrid(resolution=16, delta=0.01), source=s, path=pa.VacuumPath(length=1e3))
+    s.output()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="capture"):
+        s.output()
