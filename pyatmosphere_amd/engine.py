@@ -587,16 +587,26 @@ class StepRunner:
                    stream=None) -> Optional[torch.Tensor]:
         """Spectra, tables and GEMM of screen `step` into (ang, esc) (default:
         the workspace's single buffers) on `stream` (default: the runner's).  With
-        `compose`, also returns the full phase screen (B, n, n) float32."""
+        `compose`, also returns the full phase screen (B, n, n) float32: an element
+        past its last screen keeps that one, one without screens has zeros."""
         ws = self.ws
         st = self.stream if stream is None else stream
         if host is not None:
             upload_spectra(ws, *host, batch=self.B)
         else:
             draw_prep_device(ws, self.tables, seed, step, self.B, self.ns, st)
+        ang = ws.ang if ang is None else ang
         phi = torch.empty(self.B, ws.n, ws.n, dtype=torch.float32, device=ws.device) if compose else None
-        synth_screen(ws, self.tables, step, self.B, self.ns, st, esc=esc, ang=ws.ang if ang is None else ang,
-                     prepped=host is None, phi=phi)
+        if compose and self.ns is not None:
+            # the GEMM skips elements without this screen; the compose pass takes
+            # every element, and these have their last screen's parts still
+            p2 = ws.phi2_buffer()
+            synth_screen(ws, self.tables, step, self.B, self.ns, st, esc=esc, phi2=p2, ang=ang, prepped=host is None)
+            call("pa_screen_compose", ws.n, ptr(ws.sparam), ptr(ws.hg), ptr(p2), ptr(phi), self.B, st)
+            if self.smin == 0:
+                phi[torch.from_numpy(self.nscreens_np == 0).to(ws.device)] = 0.0
+            return phi
+        synth_screen(ws, self.tables, step, self.B, self.ns, st, esc=esc, ang=ang, prepped=host is None, phi=phi)
         return phi
 
     def apply(self, step: int, ang: Optional[torch.Tensor] = None) -> None:

@@ -869,3 +869,37 @@ def test_small_launches_take_the_same_products(dev, n, batch, points, mode):
         engine.screen_gemm(ws, 0, batch, None, None, phi=phi, tile=tile)
         got.append((ang, phi2, phi))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("draws", ["device", "host"])
+def test_composed_screens_of_a_ragged_batch(dev, draws):
+    """run_batch(screens_out=...) with 5, 2 and 0 screens: an element's screens are
+    those of a run of its own, bit for bit; past its last one it keeps that, and an
+    element without screens has zeros."""
+    s5 = channel_spec(128, 0.004, 808e-9, 0.05, 3e3, 5, 64, 1e-15)
+    s2 = channel_spec(128, 0.003, 1550e-9, 0.04, 2e3, 2, 64, 3e-15)
+    vac = engine.ChannelSpec(n=128, delta=0.004, wvl=808e-9, w0=0.05, F0=np.inf, length=3e3,
+                             positions=np.zeros(0), points=64, base=s5.base, psd=s5.psd)
+    specs = [s2, vac, s5]
+    ns = np.array([s.nscreens for s in specs])
+    rs = np.random.RandomState(6)
+    host = [(np.exp(rs.uniform(-5, 4, (3, 64))), rs.uniform(0, 6, (3, 64)),
+             0.1 * (rs.normal(size=(3, 64)) + 1j * rs.normal(size=(3, 64)))) for _ in range(5)]
+
+    def run(members):
+        tables = engine.DeviceTables([specs[m] for m in members], dev)
+        ws = engine.Workspace(128, 64, len(members), "f16x3", dev)
+        screens = []
+        torch.full((len(members), 128, 128), float("nan"), device=dev)      # what a new allocation may hold
+        engine.run_batch(ws, tables, np.arange(len(members)), ns[members], seed=3, rid=np.array(members) + 7,
+                         screens_out=screens,
+                         host_spectra=[tuple(a[members] for a in h) for h in host] if draws == "host" else None)
+        return [s.cpu().numpy() for s in screens]
+
+    together = run([0, 1, 2])
+    assert len(together) == 5
+    for m in (0, 2):
+        alone = run([m])
+        for i in range(5):
+            assert np.array_equal(together[i][m], alone[min(i, ns[m] - 1)][0]), (m, i)
+    assert all((s[1] == 0).all() for s in together)
