@@ -849,6 +849,9 @@ class GraphedBatch:
                 if i < run.smax:
                     run.screen(i, seed=self.seed)
         run.finish(self.field_out, True)
+        # the graph holds addresses in these: a run with more screens on this
+        # workspace replaces them there
+        self._synth = getattr(ws, "_synth", None)
 
 
 class Ensemble:

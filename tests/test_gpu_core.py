@@ -903,3 +903,29 @@ def test_composed_screens_of_a_ragged_batch(dev, draws):
         for i in range(5):
             assert np.array_equal(together[i][m], alone[min(i, ns[m] - 1)][0]), (m, i)
     assert all((s[1] == 0).all() for s in together)
+
+
+def test_graph_keeps_its_synthesis_buffers(dev):
+    """A captured batch whose workspace a run with more screens then uses (its
+    synthesis buffers are replaced by larger ones) replays with the same moments, and
+    the buffers that it holds are given back with it."""
+    import gc
+    import weakref
+    s3 = channel_spec(128, 0.004, 808e-9, 0.05, 3e3, 3, 64, 1e-15)
+    s5 = channel_spec(128, 0.003, 1550e-9, 0.04, 2e3, 5, 64, 3e-15)
+    t3, t5 = engine.DeviceTables([s3], dev), engine.DeviceTables([s5], dev)
+    ws = engine.Workspace(128, 64, 2, "f16x3", dev)
+    gb = engine.GraphedBatch(ws, t3, np.zeros(2), np.full(2, 3), 11)
+    want = gb.run(np.arange(2)).cpu().numpy()
+    own = weakref.ref(ws._synth)
+    engine.run_batch(ws, t5, np.zeros(2), np.full(2, 5), seed=1, rid=np.arange(2))
+    torch.cuda.synchronize()
+    assert ws._synth is not own() and own() is not None
+    filler = [torch.full((1 << k,), float("nan"), device=dev) for k in range(10, 24)]
+    for _ in range(2):
+        assert np.array_equal(gb.run(np.arange(2)).cpu().numpy(), want)
+        torch.cuda.synchronize()
+    assert all(torch.isnan(f).all() for f in filler)
+    del gb
+    gc.collect()
+    assert own() is None
