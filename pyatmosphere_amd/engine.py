@@ -320,15 +320,22 @@ class Workspace:
             self.side = torch.cuda.Stream(device=self.device)   # default priority
 
     def upload_ids(self, chan, nsteps, rid=None) -> None:
-        """Channels, screen counts and (when given) realization ids of a batch."""
+        """Channels, screen counts and (when given) realization ids of a batch; the
+        workspace's further elements keep theirs."""
         B, n = self.batch, len(chan)
-        stage = torch.zeros(16 * B, dtype=torch.uint8, pin_memory=True)
+        if n < B:
+            upload(self.chan[:n], chan, np.int32)
+            upload(self.nsteps[:n], nsteps, np.int32)
+            if rid is not None:
+                upload(self.rid[:n], rid, np.int64)
+            return
+        stage = torch.empty(16 * B, dtype=torch.uint8, pin_memory=True)
         h = stage.numpy()
-        h[8 * B:12 * B].view(np.int32)[:n] = chan
-        h[12 * B:].view(np.int32)[:n] = nsteps
+        h[8 * B:12 * B].view(np.int32)[:] = chan
+        h[12 * B:].view(np.int32)[:] = nsteps
         lo = 8 * B
         if rid is not None:
-            h[:lo].view(np.int64)[:n] = rid
+            h[:lo].view(np.int64)[:] = rid
             lo = 0
         self._ids[0][lo:].copy_(stage[lo:], non_blocking=True)
 

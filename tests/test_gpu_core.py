@@ -929,3 +929,14 @@ def test_graph_keeps_its_synthesis_buffers(dev):
     del gb
     gc.collect()
     assert own() is None
+
+
+@pytest.mark.parametrize("rid", [None, [5]])
+def test_smaller_batch_leaves_other_elements_ids(dev, rid):
+    """Uploading a batch's ids leaves those past it, which a captured batch on the
+    same workspace replays with."""
+    ws = engine.Workspace(128, 64, 3, "f16x3", dev)
+    ws.upload_ids([0, 1, 1], [5, 2, 3], [7, 8, 9])
+    ws.upload_ids([2], [4], rid)
+    assert ws.chan.tolist() == [2, 1, 1] and ws.nsteps.tolist() == [4, 2, 3]
+    assert ws.rid.tolist() == [7 if rid is None else 5, 8, 9]
