@@ -363,6 +363,14 @@ def synth_bytes_per_element(n: int, points: int, mode: int) -> int:
     return 2 * opb + points * (32 + 16) + _lib.PA_SCREEN_PARAMS * 8 + 2 * n * (8 + 8) + n * n * 4 + 12
 
 
+def whole_batch_fits(ws: "Workspace", screens: int, batch: int) -> bool:
+    """Whether the synthesis of `screens` screens of a batch as one virtual batch
+    stays within SYNTH_BATCH_MAX_BYTES and within a launch (the tables and the
+    polynomial block have the pairs on a grid axis of at most 65535 blocks)."""
+    pairs = screens * batch
+    return 0 < pairs <= 65535 and pairs * synth_bytes_per_element(ws.n, ws.points, ws.mode) <= SYNTH_BATCH_MAX_BYTES
+
+
 class SynthBuffers:
     """Screen synthesis of every screen of a batch as one virtual batch:
     element v = i * B + b is screen i of realization b (B the run's batch).
@@ -520,10 +528,8 @@ class StepRunner:
         self.chan_np, self.nscreens_np = np.asarray(chan), np.asarray(nscreens)
 
     def whole_batch_synthesis(self) -> bool:
-        """Whether synthesize_all fits SYNTH_BATCH_MAX_BYTES for this batch."""
-        ws = self.ws
-        need = self.smax * self.B * synth_bytes_per_element(ws.n, ws.points, ws.mode)
-        return self.smax > 0 and need <= SYNTH_BATCH_MAX_BYTES
+        """Whether synthesize_all takes this batch (whole_batch_fits)."""
+        return whole_batch_fits(self.ws, self.smax, self.B)
 
     def synthesize_all(self, seed: Optional[int], stream=None, timed=None, upload_ids: bool = True,
                        host: Optional[Sequence] = None) -> List[torch.Tensor]:
@@ -683,7 +689,7 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
         # a screen without a draw is an IndexError here, before anything is launched
         host_spectra = [host_spectra[i] for i in range(int(np.max(nscreens)) if len(nscreens) else 0)]
     single = single and host_spectra is not None and screens_out is None and SYNTH_WHOLE_BATCH and \
-        tables.max_screens * len(chan) * synth_bytes_per_element(ws.n, ws.points, ws.mode) <= SYNTH_BATCH_MAX_BYTES
+        whole_batch_fits(ws, tables.max_screens, len(chan))
     run = StepRunner(ws, tables, chan, nscreens, rid, single=single)
     sep = SEPARABLE_SOURCE if separable is None else bool(separable)
     if overlap is None:

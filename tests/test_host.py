@@ -512,3 +512,15 @@ def test_source_output_under_capture_is_refused_with_kept_factors(outer, monkeyp
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     with pytest.raises(RuntimeError, match="capture"):
         s.output()
+
+
+@pytest.mark.parametrize("screens, batch, whole", [(5, 13107, True), (5, 13108, False), (1, 65536, False), (0, 4, False),
+                                                   (1, 1 << 20, False)])
+def test_whole_batch_synthesis_stays_within_a_launch(screens, batch, whole):
+    """The tables' and the polynomial block's launches have the pairs on a grid axis
+    of at most 65535 blocks; larger batches are synthesized screen by screen."""
+    class Ws:
+        n, points, mode = 64, 16, 0
+    run = engine.StepRunner.__new__(engine.StepRunner)
+    run.ws, run.smax, run.B = Ws, screens, batch
+    assert run.whole_batch_synthesis() == whole
