@@ -348,6 +348,15 @@ class Workspace:
             sb = self._synth = SynthBuffers(self, screens)
         return sb
 
+    def has_room_for_host_draws(self, screens: int) -> bool:
+        """Whether the device holds the buffers that synthesize_all needs for host
+        draws; allocates them."""
+        try:
+            self.synth_buffers(screens).host_buffer()
+        except torch.OutOfMemoryError:
+            return False
+        return True
+
     def bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in vars(self).values() if isinstance(t, torch.Tensor))
 
@@ -400,6 +409,12 @@ class SynthBuffers:
 
         self.spectra: Optional[torch.Tensor] = None    # host draws (upload), allocated on first use
 
+    def host_buffer(self) -> torch.Tensor:
+        """The device buffer of host draws, allocated on first use."""
+        if self.spectra is None:
+            self.spectra = torch.empty(4 * self.capacity * self.points, dtype=torch.float32, device=self.ang.device)
+        return self.spectra
+
     def upload(self, host_spectra, batch: int):
         """The host draws of every screen, (rho, theta, value) arrays (B, P) each, in
         one copy; returns the device addresses of rho, theta, value in pair order."""
@@ -411,10 +426,9 @@ class SynthBuffers:
         for i, (r, t, v) in enumerate(host_spectra):
             rho[i * batch:(i + 1) * batch], theta[i * batch:(i + 1) * batch] = r, t
             value[i * batch:(i + 1) * batch] = v
-        if self.spectra is None:
-            self.spectra = torch.empty(4 * self.capacity * P, dtype=torch.float32, device=self.ang.device)
-        self.spectra[:4 * V * P].copy_(stage, non_blocking=True)
-        at = self.spectra.data_ptr()
+        spectra = self.host_buffer()
+        spectra[:4 * V * P].copy_(stage, non_blocking=True)
+        at = spectra.data_ptr()
         return at, at + 4 * V * P, at + 8 * V * P
 
 
@@ -685,17 +699,20 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
     its screens: host-drawn batches then upload no ids (ws.chan and ws.nsteps
     stay as they are).
     """
+    smax = int(np.max(nscreens)) if len(nscreens) else 0
     if host_spectra is not None:
         # a screen without a draw is an IndexError here, before anything is launched
-        host_spectra = [host_spectra[i] for i in range(int(np.max(nscreens)) if len(nscreens) else 0)]
-    single = single and host_spectra is not None and screens_out is None and SYNTH_WHOLE_BATCH and \
-        whole_batch_fits(ws, tables.max_screens, len(chan))
+        host_spectra = [host_spectra[i] for i in range(smax)]
+    whole = screens_out is None and SYNTH_WHOLE_BATCH and whole_batch_fits(ws, smax, len(chan))
+    if host_spectra is not None:
+        # these did with one screen's buffers: without room for all, screen by screen
+        whole = whole and ws.has_room_for_host_draws(smax)
+    single = single and whole and host_spectra is not None
     run = StepRunner(ws, tables, chan, nscreens, rid, single=single)
     sep = SEPARABLE_SOURCE if separable is None else bool(separable)
     if overlap is None:
-        overlap = use_overlap(ws, len(chan), int(np.max(nscreens)) if len(nscreens) else 0)
+        overlap = use_overlap(ws, len(chan), smax)
     device_draws = host_spectra is None and screens_out is None and run.smax > 0
-    whole = screens_out is None and run.smax > 0 and SYNTH_WHOLE_BATCH and run.whole_batch_synthesis()
     if device_draws and overlap:
         overlapped_body(run, seed, field_in, sep, whole)
     elif whole:

@@ -940,3 +940,30 @@ def test_smaller_batch_leaves_other_elements_ids(dev, rid):
     ws.upload_ids([2], [4], rid)
     assert ws.chan.tolist() == [2, 1, 1] and ws.nsteps.tolist() == [4, 2, 3]
     assert ws.rid.tolist() == [7 if rid is None else 5, 8, 9]
+
+
+def test_host_drawn_batch_without_room_for_all_screens(dev, monkeypatch):
+    """Where the device cannot hold the synthesis buffers of all screens at once, a
+    host-drawn batch goes screen by screen, with the same bits."""
+    specs = [channel_spec(128, 0.004, 808e-9, 0.05, 3e3, 4, 64, 1e-15),
+             channel_spec(128, 0.003, 1550e-9, 0.04, 2e3, 2, 64, 3e-15)]
+    tables = engine.DeviceTables(specs, dev)
+    rs = np.random.RandomState(6)
+    host = [(np.exp(rs.uniform(-5, 4, (2, 64))), rs.uniform(0, 6, (2, 64)),
+             0.1 * (rs.normal(size=(2, 64)) + 1j * rs.normal(size=(2, 64)))) for _ in range(4)]
+
+    def run(chan, single=False):
+        ws = engine.Workspace(128, 64, 2, "f16x3", dev)
+        out = torch.empty(len(chan), 128, 128, dtype=torch.complex64, device=dev)
+        engine.run_batch(ws, tables if not single else engine.DeviceTables(specs[:1], dev), np.array(chan),
+                         np.array([specs[c].nscreens for c in chan]), host_spectra=[tuple(a[:len(chan)] for a in h) for h in host],
+                         field_out=out, reduce=False, single=single)
+        return out
+
+    want = run([0, 1]), run([0], single=True)
+
+    def no_room(self, *args):
+        raise torch.OutOfMemoryError("no room")
+    monkeypatch.setattr(engine.SynthBuffers, "__init__", no_room)
+    got = run([0, 1]), run([0], single=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
