@@ -705,8 +705,9 @@ def run_batch(ws: Workspace, tables: DeviceTables, chan: np.ndarray, nscreens: n
         host_spectra = [host_spectra[i] for i in range(smax)]
     whole = screens_out is None and SYNTH_WHOLE_BATCH and whole_batch_fits(ws, smax, len(chan))
     if host_spectra is not None:
-        # these did with one screen's buffers: without room for all, screen by screen
-        whole = whole and ws.has_room_for_host_draws(smax)
+        # these did with one screen's buffers: where those of all screens for the
+        # workspace's whole batch are too much, screen by screen
+        whole = whole and whole_batch_fits(ws, smax, ws.batch) and ws.has_room_for_host_draws(smax)
     single = single and whole and host_spectra is not None
     run = StepRunner(ws, tables, chan, nscreens, rid, single=single)
     sep = SEPARABLE_SOURCE if separable is None else bool(separable)

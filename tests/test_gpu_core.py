@@ -967,3 +967,22 @@ def test_host_drawn_batch_without_room_for_all_screens(dev, monkeypatch):
     monkeypatch.setattr(engine.SynthBuffers, "__init__", no_room)
     got = run([0, 1]), run([0], single=True)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_host_drawn_buffers_stay_within_their_limit(dev, monkeypatch):
+    """SYNTH_BATCH_MAX_BYTES bounds what a workspace keeps for host draws: its buffers
+    are as large as its own batch, however small the batch that asks for them."""
+    spec = channel_spec(128, 0.004, 808e-9, 0.05, 3e3, 4, 64, 1e-15)
+    tables = engine.DeviceTables([spec], dev)
+    rs = np.random.RandomState(6)
+    host = [(np.exp(rs.uniform(-5, 4, (1, 64))), rs.uniform(0, 6, (1, 64)),
+             0.1 * (rs.normal(size=(1, 64)) + 1j * rs.normal(size=(1, 64)))) for _ in range(4)]
+    fields = []
+    for room in (4, 3):           # workspace batches' worth of buffers
+        ws = engine.Workspace(128, 64, 3, "f16x3", dev)
+        monkeypatch.setattr(engine, "SYNTH_BATCH_MAX_BYTES", room * 3 * engine.synth_bytes_per_element(128, 64, ws.mode))
+        out = torch.empty(1, 128, 128, dtype=torch.complex64, device=dev)
+        engine.run_batch(ws, tables, np.zeros(1), np.array([4]), host_spectra=host, field_out=out, reduce=False)
+        fields.append(out)
+        assert (getattr(ws, "_synth", None) is not None) == (room == 4)
+    assert torch.equal(*fields)
