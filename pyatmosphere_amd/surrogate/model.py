@@ -244,8 +244,9 @@ def _distributions(members: Sequence[PDTSurrogate], x: np.ndarray):
     host = torch.empty(dist.shape, dtype=dist.dtype, pin_memory=True)
     host.copy_(dist, non_blocking=True)
     torch.cuda.current_stream(dist.device).synchronize()
-    flat = host.numpy()
-    return flat[:M * NB].reshape(M, NB), flat[M * NB:M * (NB + 1)], flat[M * (NB + 1):]
+    # copied out of the staging memory, which an answer that is kept would hold
+    parts = host[:M * NB].clone(), host[M * NB:M * (NB + 1)].clone(), host[M * (NB + 1):].clone()
+    return parts[0].numpy().reshape(M, NB), parts[1].numpy(), parts[2].numpy()
 
 
 def ks_binned(p: np.ndarray, q: np.ndarray) -> np.ndarray:

@@ -206,3 +206,16 @@ def test_ensemble_statistics(dev, widths, M):
         np.testing.assert_allclose(a, b, rtol=0, atol=1e-13 * max(1.0, np.nanmax(np.abs(b))), equal_nan=True)
     inside = np.all(np.abs(x) <= 1 + 1e-6, axis=1)
     assert np.array_equal(got[3], (spread > 0.04) | ~inside)
+
+
+@pytest.mark.parametrize("requests", [1, 300])
+def test_answers_hold_no_pinned_memory(dev, requests):
+    """What predict and pdt return is ordinary memory, each array its own: keeping an
+    answer, or one array of it, keeps nothing else."""
+    from pyatmosphere_amd.surrogate import SurrogateEnsemble
+    x = np.random.default_rng(0).uniform(-1, 1, (requests, 5)).astype(np.float32)
+    nets = [PDTSurrogate(width=64, depth=3, seed=s, device=dev) for s in range(2)]
+    for answer in (nets[0].predict(x), SurrogateEnsemble(nets, 0.1).pdt(x)[:3]):
+        for a in answer:
+            assert a.dtype == np.float64 and not torch.from_numpy(a).is_pinned()
+            assert a.base is None or a.base.nbytes == a.nbytes
