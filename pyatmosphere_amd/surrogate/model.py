@@ -178,7 +178,7 @@ class PDTSurrogate:
     def _bf16_layers(self):
         """Per layer (weights, bias, width, padded width, inputs) for the networks
         that the fused launch does not take."""
-        if self._bf16 is None:
+        if not isinstance(self._bf16, list):
             layers = []
             for W, b in self.params:
                 fo, fi = W.shape
@@ -204,13 +204,23 @@ class PDTSurrogate:
             h = y if fo_p == fo else y[:, :fo].contiguous()
         return h
 
+    def _plain(self, *names: str) -> bool:
+        """Whether neither a subclass nor the instance has its own methods `names`."""
+        return all(getattr(getattr(self, f), "__func__", None) is getattr(PDTSurrogate, f) for f in names)
+
     def predict_raw(self, x: np.ndarray) -> np.ndarray:
         """(M, NB + 1) outputs on bf16 MFMA."""
-        return _outputs([self], x)[0].cpu().numpy().astype(np.float64)
+        out = _outputs([self], x)[0] if self._plain("_pad") else self._layer_by_layer(x)[:, :NB + 1]
+        return out.cpu().numpy().astype(np.float64)
 
     def predict(self, x: np.ndarray) -> Tuple[np.ndarray, np.ndarray]:
         """Bin probabilities (M, NB) of the transmittance PDT and log sigma_BW,x^2."""
-        return _distributions([self], x)[:2]
+        if self._plain("_pad", "predict_raw"):
+            return _distributions([self], x)[:2]
+        out = self.predict_raw(x)
+        lg = out[:, :NB]
+        p = np.exp(lg - lg.max(axis=1, keepdims=True))
+        return p / p.sum(axis=1, keepdims=True), out[:, NB]
 
 
 def _outputs(members: Sequence[PDTSurrogate], x: np.ndarray) -> torch.Tensor:
@@ -267,8 +277,8 @@ class SurrogateEnsemble:
         self.max_spread = max_spread
 
     def pdt(self, x: np.ndarray):
-        if 0 < len(self.members) <= MAX_FUSED_MEMBERS and all(type(m) is PDTSurrogate for m in self.members) \
-                and len({m.device for m in self.members}) == 1:
+        if 0 < len(self.members) <= MAX_FUSED_MEMBERS and len({m.device for m in self.members}) == 1 \
+                and all(type(m) is PDTSurrogate and m._plain("_pad", "predict_raw", "predict") for m in self.members):
             mean, lv, spread = _distributions(self.members, x)
         else:
             preds = [m.predict(x) for m in self.members]

@@ -34,3 +34,53 @@ def test_softmax_ce_minimum_at_target():
     x = np.concatenate([np.log(t), [[0.5]]], axis=1)
     _, grads = mlp.loss_and_grad(params, x, t, np.array([0.5]), 1.0)
     assert np.abs(grads[0][1]).max() < 1e-12
+
+
+def test_prediction_goes_through_an_overridden_output():
+    """predict and SurrogateEnsemble.pdt take what a subclass's or an instance's own
+    predict_raw or predict gives (no device is touched)."""
+    import torch
+    from pyatmosphere_amd.surrogate import NB, PDTSurrogate, SurrogateEnsemble
+    rng = np.random.default_rng(0)
+    out = rng.normal(size=(6, NB + 1))
+    x = rng.uniform(-1, 1, (6, 5)).astype(np.float32)
+
+    class Fixed(PDTSurrogate):
+        def predict_raw(self, x):
+            return out
+
+    lg = out[:, :NB]
+    want = np.exp(lg) / np.exp(lg).sum(axis=1, keepdims=True)
+    net = Fixed(width=16, depth=2, device=torch.device("cpu"))
+    p, lv = net.predict(x)
+    assert np.allclose(p, want, rtol=1e-13) and np.array_equal(lv, out[:, NB])
+    assert np.allclose(SurrogateEnsemble([net, net], 0.1).pdt(x)[0], want, rtol=1e-13)
+    plain = PDTSurrogate(width=16, depth=2, device=torch.device("cpu"))
+    plain.predict = lambda x: (want, out[:, NB])
+    mean, lv, spread, _ = SurrogateEnsemble([plain, net], 0.1).pdt(x)
+    assert np.allclose(mean, want, rtol=1e-13) and np.allclose(lv, out[:, NB]) and spread.max() < 1e-13
+
+
+def test_inputs_go_through_an_overridden_pad(monkeypatch):
+    """A subclass with its own input padding predicts from what it gives."""
+    import torch
+    from pyatmosphere_amd.surrogate import NB, PDTSurrogate
+    from pyatmosphere_amd.surrogate import model
+
+    seen = []
+
+    class Scaled(PDTSurrogate):
+        def _pad(self, x):
+            return super()._pad(2 * x)
+
+    def call(name, M, fo, fi, h, W, b, y, act, stream):
+        assert name == "pa_mlp_layer_bf16"
+        if not seen:
+            import ctypes
+            seen.append(np.ctypeslib.as_array((ctypes.c_float * (M * fi)).from_address(h)).reshape(M, fi).copy())
+
+    monkeypatch.setattr(model, "call", lambda name, *a: call(name, *a) if name != "pa_mlp_to_bf16" else None)
+    monkeypatch.setattr(model._lib, "stream_handle", lambda: 0)
+    x = np.random.default_rng(1).uniform(-1, 1, (3, 5)).astype(np.float32)
+    Scaled(width=32, depth=2, device=torch.device("cpu")).predict_raw(x)
+    assert np.array_equal(seen[0][:, :5], 2 * x)
