@@ -235,10 +235,7 @@ class Simulation:
             spec = path._spec((0.0, 0.0), with_total=False)  # Channel.generator output
             spec.pupils = [(r, sx, sy) for (r, sx, sy) in p["pupils"]]
             prepared.append((p, spec, path._tables(spec, dev)))
-        # with nothing to do between realizations a batch's values go in at once
-        measures = list(self.flattened_measures())
-        at_once = not (plot_step or save_step) and type(self).process_output is Simulation.process_output \
-            and all(type(m) is Measure for m in measures) and len({id(m) for m in measures}) == len(measures)
+        at_once = self._values_at_once(prepared, plot_step, save_step)
         iteration = 0
         while not self.is_measures_done():
             remaining = self._remaining()
@@ -295,6 +292,17 @@ class Simulation:
                 self.process_output(iteration, plot_step=plot_step, save_step=save_step)
                 if self.is_measures_done():
                     break
+
+    def _values_at_once(self, prepared, plot_step, save_step):
+        """Whether a batch's values can go in at once: there is nothing to do between
+        realizations, and nobody to see them one by one (a subclass's or an
+        instance's own end, output hook, measures or tracked results)."""
+        measures = list(self.flattened_measures())
+        own = any(getattr(getattr(self, f), "__func__", None) is not getattr(Simulation, f)
+                  for f in ("process_output", "is_measures_done", "flattened_measures"))
+        tracked = [m.operations[0].__self__ for p, _, _ in prepared for m, c in p["items"] if c[0] == "tracked"]
+        return not (plot_step or save_step or own) and all(type(m) is Measure for m in measures) \
+            and all(type(r) is TrackedPDTResult for r in tracked) and len({id(m) for m in measures}) == len(measures)
 
     @staticmethod
     def _column(c, mom, tr):

@@ -217,3 +217,55 @@ def test_batch_values_taken_at_once(sizes, batch):
         Simulation([])._take([(plan, None, None)], {id(plan): (mom, tr)}, batch)
         assert [(m.data, m.iteration_data) for m, _ in items2] == [(m.data, m.iteration_data) for m, _ in items]
         assert owner2.pupil_shift == owner.pupil_shift
+
+
+@pytest.mark.parametrize("own", ["none", "method_done", "method_output", "instance_output", "property_shift"])
+def test_batch_goes_by_realization_where_the_driver_is_overridden(monkeypatch, own):
+    """A Simulation whose end, output hook or tracked result a subclass or the
+    instance has made its own sees every realization, as one at a time would."""
+    import torch
+    from pyatmosphere_amd import engine
+    from pyatmosphere_amd.simulations import TrackedPDTResult, simulation
+    seen, shifts = [], []
+
+    class Stop(Simulation):
+        def is_measures_done(self, measures=None):
+            return len(m) >= 5
+
+    class Hook(Simulation):
+        def process_output(self, iteration, plot_step, save_step):
+            seen.append((iteration, len(m)))
+
+    class Tracked(TrackedPDTResult):
+        @property
+        def pupil_shift(self):
+            return (0.0, 0.0)
+
+        @pupil_shift.setter
+        def pupil_shift(self, value):
+            shifts.append(value)
+
+    class Spec:
+        n, points, nscreens = 64, 16, 1
+
+    ch = FakeChannel()
+    ch.path.init_phase_screens = lambda: None
+    ch.path._spec = lambda shift, with_total: Spec()
+    ch.path._tables = lambda spec, dev: None
+    mom = torch.from_numpy(np.random.default_rng(0).normal(size=(8, 15)))
+    monkeypatch.setattr(simulation, "device", lambda: None)
+    monkeypatch.setattr(engine, "get_workspace", lambda *a: None)
+    tracked = own == "property_shift"
+    monkeypatch.setattr(engine, "run_batch", lambda *a, **k: (mom, mom) if tracked else mom)
+    sim = {"method_done": Stop, "method_output": Hook}.get(own, Simulation)(batch=8, rng="device")
+    if own == "instance_output":
+        sim.process_output = lambda iteration, plot_step, save_step: seen.append((iteration, len(m)))
+    res = Tracked.__new__(Tracked)
+    m = Measure(ch, "atmosphere", res.set_pupil_position, max_size=None if own == "method_done" else 8)
+    sim.add_measures(m)
+    plan = dict(channel=ch, items=[(m, ("tracked", 0) if tracked else ("moment", 1))], pupils=[],
+                tracked=[0.1] if tracked else [])
+    sim._run_fused([plan], None, None)
+    assert m.data == mom[:5 if own == "method_done" else 8, 7 if tracked else 1].tolist()
+    assert seen == ([(i, i) for i in range(1, 9)] if own.endswith("_output") else [])
+    assert shifts == ([(float(a), float(b)) for a, b in mom[:, 1:3]] if tracked else [])
