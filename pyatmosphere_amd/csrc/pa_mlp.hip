@@ -547,26 +547,38 @@ static bool quads(const float* p, int ld, int K) {
   return K % 4 == 0 && ld % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
 }
 
+// Row tiles lie on a grid axis of at most 65535 blocks: calls f(first row, rows) for
+// as many launches as M rows take.
+constexpr int kGridRows = 65535 * GT;
+template <class F>
+static void row_launches(int M, F f) {
+  for (long long m = 0; m < M; m += kGridRows) f((size_t)m, (int)(M - m < kGridRows ? M - m : kGridRows));
+}
+
 int mlp_gemm_f32(int M, int N, int K, const float* A, int lda, int ta, const float* B, int ldb, int tb, float* C,
                  int ldc, float alpha, float beta, hipStream_t s) {
-  const dim3 g((N + GT - 1) / GT, (M + GT - 1) / GT);
   const bool va = !ta && quads(A, lda, K), vb = tb && quads(B, ldb, K);
-#define G_(TA, TB, VA, VB)                                                                                      \
-  hipLaunchKernelGGL((k_gemm_f32<TA, TB, VA, VB>), g, dim3(64 * kGemmWaves), 0, s, M, N, K, A, lda, B, ldb, C, \
+  row_launches(M, [&](size_t m, int rows) {
+    const dim3 g((N + GT - 1) / GT, (rows + GT - 1) / GT);
+    const float* a = A + (ta ? m : m * lda);
+    float* c = C + m * ldc;
+#define G_(TA, TB, VA, VB)                                                                                         \
+  hipLaunchKernelGGL((k_gemm_f32<TA, TB, VA, VB>), g, dim3(64 * kGemmWaves), 0, s, rows, N, K, a, lda, B, ldb, c, \
                      ldc, alpha, beta)
-  if (ta && tb) {
-    if (vb) G_(true, true, false, true);
-    else G_(true, true, false, false);
-  } else if (ta) {
-    G_(true, false, false, false);
-  } else if (tb) {
-    if (va && vb) G_(false, true, true, true);
-    else G_(false, true, false, false);
-  } else {
-    if (va) G_(false, false, true, false);
-    else G_(false, false, false, false);
-  }
+    if (ta && tb) {
+      if (vb) G_(true, true, false, true);
+      else G_(true, true, false, false);
+    } else if (ta) {
+      G_(true, false, false, false);
+    } else if (tb) {
+      if (va && vb) G_(false, true, true, true);
+      else G_(false, true, false, false);
+    } else {
+      if (va) G_(false, false, true, false);
+      else G_(false, false, false, false);
+    }
 #undef G_
+  });
   return check_launch("mlp_gemm_f32");
 }
 
@@ -590,13 +602,19 @@ int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const fl
   float *z = scratch, *d = scratch + all, *y = scratch + 2 * all;
   for (int i = 0; i < layers; ++i) {
     const int fi = sizes[i], fo = sizes[i + 1];
-    const dim3 g((fo + GT - 1) / GT, (M + GT - 1) / GT);
-    const float* W = params[2 * i];
+    const float *W = params[2 * i], *bias = params[2 * i + 1];
     float* Y = i < layers - 1 ? y : nullptr;
-    if (quads(h, fi, fi) && quads(W, fi, fi))
-      hipLaunchKernelGGL(k_layer_forward<true>, g, dim3(64 * kGemmWaves), 0, s, M, fo, fi, h, W, params[2 * i + 1], z, Y);
-    else
-      hipLaunchKernelGGL(k_layer_forward<false>, g, dim3(64 * kGemmWaves), 0, s, M, fo, fi, h, W, params[2 * i + 1], z, Y);
+    const bool vec = quads(h, fi, fi) && quads(W, fi, fi);
+    row_launches(M, [&](size_t m, int rows) {
+      const dim3 g((fo + GT - 1) / GT, (rows + GT - 1) / GT);
+      float* Ym = Y ? Y + m * fo : nullptr;
+      if (vec)
+        hipLaunchKernelGGL(k_layer_forward<true>, g, dim3(64 * kGemmWaves), 0, s, rows, fo, fi, h + m * fi, W, bias,
+                           z + m * fo, Ym);
+      else
+        hipLaunchKernelGGL(k_layer_forward<false>, g, dim3(64 * kGemmWaves), 0, s, rows, fo, fi, h + m * fi, W, bias,
+                           z + m * fo, Ym);
+    });
     if (i < layers - 1) {
       h = y;
       y += padded((size_t)M * fo);
@@ -616,11 +634,16 @@ int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const fl
       z -= padded((size_t)M * fi);
       float* dn = d - padded((size_t)M * fi);
       hl[i] = y;
-      const dim3 g((fi + GT - 1) / GT, (M + GT - 1) / GT);
-      if (quads(d, fo, fo))
-        hipLaunchKernelGGL(k_layer_backward<true>, g, dim3(64 * kGemmWaves), 0, s, M, fi, fo, d, params[2 * i], z, dn);
-      else
-        hipLaunchKernelGGL(k_layer_backward<false>, g, dim3(64 * kGemmWaves), 0, s, M, fi, fo, d, params[2 * i], z, dn);
+      const bool vec = quads(d, fo, fo);
+      row_launches(M, [&](size_t m, int rows) {
+        const dim3 g((fi + GT - 1) / GT, (rows + GT - 1) / GT);
+        if (vec)
+          hipLaunchKernelGGL(k_layer_backward<true>, g, dim3(64 * kGemmWaves), 0, s, rows, fi, fo, d + m * fo,
+                             params[2 * i], z + m * fi, dn + m * fi);
+        else
+          hipLaunchKernelGGL(k_layer_backward<false>, g, dim3(64 * kGemmWaves), 0, s, rows, fi, fo, d + m * fo,
+                             params[2 * i], z + m * fi, dn + m * fi);
+      });
       d = dn;
     } else {
       hl[i] = X;

@@ -219,3 +219,56 @@ def test_answers_hold_no_pinned_memory(dev, requests):
         for a in answer:
             assert a.dtype == np.float64 and not torch.from_numpy(a).is_pinned()
             assert a.base is None or a.base.nbytes == a.nbytes
+
+
+ROWS_PER_LAUNCH = 65535 * 32       # row tiles of 32 on a grid axis of at most 65535 blocks
+
+
+@pytest.mark.parametrize("ta, tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_past_one_launch_of_rows(dev, ta, tb):
+    """Products of more rows than one launch takes, against float64: K = 4 products and
+    the sum of 4 partial tiles, (K + 5) 2^-24 of the sum of their magnitudes."""
+    from pyatmosphere_amd._lib import call, ptr
+    M, N, K = ROWS_PER_LAUNCH + 33, 3, 4
+    g = torch.Generator(device=dev).manual_seed(ta + 2 * tb)
+    A = torch.randn((K, M) if ta else (M, K), device=dev, generator=g)
+    B = torch.randn((N, K) if tb else (K, N), device=dev, generator=g)
+    C = torch.full((M, N), float("nan"), device=dev)
+    call("pa_mlp_gemm_f32", M, N, K, ptr(A), A.shape[1], ta, ptr(B), B.shape[1], tb, ptr(C), N, 1.0, 0.0,
+         torch.cuda.current_stream().cuda_stream)
+    a, b = (A.T if ta else A).double(), (B.T if tb else B).double()
+    want = sum(a[:, k:k + 1] * b[k] for k in range(K))
+    size = sum((a[:, k:k + 1] * b[k]).abs() for k in range(K))
+    assert ((C - want).abs() <= (K + 5) * 2.0 ** -24 * size).all()
+
+
+def test_training_past_one_launch_of_rows(dev):
+    """Loss and gradients of a minibatch of more rows than one launch takes, against
+    float64.  The rows of the last launch carry the log-variance's whole error.  A
+    wave adds up to M / 16 terms of a weight gradient one by one: M / 16 2^-24 of the
+    sum of their magnitudes, and 1e-5 for the terms."""
+    M, last = ROWS_PER_LAUNCH + 33, 33
+    net = PDTSurrogate(width=16, depth=2, seed=1, device=dev, wv=1.0, wc=0.0)
+    g = torch.Generator(device=dev).manual_seed(5)
+    x = torch.rand(M, 16, device=dev, generator=g) * 2 - 1
+    t = torch.zeros(M, NB, device=dev)
+    with torch.no_grad():
+        (W0, b0), (W1, b1) = [(W.double(), b.double()) for W, b in net.params]
+        z = x.double() @ W0.T + b0
+        h = torch.nn.functional.silu(z)
+        out = h @ W1.T + b1
+        tv = out[:, NB].float()
+        tv[-last:] += 1e6
+        loss, grads = net.loss_and_grads(x, t, tv)
+        e = out[:, NB] - tv.double()
+        want = (e ** 2).mean().item()
+        assert abs(loss.item() - want) <= 1e-4 * want
+        d1 = torch.cat([torch.softmax(out[:, :NB], 1), 2 * e[:, None]], 1) / M
+        del out
+        s = torch.sigmoid(z)
+        d0 = (d1 @ W1) * s * (1 + z * (1 - s))
+        size0 = (d1.abs() @ W1.abs()) * (s * (1 + z * (1 - s))).abs()     # what d0 is formed from
+        for (gW, gb), d, size, inp in ((grads[0], d0, size0, x.double()), (grads[1], d1, d1.abs(), h)):
+            bound = M / 16 * 2.0 ** -24 + 1e-5
+            assert ((gW - d.T @ inp).abs() <= bound * (size.T @ inp.abs())).all()
+            assert ((gb - d.sum(0)).abs() <= bound * size.sum(0)).all()
