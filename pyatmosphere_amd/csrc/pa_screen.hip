@@ -1555,10 +1555,13 @@ static void gemm_split_launch(int Kp, const void* opa, const void* opb, const do
 // graph (80 tiles) 134 against 140; 192 tiles 18.0 against 19.2 but, beside the field
 // passes, three 512^2 realizations (240 tiles) 169 against 166; 256 tiles (one
 // 2048^2) 26.7 against 22.5.  (With five or eight stages 128 x 128 is no faster;
-// with four or eight 64 x 64 is up to 1.4 us slower.)
+// with four or eight 64 x 64 is up to 1.4 us slower.)  At 64^2, where every tile is
+// 64 x 64, the line is the same number of points: 4096 screens of 64 points take
+// 33.3 us with the four stages of the larger tiles' kernel, 38.5 with six.
 static int gemm_tile_default(int n, int batch) {
-  if (n >= 512 && (long long)(n / 256) * (n / 256) * batch >= 512) return 1;
-  return (long long)(n / 128) * (n / 128) * batch <= 128 ? 3 : 2;
+  const long long points = (long long)n * n * batch;
+  if (n >= 512 && points >= 512ll * 256 * 256) return 1;
+  return points <= 128ll * 128 * 128 ? 3 : 2;
 }
 
 template <int N>
