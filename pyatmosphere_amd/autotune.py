@@ -4,11 +4,11 @@ The results of the kernels do not depend on their launch shapes, only their
 speed does, so the shapes are chosen by measurement on the device at hand:
 
 * per (grid n, spectral points P, batch B, GEMM mode): the screen GEMM's
-  block tile (256 x 256 with 8 waves, or 128 x 128 with 4 waves), the rows
-  per plane-wave-table block (4, 8, 16 or 32) and the columns per block of
-  the column FFT pass (pa_col_groups: the layout's default, half or twice
-  it), each kernel timed alone with HIP events on the same inputs
-  (`tune_screen`);
+  block tile (256 x 256 with 8 waves, 128 x 128 with 4 waves, or the library's
+  own choice, which takes smaller ones for small launches), the rows per
+  plane-wave-table block (4, 8, 16 or 32) and the columns per block of the
+  column FFT pass (pa_col_groups: the layout's default, half or twice it),
+  each kernel timed alone with HIP events on the same inputs (`tune_screen`);
 * per (n, P, screens, mode): the batch size and whether screen synthesis runs
   on a second stream, by timing whole graph-replayed batches (`tune_batch`).
 
@@ -27,7 +27,7 @@ from typing import Any, Callable, Dict, Iterable, Optional
 import numpy as np
 import torch
 
-GEMM_TILES = (1, 2)
+GEMM_TILES = (0, 1, 2)     # 0: the library's own choice
 TABLE_ROWS = (4, 8, 16, 32)
 _DEVICE_NAMES: Dict[int, str] = {}
 
@@ -159,7 +159,7 @@ def tune_screen(n: int, points: int, batch: int, mode: str, device: torch.device
     engine.prep_screen(ws, tables, 0, batch, None, st)
     rows_ms = {r: time_ms(lambda r=r: engine.plane_wave_tables(ws, tables, 0, batch, None, st, rows=r), reps)
                for r in TABLE_ROWS}
-    tiles = GEMM_TILES if n >= 512 else (2,)
+    tiles = GEMM_TILES if n >= 512 else (0, 2)
     tile_ms = {t: time_ms(lambda t=t: engine.screen_gemm(ws, 0, batch, None, st, ang=ws.ang, tile=t), reps)
                for t in tiles}
     ws.work[:batch].zero_()

@@ -84,3 +84,13 @@ def test_column_groups_give_the_same_field(dev, n):
         outs.append(out.cpu())
     for c, o in zip(groups[1:], outs[1:]):
         assert torch.equal(o, outs[0]), c
+
+
+@pytest.mark.parametrize("n", [256, 512])
+def test_the_library_choice_is_a_candidate(dev, cache, n):
+    """Tuning measures the library's own GEMM tile too, so what it stores is no slower
+    than not tuning."""
+    e = autotune.tune_screen(n, 64, 1, "f16x3", dev, reps=2)
+    assert set(e["gemm_ms"]) == ({"0", "1", "2"} if n >= 512 else {"0", "2"})
+    assert e["gemm_ms"][str(e["gemm_tile"])] <= e["gemm_ms"]["0"]
+    assert autotune.lookup(n, 64, 1, "f16x3", dev)["gemm_tile"] == e["gemm_tile"]
