@@ -14,7 +14,8 @@ speed does, so the shapes are chosen by measurement on the device at hand:
 
 Choices are kept in a JSON cache ($PA_TUNE_CACHE, else
 ~/.cache/pyatmosphere_amd/tune.json) keyed by the device's name and
-architecture, the library version and the problem shape.  Workspaces pick up
+architecture, the library version, the version of its launch shapes and the
+problem shape.  Workspaces pick up
 a cached screen shape when they are created; without an entry the library's
 own defaults apply (pa_screen_gemm / pa_screen_tables with shape 0).
 """
@@ -29,6 +30,9 @@ import torch
 
 GEMM_TILES = (0, 1, 2)     # 0: the library's own choice
 TABLE_ROWS = (4, 8, 16, 32)
+# the kernels' tiles and launch shapes that cached choices were measured on: raised
+# when these change
+SHAPES = 2
 _DEVICE_NAMES: Dict[int, str] = {}
 
 
@@ -70,7 +74,7 @@ def device_name(device: torch.device) -> str:
 
 def _prefix(device: torch.device) -> str:
     from . import _lib
-    return f"{device_name(device)}|lib{_lib.call('pa_version')}"
+    return f"{device_name(device)}|lib{_lib.call('pa_version')}|shapes{SHAPES}"
 
 
 def screen_key(n: int, points: int, batch: int, mode: str, device: torch.device) -> str:

@@ -45,3 +45,20 @@ def test_corrupt_cache_reads_as_empty(cache):
     assert autotune.lookup(512, 1024, 8, "f16x3", None) is None
     autotune._store(autotune.screen_key(512, 1024, 8, "f16x3", None), {"gemm_tile": 2, "table_rows": 8})
     assert autotune.lookup(512, 1024, 8, "f16x3", None)["table_rows"] == 8
+
+
+def test_choices_measured_on_other_launch_shapes_are_not_used(tmp_path, monkeypatch):
+    """A cache written before the kernels' tiles and launch shapes were what they are
+    has choices among others: its entries miss, and stay in the file."""
+    path = tmp_path / "tune.json"
+    monkeypatch.setenv("PA_TUNE_CACHE", str(path))
+    monkeypatch.setattr(autotune, "device_name", lambda device: "testdev")
+    old = {"testdev|lib1|screen|n1024|P1024|B32|f16x3": {"gemm_tile": 2, "table_rows": 8, "col_group": 8},
+           "testdev|lib1|batch|n1024|P1024|S5|f16x3": {"batch": 64, "overlap": False}}
+    path.write_text(json.dumps(old))
+    assert autotune.lookup(1024, 1024, 32, "f16x3", None) is None
+    assert autotune.lookup_batch(1024, 1024, 5, "f16x3", None) is None
+    new = {"gemm_tile": 0, "table_rows": 32, "col_group": 4}
+    autotune._store(autotune.screen_key(1024, 1024, 32, "f16x3", None), new)
+    assert autotune.lookup(1024, 1024, 32, "f16x3", None) == new
+    assert set(old) < set(json.loads(path.read_text()))
