@@ -358,8 +358,7 @@ int pa_mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, f
  * sizes[layers] - 1 <= 64 bins at the end): X[M][sizes[0]], params = (W0, b0,
  * W1, b1, ...) with W_i [sizes[i + 1]][sizes[i]], loss[M], mean (nullable) the
  * mean of loss, grads laid out as params (host arrays of device pointers).  The launches of a step in one call.
- * scratch: pa_mlp_loss_grads_scratch(layers, sizes, M) bytes, 16-byte aligned.
- * layers <= 256. */
+ * scratch: pa_mlp_loss_grads_scratch(layers, sizes, M) bytes, 16-byte aligned. */
 long long pa_mlp_loss_grads_scratch(int layers, const int* sizes, int M);
 int pa_mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
                       const float* target, const float* tvar, float wv, float wc, float* loss, float* mean,

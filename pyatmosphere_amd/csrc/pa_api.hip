@@ -411,7 +411,7 @@ int pa_mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, f
   return mlp_adam(n, w, g, m, v, lr, b1, b2, eps, t, STREAM(stream));
 }
 static bool mlp_sizes_ok(int layers, const int* sizes, int M) {
-  if (!sizes || layers < 1 || layers > kMlpMaxLayers || M < 1) return false;
+  if (!sizes || layers < 1 || M < 1) return false;
   for (int i = 0; i <= layers; ++i)
     if (sizes[i] < 1) return false;
   return sizes[layers] >= 2 && sizes[layers] <= 65;
@@ -448,7 +448,7 @@ int pa_mlp_layer_bf16(int M, int N, int K, const float* X, const void* W, const 
 }
 
 static bool mlp_layers_ok(int layers, const int* sizes) {
-  if (!sizes || layers < 1 || layers > kMlpMaxLayers) return false;
+  if (!sizes || layers < 1) return false;
   for (int i = 0; i <= layers; ++i)
     if (sizes[i] < 1) return false;
   return true;

@@ -11,7 +11,6 @@ constexpr int kMaxPupils = PA_MAX_PUPILS;     // pupils evaluated per channel in
 constexpr int kMaxSums = 6 + kMaxPupils;      // partial sums per tile
 constexpr int kChParams = 4;                  // per channel: delta, shift_x, shift_y, spare
 constexpr int kMoments = PA_NUM_MOMENTS;      // finalized values per element (see pa_hip.h)
-constexpr int kMlpMaxLayers = 256;            // layers of a network in one pa_mlp_loss_grads call
 constexpr int kMaxDevices = 64;               // devices whose static scratch address is kept
 
 // Pupil membership (pupils.py:8-10): (x - sx)^2 + (y + sy)^2 <= a^2 with

@@ -624,43 +624,40 @@ int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const fl
   }
   // z, d: the last layer's
   hipLaunchKernelGGL(k_head_loss, dim3(M), dim3(64), 0, s, M, NB, z, target, tvar, wv, wc, loss, d);
-  const float* dl[kMlpMaxLayers];
-  const float* hl[kMlpMaxLayers];
-  for (int i = layers - 1; i >= 0; --i) {
+  for (int i = layers - 1; i > 0; --i) {
     const int fi = sizes[i], fo = sizes[i + 1];
-    dl[i] = d;
-    if (i > 0) {
-      y -= padded((size_t)M * fi);
-      z -= padded((size_t)M * fi);
-      float* dn = d - padded((size_t)M * fi);
-      hl[i] = y;
-      const bool vec = quads(d, fo, fo);
-      row_launches(M, [&](size_t m, int rows) {
-        const dim3 g((fi + GT - 1) / GT, (rows + GT - 1) / GT);
-        if (vec)
-          hipLaunchKernelGGL(k_layer_backward<true>, g, dim3(64 * kGemmWaves), 0, s, rows, fi, fo, d + m * fo,
-                             params[2 * i], z + m * fi, dn + m * fi);
-        else
-          hipLaunchKernelGGL(k_layer_backward<false>, g, dim3(64 * kGemmWaves), 0, s, rows, fi, fo, d + m * fo,
-                             params[2 * i], z + m * fi, dn + m * fi);
-      });
-      d = dn;
-    } else {
-      hl[i] = X;
-    }
+    z -= padded((size_t)M * fi);
+    float* dn = d - padded((size_t)M * fi);
+    const bool vec = quads(d, fo, fo);
+    row_launches(M, [&](size_t m, int rows) {
+      const dim3 g((fi + GT - 1) / GT, (rows + GT - 1) / GT);
+      if (vec)
+        hipLaunchKernelGGL(k_layer_backward<true>, g, dim3(64 * kGemmWaves), 0, s, rows, fi, fo, d + m * fo,
+                           params[2 * i], z + m * fi, dn + m * fi);
+      else
+        hipLaunchKernelGGL(k_layer_backward<false>, g, dim3(64 * kGemmWaves), 0, s, rows, fi, fo, d + m * fo,
+                           params[2 * i], z + m * fi, dn + m * fi);
+    });
+    d = dn;
   }
+  // d: the first layer's; every layer's dZ and inputs follow one another
+  y = scratch + 2 * all;
+  h = X;
   for (int i0 = 0; i0 < layers; i0 += kGradLayers) {
     const int cnt = layers - i0 < kGradLayers ? layers - i0 : kGradLayers;
     GradLayers g = {};
     for (int j = 0; j < cnt; ++j) {
       const int fi = sizes[i0 + j], fo = sizes[i0 + j + 1];
-      g.d[j] = dl[i0 + j];
-      g.h[j] = hl[i0 + j];
+      g.d[j] = d;
+      g.h[j] = h;
       g.dw[j] = grads[2 * (i0 + j)];
       g.db[j] = grads[2 * (i0 + j) + 1];
       g.fo[j] = fo;
       g.fi[j] = fi;
       g.first[j + 1] = g.first[j] + ((fo + GT - 1) / GT) * ((fi + GT - 1) / GT);
+      d += padded((size_t)M * fo);
+      h = y;
+      y += padded((size_t)M * fo);
     }
     const bool last = i0 + cnt == layers;
     hipLaunchKernelGGL(k_weight_grads, dim3(g.first[cnt] + (last && mean ? 1 : 0)), dim3(64 * kGradWaves), 0, s, cnt, M,

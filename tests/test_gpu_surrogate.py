@@ -272,3 +272,59 @@ def test_training_past_one_launch_of_rows(dev):
             bound = M / 16 * 2.0 ** -24 + 1e-5
             assert ((gW - d.T @ inp).abs() <= bound * (size.T @ inp.abs())).all()
             assert ((gb - d.sum(0)).abs() <= bound * size.sum(0)).all()
+
+
+def _by_single_kernels(net, X, T, TV):
+    """Loss per row and gradients from the entry points of one operation each."""
+    from pyatmosphere_amd._lib import call, ptr
+    s = torch.cuda.current_stream().cuda_stream
+    M, hs, zs = X.shape[0], [X], []
+    new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=X.device)
+    for i, (W, b) in enumerate(net.params):
+        fo, fi = W.shape
+        Z, Y = new(M, fo), new(M, fo)
+        call("pa_mlp_gemm_f32", M, fo, fi, ptr(hs[-1]), fi, 0, ptr(W), fi, 1, ptr(Z), fo, 1.0, 0.0, s)
+        call("pa_mlp_bias_act", M, fo, ptr(Z), ptr(b), ptr(Y), int(i < len(net.params) - 1), s)
+        zs.append(Z)
+        hs.append(Y)
+    loss, d, grads = new(M), new(M, NB + 1), []
+    call("pa_mlp_head_loss", M, NB, ptr(hs[-1]), ptr(T), ptr(TV), net.wv, net.wc, ptr(loss), ptr(d), s)
+    for i in reversed(range(len(net.params))):
+        W, b = net.params[i]
+        fo, fi = W.shape
+        if i < len(net.params) - 1:
+            dz = new(M, fo)
+            call("pa_mlp_act_backward", M, fo, ptr(zs[i]), ptr(d), ptr(dz), s)
+            d = dz
+        gW, gb, dh = torch.empty_like(W), torch.empty_like(b), new(M, fi)
+        call("pa_mlp_gemm_f32", fo, fi, M, ptr(d), fo, 1, ptr(hs[i]), fi, 0, ptr(gW), fi, 1.0, 0.0, s)
+        call("pa_mlp_bias_grad", M, fo, ptr(d), ptr(gb), s)
+        call("pa_mlp_gemm_f32", M, fi, fo, ptr(d), fo, 0, ptr(W), fi, 0, ptr(dh), fi, 1.0, 0.0, s)
+        d, grads = dh, [(gW, gb)] + grads
+    return loss, grads
+
+
+@pytest.mark.parametrize("depth", [256, 257, 300])
+def test_networks_of_many_layers(dev, depth):
+    """Gradients, an update and predictions of networks of more layers than any group
+    of launches takes, against one launch per operation: the forward values have the
+    same bits, and the backward chain adds (16 + 5) 2^-24 of its terms per layer,
+    whose magnitudes add up to at most 16 times the result."""
+    rng = np.random.default_rng(depth)
+    net = PDTSurrogate(width=16, depth=depth, seed=4, device=dev, wv=0.5, wc=2.0)
+    net.params = [(W * 0.9, b + 0.2) for W, b in net.params]      # gradients shrink by 0.65 to 0.85 a layer
+    x, t, tv = _batch(rng, 19)
+    X, T, TV = net._pad(x), torch.from_numpy(t).to(dev), torch.from_numpy(tv).to(dev)
+    loss, grads = net.loss_and_grads(X, T, TV)
+    ref_loss, ref = _by_single_kernels(net, X, T, TV)
+    assert abs(loss.item() - ref_loss.double().mean().item()) <= 1e-5 * abs(loss.item())
+    bound = depth * 21 * 2.0 ** -24 * 16
+    for i, (got, want) in enumerate(zip(grads, ref)):
+        for a, b in zip(got, want):
+            # (float32 norms far below 1e-19 lose their squares)
+            a, b = a.double(), b.double()
+            assert (a - b).norm() <= bound * b.norm() + 1e-36, i
+    assert grads[100][0].double().norm() > 1e-32
+    net.adam_step(grads, 1e-3)
+    p, lv = net.predict(x)
+    assert p.shape == (19, NB) and np.isfinite(lv).all() and np.allclose(p.sum(axis=1), 1)

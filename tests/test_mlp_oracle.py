@@ -1,5 +1,6 @@
 """The float64 MLP oracle's gradients against central finite differences."""
 import numpy as np
+import pytest
 
 from oracle import mlp
 
@@ -84,3 +85,14 @@ def test_inputs_go_through_an_overridden_pad(monkeypatch):
     x = np.random.default_rng(1).uniform(-1, 1, (3, 5)).astype(np.float32)
     Scaled(width=32, depth=2, device=torch.device("cpu")).predict_raw(x)
     assert np.array_equal(seen[0][:, :5], 2 * x)
+
+
+@pytest.mark.parametrize("layers", [16, 17, 256, 257, 1000])
+def test_any_number_of_layers(layers):
+    """The scratch of a training step and the packed size (0: not for the fused network,
+    which takes 16 layers) of networks of any depth (host functions)."""
+    from pyatmosphere_amd._lib import call, int_array
+    sizes = int_array([16] * layers + [65])
+    rows = 5
+    assert call("pa_mlp_loss_grads_scratch", layers, sizes, rows) == 4 * (3 * 80 * (layers - 1) + 2 * 328)
+    assert (call("pa_mlp_pack_bytes", layers, sizes) > 0) == (layers <= 16)
