@@ -328,3 +328,67 @@ def test_networks_of_many_layers(dev, depth):
     net.adam_step(grads, 1e-3)
     p, lv = net.predict(x)
     assert p.shape == (19, NB) and np.isfinite(lv).all() and np.allclose(p.sum(axis=1), 1)
+
+
+@pytest.mark.parametrize("M, N", [(1, 1), (37, 65), (300, 17)])
+def test_single_operations_match_float64(dev, M, N):
+    """The entry points of one training operation each, against float64 (u = 2^-24):
+    SiLU to 16 u, its derivative to 32 u of |dY| s (1 + |z|), a column sum to M u of
+    its terms' magnitudes, the head to 256 u of those (64-term sums and exponentials),
+    Adam to its few roundings, of which 1 - b^t loses u / (1 - b^t)."""
+    from pyatmosphere_amd._lib import call, ptr
+    u, s = 2.0 ** -24, torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(M + N)
+    f32 = lambda *shape: (3 * rng.normal(size=shape)).astype(np.float32)
+    held = []          # a temporary's memory would go to the next one before the launch
+
+    def put(a):
+        held.append(torch.from_numpy(a.copy()).to(dev))
+        return held[-1]
+    get = lambda t: t.cpu().numpy().astype(np.float64)
+
+    z0, bias, dy = f32(M, N), f32(N), f32(M, N)
+    for act in (0, 1):
+        Z, Y = put(z0), torch.empty(M, N, device=dev)
+        call("pa_mlp_bias_act", M, N, ptr(Z), ptr(put(bias)), ptr(Y), act, s)
+        assert np.array_equal(Z.cpu().numpy(), z0 + bias)
+        z = get(Z)
+        want = omlp.silu(z) if act else z
+        assert (np.abs(get(Y) - want) <= 16 * u * np.abs(want) * act).all()
+    dz, db = torch.empty(M, N, device=dev), torch.empty(N, device=dev)
+    call("pa_mlp_act_backward", M, N, ptr(Z), ptr(put(dy)), ptr(dz), s)
+    assert (np.abs(get(dz) - dy * omlp.dsilu(z)) <= 32 * u * np.abs(dy) / (1 + np.exp(-z)) * (1 + np.abs(z))).all()
+    call("pa_mlp_bias_grad", M, N, ptr(put(dy)), ptr(db), s)
+    d64 = dy.astype(np.float64)
+    assert (np.abs(get(db) - d64.sum(axis=0)) <= M * u * np.abs(d64).sum(axis=0)).all()
+
+    nb = min(N, 64)
+    out, tv = f32(M, nb + 1), f32(M)
+    t = rng.random((M, nb)).astype(np.float32)
+    t /= t.sum(axis=1, keepdims=True)
+    loss, dout = torch.empty(M, device=dev), torch.empty(M, nb + 1, device=dev)
+    wv, wc = 0.5, 2.0
+    call("pa_mlp_head_loss", M, nb, ptr(put(out)), ptr(put(t)), ptr(put(tv)), wv, wc, ptr(loss), ptr(dout), s)
+    o, t64, lv = out[:, :nb].astype(np.float64), t.astype(np.float64), out[:, nb].astype(np.float64)
+    lse = np.log(np.exp(o).sum(axis=1, keepdims=True))
+    p = np.exp(o - lse)
+    P, T, e = np.cumsum(p, axis=1), np.cumsum(t64, axis=1), lv - tv
+    g, gmag = (2 * wc * np.cumsum(a[:, ::-1], axis=1)[:, ::-1] for a in (P - T, P + T))
+    want = -(t64 * (o - lse)).sum(axis=1) + wc * ((P - T) ** 2).sum(axis=1) + wv * e ** 2
+    size = (t64 * (np.abs(o) + np.abs(lse))).sum(axis=1) + wc * ((P + T) ** 2).sum(axis=1) + wv * (np.abs(lv) + np.abs(tv)) ** 2
+    assert (np.abs(get(loss) - want) <= 256 * u * size).all()
+    want = np.concatenate([p - t64 + p * (g - (p * g).sum(axis=1, keepdims=True)), 2 * wv * e[:, None]], axis=1) / M
+    size = np.concatenate([p + t64 + p * (gmag + (p * gmag).sum(axis=1, keepdims=True)),
+                           2 * wv * (np.abs(lv) + np.abs(tv))[:, None]], axis=1) / M
+    assert (np.abs(get(dout) - want) <= 256 * u * size).all()
+
+    w, gr, m, v = f32(M, N), f32(M, N), f32(M, N), f32(M, N) ** 2
+    lr, b1, b2, eps, step = (np.float32(a) for a in (1e-2, 0.9, 0.999, 1e-8, 3))
+    W, Mm, V = put(w), put(m), put(v)
+    call("pa_mlp_adam", M * N, ptr(W), ptr(put(gr)), ptr(Mm), ptr(V), lr, b1, b2, eps, 3, s)
+    w, gr, m, v, lr, b1, b2, eps = (np.float64(a) for a in (w, gr, m, v, lr, b1, b2, eps))
+    m1, v1, c1, c2 = b1 * m + (1 - b1) * gr, b2 * v + (1 - b2) * gr ** 2, 1 - b1 ** 3, 1 - b2 ** 3
+    msize, move = b1 * np.abs(m) + (1 - b1) * np.abs(gr), lr / c1 / (np.sqrt(v1 / c2) + eps)
+    assert (np.abs(get(Mm) - m1) <= 4 * u * msize).all() and (np.abs(get(V) - v1) <= 4 * u * v1).all()
+    bound = u * np.abs(w) + (16 + 2 / c1 + 2 / c2) * u * msize * move
+    assert (np.abs(get(W) - (w - move * m1)) <= bound).all()
