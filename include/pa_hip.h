@@ -363,7 +363,8 @@ long long pa_mlp_loss_grads_scratch(int layers, const int* sizes, int M);
 int pa_mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const float* const* params,
                       const float* target, const float* tvar, float wv, float wc, float* loss, float* mean,
                       float* const* grads, void* scratch, void* stream);
-/* pa_mlp_adam of `count` tensors (host arrays of sizes and device pointers). */
+/* pa_mlp_adam of `count` tensors (host arrays of sizes and device pointers); one
+ * that is there more than once is updated in turn. */
 int pa_mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
                       float* const* v, float lr, float b1, float b2, float eps, int t, void* stream);
 /* float32 -> bf16 (round to nearest even); y holds n uint16. */

@@ -669,19 +669,26 @@ int mlp_loss_grads(int layers, const int* sizes, int M, const float* X, const fl
 int mlp_adam_multi(int count, const int* n, float* const* w, const float* const* g, float* const* m,
                    float* const* v, float lr, float b1, float b2, float eps, int t, hipStream_t s) {
   const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
-  for (int i0 = 0; i0 < count; i0 += kAdamTensors) {
-    const int cnt = count - i0 < kAdamTensors ? count - i0 : kAdamTensors;
+  for (int i0 = 0; i0 < count;) {
     AdamTensors a = {};
-    int blocks = 0;
-    for (int j = 0; j < cnt; ++j) {
-      a.w[j] = w[i0 + j];
-      a.g[j] = g[i0 + j];
-      a.m[j] = m[i0 + j];
-      a.v[j] = v[i0 + j];
-      a.n[j] = n[i0 + j];
-      a.first[j] = blocks;
-      blocks += (n[i0 + j] + kAdamPer - 1) / kAdamPer;
+    int blocks = 0, cnt = 0;
+    // a tensor that is there already (weights that layers share) is updated again
+    // in the next launch, after the first update
+    auto there = [&](int i) {
+      for (int j = 0; j < cnt; ++j)
+        if (a.w[j] == w[i] || a.m[j] == m[i] || a.v[j] == v[i]) return true;
+      return false;
+    };
+    for (int i = i0; i < count && cnt < kAdamTensors && !there(i); ++i, ++cnt) {
+      a.w[cnt] = w[i];
+      a.g[cnt] = g[i];
+      a.m[cnt] = m[i];
+      a.v[cnt] = v[i];
+      a.n[cnt] = n[i];
+      a.first[cnt] = blocks;
+      blocks += (n[i] + kAdamPer - 1) / kAdamPer;
     }
+    i0 += cnt;
     hipLaunchKernelGGL(k_adam_multi, dim3(blocks), dim3(256), 0, s, cnt, a, lr, b1, b2, eps, c1, c2);
   }
   return check_launch("mlp_adam_multi");

@@ -392,3 +392,31 @@ def test_single_operations_match_float64(dev, M, N):
     assert (np.abs(get(Mm) - m1) <= 4 * u * msize).all() and (np.abs(get(V) - v1) <= 4 * u * v1).all()
     bound = u * np.abs(w) + (16 + 2 / c1 + 2 / c2) * u * msize * move
     assert (np.abs(get(W) - (w - move * m1)) <= bound).all()
+
+
+@pytest.mark.parametrize("depth, shared", [(4, {2: 1}), (12, {2: 1, 3: 1, 10: 4})])
+@pytest.mark.parametrize("moments", [False, True])
+def test_adam_updates_shared_weights_in_turn(dev, depth, shared, moments):
+    """Layers that share their weights (and moments): one update after the other, as
+    pa_mlp_adam tensor by tensor gives (32 roundings of a weight and its moves)."""
+    from pyatmosphere_amd._lib import call, ptr
+    net, lr = PDTSurrogate(width=40, depth=depth, seed=5, device=dev), 0.01
+    for i, j in shared.items():
+        net.params[i] = net.params[j]
+        if moments:
+            net.m[i], net.v[i] = net.m[j], net.v[j]
+    rng = np.random.default_rng(depth)
+    grads = [tuple(torch.from_numpy(rng.normal(size=t.shape).astype(np.float32)).to(dev) for t in p)
+             for p in net.params]
+    copies = {}
+    want = [[copies.setdefault(t.data_ptr(), t.clone()) for p in layer for t in p]
+            for layer in zip(net.params, net.m, net.v)]
+    for step in (1, 2):
+        for (w, b, mw, mb, vw, vb), (gw, gb) in zip(want, grads):
+            for p, g, m, v in ((w, gw, mw, vw), (b, gb, mb, vb)):
+                call("pa_mlp_adam", p.numel(), ptr(p), ptr(g), ptr(m), ptr(v), lr, 0.9, 0.999, 1e-8, step,
+                     torch.cuda.current_stream().cuda_stream)
+        net.adam_step(grads, lr)
+    for layer, ref in zip(zip(net.params, net.m, net.v), want):
+        for t, r in zip((t for p in layer for t in p), ref):
+            assert ((t - r).abs() <= 32 * 2.0 ** -24 * (r.abs() + 8 * lr)).all()
