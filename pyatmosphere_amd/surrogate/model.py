@@ -179,6 +179,7 @@ class PDTSurrogate:
         """Per layer (weights, bias, width, padded width, inputs) for the networks
         that the fused launch does not take."""
         if not isinstance(self._bf16, list):
+            s = _lib.stream_handle()
             layers = []
             for W, b in self.params:
                 fo, fi = W.shape
@@ -188,7 +189,7 @@ class PDTSurrogate:
                 bp = torch.zeros(fo_p, dtype=torch.float32, device=self.device)
                 bp[:fo] = b
                 Wb = torch.empty(fo_p, fi, dtype=torch.int16, device=self.device)
-                call("pa_mlp_to_bf16", Wp.numel(), ptr(Wp), ptr(Wb), _lib.stream_handle())
+                call("pa_mlp_to_bf16", Wp.numel(), ptr(Wp), ptr(Wb), s)
                 layers.append((Wb, bp, fo, fo_p, fi))
             self._bf16 = layers
         return self._bf16
@@ -196,11 +197,10 @@ class PDTSurrogate:
     def _layer_by_layer(self, x: np.ndarray) -> torch.Tensor:
         """(M, outputs) device outputs, one launch per layer."""
         h = self._pad(x)
-        M, layers = h.shape[0], self._bf16_layers()
+        M, layers, s = h.shape[0], self._bf16_layers(), _lib.stream_handle()
         for i, (Wb, bp, fo, fo_p, fi) in enumerate(layers):
             y = torch.empty(M, fo_p, dtype=torch.float32, device=self.device)
-            call("pa_mlp_layer_bf16", M, fo_p, fi, ptr(h), ptr(Wb), ptr(bp), ptr(y), int(i < len(layers) - 1),
-                 _lib.stream_handle())
+            call("pa_mlp_layer_bf16", M, fo_p, fi, ptr(h), ptr(Wb), ptr(bp), ptr(y), int(i < len(layers) - 1), s)
             h = y if fo_p == fo else y[:, :fo].contiguous()
         return h
 
@@ -227,9 +227,9 @@ def _outputs(members: Sequence[PDTSurrogate], x: np.ndarray) -> torch.Tensor:
     """(members, M, NB + 1) float32 device outputs; the members share a device.
     Networks of one shape run in one launch."""
     dev, M = members[0].device, x.shape[0]
-    shapes = {tuple(p.shape for p in _flat(m.params)) for m in members}
     packs = [m._packed() for m in members]
-    if len(shapes) > 1 or any(p is None for p in packs):
+    if any(p is None for p in packs) or \
+            len(members) > 1 and len({tuple(p.shape for p in _flat(m.params)) for m in members}) > 1:
         if len(members) > 1:
             return torch.cat([_outputs([m], x) for m in members])
         return members[0]._layer_by_layer(x)[None, :, :NB + 1].contiguous()

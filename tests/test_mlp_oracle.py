@@ -96,3 +96,21 @@ def test_any_number_of_layers(layers):
     rows = 5
     assert call("pa_mlp_loss_grads_scratch", layers, sizes, rows) == 4 * (3 * 80 * (layers - 1) + 2 * 328)
     assert (call("pa_mlp_pack_bytes", layers, sizes) > 0) == (layers <= 16)
+
+
+@pytest.mark.parametrize("layers", [2, 20])
+def test_layers_one_by_one_ask_for_the_stream_once(monkeypatch, layers):
+    """Networks that go layer by layer do not pay for the current stream at each layer."""
+    import torch
+    from pyatmosphere_amd.surrogate import PDTSurrogate
+    from pyatmosphere_amd.surrogate import model
+    asked = []
+    monkeypatch.setattr(model, "call", lambda name, *a: None)
+    monkeypatch.setattr(model._lib, "stream_handle", lambda: asked.append(1) or 0)
+    net = PDTSurrogate(width=32, depth=layers, device=torch.device("cpu"))
+    x = np.zeros((3, 5), np.float32)
+    net._layer_by_layer(x)          # lays the weights out too
+    assert len(asked) <= 2
+    asked.clear()
+    net._layer_by_layer(x)
+    assert len(asked) == 1
