@@ -226,13 +226,18 @@ def value_key(*values) -> tuple:
     """The values themselves, to compare with others by: numbers as they are, arrays
     (and whatever numpy takes as one) by their bytes, as they may change in place;
     the types too, which numpy's promotion depends on."""
-    out = []
-    for v in values:
-        if not isinstance(v, (int, float, np.number, type(None))):
-            a = np.asarray(v)
-            v = (type(v), a.dtype.str, a.shape, a.tobytes())
-        out.append((type(v), v))
-    return tuple(out)
+    types = tuple(map(type, values))
+    if not _NUMBERS.issuperset(types):
+        values = [v if isinstance(v, (int, float, np.number, type(None))) else _array_key(v) for v in values]
+    return types, tuple(values)
+
+
+_NUMBERS = {int, float, np.float64, np.float32, type(None)}
+
+
+def _array_key(v) -> tuple:
+    a = np.asarray(v)
+    return a.dtype.str, a.shape, a.tobytes()
 
 
 class KeptTables:
@@ -248,9 +253,9 @@ class KeptTables:
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the tables of a channel cannot be uploaded or shared under graph capture: "
                                "capture engine.run_batch on DeviceTables of its own")
-        key = value_key(spec.n, spec.delta, spec.wvl, spec.w0, spec.F0, spec.length, spec.positions, spec.points,
-                        *spec.shift, *(() if spec.gains is None else spec.gains), *spec.pupils), \
-            len(spec.pupils), device, _lib.stream_handle()
+        key = value_key(spec.n, spec.delta, spec.wvl, spec.w0, spec.F0, spec.length, spec.points,
+                        *spec.shift, *(() if spec.gains is None else spec.gains)), \
+            value_key(spec.positions, *spec.pupils), device, _lib.stream_handle()
         for k, base, psd, tables in self._kept:
             if k == key and np.array_equal(base, spec.base) and np.array_equal(psd, spec.psd):
                 return tables

@@ -114,7 +114,8 @@ class RandLogPolarGrid(Grid):
     def _plain_limits(self):
         """Whether the annuli can be kept by value: numbers, not arrays or
         tensors, which hash by identity (or not at all) and may change in place."""
-        return all(isinstance(v, (int, float, np.number)) for v in (self.points, self.f_min, self.f_max))
+        plain = (int, float, np.number)
+        return isinstance(self.points, plain) and isinstance(self.f_min, plain) and isinstance(self.f_max, plain)
 
     def _annuli(self):
         if type(self).base is not RandLogPolarGrid.base or not self._plain_limits():
