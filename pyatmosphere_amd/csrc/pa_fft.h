@@ -147,9 +147,10 @@ struct Plan;
 // E: points per thread; R0..R2: radices (0 = unused); T: rows per tile of the
 // field layout and per row-pass block; C: columns per column-pass block.  T
 // makes row-pass blocks of 128 (256^2) to 256 or 512 threads: the fewer waves
-// meet at a block's barriers the better its loads overlap its transforms, down
-// to the T C 8-byte runs of the column pass (128 bytes and more where T is not
-// 2).  Measured, T against twice that: k_row_mid 8.4 against 10.8 us (one
+// meet at a block's barriers the better its loads overlap its transforms, until
+// the column pass's runs (8 T bytes a column: with the columns it takes by default
+// 128 bytes and more up to 1024^2, 64 or 128 at 2048^2, 32 at 4096^2) become too
+// short.  Measured, T against twice that: k_row_mid 8.4 against 10.8 us (one
 // 1024^2 field), 100 against 108 (27), 5.0 against 6.5 (one 512^2), 230 against
 // 242 (256); k_row_last 242 against 276 (128 of 1024^2).  At 2048 half the T
 // slows the column pass (967 against 867 us, 64 fields), at 4096 twice the T

@@ -606,11 +606,11 @@ __device__ __forceinline__ uint32_t split_pack(double v0, double v1, uint32_t& l
 //
 // AXIS 0 and 1 fill one operand each; AXIS 2 fills both, axis blockIdx.z: the
 // polynomial part of A's blocks is a chain of latencies (sincos, barriers,
-// recurrences) and B's blocks are stores, so they overlap.  Measured with A's
-// columns on MFMA, all of pa_screen_tables with one launch against two: 16.3 against
-// 22.4 us of kernels for one 2048^2 screen, 50 against 62 us (ten of 2048^2), 57
-// against 67 (60 of 512^2), 260 against 280 (189 of 1024^2), 944 against 975 (320 of
-// 2048^2).
+// recurrences) and B's blocks are stores, so they overlap.  Measured, all of
+// pa_screen_tables at 1024 points with one launch against two: 29.5 against 35.0 us
+// for one 2048^2 screen, 54 against 67 (ten of 2048^2), 63 against 73 (60 of 512^2),
+// 317 against 333 (189 of 1024^2), the same for 320 of 2048^2 (1088), 1059 against
+// 1029 for 1280 of 512^2.
 template <int AXIS, int TC, int RG>
 struct TablesLds {
   static constexpr int RT = TC * RG;
@@ -1037,9 +1037,7 @@ __device__ __forceinline__ void gemm_epilogue(const f16v (&acc)[MI][NI], int m0,
 //   byte ((q N + row) 16 + k % 16) 2 of the plane, q = k / 16,
 // so one chunk of a block's rows is a contiguous run of HBM.
 // Geometry: BM x BN block tile, WGM x WGN waves, each wave owning a
-// (BM/WGM) x (BN/WGN) tile of 32x32 MFMA blocks.  Grids of 512 and up use
-// 256 x 256 block tiles (8 waves of 128 x 64); smaller grids 128 x 128 (or
-// N x N) with 4 waves.
+// (BM/WGM) x (BN/WGN) tile of 32x32 MFMA blocks.
 // CFG 1: 256 x 256 block tiles (8 waves of 128 x 64) for grids of 512 and up;
 // CFG 2: 128 x 128 (or N x N) tiles with 4 waves of 64 x 64, 4x the blocks;
 // CFG 3: 64 x 64 tiles with 4 waves of 32 x 32 and six stages, for launches whose
@@ -1516,8 +1514,10 @@ int screen_tables(int n, int P, double* fxy, double* sparam,
   const long long partial = (long long)lowrank_chunks(P) * kLRSums * (long long)sizeof(double);
   if (P >= 32 && partial > opbytes)
     return set_error(PA_ERR_SIZE, "screen_tables: B operand too small for the polynomial block's partial sums");
-  // column-smooth points per element: as many P_km rows as the B operand's
-  // room after the partial sums holds, at most kColLowMax
+  // column-smooth points per element: at most kColLowMax, and at most half of the
+  // P_km rows that the B operand's room after the partial sums holds (which binds at
+  // 64^2 with up to 96 points only; it decides which points the block takes, and so
+  // the roundings of such screens)
   const int nc_max = (int)std::max(0LL, std::min<long long>(kColLowMax, (opbytes - partial) / (kLR * 16)));
   switch (mode) {
     case PA_GEMM_F16X3:
@@ -1558,10 +1558,11 @@ static void gemm_split_launch(int Kp, const void* opa, const void* opb, const do
 // with four or eight 64 x 64 is up to 1.4 us slower.)  At 64^2, where every tile is
 // 64 x 64, the line is the same number of points: 4096 screens of 64 points take
 // 33.3 us with the four stages of the larger tiles' kernel, 38.5 with six.
+constexpr long long kSmallGemmPoints = 128ll * 128 * 128;
 static int gemm_tile_default(int n, int batch) {
   const long long points = (long long)n * n * batch;
   if (n >= 512 && points >= 512ll * 256 * 256) return 1;
-  return points <= 128ll * 128 * 128 ? 3 : 2;
+  return points <= kSmallGemmPoints ? 3 : 2;
 }
 
 template <int N>
@@ -1572,18 +1573,26 @@ static int gemm_n(int P, const void* opa, const void* opb, const double* sparam,
   if (tile != 0 && tile != 1 && tile != 2) return set_error(PA_ERR_ARG, "screen_gemm: tile must be 0, 1 or 2");
   if (N < 512 && tile == 1) tile = 2;   // no 256 x 256 tiles below 512
   if (tile == 0) tile = gemm_tile_default(N, batch);
+  // (the tiles that no launch of this size takes are not compiled)
+  constexpr bool BIG = N >= 512, SMALL = (long long)N * N <= kSmallGemmPoints;
 #define G_(MODE, CFG) \
   gemm_split_launch<N, MODE, CFG>(Kp, opa, opb, sparam, esc, phi2, ang, fac, hg, phi, nsteps, step, batch, s)
+#define S_(MODE)                      \
+  do {                                \
+    if constexpr (BIG) {              \
+      if (tile == 1) G_(MODE, 1);     \
+    }                                 \
+    if constexpr (SMALL) {            \
+      if (tile == 3) G_(MODE, 3);     \
+    }                                 \
+    if (tile == 2) G_(MODE, 2);       \
+  } while (0)
   switch (mode) {
     case PA_GEMM_F16X3:
-      if (tile == 1) G_(PA_GEMM_F16X3, 1);
-      else if (tile == 2) G_(PA_GEMM_F16X3, 2);
-      else G_(PA_GEMM_F16X3, 3);
+      S_(PA_GEMM_F16X3);
       break;
     case PA_GEMM_BF16X3:
-      if (tile == 1) G_(PA_GEMM_BF16X3, 1);
-      else if (tile == 2) G_(PA_GEMM_BF16X3, 2);
-      else G_(PA_GEMM_BF16X3, 3);
+      S_(PA_GEMM_BF16X3);
       break;
     case PA_GEMM_F32: {
 #define F_(BT)                                                                                                        \
@@ -1596,19 +1605,20 @@ static int gemm_n(int P, const void* opa, const void* opb, const double* sparam,
       hipLaunchKernelGGL((k_screen_gemm_f32<N, BT, false>), gf, dim3(256), 0, s, opa, opb, sparam, esc, phi2, ang,    \
                          fac, Kp, nsteps, step, batch, hg, phi);                                                      \
   } while (0)
+      const bool wide = (long long)N * N * batch >= 256ll * 128 * 128;
       if constexpr (N >= 128) {
-        if ((long long)(N / 128) * (N / 128) * batch >= 256) {
-          F_(128);
-          break;
-        }
+        if (wide) F_(128);
       }
-      F_(64);
+      if constexpr (N < 2048) {
+        if (N < 128 || !wide) F_(64);
+      }
       break;
 #undef F_
     }
     default:
       return set_error(PA_ERR_ARG, "unknown GEMM mode");
   }
+#undef S_
 #undef G_
   return check_launch("screen_gemm");
 }
