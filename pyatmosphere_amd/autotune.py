@@ -1,7 +1,8 @@
 """Launch-shape autotuner for the split-step path.
 
-The results of the kernels do not depend on their launch shapes, only their
-speed does, so the shapes are chosen by measurement on the device at hand:
+The results of the kernels do not depend on their launch shapes (but for the
+last bit of the tables' float64 recurrences), only their speed does, so the
+shapes are chosen by measurement on the device at hand:
 
 * per (grid n, spectral points P, batch B, GEMM mode): the screen GEMM's
   block tile (256 x 256 with 8 waves, 128 x 128 with 4 waves, or the library's
